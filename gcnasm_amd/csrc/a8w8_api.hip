@@ -66,6 +66,13 @@ bool raise_lds_limits_of_mode()
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, narrow_stages(MODE), 64>, small_lds_bytes(MODE, narrow_stages(MODE), 64)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, narrow_stages(MODE), 64>, small_lds_bytes(MODE, narrow_stages(MODE), 64));
     }
+    if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BF16)
+        ok = ok && raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, 2, SM_BN, true>, small_lds_bytes(MODE, 2)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 2, SM_BN, true>, small_lds_bytes(MODE, 2)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, 4, SM_BN, true>, small_lds_bytes(MODE, 4)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 4, SM_BN, true>, small_lds_bytes(MODE, 4)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, narrow_stages(MODE), 64, true>, small_lds_bytes(MODE, narrow_stages(MODE), 64)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, narrow_stages(MODE), 64, true>, small_lds_bytes(MODE, narrow_stages(MODE), 64));
     return ok;
 }
 
@@ -181,6 +188,13 @@ GemmParams make_params(const a8w8_gemm_args* g)
     return p;
 }
 
+// 16-byte aligned rows in A and B.
+bool rows_aligned(const a8w8_gemm_args* g)
+{
+    return g->stride_a % 16 == 0 && g->stride_b % 16 == 0 && aligned16(g->a) && aligned16(g->b) &&
+           (g->batch == 1 || (g->stride_a_batch % 16 == 0 && g->stride_b_batch % 16 == 0));
+}
+
 // The tiled kernels need whole 128-wide K steps and 16-byte aligned rows in A and B; the MX
 // variant also stages its scale bytes with dword-granular loads.
 bool tiled_ok(const a8w8_gemm_args* g)
@@ -193,9 +207,21 @@ bool tiled_ok(const a8w8_gemm_args* g)
         (!aligned16(g->sfa) || !aligned16(g->sfb) ||
          (g->batch > 1 && (g->stride_sfa_batch % 16 != 0 || g->stride_sfb_batch % 16 != 0))))
         return false;
-    return g->k % BK == 0 && g->stride_a % 16 == 0 && g->stride_b % 16 == 0 && aligned16(g->a) && aligned16(g->b) &&
-           (g->batch == 1 || (g->stride_a_batch % 16 == 0 && g->stride_b_batch % 16 == 0)) &&
-           (long long)((g->m + BM - 1) / BM) * ((g->n + BN - 1) / BN) < (1ll << 31);
+    return g->k % BK == 0 && rows_aligned(g) && (long long)((g->m + BM - 1) / BM) * ((g->n + BN - 1) / BN) < (1ll << 31);
+}
+
+// Rows of whole 16-byte pieces whose length is no multiple of the 128-byte K step: the 128-tile kernel with a partial last
+// step (scales that do not change with K; k in bytes here).  It is the faster one at any size, since the one-thread-per-element
+// kernel takes 86 ns per K element however small the problem (128 x 256 x 240: 20.9 us against 5.4, 1000 x 3000 x 2000: 7545
+// against 21, 4096 x 4096 x 4080: 84 ms against 0.116); problems of a few rows, columns and K elements, where that is no more
+// than a launch or two, stay there, in the order of operations of the CPU reference.
+constexpr int RAGGED_MIN_K_BYTES = 256;
+constexpr long long RAGGED_MIN_MACS = 1ll << 19;
+bool ragged_ok(const a8w8_gemm_args* g)
+{
+    return (g->scale_mode == A8W8_SCALE_TENSOR || g->scale_mode == A8W8_SCALE_ROWCOL) && !g->b_preshuffled && g->k % BK != 0 &&
+           g->k % 16 == 0 && rows_aligned(g) && (long long)((g->m + SM_BM - 1) / SM_BM) * ((g->n + 63) / 64) < (1ll << 31) &&
+           (g->k >= RAGGED_MIN_K_BYTES || (double)g->batch * g->m * g->n * g->k >= (double)RAGGED_MIN_MACS);
 }
 
 // B in the a8w8_preshuffle_b layout is read by the MFMA kernels only (the one-thread-per-element kernel reads
@@ -269,16 +295,16 @@ bool narrow_tiles_pay(long long items128, int n, int k)
     return 2 * items128 <= num_cus() && n > 64 && k / BK >= A8W8_NARROW_MIN_KSTEPS;
 }
 
-template <int MODE, int CDT, int STAGES>
+template <int MODE, int CDT, int STAGES, bool RAGGED>
 int launch_small_stages(const GemmParams& q, int batch, hipStream_t stream)
 {
     dim3 grid((unsigned)(q.tiles_m * q.tiles_n), 1, (unsigned)batch);
-    return launch(gemm_a8w8_tile128<MODE, CDT, STAGES>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, STAGES), stream, q);
+    return launch(gemm_a8w8_tile128<MODE, CDT, STAGES, SM_BN, RAGGED>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, STAGES), stream, q);
 }
 
 // Up to one workgroup per compute unit: four LDS stages (deep prefetch, one workgroup per compute unit).  More: two
 // stages, so that two workgroups share a compute unit and hide each other's waits.
-template <int MODE, int CDT>
+template <int MODE, int CDT, bool RAGGED = false>
 int launch_small(const GemmParams& p, int batch, hipStream_t stream)
 {
     if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BLOCK || MODE == MODE_MX || MODE == MODE_MXT ||
@@ -293,11 +319,11 @@ int launch_small(const GemmParams& p, int batch, hipStream_t stream)
             q.tiles_n = (p.n + 63) / 64;
             dim3 grid((unsigned)(q.tiles_m * q.tiles_n), 1, (unsigned)batch);
             constexpr int ST = narrow_stages(MODE);
-            return launch(gemm_a8w8_tile128<MODE, CDT, ST, 64>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, ST, 64), stream, q);
+            return launch(gemm_a8w8_tile128<MODE, CDT, ST, 64, RAGGED>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, ST, 64), stream, q);
         }
         if (items <= (long long)A8W8_SMALL_DEEP_UP_TO * num_cus())
-            return launch_small_stages<MODE, CDT, 4>(q, batch, stream);
-        return launch_small_stages<MODE, CDT, 2>(q, batch, stream);
+            return launch_small_stages<MODE, CDT, 4, RAGGED>(q, batch, stream);
+        return launch_small_stages<MODE, CDT, 2, RAGGED>(q, batch, stream);
     } else {
         return A8W8_ERR_BAD_MODE;
     }
@@ -378,6 +404,12 @@ int dispatch_wide(const a8w8_gemm_args* g, const GemmParams& p, hipStream_t s)
 int dispatch_small(const a8w8_gemm_args* g, const GemmParams& p, hipStream_t s)
 {
     A8W8_DISPATCH(launch_small, g->scale_mode, g->c_dtype, p, g->batch, s)
+}
+int dispatch_ragged(const a8w8_gemm_args* g, const GemmParams& p, hipStream_t s)
+{
+    if (g->scale_mode == A8W8_SCALE_TENSOR)
+        return g->c_dtype == A8W8_C_BF16 ? launch_small<MODE_TENSOR, C_BF16, true>(p, g->batch, s) : launch_small<MODE_TENSOR, C_FP32, true>(p, g->batch, s);
+    return g->c_dtype == A8W8_C_BF16 ? launch_small<MODE_ROWCOL, C_BF16, true>(p, g->batch, s) : launch_small<MODE_ROWCOL, C_FP32, true>(p, g->batch, s);
 }
 int dispatch_general(const a8w8_gemm_args* g, const GemmParams& p, hipStream_t s)
 {
@@ -564,6 +596,7 @@ bool c_stride_too_large(const a8w8_gemm_args* g, const a8w8_gemm_args* byte_view
 int launch_dense_fp8(const a8w8_gemm_args* g, hipStream_t s)
 {
     const GemmParams p = make_params(g);
+    if (ragged_ok(g)) return dispatch_ragged(g, p, s);
     if (!tiled_ok(g)) return dispatch_general(g, p, s);
     if (small_ok(g)) return dispatch_small(g, p, s);
     if (wide_ok(g)) return dispatch_wide(g, p, s);
@@ -642,6 +675,12 @@ static int a16w16_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allo
                                              : launch_wide<MODE_BF16, C_FP32>(p, g->batch, s);
         return g->c_dtype == A8W8_C_BF16 ? launch_persist<MODE_BF16, C_BF16>(p, g->batch, s)
                                          : launch_persist<MODE_BF16, C_FP32>(p, g->batch, s);
+    }
+    if (fits && ragged_ok(&bytes)) {     // a partial last K step
+        GemmParams p = make_params(&bytes);
+        p.sfa = p.sfb = nullptr;
+        return g->c_dtype == A8W8_C_BF16 ? launch_small<MODE_BF16, C_BF16, true>(p, g->batch, s)
+                                         : launch_small<MODE_BF16, C_FP32, true>(p, g->batch, s);
     }
     dim3 grid((unsigned)((g->n + 15) / 16), (unsigned)((g->m + 15) / 16), (unsigned)g->batch);
     if (g->c_dtype == A8W8_C_BF16)
@@ -1175,6 +1214,7 @@ const char* a8w8_kernel_name(const a8w8_gemm_args* g)
     if (g->b_preshuffled && validate_flat(g) == A8W8_OK && (prefer_flat_fp8(g) || !dense_ok)) return "flatmm_a8w8";
     if (dense_ok && flat_rowmajor_ok(g) && prefer_flat_fp8(g)) return "flatmm_a8w8";
     if (!dense_ok) return nullptr;
+    if (ragged_ok(g)) return "gemm_a8w8_tile128";
     if (!tiled_ok(g)) return "gemm_a8w8_general";
     if (small_ok(g)) return "gemm_a8w8_tile128";
     if (wide_ok(g)) return "gemm_a8w8_wide";

@@ -2,7 +2,8 @@
 // One thread per element of C, sequential K, one product-times-scale per MAC without fused
 // multiply-add, i.e. the arithmetic order of the reference CPU GEMM
 // (opus_gemm/block_scale_gemm/gemm_a8w8_blockscale_host.cc:66-90).  It is the path for
-// shapes the tiled kernels do not take (k % 128 != 0, unaligned rows); it is not fast.
+// shapes the tiled kernels do not take (unaligned rows, k no multiple of 128 with scales that change along K, k no multiple
+// of 16 at all, a few thousand outputs over a short K); it is not fast.
 #pragma once
 #include "a8w8_device.hpp"
 

@@ -55,9 +55,19 @@ constexpr int small_lds_bytes(int mode, int stages, int bn = SM_BN)
 // alone on its compute unit streams its share of the weights through a long K loop: SM_STAGES = 6 there (five K
 // steps of loads ahead, 144-154 KiB of LDS; 5 with tiled MX scales, whose 4 KiB per stage would not fit six; measured,
 // five and six stages run alike, and so does a separate ring of ten stages for the weights).
-template <int MODE, int CDT, int SM_STAGES, int BN_ = SM_BN>
+// RAGGED: k is no multiple of 128 (bytes).  The last K step is a partial one: the 16-byte pieces past k are fetched with a
+// lane offset beyond the buffer descriptor and read as zero on both sides (k % 16 == 0, so a piece is never split).  FP8
+// operands then run on the bf16 MFMA: the one-thread-per-element kernel that took these shapes before adds products in
+// fp32 one after the other, and the FP8 MFMA, which aligns its products to the largest one, is about 40 times less
+// precise than that (1.4e-5 against 8e-8 of the result in norm over K = 4096 normal data), while E4M3 -> bf16 is exact
+// and the bf16 MFMA keeps fp32 sums (8e-8).  A K step is four quarters of 32 elements; the fragments of the next quarter
+// are converted between the MFMAs of this one.  Half the MFMA rate, and still bound by it.
+// 1000 x 3000 x 2000 row/col: 7545 us on the one-thread-per-element kernel, 21 us here; 4096 x 4096 x 4080: 1.2 PFLOP/s.
+template <int MODE, int CDT, int SM_STAGES, int BN_ = SM_BN, bool RAGGED = false>
 __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
 {
+    static_assert(!RAGGED || MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BF16, "partial K steps: no scales that change with K");
+    constexpr bool BY_BF16 = RAGGED && MODE != MODE_BF16;      // FP8 operands converted to bf16
     static_assert(SM_STAGES == 2 || SM_STAGES == 4 || SM_STAGES == 5 || SM_STAGES == 6, "two, four, five or six LDS stages");
     static_assert(BN_ == 128 || BN_ == 64, "tile width");
     constexpr int SM_BN = BN_;
@@ -84,7 +94,7 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
     int tile_m, tile_n;
     tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
     const int m0 = tile_m * SM_BM, n0 = tile_n * SM_BN;
-    const int nk = p.k / BK;
+    const int nk = RAGGED ? (p.k + BK - 1) / BK : p.k / BK;
 
     const uint8_t* a_base = p.a + (long long)batch * p.a_batch;
     const uint8_t* b_base = p.b + (long long)batch * p.b_batch;
@@ -103,6 +113,9 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
     for (int j = 0; j < 4; ++j) voff_a[j] = min(m0 + ld_row + 32 * j, p.m - 1) * p.lda + ld_piece16;
 #pragma unroll
     for (int j = 0; j < B_LOADS; ++j) voff_b[j] = b_lane_offset(p, min(n0 + ld_row + 32 * j, p.n - 1), ld_piece16);
+    // the lane's piece of the last, partial K step lies past k: out of every descriptor's range (an extent is below 2^31)
+    const int past_k = RAGGED && (nk - 1) * BK + ld_piece16 >= p.k ? (int)0x80000000u : 0;
+    auto lane_offset = [&](int voff, int kstep) __attribute__((always_inline)) { return RAGGED ? voff | (kstep == nk - 1 ? past_k : 0) : voff; };
     // block mode: waves 0 and 1 fetch the step's 128 A-row scales (64 each), waves 2 and 3 the B scale
     // of the tile's 128 x 128 block (every lane the same dword: the stage's copy at +512 is the one read)
     constexpr int LOADS_PER_STAGE = 4 + B_LOADS + (MODE == MODE_F4 ? 2 : STEP_SCALES ? 1 : 0);
@@ -151,9 +164,9 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
         A8W8_LDS char* s = (A8W8_LDS char*)smem + stage * SM_STAGE_BYTES + wave * 1024;
         const int koff = kstep * BK;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) load_to_lds_16(rsrc_a, s + j * 4096, voff_a[j], koff);
+        for (int j = 0; j < 4; ++j) load_to_lds_16(rsrc_a, s + j * 4096, lane_offset(voff_a[j], kstep), koff);
 #pragma unroll
-        for (int j = 0; j < B_LOADS; ++j) load_to_lds_16(rsrc_b, s + SM_BM * BK + j * 4096, voff_b[j], kstep << p.b_kshift);
+        for (int j = 0; j < B_LOADS; ++j) load_to_lds_16(rsrc_b, s + SM_BM * BK + j * 4096, lane_offset(voff_b[j], kstep), kstep << p.b_kshift);
         if constexpr (TILED_SCALES) {
             A8W8_LDS char* sc = (A8W8_LDS char*)smem + SM_STAGES * SM_STAGE_BYTES + stage * SM_SCALE_BYTES + wave * 1024;
             // the pair of 128-element K steps this step belongs to (FP8: two byte steps) or is (FP4: 256 elements)
@@ -218,8 +231,9 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
     // ks + 2) between them; the other workgroup's MFMAs run beside this one's LDS reads.
     constexpr bool TWO = SM_STAGES == 2;
     constexpr bool PIPELINED = TWO ? A8W8_SMALL_PIPELINED_TWO != 0 : A8W8_SMALL_PIPELINED != 0;
+    static_assert(PIPELINED || !RAGGED, "partial K steps exist in the overlapped loop only");
     if constexpr (PIPELINED) {
-        constexpr int HALVES = (IS_F4 || MODE == MODE_BF16) ? 2 : 1;      // MFMAs per pair of fragments
+        constexpr int HALVES = BY_BF16 ? 4 : (IS_F4 || MODE == MODE_BF16) ? 2 : 1;      // MFMAs per pair of fragments
         constexpr int NFRAG = SM_TM + SM_TN, NSLOT = SM_TM * SM_TN * HALVES, NLOAD = LOADS_PER_STAGE;
         constexpr int LOAD_EVERY = NSLOT / NLOAD, READ_EVERY = NSLOT / NFRAG;
         constexpr int BLK_LAG = MODE == MODE_BLOCK ? 4 : 0;
@@ -272,11 +286,19 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
                 for (int t = 0; t < SM_TN; ++t) sb[t] = u[mxt_unit_b + mxt_off_b[t]];
             }
         };
+        // eight E4M3 codes (two dwords: quarter `h` of a fragment) as bf16
+        auto quarter_to_bf16 = [&](const v8i& f, int h) __attribute__((always_inline)) -> v8bf {
+            const v2bf x0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)f[2 * h], 1.0f, false);
+            const v2bf x1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)f[2 * h], 1.0f, true);
+            const v2bf x2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)f[2 * h + 1], 1.0f, false);
+            const v2bf x3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)f[2 * h + 1], 1.0f, true);
+            return v8bf{x0[0], x0[1], x1[0], x1[1], x2[0], x2[1], x3[0], x3[1]};
+        };
         // load n of a stage: four chunks of A, the chunks of B, then the step's scales
         auto load_one = [&](int stage, int kstep, int n) __attribute__((always_inline)) {
             A8W8_LDS char* s = (A8W8_LDS char*)smem + stage * SM_STAGE_BYTES + wave * 1024;
-            if (n < 4) load_to_lds_16(rsrc_a, s + n * 4096, voff_a[n], kstep * BK);
-            else if (n < 4 + B_LOADS) load_to_lds_16(rsrc_b, s + SM_BM * BK + (n - 4) * 4096, voff_b[n - 4], kstep << p.b_kshift);
+            if (n < 4) load_to_lds_16(rsrc_a, s + n * 4096, lane_offset(voff_a[n], kstep), kstep * BK);
+            else if (n < 4 + B_LOADS) load_to_lds_16(rsrc_b, s + SM_BM * BK + (n - 4) * 4096, lane_offset(voff_b[n - 4], kstep), kstep << p.b_kshift);
             else if constexpr (TILED_SCALES) {
                 A8W8_LDS char* sc = (A8W8_LDS char*)smem + SM_STAGES * SM_STAGE_BYTES + stage * SM_SCALE_BYTES + wave * 1024;
                 const int pair = MODE == MODE_F4T ? kstep : kstep >> 1;
@@ -316,12 +338,20 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
             A8W8_RAW_BARRIER();
             const int kload = min(ks + SM_STAGES, nk - 1);      // past the end: the last step again, into a stage nobody reads
             v4f part[BLK_LAG + 1];
+            v8bf quarter[BY_BF16 ? 2 : 1][NFRAG];
+            if constexpr (BY_BF16) {
+#pragma unroll
+                for (int n = 0; n < NFRAG; ++n) quarter[0][n] = quarter_to_bf16(have[n], 0);
+            }
 #pragma unroll
             for (int t = 0; t < NSLOT + BLK_LAG; ++t) {
                 if (t < NSLOT) {
                     // fragments pairs column by column; two-MFMA pairs: first halves of the column's four tiles, then second
                     // halves (back-to-back MFMAs on one accumulator stall)
-                    const int i = t % SM_TM, h = (t / SM_TM) % HALVES, j = t / (SM_TM * HALVES);
+                    // (converted operands: quarter by quarter over all tiles)
+                    constexpr int TILES = SM_TM * SM_TN;
+                    const int i = t % SM_TM;
+                    const int h = BY_BF16 ? t / TILES : (t / SM_TM) % HALVES, j = BY_BF16 ? t % TILES / SM_TM : t / (SM_TM * HALVES);
                     const v8i& fb = have[SM_TM + j];
                     const v8i& fa = have[i];
                     if constexpr (MODE == MODE_BLOCK) {
@@ -339,6 +369,9 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
                                 sb[j], 1, sa[i]);
                     } else if constexpr (MODE == MODE_MX || MODE == MODE_MXT) {
                         acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb, fa, acc[i][j], 0, 0, 0, sb[j], 0, sa[i]);
+                    } else if constexpr (BY_BF16) {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(quarter[h & 1][SM_TM + j], quarter[h & 1][i], acc[i][j], 0, 0, 0);
+                        if (t % TILES < NFRAG && h + 1 < HALVES) quarter[(h + 1) & 1][t % TILES] = quarter_to_bf16(have[t % TILES], h + 1);
                     } else if constexpr (MODE == MODE_BF16) {
                         // a 128-byte row is 64 bf16: the fragment's two 16-byte halves feed one 16x16x32 MFMA each
                         const v4i bh = {fb[4 * h], fb[4 * h + 1], fb[4 * h + 2], fb[4 * h + 3]};

@@ -98,8 +98,8 @@ typedef struct {
 /* Dense GEMM, any scale mode.  Replaces the launch
  *   gemm_a8w8_blockscale_kernel<Traits><<<grid, 512>>>(kargs)   (host.cc:14-15, 249-257)
  * and the launches of the absent siblings gemm_a8w8_8wave (opus_gemm/rebuild.sh:3) for the
- * per-tensor and row/column modes.  Needs k % 128 == 0 and 16-byte aligned A/B rows for
- * the tiled kernels; other shapes run on a slower general kernel.  m, n edges are handled.
+ * per-tensor and row/column modes.  Needs 16-byte aligned A/B rows and k % 128 == 0 (per-tensor and row/column scales:
+ * k % 16 == 0) for the tiled kernels; other shapes run on a slower general kernel.  m, n edges are handled.
  * b_preshuffled != 0: B is in the a8w8_preshuffle_b layout (the weights a8w8_flatmm streams), so that one copy
  * of the weights serves prefill and decode; needs n % 16 == 0, k % 128 == 0 and 16-byte aligned pointers.
  * a16w16_gemm and a4w4_gemm accept it likewise for the weights their flat siblings stream (shuffled as bytes).
@@ -112,7 +112,8 @@ A8W8_API int a8w8_gemm(const a8w8_gemm_args* args, void* hip_stream);
  * absent from the reference): A [batch, m, k] and B [batch, n, k] hold bf16, C = A * B^T in bf16 or
  * fp32, fp32 accumulation, no scales (sfa, sfb, stride_sf*, scale_mode are ignored).  Runs on the
  * same pipelined kernel as a8w8_gemm with the 16x16x32 bf16 MFMA when k % 64 == 0, k >= 128 and rows
- * are 16-byte aligned; other shapes take a general kernel that follows the CPU order of operations. */
+ * are 16-byte aligned, on its 128-tile variant when k % 8 == 0; other shapes take a general kernel that follows the CPU
+ * order of operations. */
 A8W8_API int a16w16_gemm(const a8w8_gemm_args* args, void* hip_stream);
 
 /* The bf16 flat GEMM (flatmm_a16w16_gfx950, opus_fmm/README.md:10,51-57; source absent): A [batch, m, k]
