@@ -73,3 +73,25 @@ def test_device_preshuffle(orc):
     b = rng.integers(0, 256, (96, 320)).astype(np.uint8)
     got = g.preshuffle_b_device(dev(b)).cpu().numpy()
     assert (got == orc.preshuffle_b(b)).all()
+
+
+@pytest.mark.parametrize("dialect", [0, 1])
+@pytest.mark.parametrize("n", [4, 7, 2047, 2048, 2049, 2051, 4095, 6151])
+def test_vectorised_and_unaligned_conversions_agree(orc, dialect, n):
+    """Lengths around a workgroup's 2048 elements with every remainder of 4; arrays that start on and off the 16 (floats)
+    and 4 (codes) bytes the vectorised kernels need; nothing is written behind the end."""
+    x = np.random.default_rng(n).standard_normal(n).astype(np.float32) * 100
+    want = orc.encode(x, dialect, clamp240=True)
+    want_back = orc.decode(want, dialect)
+    for shift in (0, 1):
+        src = torch.zeros(n + 8, device="cuda")
+        src[shift: shift + n] = torch.from_numpy(x).cuda()
+        codes = torch.full((n + 8,), 0x55, dtype=torch.uint8, device="cuda")
+        back = torch.full((n + 8,), 7.0, device="cuda")
+        L, s = g.lib(), g.api._stream()
+        assert L.a8w8_cvt_f32_to_e4m3(src[shift:].data_ptr(), codes[shift:].data_ptr(), n, dialect, 1, s) == 0
+        assert L.a8w8_cvt_e4m3_to_f32(codes[shift:].data_ptr(), back[shift:].data_ptr(), n, dialect, s) == 0
+        torch.cuda.synchronize()
+        assert (codes[shift: shift + n].cpu().numpy() == want).all()
+        assert (back[shift: shift + n].cpu().numpy() == want_back).all()
+        assert (codes[shift + n:] == 0x55).all() and (back[shift + n:] == 7.0).all()
