@@ -1025,8 +1025,12 @@ int a8w8_quantize(const float* src, int rows, int k, int ld, uint8_t* q, void* s
             if (group_rows == 1) {
                 if (const int ds = device_status(); ds != A8W8_OK) return ds;
                 const long long waves = (long long)rows * (k / 128);
-                if (quant_vec_ok(src, rows, k, ld, q, 4))
-                    A8W8_LAUNCH_OR_RETURN(quant_1x128_vec_kernel, dim3((unsigned)((waves + 8 * QUANT_1X128_GROUPS - 1) / (8 * QUANT_1X128_GROUPS))), dim3(256), 0, s, src, rows, k, ld, q,
+                const unsigned groups = (unsigned)(k / 128);
+                if (quant_vec_ok(src, rows, k, ld, q, 4) && waves <= QUANT_1X128_FEW)
+                    A8W8_LAUNCH_OR_RETURN(quant_1x128_vec_kernel<8>, dim3(groups * ((rows + 7) / 8)), dim3(256), 0, s, src, rows, k, ld, q,
+                                       (float*)scale);
+                else if (quant_vec_ok(src, rows, k, ld, q, 4))
+                    A8W8_LAUNCH_OR_RETURN(quant_1x128_vec_kernel<32>, dim3(groups * ((rows + 31) / 32)), dim3(256), 0, s, src, rows, k, ld, q,
                                        (float*)scale);
                 else
                     A8W8_LAUNCH_OR_RETURN(quant_1x128_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, src, rows, k,
@@ -1036,8 +1040,12 @@ int a8w8_quantize(const float* src, int rows, int k, int ld, uint8_t* q, void* s
             if (group_rows == 128) {
                 if (rows % 128 != 0) return A8W8_ERR_BAD_GROUP;
                 if (const int ds = device_status(); ds != A8W8_OK) return ds;
-                A8W8_LAUNCH_OR_RETURN(quant_128x128_kernel, dim3((unsigned)(k / 128), (unsigned)(rows / 128)), dim3(256), 0,
-                                   s, src, k, ld, q, (float*)scale);
+                if (quant_vec_ok(src, rows, k, ld, q, 4))
+                    A8W8_LAUNCH_OR_RETURN(quant_128x128_vec_kernel, dim3((unsigned)(k / 128), (unsigned)(rows / 128)), dim3(256), 0,
+                                       s, src, k, ld, q, (float*)scale);
+                else
+                    A8W8_LAUNCH_OR_RETURN(quant_128x128_kernel, dim3((unsigned)(k / 128), (unsigned)(rows / 128)), dim3(256), 0,
+                                       s, src, k, ld, q, (float*)scale);
                 return A8W8_OK;
             }
             return A8W8_ERR_BAD_MODE;

@@ -136,3 +136,21 @@ def test_vector_and_scalar_kernels_agree_with_the_oracle_on_views(orc):
     q, s = _run(long_rows, g.ROWCOL)
     qr, sr = orc.quantize(long_rows, orc.ROWCOL)
     assert (q == qr).all() and (s.view(np.uint32) == sr.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 31, 33, 1025])
+@pytest.mark.parametrize("k", [128, 2176])
+def test_1x128_row_tiles(orc, rows, k):
+    """Tiles of 8 rows (few blocks) and of 32 (1025 x 2176: more than 2^14 blocks), whole and ragged; rows in a wider buffer."""
+    x = np.random.default_rng(rows + k).standard_normal((rows, k)).astype(np.float32)
+    x[0, :128] = 0
+    whole = torch.full((rows, k + 4), 1e30, device="cuda")
+    whole[:, :k] = dev(x)
+    q, s = g.quantize(whole[:, :k], g.BLOCK)
+    qr, sr = orc.quantize(x, orc.BLOCK, 1)
+    assert (q.cpu().numpy() == qr).all() and (s.cpu().numpy() == sr).all()
+    if rows >= 128:
+        x, whole = x[:1024], whole[:1024]
+        q, s = g.quantize(whole[:, :k], g.BLOCK, 128)
+        qr, sr = orc.quantize(x, orc.BLOCK, 128)
+        assert (q.cpu().numpy() == qr).all() and (s.cpu().numpy() == sr).all()
