@@ -605,6 +605,48 @@ int launch_dense_fp8(const a8w8_gemm_args* g, hipStream_t s)
     return persist_ok(g) ? dispatch_persist(g, p, s) : dispatch_small(g, p, s);
 }
 
+// the vectorised quantisers read 16 bytes per lane and write packed words
+bool quant_vec_ok(const float* src, int rows, int k, int ld, const uint8_t* q, int q_align)
+{
+    return aligned16(src) && ld % 4 == 0 && k % 4 == 0 && ((uintptr_t)q & (uintptr_t)(q_align - 1)) == 0 &&
+           (long long)rows * k < (1ll << 31);
+}
+
+// 127 at the positions of the tiled layout that no (row, block) owns, for quantisers that write the real ones only
+int fill_mx_tiled(int rows, int k, uint8_t* scale, hipStream_t s)
+{
+    if (rows % 64 == 0 && k % 512 == 0) return A8W8_OK;
+    const size_t dwords = mx_tiled_bytes(rows, k) / 4;
+    return launch(mx_tiled_fill_kernel, dim3((unsigned)((dwords + 255) / 256)), dim3(256), 0, s, (uint32_t*)scale, dwords);
+}
+
+// The vectorised MX quantisers: as many chunks per wave as the array fills the chip with (quant_mx_vec_kernel), over the padded
+// array where its elements can be counted with 31 bits.
+template <bool FP4, bool TILED>
+int launch_quant_mx(const float* src, int rows, int k, int ld, uint8_t* q, uint8_t* scale, hipStream_t s)
+{
+    int rows_p = rows, k_p = k;
+    if constexpr (TILED) {
+        const long long rp = (rows + 63ll) / 64 * 64, kp = (k + 511ll) / 512 * 512;
+        if (rp * kp < (1ll << 31)) {
+            rows_p = (int)rp;
+            k_p = (int)kp;
+        } else if (const int st = fill_mx_tiled(rows, k, scale, s); st != A8W8_OK) {
+            return st;
+        }
+    }
+    const long long total = (long long)rows_p * k_p;
+    const auto grid = [&](int per_thread) { return dim3((unsigned)((total / per_thread + 255) / 256)); };
+    if (total >= QUANT_MX_FULL) return launch(quant_mx_vec_kernel<FP4, TILED, 4>, grid(16), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
+    if constexpr (FP4) {
+        return launch(quant_mxfp4_few_kernel<TILED>, grid(8), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
+    } else {
+        if (total > QUANT_MX_FEW)
+            return launch(quant_mx_vec_kernel<false, TILED, 2>, grid(8), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
+        return launch(quant_mx_vec_kernel<false, TILED, 1>, grid(4), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -809,13 +851,6 @@ static int a4w4_flat_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
 
 int a4w4_flatmm(const a8w8_gemm_args* g, void* hip_stream) { return a4w4_flat_impl(g, hip_stream, true); }
 
-// the vectorised quantisers read 16 bytes per lane and write packed words
-static bool quant_vec_ok(const float* src, int rows, int k, int ld, const uint8_t* q, int q_align)
-{
-    return aligned16(src) && ld % 4 == 0 && k % 4 == 0 && ((uintptr_t)q & (uintptr_t)(q_align - 1)) == 0 &&
-           (long long)rows * k < (1ll << 31);
-}
-
 int a4w4_quantize_mx(const float* src, int rows, int k, int ld, uint8_t* q, uint8_t* scale, int tiled, void* hip_stream)
 {
     if (!src || !q || !scale) return A8W8_ERR_NULL_POINTER;
@@ -826,22 +861,12 @@ int a4w4_quantize_mx(const float* src, int rows, int k, int ld, uint8_t* q, uint
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     hipStream_t s = (hipStream_t)hip_stream;
     const long long threads = (long long)rows * k;
-    if (tiled) {
-        if (rows % 64 != 0 || k % 512 != 0) {
-            const size_t dwords = mx_tiled_bytes(rows, k) / 4;
-            A8W8_LAUNCH_OR_RETURN(mx_tiled_fill_kernel, dim3((unsigned)((dwords + 255) / 256)), dim3(256), 0, s, (uint32_t*)scale, dwords);
-        }
-        if (quant_vec_ok(src, rows, k, ld, q, 4))
-            A8W8_LAUNCH_OR_RETURN(quant_mxfp4_vec_kernel<true>, dim3((unsigned)((threads / 8 + 255) / 256)), dim3(256), 0, s, src, rows, k, ld, q, scale);
-        else
-            A8W8_LAUNCH_OR_RETURN(quant_mxfp4_kernel<true>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, src, rows, k, ld, q, scale);
-    } else {
-        if (quant_vec_ok(src, rows, k, ld, q, 4))
-            A8W8_LAUNCH_OR_RETURN(quant_mxfp4_vec_kernel<false>, dim3((unsigned)((threads / 8 + 255) / 256)), dim3(256), 0, s, src, rows, k, ld, q, scale);
-        else
-            A8W8_LAUNCH_OR_RETURN(quant_mxfp4_kernel<false>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, src, rows, k, ld, q, scale);
-    }
-    return A8W8_OK;
+    if (quant_vec_ok(src, rows, k, ld, q, 4))
+        return tiled ? launch_quant_mx<true, true>(src, rows, k, ld, q, scale, s) : launch_quant_mx<true, false>(src, rows, k, ld, q, scale, s);
+    const dim3 grid((unsigned)((threads + 255) / 256));
+    if (!tiled) return launch(quant_mxfp4_kernel<false>, grid, dim3(256), 0, s, src, rows, k, ld, q, scale);
+    if (const int st = fill_mx_tiled(rows, k, scale, s); st != A8W8_OK) return st;
+    return launch(quant_mxfp4_kernel<true>, grid, dim3(256), 0, s, src, rows, k, ld, q, scale);
 }
 
 static int a16w16_flat_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_dense)
@@ -1052,32 +1077,18 @@ int a8w8_quantize(const float* src, int rows, int k, int ld, uint8_t* q, void* s
         case A8W8_SCALE_MX_E8M0_1x32: {
             if (k % 32 != 0) return A8W8_ERR_BAD_GROUP;
             if (const int ds = device_status(); ds != A8W8_OK) return ds;
-            const long long threads = (long long)rows * k;
-            if (quant_vec_ok(src, rows, k, ld, q, 4))
-                A8W8_LAUNCH_OR_RETURN(quant_mx_vec_kernel<false>, dim3((unsigned)((threads / (4 * QUANT_MX_CHUNKS) + 255) / 256)), dim3(256), 0, s, src,
-                                   rows, k, ld, q, (uint8_t*)scale);
-            else
-                A8W8_LAUNCH_OR_RETURN(quant_mx_kernel<false>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, src, rows, k,
-                                   ld, q, (uint8_t*)scale);
-            return A8W8_OK;
+            if (quant_vec_ok(src, rows, k, ld, q, 4)) return launch_quant_mx<false, false>(src, rows, k, ld, q, (uint8_t*)scale, s);
+            return launch(quant_mx_kernel<false>, dim3((unsigned)(((long long)rows * k + 255) / 256)), dim3(256), 0, s, src, rows, k, ld, q,
+                          (uint8_t*)scale);
         }
         case A8W8_SCALE_MX_E8M0_TILED: {
             if (k % 32 != 0) return A8W8_ERR_BAD_GROUP;
             if (const int ds = device_status(); ds != A8W8_OK) return ds;
             if (((uintptr_t)scale & 3) != 0) return A8W8_ERR_MISALIGNED;
-            const long long threads = (long long)rows * k;
-            if (rows % 64 != 0 || k % 512 != 0) {   // positions no (row, block) owns: 127 first
-                const size_t dwords = mx_tiled_bytes(rows, k) / 4;
-                A8W8_LAUNCH_OR_RETURN(mx_tiled_fill_kernel, dim3((unsigned)((dwords + 255) / 256)), dim3(256), 0, s,
-                                   (uint32_t*)scale, dwords);
-            }
-            if (quant_vec_ok(src, rows, k, ld, q, 4))
-                A8W8_LAUNCH_OR_RETURN(quant_mx_vec_kernel<true>, dim3((unsigned)((threads / (4 * QUANT_MX_CHUNKS) + 255) / 256)), dim3(256), 0, s, src,
-                                   rows, k, ld, q, (uint8_t*)scale);
-            else
-                A8W8_LAUNCH_OR_RETURN(quant_mx_kernel<true>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, src, rows,
-                                   k, ld, q, (uint8_t*)scale);
-            return A8W8_OK;
+            if (quant_vec_ok(src, rows, k, ld, q, 4)) return launch_quant_mx<false, true>(src, rows, k, ld, q, (uint8_t*)scale, s);
+            if (const int st = fill_mx_tiled(rows, k, (uint8_t*)scale, s); st != A8W8_OK) return st;
+            return launch(quant_mx_kernel<true>, dim3((unsigned)(((long long)rows * k + 255) / 256)), dim3(256), 0, s, src, rows, k, ld, q,
+                          (uint8_t*)scale);
         }
         default:
             return A8W8_ERR_BAD_MODE;

@@ -275,8 +275,24 @@ __global__ void __launch_bounds__(256) quant_128x128_kernel(const float* src, in
         o[(long long)(i >> 7) * k + (i & 127)] = quant_one(x[(long long)(i >> 7) * ld + (i & 127)], s);
 }
 
-// MX: one E8M0 exponent per 32 K-elements, e = ceil(log2(amax/448)) clamped to [-127, 127]
-// computed exactly from the fp32 exponent/mantissa fields; 32 lanes per block.
+// clamp(ceil(log2(amax / top)), -127, 127) for top = (1 + TOP_MANT / 2^23) 2^TOP_EXP: the exponent difference, one more when
+// amax's mantissa is above top's.  It equals the exponent of the rounded fp32 quotient for every amax: the quotient of the first
+// mantissa above top's rounds up, except where it is subnormal, once (TOP_MANT + 1 at quotient exponent -127), where it rounds
+// back to the power of two; amax = Inf keeps the exponent 0 that frexp gave it, NaN counts as zero.  Five integer operations
+// where the divide and frexp took about twenty.
+template <int TOP_EXP, unsigned TOP_MANT>
+A8W8_DEV int mx_block_exponent(float amax)
+{
+    const unsigned u = __float_as_uint(amax);
+    const int field = (int)(u >> 23);
+    const unsigned above = (u & 0x7fffffu) > TOP_MANT + (field == TOP_EXP ? 1u : 0u) ? 1u : 0u;
+    const int e = max(-127, field - 127 - TOP_EXP + (int)above);
+    return u < 0x7f800000u ? e : u == 0x7f800000u ? 0 : -127;
+}
+A8W8_DEV int mx_exponent_e4m3(float amax) { return mx_block_exponent<8, 0x600000u>(amax); }      // 448 = 1.75 * 2^8
+A8W8_DEV int mx_exponent_e2m1(float amax) { return mx_block_exponent<2, 0x400000u>(amax); }      // 6 = 1.5 * 2^2
+
+// MX: one E8M0 exponent per 32 K-elements, e = ceil(log2(amax/448)) clamped to [-127, 127]; 32 lanes per block.
 template <bool TILED>
 __global__ void __launch_bounds__(256) quant_mx_kernel(const float* src, int rows, int k, int ld, uint8_t* q,
                                                        uint8_t* scale)
@@ -290,14 +306,7 @@ __global__ void __launch_bounds__(256) quant_mx_kernel(const float* src, int row
     float amax = fabsf(v);
 #pragma unroll
     for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-    const float t = __fdiv_rn(amax, 448.0f);
-    int e = -127;
-    if (t > 0.f) {
-        int ex;
-        const float f = frexpf(t, &ex);          // t = f * 2^ex, f in [0.5, 1)
-        e = (f == 0.5f) ? ex - 1 : ex;
-        e = max(-127, min(127, e));
-    }
+    const int e = mx_exponent_e4m3(amax);
     if (l == 0) scale[TILED ? mx_tiled_index(rows, row, g) : (size_t)row * blocks + g] = (uint8_t)(e + 127);
     const float qv = ldexpf(v, -e);
     const uint32_t w = __builtin_amdgcn_cvt_pk_fp8_f32(qv, qv, 0, false);
@@ -330,14 +339,7 @@ __global__ void __launch_bounds__(256) quant_mxfp4_kernel(const float* src, int 
     float amax = fabsf(v);
 #pragma unroll
     for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-    const float t = __fdiv_rn(amax, 6.0f);
-    int e = -127;
-    if (t > 0.f) {
-        int ex;
-        const float f = frexpf(t, &ex);          // t = f * 2^ex, f in [0.5, 1)
-        e = (f == 0.5f) ? ex - 1 : ex;
-        e = max(-127, min(127, e));
-    }
+    const int e = mx_exponent_e2m1(amax);
     if (l == 0) scale[TILED ? mx_tiled_index(rows, row, g) : (size_t)row * blocks + g] = (uint8_t)(e + 127);
     const unsigned code = e2m1_encode(ldexpf(v, -e));
     const unsigned hi = __shfl_down(code, 1, 64);
@@ -353,17 +355,12 @@ A8W8_DEV uint32_t pack4_e4m3(float a, float b, float c, float d)
     uint32_t w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
     return __builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);
 }
-A8W8_DEV int mx_block_exponent(float amax, float top)
+// two floats, divided by 2^e, as E2M1 codes in byte BYTE of `word`: the hardware convert, the same code as e2m1_encode(ldexpf(x, -e))
+// for all 2^32 inputs (NaN and Inf included) at every e tried, -127 and 127 among them
+template <int BYTE>
+A8W8_DEV unsigned e2m1_pair(unsigned word, float x, float y, float scale)
 {
-    const float t = __fdiv_rn(amax, top);
-    int e = -127;
-    if (t > 0.f) {
-        int ex;
-        const float f = frexpf(t, &ex);          // t = f * 2^ex, f in [0.5, 1)
-        e = (f == 0.5f) ? ex - 1 : ex;
-        e = max(-127, min(127, e));
-    }
-    return e;
+    return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(word, x, y, scale, BYTE);
 }
 
 // 16 bytes of an input that is read once: a non-temporal load (the line is not kept in L2 in place of something that
@@ -374,80 +371,95 @@ A8W8_DEV float4 load_once4(const float* p)
     return make_float4(t.x, t.y, t.z, t.w);
 }
 
-// MX E4M3 with one E8M0 exponent per 32 elements.  A wave takes 1024 consecutive elements of the
-// flattened [rows, k] array as four chunks of 256: lane l owns elements 4l..4l+3 of each chunk, eight
-// lanes share a block.  Every load and store instruction of a wave covers one contiguous run of memory;
-// all loads are issued before any chunk is processed.
-constexpr int QUANT_MX_CHUNKS = 4;
-template <bool TILED>
-__global__ void __launch_bounds__(256) quant_mx_vec_kernel(const float* __restrict__ src, int rows, int k, int ld,
+// MX formats with one E8M0 exponent per 32 elements (bound: HBM).  A wave takes 256 CHUNKS consecutive elements of the
+// flattened [rows, k] array: lane l owns elements 4l..4l+3 of each chunk of 256, eight lanes share a block.  Every load and
+// store instruction of a wave covers one contiguous run of memory; all loads are issued before any chunk is processed.
+// Four chunks are what large arrays want (8192 x 8192 E4M3, tiled scales: 56.3 us, two 58.3, one 64.9), fewer where there are
+// not enough of them to fill the chip and a wave's own latency is the time (2560 x 2560: 8.2 / 7.4 / 8.5; 64 x 7168: 3.8 / 2.7 /
+// 2.7; 16 x 7168: 3.7 / 2.6 / 2.3).
+// TILED: the grid covers the padded [rows_p, k_p] array of the tiled layout (rows_p % 64 == 0, k_p % 512 == 0), so that the
+// positions no (row, block) owns get their 127 here instead of from a launch of their own before this one (2.3 us).  Otherwise,
+// and where the caller filled the scales beforehand, rows_p = rows and k_p = k.
+// FP4: packed E2M1, two bytes per lane and chunk; the hardware convert instead of seven comparisons per element (8192 x 8192
+// 62.6 -> 50.3 us, 4096 x 4096 16.8 -> 13.6).
+template <bool FP4, bool TILED, int CHUNKS>
+__global__ void __launch_bounds__(256) quant_mx_vec_kernel(const float* __restrict__ src, int rows, int k, int rows_p, int k_p, int ld,
                                                            uint8_t* __restrict__ q, uint8_t* __restrict__ scale)
 {
-    const unsigned total = (unsigned)rows * (unsigned)k;            // < 2^31 (checked by the host)
+    const unsigned total = (unsigned)rows_p * (unsigned)k_p;        // < 2^31 (checked by the host)
     const unsigned wave = (blockIdx.x * 256u + threadIdx.x) >> 6;
     const unsigned lane = threadIdx.x & 63;
     const int blocks = k >> 5;
-    constexpr int CH = QUANT_MX_CHUNKS;
-    unsigned row[CH], col[CH];
-    bool live[CH];
-    float4 v[CH];
+    unsigned row[CHUNKS], col[CHUNKS];
+    bool live[CHUNKS], owned[CHUNKS];
+    float4 v[CHUNKS];
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const unsigned e0 = wave * (256u * CH) + c * 256u + lane * 4u;
+    for (int c = 0; c < CHUNKS; ++c) {
+        const unsigned e0 = wave * (256u * CHUNKS) + c * 256u + lane * 4u;
         live[c] = e0 < total;
-        row[c] = live[c] ? e0 / (unsigned)k : 0u;
-        col[c] = live[c] ? e0 % (unsigned)k : 0u;
+        row[c] = live[c] ? e0 / (unsigned)k_p : 0u;
+        col[c] = live[c] ? e0 % (unsigned)k_p : 0u;
+        owned[c] = live[c] && (!TILED || (row[c] < (unsigned)rows && col[c] < (unsigned)k));
         v[c] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (live[c]) v[c] = load_once4(src + (size_t)row[c] * ld + col[c]);
+        if (owned[c]) v[c] = load_once4(src + (size_t)row[c] * ld + col[c]);
     }
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
+    for (int c = 0; c < CHUNKS; ++c) {
         float amax = fmaxf(fmaxf(fabsf(v[c].x), fabsf(v[c].y)), fmaxf(fabsf(v[c].z), fabsf(v[c].w)));
 #pragma unroll
         for (int off = 4; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-        const int e = mx_block_exponent(amax, 448.0f);
+        const int e = FP4 ? mx_exponent_e2m1(amax) : mx_exponent_e4m3(amax);
         if (!live[c]) continue;
         if ((lane & 7) == 0) {
             const int g = (int)(col[c] >> 5);
-            scale[TILED ? mx_tiled_index(rows, (int)row[c], g) : (size_t)row[c] * blocks + g] = (uint8_t)(e + 127);
+            scale[TILED ? mx_tiled_index(rows, (int)row[c], g) : (size_t)row[c] * blocks + g] = (uint8_t)((owned[c] ? e : 0) + 127);
         }
-        *(uint32_t*)(q + (size_t)row[c] * k + col[c]) =
-            pack4_e4m3(ldexpf(v[c].x, -e), ldexpf(v[c].y, -e), ldexpf(v[c].z, -e), ldexpf(v[c].w, -e));
+        if (!owned[c]) continue;
+        if constexpr (FP4) {
+            const float s = __uint_as_float((unsigned)(e + 127) << 23);      // (2^-127: the convert takes the exponent field)
+            *(uint16_t*)(q + (((size_t)row[c] * k + col[c]) >> 1)) = (uint16_t)e2m1_pair<1>(e2m1_pair<0>(0u, v[c].x, v[c].y, s), v[c].z, v[c].w, s);
+        } else {
+            *(uint32_t*)(q + (size_t)row[c] * k + col[c]) =
+                pack4_e4m3(ldexpf(v[c].x, -e), ldexpf(v[c].y, -e), ldexpf(v[c].z, -e), ldexpf(v[c].w, -e));
+        }
     }
 }
 
-// MXFP4 (packed E2M1): lane l owns eight consecutive elements (two 16-byte loads, one 4-byte store),
-// four lanes share a block, a wave takes 512 consecutive elements.
+// MXFP4 below the size that fills the chip: lane l owns eight consecutive elements (two 16-byte loads, one 4-byte store), four
+// lanes share a block, a wave takes 512 consecutive elements (256 x 8192: 2.7 us against 3.2-3.8 with chunks, 64 x 7168: 2.3
+// against 2.6; 4096 x 2048: 7.8 against 7.5).
 template <bool TILED>
-__global__ void __launch_bounds__(256) quant_mxfp4_vec_kernel(const float* __restrict__ src, int rows, int k, int ld,
+__global__ void __launch_bounds__(256) quant_mxfp4_few_kernel(const float* __restrict__ src, int rows, int k, int rows_p, int k_p, int ld,
                                                               uint8_t* __restrict__ q, uint8_t* __restrict__ scale)
 {
-    const unsigned total = (unsigned)rows * (unsigned)k;            // < 2^31 (checked by the host)
+    const unsigned total = (unsigned)rows_p * (unsigned)k_p;        // < 2^31 (checked by the host)
     const unsigned e0 = (blockIdx.x * 256u + threadIdx.x) * 8u;
     const bool live = e0 < total;
-    const unsigned row = live ? e0 / (unsigned)k : 0u, col = live ? e0 % (unsigned)k : 0u;
+    const unsigned row = live ? e0 / (unsigned)k_p : 0u, col = live ? e0 % (unsigned)k_p : 0u;
+    const bool owned = live && (!TILED || (row < (unsigned)rows && col < (unsigned)k));
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-    if (live) {
-        const float4* p = (const float4*)(src + (size_t)row * ld + col);
-        a = p[0];
-        b = p[1];
+    if (owned) {
+        const float* p = src + (size_t)row * ld + col;
+        a = load_once4(p);
+        b = load_once4(p + 4);
     }
     float amax = fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))),
                        fmaxf(fmaxf(fabsf(b.x), fabsf(b.y)), fmaxf(fabsf(b.z), fabsf(b.w))));
 #pragma unroll
     for (int off = 2; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-    const int e = mx_block_exponent(amax, 6.0f);
+    const int e = mx_exponent_e2m1(amax);
     if (!live) return;
     if ((threadIdx.x & 3) == 0) {
         const int g = (int)(col >> 5);
-        scale[TILED ? mx_tiled_index(rows, (int)row, g) : (size_t)row * (k >> 5) + g] = (uint8_t)(e + 127);
+        scale[TILED ? mx_tiled_index(rows, (int)row, g) : (size_t)row * (k >> 5) + g] = (uint8_t)((owned ? e : 0) + 127);
     }
-    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    unsigned w = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) w |= e2m1_encode(ldexpf(x[i], -e)) << (4 * i);     // even K in the low nibble
-    *(uint32_t*)(q + (size_t)row * (k >> 1) + (col >> 1)) = w;
+    if (!owned) return;
+    const float s = __uint_as_float((unsigned)(e + 127) << 23);
+    *(uint32_t*)(q + (((size_t)row * k + col) >> 1)) =
+        e2m1_pair<3>(e2m1_pair<2>(e2m1_pair<1>(e2m1_pair<0>(0u, a.x, a.y, s), a.z, a.w, s), b.x, b.y, s), b.z, b.w, s);
 }
+// elements from which the chip is full
+constexpr long long QUANT_MX_FULL = 1ll << 23, QUANT_MX_FEW = 1ll << 18;
 
 // per-row scale, one workgroup per row.  HOLD: the row has at most 8192 elements and stays in registers
 // between the amax pass and the quantisation (one read of the input); otherwise it is read twice.

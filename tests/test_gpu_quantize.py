@@ -154,3 +154,26 @@ def test_1x128_row_tiles(orc, rows, k):
         q, s = g.quantize(whole[:, :k], g.BLOCK, 128)
         qr, sr = orc.quantize(x, orc.BLOCK, 128)
         assert (q.cpu().numpy() == qr).all() and (s.cpu().numpy() == sr).all()
+
+
+@pytest.mark.parametrize("rows,k", [(1, 32), (1, 4096), (63, 4096), (65, 992), (129, 2016), (300, 1024), (2049, 4096)])
+def test_mx_quantisers_at_every_chunk_count(orc, rows, k):
+    """Arrays of up to 2^18 elements, up to 2^23 and beyond (one, two and four chunks per wave; MXFP4 has two kernels), tiled
+    layouts with padding rows and blocks; blocks whose largest value lies at, one ulp above and one ulp below a power of two times
+    448 or 6, the smallest exponent with its subnormal quotients, Inf and NaN."""
+    r = np.random.default_rng(rows + k)
+    x = (r.standard_normal((rows, k)) * np.exp2(r.integers(-30, 30, (rows, k // 32)).repeat(32, axis=1))).astype(np.float32)
+    for i, top in enumerate([448.0, 6.0]):
+        for j, (e, ulp) in enumerate([(0, 0), (0, 1), (0, -1), (5, 1), (-127, 0), (-127, 1), (-127, 2), (-127, -1), (-128, 1)]):
+            n = (2 * j + i) % (rows * (k // 32))
+            v = np.float32(np.ldexp(top, e))
+            block = x.reshape(-1, 32)[n]
+            block[:] = 0
+            block[7] = np.int32(v.view(np.int32) + ulp).view(np.float32)
+    for mode, quantise, reference in [("e4m3", lambda t, tiled: g.quantize(t, g.MX_TILED if tiled else g.MX), lambda a: orc.quantize(a, orc.MX)),
+                                      ("e2m1", lambda t, tiled: g.quantize_mxfp4(t, tiled=tiled), orc.quantize_mxfp4)]:
+        qr, sr = reference(x)
+        q, s = quantise(dev(x), False)
+        assert (q.cpu().numpy() == qr).all() and (s.cpu().numpy() == sr).all(), mode
+        qt, st = quantise(dev(x), True)
+        assert torch.equal(qt, q) and (st.cpu().numpy() == orc.mx_tile_scales(sr)).all(), mode
