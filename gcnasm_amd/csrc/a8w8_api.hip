@@ -1021,27 +1021,31 @@ int a8w8_quantize(const float* src, int rows, int k, int ld, uint8_t* q, void* s
         case A8W8_SCALE_TENSOR: {
             if (const int ds = device_status(); ds != A8W8_OK) return ds;
             const long long total = (long long)rows * k;
-            const unsigned grid = (unsigned)(total / 256 + 1 < 4096 ? total / 256 + 1 : 4096);
-            A8W8_LAUNCH_OR_RETURN(quant_tensor_clear_kernel, dim3(1), dim3(1), 0, s, (float*)scale);
             if (ld == k && total % 4 == 0 && aligned16(src) && ((uintptr_t)q & 3) == 0) {
                 const size_t units = (size_t)(total / 4);
-                const unsigned vgrid = (unsigned)(units / 1024 + 1 < 2048 ? units / 1024 + 1 : 2048);
-                A8W8_LAUNCH_OR_RETURN(quant_tensor_amax_vec_kernel, dim3(vgrid), dim3(256), 0, s, (const float4*)src, units, (float*)scale);
-                A8W8_LAUNCH_OR_RETURN(quant_tensor_apply_vec_kernel, dim3(vgrid), dim3(256), 0, s, (const float4*)src, units, (uint32_t*)q,
-                                   (const float*)scale);
-            } else {
-                A8W8_LAUNCH_OR_RETURN(quant_tensor_amax_kernel, dim3(grid), dim3(256), 0, s, src, rows, k, ld, (float*)scale);
-                A8W8_LAUNCH_OR_RETURN(quant_tensor_apply_kernel, dim3(grid), dim3(256), 0, s, src, rows, k, ld, q, (const float*)scale);
+                if (units <= QUANT_TENSOR_ONE)
+                    return launch(quant_tensor_one_kernel, dim3(1), dim3(1024), 0, s, (const float4*)src, (int)units, (uint32_t*)q, (float*)scale);
+                const unsigned parts = (unsigned)std::min<size_t>((units + 1023) / 1024, QUANT_TENSOR_PARTS);
+                const size_t apply = (units + 256 * QUANT_TENSOR_UNITS - 1) / (256 * QUANT_TENSOR_UNITS);
+                if (apply < (1u << 31)) {
+                    A8W8_LAUNCH_OR_RETURN(quant_tensor_amax_vec_kernel, dim3(parts), dim3(256), 0, s, (const float4*)src, units, (float*)q);
+                    A8W8_LAUNCH_OR_RETURN(quant_tensor_fold_kernel, dim3(1), dim3(256), 0, s, (const float*)q, (int)parts, (float*)scale);
+                    return launch(quant_tensor_apply_vec_kernel, dim3((unsigned)apply), dim3(256), 0, s, (const float4*)src, units, (uint32_t*)q,
+                                  (const float*)scale);
+                }
             }
-            A8W8_LAUNCH_OR_RETURN(quant_tensor_finish_kernel, dim3(1), dim3(1), 0, s, (float*)scale);
-            return A8W8_OK;
+            const unsigned grid = (unsigned)(total / 256 + 1 < 4096 ? total / 256 + 1 : 4096);
+            A8W8_LAUNCH_OR_RETURN(quant_tensor_clear_kernel, dim3(1), dim3(1), 0, s, (float*)scale);
+            A8W8_LAUNCH_OR_RETURN(quant_tensor_amax_kernel, dim3(grid), dim3(256), 0, s, src, rows, k, ld, (float*)scale);
+            A8W8_LAUNCH_OR_RETURN(quant_tensor_apply_kernel, dim3(grid), dim3(256), 0, s, src, rows, k, ld, q, (const float*)scale);
+            return launch(quant_tensor_finish_kernel, dim3(1), dim3(1), 0, s, (float*)scale);
         }
         case A8W8_SCALE_ROWCOL:
             if (const int ds = device_status(); ds != A8W8_OK) return ds;
-            if (quant_vec_ok(src, rows, k, ld, q, 4) && k <= 8192)
-                A8W8_LAUNCH_OR_RETURN(quant_rowwise_vec_kernel<true>, dim3((unsigned)rows), dim3(256), 0, s, src, k, ld, q, (float*)scale);
-            else if (quant_vec_ok(src, rows, k, ld, q, 4))
-                A8W8_LAUNCH_OR_RETURN(quant_rowwise_vec_kernel<false>, dim3((unsigned)rows), dim3(256), 0, s, src, k, ld, q, (float*)scale);
+            if (quant_vec_ok(src, rows, k, ld, q, 4))
+                return launch(k <= 4096 ? quant_rowwise_vec_kernel<256, true> : k <= 8192 ? quant_rowwise_vec_kernel<512, true>
+                              : k <= 16384 ? quant_rowwise_vec_kernel<1024, true> : quant_rowwise_vec_kernel<256, false>,
+                              dim3((unsigned)rows), dim3(k <= 4096 || k > 16384 ? 256 : k <= 8192 ? 512 : 1024), 0, s, src, k, ld, q, (float*)scale);
             else
                 A8W8_LAUNCH_OR_RETURN(quant_rowwise_kernel, dim3((unsigned)rows), dim3(256), 0, s, src, k, ld, q, (float*)scale);
             return A8W8_OK;

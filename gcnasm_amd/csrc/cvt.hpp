@@ -461,26 +461,31 @@ __global__ void __launch_bounds__(256) quant_mxfp4_few_kernel(const float* __res
 // elements from which the chip is full
 constexpr long long QUANT_MX_FULL = 1ll << 23, QUANT_MX_FEW = 1ll << 18;
 
-// per-row scale, one workgroup per row.  HOLD: the row has at most 8192 elements and stays in registers
-// between the amax pass and the quantisation (one read of the input); otherwise it is read twice.
-template <bool HOLD>
-__global__ void __launch_bounds__(256) quant_rowwise_vec_kernel(const float* __restrict__ src, int k, int ld,
-                                                                uint8_t* __restrict__ q, float* __restrict__ scale)
+// per-row scale, one workgroup per row.  HOLD: the row (at most 16 THREADS elements) stays in registers between the amax pass
+// and the quantisation, four 16-byte loads per thread (one read of the input); otherwise it is read twice.  256 threads up to
+// 4096 elements, 512 to 8192, 1024 to 16384: fewer registers and a shorter chain per thread than 256 threads with eight loads
+// each (8192 x 8192 54.2 -> 52.0 us, 256 x 8192 4.2 -> 4.0, 16 x 7168 3.4 -> 3.2, 4096 x 2048 9.1 -> 8.5); more threads
+// than that idle (4096 x 4096 15.2 us with 256, 17.8 with 512).
+template <int THREADS, bool HOLD>
+__global__ void __launch_bounds__(THREADS) quant_rowwise_vec_kernel(const float* __restrict__ src, int k, int ld,
+                                                                    uint8_t* __restrict__ q, float* __restrict__ scale)
 {
-    __shared__ float part[4];
+    __shared__ float part[THREADS / 64];
     const int row = blockIdx.x;
     const float* x = src + (size_t)row * ld;
-    float4 held[8];
+    float4 held[4];
     float amax = 0.f;
     if constexpr (HOLD) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int i = threadIdx.x * 4 + u * 1024;
+        for (int u = 0; u < 4; ++u) {
+            const int i = threadIdx.x * 4 + u * (4 * THREADS);
             held[u] = i < k ? load_once4(x + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-            amax = fmaxf(amax, fmaxf(fmaxf(fabsf(held[u].x), fabsf(held[u].y)), fmaxf(fabsf(held[u].z), fabsf(held[u].w))));
         }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            amax = fmaxf(amax, fmaxf(fmaxf(fabsf(held[u].x), fabsf(held[u].y)), fmaxf(fabsf(held[u].z), fabsf(held[u].w))));
     } else {
-        for (int i = threadIdx.x * 4; i < k; i += 1024) {
+        for (int i = threadIdx.x * 4; i < k; i += 4 * THREADS) {
             const float4 v = *(const float4*)(x + i);
             amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
         }
@@ -488,19 +493,21 @@ __global__ void __launch_bounds__(256) quant_rowwise_vec_kernel(const float* __r
     amax = wave_max(amax);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = amax;
     __syncthreads();
-    amax = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+    amax = part[0];
+#pragma unroll
+    for (int w = 1; w < THREADS / 64; ++w) amax = fmaxf(amax, part[w]);
     const float s = amax > 0.f ? __fdiv_rn(amax, 448.0f) : 1.0f;   // an all-zero group keeps scale 1
     if (threadIdx.x == 0) scale[row] = s;
     if constexpr (HOLD) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int i = threadIdx.x * 4 + u * 1024;
+        for (int u = 0; u < 4; ++u) {
+            const int i = threadIdx.x * 4 + u * (4 * THREADS);
             if (i < k)
                 *(uint32_t*)(q + (size_t)row * k + i) = pack4_e4m3(__fdiv_rn(held[u].x, s), __fdiv_rn(held[u].y, s),
                                                                    __fdiv_rn(held[u].z, s), __fdiv_rn(held[u].w, s));
         }
     } else {
-        for (int i = threadIdx.x * 4; i < k; i += 1024) {
+        for (int i = threadIdx.x * 4; i < k; i += 4 * THREADS) {
             const float4 v = *(const float4*)(x + i);
             *(uint32_t*)(q + (size_t)row * k + i) =
                 pack4_e4m3(__fdiv_rn(v.x, s), __fdiv_rn(v.y, s), __fdiv_rn(v.z, s), __fdiv_rn(v.w, s));
@@ -571,9 +578,16 @@ __global__ void __launch_bounds__(256) quant_128x128_vec_kernel(const float* __r
             pack4_e4m3(__fdiv_rn(v[u].x, s), __fdiv_rn(v[u].y, s), __fdiv_rn(v[u].z, s), __fdiv_rn(v[u].w, s));
 }
 
-// per-tensor scale over a contiguous array (ld == k): the amax and apply passes on 16-byte units, four
-// units per thread and iteration (loads first)
-__global__ void __launch_bounds__(256) quant_tensor_amax_vec_kernel(const float4* __restrict__ src, size_t units, float* scale)
+// per-tensor scale over a contiguous array (ld == k) of 16-byte units (bound: HBM, two passes), in three launches:
+//  1. every workgroup writes the maximum of its share, a plain store, into the first bytes of the output array, which nothing
+//     has been written to yet (thousands of atomics on the scale slot, which had to be cleared by a launch of its own before,
+//     took longer than the pass over the data);
+//  2. one workgroup folds these into the scale;
+//  3. the quantisation, from the end of the array to its start: what the first pass read last is still in the Infinity Cache.
+// 2560 x 2560: 23.6 us with atomics (four launches), 15.2 here; 8192 x 8192 115.8 -> 96.8 (98.1 with four units per
+// thread in pass 3, 100.1 from start to end as well); 1 x 4096 7.4 -> 5.6.
+constexpr int QUANT_TENSOR_PARTS = 1024;      // workgroups of pass 1 at most
+__global__ void __launch_bounds__(256) quant_tensor_amax_vec_kernel(const float4* __restrict__ src, size_t units, float* __restrict__ parts)
 {
     __shared__ float part[4];
     float amax = 0.f;
@@ -589,28 +603,69 @@ __global__ void __launch_bounds__(256) quant_tensor_amax_vec_kernel(const float4
     amax = wave_max(amax);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = amax;
     __syncthreads();
+    if (threadIdx.x == 0) parts[blockIdx.x] = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+}
+__global__ void __launch_bounds__(256) quant_tensor_fold_kernel(const float* __restrict__ parts, int n, float* __restrict__ scale)
+{
+    __shared__ float part[4];
+    float amax = 0.f;
+#pragma unroll
+    for (int u = 0; u < QUANT_TENSOR_PARTS / 256; ++u) {
+        const int i = threadIdx.x + 256 * u;
+        if (i < n) amax = fmaxf(amax, parts[i]);
+    }
+    amax = wave_max(amax);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = amax;
+    __syncthreads();
     if (threadIdx.x == 0) {
         amax = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
-        // thousands of atomics on one address take longer than the pass over the data: only a
-        // workgroup that would raise the maximum sends one
-        if (__float_as_uint(amax) > __hip_atomic_load((unsigned int*)scale, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            atomicMax((unsigned int*)scale, __float_as_uint(amax));
+        *scale = amax > 0.f ? __fdiv_rn(amax, 448.0f) : 1.0f;
     }
 }
+constexpr int QUANT_TENSOR_UNITS = 2;
 __global__ void __launch_bounds__(256) quant_tensor_apply_vec_kernel(const float4* __restrict__ src, size_t units,
-                                                                     uint32_t* __restrict__ q, const float* __restrict__ amax_slot)
+                                                                     uint32_t* __restrict__ q, const float* __restrict__ scale)
 {
-    const float amax = *amax_slot;
-    const float s = amax > 0.f ? __fdiv_rn(amax, 448.0f) : 1.0f;
-    const size_t stride = (size_t)gridDim.x * 256;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < units; i += 4 * stride) {
-        float4 v[4];
+    constexpr int U = QUANT_TENSOR_UNITS;
+    const float s = *scale;
+    const size_t i0 = (size_t)(gridDim.x - 1 - blockIdx.x) * (256 * U) + threadIdx.x;
+    float4 v[U];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = i + u * stride < units ? src[i + u * stride] : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int u = 0; u < U; ++u) v[u] = i0 + 256 * u < units ? load_once4((const float*)(src + i0 + 256 * u)) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (i + u * stride < units)
-                q[i + u * stride] = pack4_e4m3(__fdiv_rn(v[u].x, s), __fdiv_rn(v[u].y, s), __fdiv_rn(v[u].z, s), __fdiv_rn(v[u].w, s));
+    for (int u = 0; u < U; ++u)
+        if (i0 + 256 * u < units)
+            q[i0 + 256 * u] = pack4_e4m3(__fdiv_rn(v[u].x, s), __fdiv_rn(v[u].y, s), __fdiv_rn(v[u].z, s), __fdiv_rn(v[u].w, s));
+}
+// Up to QUANT_TENSOR_ONE units: one workgroup, one launch, the array in its registers (1 x 4096 2.7 us against 6.1 in three
+// launches, 4 x 4096 4.0 against 6.2; with eight units per thread 8 x 4096 5.9 against 6.3, which one compute unit's loads bound).
+constexpr int QUANT_TENSOR_ONE = 4096;
+__global__ void __launch_bounds__(1024) quant_tensor_one_kernel(const float4* __restrict__ src, int units, uint32_t* __restrict__ q,
+                                                                float* __restrict__ scale)
+{
+    __shared__ float part[16];
+    constexpr int U = QUANT_TENSOR_ONE / 1024;
+    float4 v[U];
+    float amax = 0.f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int i = threadIdx.x + 1024 * u;
+        v[u] = i < units ? load_once4((const float*)(src + i)) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
+    amax = wave_max(amax);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = amax;
+    __syncthreads();
+    amax = part[0];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) amax = fmaxf(amax, part[w]);
+    const float s = amax > 0.f ? __fdiv_rn(amax, 448.0f) : 1.0f;   // an all-zero group keeps scale 1
+    if (threadIdx.x == 0) *scale = s;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int i = threadIdx.x + 1024 * u;
+        if (i < units) q[i] = pack4_e4m3(__fdiv_rn(v[u].x, s), __fdiv_rn(v[u].y, s), __fdiv_rn(v[u].z, s), __fdiv_rn(v[u].w, s));
     }
 }
 

@@ -177,3 +177,32 @@ def test_mx_quantisers_at_every_chunk_count(orc, rows, k):
         assert (q.cpu().numpy() == qr).all() and (s.cpu().numpy() == sr).all(), mode
         qt, st = quantise(dev(x), True)
         assert torch.equal(qt, q) and (st.cpu().numpy() == orc.mx_tile_scales(sr)).all(), mode
+
+
+@pytest.mark.parametrize("rows,k", [(1, 4), (1, 4096), (3, 5460), (4, 4096), (1, 16388), (33, 516), (1024, 4096), (1025, 4100)])
+def test_per_tensor_one_launch_and_three(orc, rows, k):
+    """One workgroup up to 16384 elements, three launches beyond (one partial maximum, a few, all 1024 of them); the largest
+    value in the last element and in the first, an all-zero array, NaN beside numbers."""
+    for place in (0, rows * k - 1, None):
+        x = np.random.default_rng(rows + k).standard_normal((rows, k)).astype(np.float32)
+        if place is None:
+            x[:] = 0
+        else:
+            x.reshape(-1)[place] = -77.5
+            if rows * k > 8:
+                x.reshape(-1)[rows * k // 2] = np.nan
+        qr, sr = orc.quantize(np.nan_to_num(x, nan=0.0), orc.TENSOR)
+        q, s = _run(x, g.TENSOR)
+        number = ~np.isnan(x)
+        assert s[0] == np.float32(sr).ravel()[0] and (q[number] == qr[number]).all()
+        assert ((q[~number] & 0x7F) == 0x7F).all()
+
+
+@pytest.mark.parametrize("k", [4, 4096, 4100, 8192, 8196, 16384, 16388])
+def test_rowwise_at_every_row_length(orc, k):
+    x = np.random.default_rng(k).standard_normal((5, k)).astype(np.float32)
+    x[1] = 0
+    x[2, k - 1] = 99.0
+    qr, sr = orc.quantize(x, orc.ROWCOL)
+    q, s = _run(x, g.ROWCOL)
+    assert (q == qr).all() and (s == sr).all()
