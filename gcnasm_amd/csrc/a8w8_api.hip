@@ -55,7 +55,7 @@ bool raise_lds_limits_of_mode()
     if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BLOCK || MODE == MODE_MX || MODE == MODE_BF16)
         ok = ok && raise_lds_limit(gemm_a8w8_persist<MODE, C_BF16>, persist_lds_bytes(MODE)) &&
              raise_lds_limit(gemm_a8w8_persist<MODE, C_FP32>, persist_lds_bytes(MODE));
-    if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16 || MODE == MODE_F4T)
+    if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16 || MODE == MODE_F4T || MODE == MODE_F4)
         ok = ok && raise_lds_limit(gemm_a8w8_wide<MODE, C_BF16>, wide_lds_bytes(MODE)) &&
              raise_lds_limit(gemm_a8w8_wide<MODE, C_FP32>, wide_lds_bytes(MODE));
     {
@@ -252,6 +252,22 @@ bool wide_ok(const a8w8_gemm_args* g)
     return persist_ok(g) && (g->k / BK) % 2 == 0;
 }
 
+int num_cus();
+bool small_ok(const a8w8_gemm_args* g);
+
+// MXFP4 with row-major scales on the four-wave kernel (`g`: byte view, k in bytes, row-major scale mode).  It fetches 16 scale
+// bytes of a row at a time (two K steps: an even number of them) with 32-bit offsets that run up to 256 rows past the end of
+// the matrix.  The line to the 128-tile kernel is the one every other mode has (small_ok): above it 256-tiles are the
+// faster ones (4096^3 with the quantiser of A: 67.5 us with the GEMM on the 128-tile kernel, 55.5 here).
+bool wide_row_scales_ok(const a8w8_gemm_args* g)
+{
+    const auto rows_ok = [&](const void* s, long long stride, long long batch_stride, long long rows) {
+        return aligned16(s) && stride % 16 == 0 && (g->batch == 1 || batch_stride % 16 == 0) && (rows + BM) * stride < (1ll << 31);
+    };
+    return !small_ok(g) && persist_ok(g) && (g->k / BK) % 2 == 0 && rows_ok(g->sfa, g->stride_sfa, g->stride_sfa_batch, g->m) &&
+           rows_ok(g->sfb, g->stride_sfb, g->stride_sfb_batch, g->n) && c_tile_fits(g->stride_c, g->c_dtype == A8W8_C_BF16 ? 2 : 4);
+}
+
 template <int MODE, int CDT>
 int launch_general(const GemmParams& p, int batch, hipStream_t stream);
 
@@ -355,7 +371,7 @@ int launch_persist(const GemmParams& p, int batch, hipStream_t stream)
 template <int MODE, int CDT>
 int launch_wide(const GemmParams& p, int batch, hipStream_t stream)
 {
-    if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16 || MODE == MODE_F4T) {
+    if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16 || MODE == MODE_F4T || MODE == MODE_F4) {
         if (!c_tile_fits(p.ldc, CDT == C_BF16 ? 2 : 4)) return A8W8_ERR_TOO_LARGE;
         PersistParams pp;
         pp.g = p;
@@ -784,12 +800,16 @@ static int a4w4_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
                              (!small_ok(&bytes) && !persist_ok(&bytes))))
         return A8W8_ERR_BAD_GROUP;
     // row-major scales: the 128-tile kernel at any size (it stages the step's eight scale bytes per row as two dwords:
-    // scale rows have to start on dwords)
+    // scale rows have to start on dwords), the four-wave kernel where the problem fills the chip with 256-tiles and the
+    // scale rows take its 16-byte loads
     if (!tiled && !g->b_preshuffled && g->k % 256 == 0) {
         a8w8_gemm_args rows = bytes;
         rows.scale_mode = A8W8_SCALE_MX_E8M0_1x32;      // what tiled_ok checks the scale strides and pointers against
         if (tiled_ok(&rows) && (long long)((g->m + SM_BM - 1) / SM_BM) * ((g->n + 63) / 64) < (1ll << 31)) {
             const GemmParams p = make_params(&bytes);
+            if (wide_row_scales_ok(&rows))
+                return g->c_dtype == A8W8_C_BF16 ? launch_wide<MODE_F4, C_BF16>(p, g->batch, s)
+                                                 : launch_wide<MODE_F4, C_FP32>(p, g->batch, s);
             return g->c_dtype == A8W8_C_BF16 ? launch_small<MODE_F4, C_BF16>(p, g->batch, s)
                                              : launch_small<MODE_F4, C_FP32>(p, g->batch, s);
         }

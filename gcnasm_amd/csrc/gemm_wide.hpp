@@ -74,8 +74,8 @@ constexpr int WIDE_THREADS = 256;
 constexpr int WIDE_T = 8;                            // 8 x 8 MFMA tiles per wave
 constexpr int wide_lds_bytes(int mode)
 {
-    // tiled MX scales: two buffers of two scale groups each, i.e. all of the 160 KiB
-    return GEMM_LDS_BYTES + ((mode == MODE_MXT || mode == MODE_F4T) ? 4 * MX_GROUP_BYTES : mode == MODE_ROWCOL ? 2 * ROWCOL_SCALE_BYTES : 0);
+    // MX scales: two buffers of two scale groups each, i.e. all of the 160 KiB
+    return GEMM_LDS_BYTES + ((mode == MODE_MXT || mode == MODE_F4T || mode == MODE_F4) ? 4 * MX_GROUP_BYTES : mode == MODE_ROWCOL ? 2 * ROWCOL_SCALE_BYTES : 0);
 }
 
 // The 64 accumulator tiles of a wave live in accumulator registers a[0:255], tile (i, j) in
@@ -143,15 +143,20 @@ template <int MODE, int CDT>
 __global__ void __launch_bounds__(WIDE_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gemm_a8w8_wide(PersistParams pp)
 {
-    static_assert(MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16 || MODE == MODE_F4T,
+    static_assert(MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16 || MODE == MODE_F4T || MODE == MODE_F4,
                   "modes of the four-wave kernel");
     // MODE_F4T (packed E2M1 operands): a 128-byte K step holds 256 elements = eight scale blocks = one
     // "pair of K steps" of the tiled scale layout: the tiled-MX plumbing serves it with a scale fetch
     // every step and two 16 x 16 x 128 FP4 MFMAs per fragment pair.  MODE_BF16: a step is 64 elements,
     // two 16 x 16 x 32 MFMAs per fragment pair, no scales.
-    constexpr bool IS_MXT = MODE == MODE_MXT || MODE == MODE_F4T;   // tiled E8M0 scales
-    constexpr int MPF = (MODE == MODE_BF16 || MODE == MODE_F4T) ? 2 : 1;     // MFMAs per fragment pair
-    constexpr int PAIR_STEPS = MODE == MODE_F4T ? 1 : 2;             // K steps served by one fetch of scales
+    // MODE_F4 (the same operands, row-major scales): a scale group in LDS is 16 bytes of each of the tile's 512 rows, two
+    // K steps of eight bytes, where the tiled layout has the same bytes in the order the lanes want them.  Everything but
+    // the fetch (one row per lane) and the read (two bytes of a row put in place by v_perm) is shared.
+    constexpr bool IS_F4 = MODE == MODE_F4T || MODE == MODE_F4;
+    constexpr bool ROW_SCALES = MODE == MODE_F4;
+    constexpr bool IS_MXT = MODE == MODE_MXT || IS_F4;               // E8M0 scales
+    constexpr int MPF = (MODE == MODE_BF16 || IS_F4) ? 2 : 1;        // MFMAs per fragment pair
+    constexpr int PAIR_STEPS = IS_F4 ? 1 : 2;                        // K steps served by one fetch of scales
     // tiled MX scales are laid out for A tiles whose rows are dealt like the B tiles' rows
     constexpr bool PERM_A = IS_MXT;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -228,8 +233,8 @@ gemm_a8w8_wide(PersistParams pp)
     };
     ScaleTile sf_cur = {}, sf_next = {};
     const int sf_nblk[2] = {(p.m + 63) >> 6, (p.n + 63) >> 6};
-    const uint32_t sf_bytes[2] = {(uint32_t)mx_tiled_bytes(p.m, MODE == MODE_F4T ? 2 * p.k : p.k),
-                                  (uint32_t)mx_tiled_bytes(p.n, MODE == MODE_F4T ? 2 * p.k : p.k)};
+    const uint32_t sf_bytes[2] = {ROW_SCALES ? (uint32_t)(p.m - 1) * p.stride_sfa + (p.k >> 4) : (uint32_t)mx_tiled_bytes(p.m, IS_F4 ? 2 * p.k : p.k),
+                                  ROW_SCALES ? (uint32_t)(p.n - 1) * p.stride_sfb + (p.k >> 4) : (uint32_t)mx_tiled_bytes(p.n, IS_F4 ? 2 * p.k : p.k)};
     auto point_scales_at = [&](ScaleTile& t, int item) __attribute__((always_inline)) {
         if constexpr (IS_MXT) {
             item = min(item, pp.items - 1);
@@ -256,7 +261,10 @@ gemm_a8w8_wide(PersistParams pp)
                     const __amdgpu_buffer_rsrc_t rs = make_rsrc(t.base[side], sf_bytes[side]);   // past the end: reads 0
                     A8W8_LDS char* s =
                         (A8W8_LDS char*)smem + GEMM_LDS_BYTES + buf * BATCH_BYTES + gi * MX_GROUP_BYTES + side * 4096 + wave_lds;
-                    load_to_lds_16(rs, s, lane16, ((batch * GPB + gi) * sf_nblk[side] + t.blk[side] + wave) * 1024);
+                    if constexpr (ROW_SCALES)      // one row per lane, the 16 bytes of the group's two K steps
+                        load_to_lds_16(rs, s, ((t.blk[side] + wave) * 64 + lane) * (side ? p.stride_sfb : p.stride_sfa), (batch * GPB + gi) * 16);
+                    else
+                        load_to_lds_16(rs, s, lane16, ((batch * GPB + gi) * sf_nblk[side] + t.blk[side] + wave) * 1024);
                 }
         }
     };
@@ -308,8 +316,26 @@ gemm_a8w8_wide(PersistParams pp)
     // MX scales in registers: per 64-row block of the wave's A rows (and B rows) one dword per tile
     // pair, whose byte 2 (tile parity) + (step parity) belongs to the MFMA; they serve two K steps.
     const int lane_rg = r16 * 4 + g;
-    const int rd_sfa = GEMM_LDS_BYTES + wave_m * 2048 + lane_rg * 8;
-    const int rd_sfb = GEMM_LDS_BYTES + 4096 + wave_n * 2048 + lane_rg * 8;
+    // (row-major: the row this lane scales in MFMA tile 0 of the wave's first block; tile parity adds 4 rows, the pair 32, the block 64)
+    const int sf_lane = ROW_SCALES ? (8 * (r16 >> 2) + (r16 & 3)) * 16 : lane_rg * 8;
+    const int rd_sfa = GEMM_LDS_BYTES + wave_m * 2048 + sf_lane;
+    const int rd_sfb = GEMM_LDS_BYTES + 4096 + wave_n * 2048 + sf_lane;
+    // Row-major scales: of the step's eight bytes of a row the lane needs g (first half of the step) and 4 + g (second
+    // half); tile parity 0's two go into the low half of the dword, parity 1's into the high half.
+    const unsigned sf_sel_even = (unsigned)g | (unsigned)(4 + g) << 8 | 0x0c0c0000u;      // 0x0c: a zero byte
+    const unsigned sf_sel_odd = (unsigned)g << 16 | (unsigned)(4 + g) << 24 | 0x0c0cu;
+    auto read_row_scales = [&](int at, v2i (&raw)[4]) __attribute__((always_inline)) {      // [pair][parity]
+#pragma unroll
+        for (int e = 0; e < 4; ++e) raw[e] = *(const v2i*)(smem + at + (e >> 1) * 512 + (e & 1) * 64);
+    };
+    auto place_row_scales = [&](const v2i (&raw)[4]) __attribute__((always_inline)) -> v2i {
+        v2i v;
+#pragma unroll
+        for (int jp = 0; jp < 2; ++jp)
+            v[jp] = (int)(__builtin_amdgcn_perm((unsigned)raw[2 * jp].y, (unsigned)raw[2 * jp].x, sf_sel_even) |
+                          __builtin_amdgcn_perm((unsigned)raw[2 * jp + 1].y, (unsigned)raw[2 * jp + 1].x, sf_sel_odd));
+        return v;
+    };
     v2i sc_a[2], sc_b[2], sc_a_next[2], sc_b_next[2];
     int sc_rd_off = 0;                              // LDS offset (buffer, pair) of the scales to fetch next
     constexpr int BATCH_STEPS = 2 * 2 * PAIR_STEPS;  // K steps served by one batch: two scale groups of two pairs
@@ -498,8 +524,16 @@ gemm_a8w8_wide(PersistParams pp)
     if constexpr (IS_MXT) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            sc_a[u] = *(const v2i*)(smem + rd_sfa + u * 1024);
-            sc_b[u] = *(const v2i*)(smem + rd_sfb + u * 1024);
+            if constexpr (ROW_SCALES) {
+                v2i raw[4];
+                read_row_scales(rd_sfa + u * 1024, raw);
+                sc_a[u] = place_row_scales(raw);
+                read_row_scales(rd_sfb + u * 1024, raw);
+                sc_b[u] = place_row_scales(raw);
+            } else {
+                sc_a[u] = *(const v2i*)(smem + rd_sfa + u * 1024);
+                sc_b[u] = *(const v2i*)(smem + rd_sfb + u * 1024);
+            }
         }
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -526,6 +560,7 @@ gemm_a8w8_wide(PersistParams pp)
         // registers and are updated in place, and the statements keep their order, so the source
         // order below is the schedule: two MFMAs, one LDS read; a load after every fourth MFMA.
         v4i half[8];
+        v2i sf_raw[2][4];
         // 16 MPF slots: with two MFMAs per fragment pair, all first halves, then all second halves
         // (two MFMAs in a row on one accumulator would wait for each other)
         static_for<16 * MPF>([&](auto SS) {
@@ -537,7 +572,7 @@ gemm_a8w8_wide(PersistParams pp)
             constexpr int j = jb + (a_outer ? inner : (t >> 2)), i = ia + (a_outer ? (t >> 2) : inner);
             constexpr int lo = (i * 8 + j) * 4;
             constexpr bool z = zc && hf == 0;
-            if constexpr (MODE == MODE_F4T) {
+            if constexpr (IS_F4) {
                 const v4i bh = hf ? v4i{fb[j][4], fb[j][5], fb[j][6], fb[j][7]} : v4i{fb[j][0], fb[j][1], fb[j][2], fb[j][3]};
                 const v4i ah = hf ? v4i{fa[i][4], fa[i][5], fa[i][6], fa[i][7]} : v4i{fa[i][0], fa[i][1], fa[i][2], fa[i][3]};
                 mfma_acc_f4<lo, z, 2 * (j & 1) + hf, 2 * (i & 1) + hf>(bh, ah, sc_b[j >> 2][(j >> 1) & 1], sc_a[i >> 2][(i >> 1) & 1]);
@@ -573,6 +608,11 @@ gemm_a8w8_wide(PersistParams pp)
             if constexpr (IS_MXT && SCR && sl % (4 * MPF) == 0) {
                 // the next pair's scales, four 8-byte reads spread over the quadrant
                 constexpr int u = sl / (4 * MPF);
+                if constexpr (ROW_SCALES) {
+                    // row-major: four reads, put in place when the next four have been issued (the last ones behind the quadrant)
+                    read_row_scales(sc_rd_off + (u < 2 ? rd_sfa : rd_sfb) + (u & 1) * 1024, sf_raw[u & 1]);
+                    if constexpr (u > 0) (u <= 2 ? sc_a_next[(u - 1) & 1] : sc_b_next[0]) = place_row_scales(sf_raw[(u & 1) ^ 1]);
+                } else {
 #ifdef A8W8_ABLATE_SCALE_READS
                 const v2i v = u < 2 ? sc_a[u] : sc_b[u - 2];
 #else
@@ -580,6 +620,7 @@ gemm_a8w8_wide(PersistParams pp)
 #endif
                 if constexpr (u < 2) sc_a_next[u] = v;
                 else sc_b_next[u - 2] = v;
+                }
             }
             if constexpr (eq >= 0 && sl % (2 * MPF) == 2 * MPF - 1) {
                 using EQT = std::integral_constant<int, eq < 0 ? 0 : eq>;
@@ -592,6 +633,10 @@ gemm_a8w8_wide(PersistParams pp)
                 }
             }
         });
+        if constexpr (ROW_SCALES && SCR) {
+            sc_b_next[1] = place_row_scales(sf_raw[1]);
+            asm volatile("" : "+v"(sc_b_next[1]));      // in front of the hand-over: not directly before the MFMA that reads it
+        }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const v4i lo = half[2 * t], hi = half[2 * t + 1];
@@ -719,7 +764,7 @@ gemm_a8w8_wide(PersistParams pp)
                     const int q = first / PAIR_STEPS;          // pair; two pairs per scale group, GPB groups per batch
                     const bool same = first < nk;
                     const int buf = same ? (cur_bbase + (q >> 2)) & 1 : (cur_bbase + batches_per_tile) & 1;
-                    sc_rd_off = buf * BATCH_BYTES + (same ? ((q >> 1) & 1) * MX_GROUP_BYTES + (q & 1) * 512 : 0);
+                    sc_rd_off = buf * BATCH_BYTES + (same ? ((q >> 1) & 1) * MX_GROUP_BYTES + (q & 1) * (ROW_SCALES ? 8 : 512) : 0);
                 }
             };
             point_scale_read_at(PAIR_STEPS == 1 ? ks + 1 : ks + 2);
