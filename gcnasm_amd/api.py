@@ -58,6 +58,14 @@ def build_library(verbose=False):
 
 
 _lib = None
+torch = None        # imported with the first call that takes tensors (the package itself needs only ctypes)
+
+
+def _need_torch():
+    global torch
+    if torch is None:
+        import torch as module
+        torch = module
 
 
 def lib():
@@ -110,9 +118,14 @@ def status_string(status):
     return lib().a8w8_status_string(int(status)).decode()
 
 
+# The host's part of a call is what a decoding step of a small layer waits for (1 x 4096 x 4096 with its quantiser: the two
+# launches take 8 us of device time).  Hence below: shapes and strides are read from a tensor once, the argument block is
+# filled by its constructor, the stream comes as the raw handle: quantize 10.3 -> 8.3 us per call, flatmm 12.8 -> 8.5 (of which the
+# library and its launch are 3.5, each allocation 1.8).
 def _stream():
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream's handle (what torch.cuda.current_stream().cuda_stream holds, without the object around it)."""
+    _need_torch()
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _check(status, where):
@@ -123,26 +136,35 @@ def _check(status, where):
 def raw_gemm_args(a, b, c, sfa, sfb, m, n, k, scale_mode, c_dtype=BF16, batch=1, stride_a=None, stride_b=None,
                   stride_c=None, stride_sfa=None, stride_sfb=None, b_preshuffled=0, batch_strides=None):
     """Fill the C argument block from raw integers (device addresses)."""
-    g = GemmArgs()
-    g.a, g.b, g.c, g.sfa, g.sfb = a, b, c, sfa, sfb
-    g.m, g.n, g.k, g.batch = m, n, k, batch
-    g.stride_a = k if stride_a is None else stride_a
-    g.stride_b = k if stride_b is None else stride_b
-    g.stride_c = n if stride_c is None else stride_c
+    if stride_a is None:
+        stride_a = k
+    if stride_b is None:
+        stride_b = k
+    if stride_c is None:
+        stride_c = n
     if stride_sfa is None:
-        stride_sfa = {TENSOR: 0, ROWCOL: 0, BLOCK: m, MX: k // 32}[scale_mode] if 0 <= scale_mode <= 3 else 0
+        stride_sfa = m if scale_mode == BLOCK else k // 32 if scale_mode == MX else 0
     if stride_sfb is None:
-        stride_sfb = {TENSOR: 0, ROWCOL: 1, BLOCK: k // 128, MX: k // 32}[scale_mode] if 0 <= scale_mode <= 3 else 0
-    g.stride_sfa, g.stride_sfb = stride_sfa, stride_sfb
-    if batch_strides is None:
-        sfa_b = {TENSOR: 1, ROWCOL: m, BLOCK: m * (k // 128), MX: m * (k // 32),
-                 MX_TILED: mx_tiled_bytes(m, k)}.get(scale_mode, 0)
-        sfb_b = {TENSOR: 1, ROWCOL: n, BLOCK: (n // 128) * (k // 128), MX: n * (k // 32),
-                 MX_TILED: mx_tiled_bytes(n, k)}.get(scale_mode, 0)
-        batch_strides = (m * g.stride_a, n * g.stride_b, m * g.stride_c, sfa_b, sfb_b)
-    (g.stride_a_batch, g.stride_b_batch, g.stride_c_batch, g.stride_sfa_batch, g.stride_sfb_batch) = batch_strides
-    g.scale_mode, g.c_dtype, g.b_preshuffled = scale_mode, c_dtype, b_preshuffled
-    return g
+        stride_sfb = 1 if scale_mode == ROWCOL else k // 128 if scale_mode == BLOCK else k // 32 if scale_mode == MX else 0
+    if batch_strides is not None:
+        a_b, b_b, c_b, sfa_b, sfb_b = batch_strides
+    else:
+        a_b, b_b, c_b = m * stride_a, n * stride_b, m * stride_c
+        if scale_mode == TENSOR:
+            sfa_b = sfb_b = 1
+        elif scale_mode == ROWCOL:
+            sfa_b, sfb_b = m, n
+        elif scale_mode == BLOCK:
+            sfa_b, sfb_b = m * (k // 128), (n // 128) * (k // 128)
+        elif scale_mode == MX:
+            sfa_b, sfb_b = m * (k // 32), n * (k // 32)
+        elif scale_mode == MX_TILED:
+            sfa_b, sfb_b = mx_tiled_bytes(m, k), mx_tiled_bytes(n, k)
+        else:
+            sfa_b = sfb_b = 0
+    # (in the order of the fields)
+    return GemmArgs(a, b, c, m, n, k, batch, stride_a, stride_b, stride_c, a_b, b_b, c_b, sfa, sfb, stride_sfa, stride_sfb, sfa_b, sfb_b,
+                    scale_mode, c_dtype, b_preshuffled)
 
 
 def mx_tiled_bytes(rows, k):
@@ -152,7 +174,6 @@ def mx_tiled_bytes(rows, k):
 
 def _out(c, shape, c_dtype, device):
     """The output tensor and its C type code: a caller's tensor decides the type (bf16 or fp32 only)."""
-    import torch
     if c is None:
         return torch.empty(shape, dtype=torch.bfloat16 if c_dtype == BF16 else torch.float32, device=device), c_dtype
     if c.dtype not in (torch.bfloat16, torch.float32):
@@ -162,20 +183,19 @@ def _out(c, shape, c_dtype, device):
     return c, (BF16 if c.dtype == torch.bfloat16 else FP32)
 
 
-def _check_operand(t, name, dims):
+def _check_operand(t, name, dims, shape, strides):
     """Operands are strided views of device memory whose rows are contiguous; anything else would be misread."""
     if not t.is_cuda:
         raise ValueError(f"{name} must live on the GPU")
-    if t.dim() not in dims:
-        raise ValueError(f"{name} must have {' or '.join(str(d) for d in dims)} dimensions, got {t.dim()}")
-    if t.dim() >= 1 and t.shape[-1] > 1 and t.stride(-1) != 1:
-        raise ValueError(f"{name}: the last dimension must be contiguous (stride {t.stride(-1)})")
+    if len(shape) not in dims:
+        raise ValueError(f"{name} must have {' or '.join(str(d) for d in dims)} dimensions, got {len(shape)}")
+    if shape and shape[-1] > 1 and strides[-1] != 1:
+        raise ValueError(f"{name}: the last dimension must be contiguous (stride {strides[-1]})")
 
 
 def _check_scales(t, name, scale_mode):
     """Scale arrays are read with the strides their shape implies: they have to be contiguous, on the GPU, and of
     the element type of the scale mode (fp32, or uint8 for the E8M0 modes)."""
-    import torch
     want = torch.uint8 if scale_mode in (MX, MX_TILED) else torch.float32
     if not t.is_cuda or not t.is_contiguous():
         raise ValueError(f"{name} must be a contiguous GPU tensor")
@@ -203,33 +223,37 @@ def _check_scale_sizes(sfa, sfb, scale_mode, m, n, k, batch, b_shared):
     need_a = batch * scale_elements(scale_mode, m, k, False)
     per_b = scale_elements(scale_mode, n, k, True)
     need_b = per_b if b_shared else batch * per_b
-    if sfa.numel() < need_a:
-        raise ValueError(f"sfa holds {sfa.numel()} elements, this problem reads {need_a}")
-    if sfb.numel() < need_b:
-        raise ValueError(f"sfb holds {sfb.numel()} elements, this problem reads {need_b}")
-    if b_shared and sfb.numel() >= batch * per_b and sfb.numel() > per_b:
+    has_a, has_b = sfa.numel(), sfb.numel()
+    if has_a < need_a:
+        raise ValueError(f"sfa holds {has_a} elements, this problem reads {need_a}")
+    if has_b < need_b:
+        raise ValueError(f"sfb holds {has_b} elements, this problem reads {need_b}")
+    if b_shared and has_b >= batch * per_b and has_b > per_b:
         raise ValueError(f"b is shared by all {batch} batch entries but sfb holds a set of scales per entry; pass one set")
 
 
 def _args_from_tensors(a, b, sfa, sfb, scale_mode, c, c_dtype, b_preshuffled, n=None, scaled=True):
-    _check_operand(a, "a", (2, 3))
-    _check_operand(b, "b", (1, 2) if b_preshuffled else (2, 3))
+    _need_torch()
+    a_shape, a_strides, b_shape, b_strides = a.shape, a.stride(), b.shape, b.stride()
+    _check_operand(a, "a", (2, 3), a_shape, a_strides)
+    _check_operand(b, "b", (1, 2) if b_preshuffled else (2, 3), b_shape, b_strides)
     if scaled:
         _check_scales(sfa, "sfa", scale_mode)
         _check_scales(sfb, "sfb", scale_mode)
-    batch = a.shape[0] if a.dim() == 3 else 1
-    m, k = a.shape[-2], a.shape[-1]
+    batched = len(a_shape) == 3
+    batch = a_shape[0] if batched else 1
+    m, k = a_shape[-2], a_shape[-1]
     if n is None:
-        n = b.shape[-2]
-    shape = (batch, m, n) if a.dim() == 3 else (m, n)
-    c, c_dtype = _out(c, shape, c_dtype, a.device)
-    if c.dim() >= 2 and c.shape[-1] > 1 and c.stride(-1) != 1:
+        n = b_shape[-2]
+    c, c_dtype = _out(c, (batch, m, n) if batched else (m, n), c_dtype, a.device)
+    c_strides = c.stride()
+    if n > 1 and c_strides[-1] != 1:
         raise ValueError("c: the last dimension must be contiguous")
     g = raw_gemm_args(a.data_ptr(), b.data_ptr(), c.data_ptr(), sfa.data_ptr(), sfb.data_ptr(), m, n, k, scale_mode,
-                      c_dtype, batch, stride_a=a.stride(-2), stride_b=(k if b_preshuffled else b.stride(-2)),
-                      stride_c=c.stride(-2), b_preshuffled=b_preshuffled)
-    if a.dim() == 3:
-        g.stride_a_batch, g.stride_c_batch = a.stride(0), c.stride(0)
+                      c_dtype, batch, stride_a=a_strides[-2], stride_b=(k if b_preshuffled else b_strides[-2]),
+                      stride_c=c_strides[-2], b_preshuffled=b_preshuffled)
+    if batched:
+        g.stride_a_batch, g.stride_c_batch = a_strides[0], c_strides[0]
         if b_preshuffled:
             # flat shuffled weights: of every batch entry back to back, or one matrix shared by all of them
             per_entry = n * k * a.element_size() // b.element_size()
@@ -240,10 +264,10 @@ def _args_from_tensors(a, b, sfa, sfb, scale_mode, c, c_dtype, b_preshuffled, n=
                 g.stride_sfb_batch = 0
             else:
                 raise ValueError(f"shuffled b holds {b.numel()} elements, expected {per_entry} or {batch} x {per_entry}")
-        elif b.dim() == 3:
-            if b.shape[0] != batch:
-                raise ValueError(f"b has {b.shape[0]} batch entries, a has {batch}")
-            g.stride_b_batch = b.stride(0)
+        elif len(b_shape) == 3:
+            if b_shape[0] != batch:
+                raise ValueError(f"b has {b_shape[0]} batch entries, a has {batch}")
+            g.stride_b_batch = b_strides[0]
         else:
             # one weight matrix shared by every batch entry, and with it one set of weight scales
             g.stride_b_batch = 0
@@ -271,7 +295,7 @@ def gemm_a16w16(a, b, c=None, c_dtype=BF16, n=None):
 
 def preshuffle_b_bf16_device(b):
     """bf16 weights [N, K] on the GPU -> the pre-shuffled byte layout a16w16_flatmm streams (flat uint8 tensor)."""
-    import torch
+    _need_torch()
     n, k = b.shape
     return preshuffle_b_device(b.contiguous().view(torch.uint8).view(n, 2 * k))
 
@@ -285,7 +309,7 @@ def flatmm_a16w16(a, b_shuffled, n, c=None, c_dtype=BF16):
 
 def quantize_mxfp4(x, tiled=False):
     """fp32 [rows, K] -> (packed E2M1 bytes [rows, K/2], E8M0 scales row-major [rows, K/32] or tiled)."""
-    import torch
+    _need_torch()
     rows, k = x.shape
     q = torch.empty((rows, k // 2), dtype=torch.uint8, device=x.device)
     s = torch.empty(mx_tiled_bytes(rows, k) if tiled else (rows, k // 32), dtype=torch.uint8, device=x.device)
@@ -297,6 +321,7 @@ def quantize_mxfp4(x, tiled=False):
 def gemm_a4w4(a, b, sfa, sfb, scale_mode=MX_TILED, c=None, c_dtype=BF16, n=None):
     """MXFP4 GEMM through a4w4_gemm: a [M, K/2], b [N, K/2] packed E2M1 (uint8 on the GPU); with `n` given, b is the
     flat pre-shuffled weight of n rows (preshuffle_b_device on the packed bytes)."""
+    _need_torch()
     m, k = a.shape[-2], a.shape[-1] * 2
     shuffled = n is not None
     if not shuffled:
@@ -312,6 +337,7 @@ def gemm_a4w4(a, b, sfa, sfb, scale_mode=MX_TILED, c=None, c_dtype=BF16, n=None)
 def flatmm_a4w4(a, b_shuffled, sfa_tiled, sfb_tiled, n, c=None, c_dtype=BF16):
     """MXFP4 skinny-M GEMM through a4w4_flatmm: a [M, K/2] packed E2M1 with M <= 128, b_shuffled from
     preshuffle_b_device on the packed weight bytes [N, K/2], both scale arrays in the MX_TILED layout."""
+    _need_torch()
     m, k = a.shape[-2], a.shape[-1] * 2
     c, c_dtype = _out(c, (m, n), c_dtype, a.device)
     g = raw_gemm_args(a.data_ptr(), b_shuffled.data_ptr(), c.data_ptr(), sfa_tiled.data_ptr(), sfb_tiled.data_ptr(), m, n, k,
@@ -354,7 +380,7 @@ def unshuffle_b(bs_np, n, k):
 
 
 def preshuffle_b_device(b):
-    import torch
+    _need_torch()
     n, k = b.shape
     out = torch.empty(n * k, dtype=torch.uint8, device=b.device)
     _check(lib().a8w8_preshuffle_b_device(b.data_ptr(), out.data_ptr(), n, k, _stream()), "a8w8_preshuffle_b_device")
@@ -362,7 +388,7 @@ def preshuffle_b_device(b):
 
 
 def cvt_f32_to_e4m3(x, dialect=OCP, clamp240=False):
-    import torch
+    _need_torch()
     x = x.contiguous()
     out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
     _check(lib().a8w8_cvt_f32_to_e4m3(x.data_ptr(), out.data_ptr(), x.numel(), dialect, int(clamp240), _stream()),
@@ -371,7 +397,7 @@ def cvt_f32_to_e4m3(x, dialect=OCP, clamp240=False):
 
 
 def cvt_e4m3_to_f32(codes, dialect=OCP):
-    import torch
+    _need_torch()
     codes = codes.contiguous()
     out = torch.empty(codes.shape, dtype=torch.float32, device=codes.device)
     _check(lib().a8w8_cvt_e4m3_to_f32(codes.data_ptr(), out.data_ptr(), codes.numel(), dialect, _stream()),
@@ -381,7 +407,7 @@ def cvt_e4m3_to_f32(codes, dialect=OCP):
 
 def quantize(x, scale_mode, group_rows=1):
     """fp32 [rows, K] -> (E4M3 bytes [rows, K], scales in the layout a8w8_gemm reads)."""
-    import torch
+    _need_torch()
     rows, k = x.shape
     q = torch.empty((rows, k), dtype=torch.uint8, device=x.device)
     if scale_mode == TENSOR:
@@ -405,7 +431,7 @@ def quantize(x, scale_mode, group_rows=1):
 
 def mx_tile_scales(sf, out=None):
     """Row-major E8M0 scales [rows, K/32] (u8, on the GPU) -> the MX_TILED layout (flat u8 tensor)."""
-    import torch
+    _need_torch()
     rows, kb = sf.shape
     if out is None:
         out = torch.empty(mx_tiled_bytes(rows, kb * 32), dtype=torch.uint8, device=sf.device)
@@ -416,7 +442,7 @@ def mx_tile_scales(sf, out=None):
 
 def mx_tile_scales_ab(sfa, sfb):
     """Both scale arrays of a GEMM ([M, K/32] and [N, K/32] u8) -> MX_TILED, one launch."""
-    import torch
+    _need_torch()
     m, kb = sfa.shape
     n = sfb.shape[0]
     ta = torch.empty(mx_tiled_bytes(m, kb * 32), dtype=torch.uint8, device=sfa.device)
