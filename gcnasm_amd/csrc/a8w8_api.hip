@@ -66,6 +66,9 @@ bool raise_lds_limits_of_mode()
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, narrow_stages(MODE), 64>, small_lds_bytes(MODE, narrow_stages(MODE), 64)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, narrow_stages(MODE), 64>, small_lds_bytes(MODE, narrow_stages(MODE), 64));
     }
+    if constexpr (MODE != MODE_BLOCK)
+        ok = ok && raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, 3, SM_BN, false, 256>, small_lds_bytes(MODE, 3, SM_BN, 256)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 3, SM_BN, false, 256>, small_lds_bytes(MODE, 3, SM_BN, 256));
     if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BF16)
         ok = ok && raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, 2, SM_BN, true>, small_lds_bytes(MODE, 2)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 2, SM_BN, true>, small_lds_bytes(MODE, 2)) &&
@@ -311,6 +314,17 @@ bool narrow_tiles_pay(long long items128, int n, int k)
     return 2 * items128 <= num_cus() && n > 64 && k / BK >= A8W8_NARROW_MIN_KSTEPS;
 }
 
+// 256 x 128 tiles where 128 x 128 ones would put two workgroups on a compute unit, 256 x 128 ones would not, and the K loop is
+// long enough to make up for a prologue and a tile's stores that no second workgroup hides.  us per launch, bf16 C, two-stage
+// 128-tiles -> 256 x 128 (row/col, row-major MX, tiled MX, MXFP4 row-major / tiled, bf16):
+//   2560^3            22.2 -> 20.3, 26.1 -> 23.5, 23.3 -> 20.3, 16.8 / 13.9 -> 16.7 / 14.1, 41.3 -> 36.5
+//   2049x3584x4096    34.6 -> 28.5, 45.1 -> 36.0, 35.7 -> 30.2, 29.0 / 21.7 -> 24.6 / 19.8, 66.4 -> 51.5
+//   512x16384x7168    67.3 -> 57.1, 88.6 -> 81.5, 71.1 -> 60.2, 42.7 / 33.3 -> 39.1 / 29.5, 126.4 -> 112.5
+//   2048x4096x2048    18.0 -> 18.1, 21.3 -> 20.2, 19.4 -> 18.6, 15.2 / 12.7 -> 15.8 / 13.5, 31.1 -> 30.1
+//   1000x8192x1024    14.2 -> 14.7, 14.9 -> 15.2, 14.3 -> 14.4, 11.8 / 10.7 -> 13.3 / 12.1, 19.1 -> 20.1
+// i.e. the line lies at 16 steps of 128 bytes, and where a step's scales cost next to nothing beside its short MFMAs at 24.
+constexpr int tall_min_ksteps(int mode) { return mode == MODE_BF16 || mode == MODE_F4T ? 24 : 16; }
+
 template <int MODE, int CDT, int STAGES, bool RAGGED>
 int launch_small_stages(const GemmParams& q, int batch, hipStream_t stream)
 {
@@ -339,6 +353,16 @@ int launch_small(const GemmParams& p, int batch, hipStream_t stream)
         }
         if (items <= (long long)A8W8_SMALL_DEEP_UP_TO * num_cus())
             return launch_small_stages<MODE, CDT, 4, RAGGED>(q, batch, stream);
+        if constexpr (MODE != MODE_BLOCK && !RAGGED) {
+            const int tall_m = (p.m + 255) / 256;
+            // (its rows past the end are left to the buffer descriptors: the 32-bit offsets of a whole tile must not wrap)
+            const bool offsets_fit = (p.m + 256ll) * p.lda + p.k < (1ll << 32) && (p.n + 128ll) * p.ldb + p.k < (1ll << 32);
+            if (offsets_fit && (long long)tall_m * q.tiles_n * batch <= num_cus() && p.k / BK >= tall_min_ksteps(MODE)) {
+                q.tiles_m = tall_m;
+                dim3 grid((unsigned)(q.tiles_m * q.tiles_n), 1, (unsigned)batch);
+                return launch(gemm_a8w8_tile128<MODE, CDT, 3, SM_BN, false, 256>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, 3, SM_BN, 256), stream, q);
+            }
+        }
         return launch_small_stages<MODE, CDT, 2, RAGGED>(q, batch, stream);
     } else {
         return A8W8_ERR_BAD_MODE;

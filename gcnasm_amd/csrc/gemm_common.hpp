@@ -13,6 +13,9 @@
 // up holding C[m = lane%16][n = 4*(lane/16) .. +3]: four consecutive n, one 8-byte store
 // of bf16, and one A-side scale per lane per tile.
 #pragma once
+#include <type_traits>
+#include <utility>
+
 #include "a8w8_device.hpp"
 
 namespace a8w8 {
@@ -97,6 +100,75 @@ A8W8_DEV void tile_of_item(const TileMap& t, int item, int& batch, int& tm, int&
         tn = div_by_known(in_group, t.rem, t.inv_rem);
         tm = first_m + in_group - tn * t.rem;
     }
+}
+
+// Accumulators in named registers, for the kernels with one wave per SIMD: the four-wave kernel's 64 tiles (i, j) of a wave
+// live in accumulator registers a[4 (8i + j) : +3], the 32 of the 256 x 128 variant of the 128-tile kernel in a[4 (4i + j) : +3].
+// (Left to the compiler, a loop of 32 tiles moved every accumulator through one register quadruple, with the idle cycles between
+// an MFMA and the read of its result each time: twice the time per K step.)  They are named in assembly statements only and never appear as variables: the
+// compiler allocates nothing there (its own registers stay below 256, which the build checks), so no
+// copy, spill or re-materialisation can come between two MFMAs of one tile.  The statements keep
+// their order; the compiler does not see the MFMAs' latency, so the code that reads an accumulator
+// makes sure that enough instructions separate it from the last MFMA into that tile.
+template <int N, class F, int... I>
+A8W8_DEV void static_for_impl(F&& f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+A8W8_DEV void static_for(F&& f)
+{
+    static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
+}
+
+// tile LO/4 += a . b, or = a . b when ZC (the tile's first K step)
+template <int LO, bool ZC>
+A8W8_DEV void mfma_acc(const v8i& a, const v8i& b)
+{
+    if constexpr (ZC) asm volatile("v_mfma_f32_16x16x128_f8f6f4 a[%2:%3], %0, %1, 0" ::"v"(a), "v"(b), "n"(LO), "n"(LO + 3));
+    else asm volatile("v_mfma_f32_16x16x128_f8f6f4 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(a), "v"(b), "n"(LO), "n"(LO + 3));
+}
+// the same with E8M0 block scales: byte OA of sa scales a's K block of the lane, byte OB of sb b's
+template <int LO, bool ZC, int OA, int OB>
+A8W8_DEV void mfma_acc_mx(const v8i& a, const v8i& b, int sa, int sb)
+{
+    if constexpr (ZC)
+        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 a[%4:%5], %0, %1, 0, %2, %3 op_sel:[%6,%7,0] op_sel_hi:[%8,%9,0]" ::"v"(a),
+                     "v"(b), "v"(sa), "v"(sb), "n"(LO), "n"(LO + 3), "n"(OA & 1), "n"(OB & 1), "n"(OA >> 1), "n"(OB >> 1));
+    else
+        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 a[%4:%5], %0, %1, a[%4:%5], %2, %3 op_sel:[%6,%7,0] op_sel_hi:[%8,%9,0]" ::"v"(a),
+                     "v"(b), "v"(sa), "v"(sb), "n"(LO), "n"(LO + 3), "n"(OA & 1), "n"(OB & 1), "n"(OA >> 1), "n"(OB >> 1));
+}
+// bf16 operands: one 16 x 16 x 32 MFMA per 16-byte half of a fragment
+template <int LO, bool ZC>
+A8W8_DEV void mfma_acc_bf16(const v4i& a, const v4i& b)
+{
+    if constexpr (ZC) asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, 0" ::"v"(a), "v"(b), "n"(LO), "n"(LO + 3));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(a), "v"(b), "n"(LO), "n"(LO + 3));
+}
+// packed E2M1 operands (format 4 for both): one 16 x 16 x 128 MFMA per 16-byte half of a fragment
+template <int LO, bool ZC, int OA, int OB>
+A8W8_DEV void mfma_acc_f4(const v4i& a, const v4i& b, int sa, int sb)
+{
+    if constexpr (ZC)
+        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 a[%4:%5], %0, %1, 0, %2, %3 op_sel:[%6,%7,0] op_sel_hi:[%8,%9,0] cbsz:4 blgp:4" ::"v"(a),
+                     "v"(b), "v"(sa), "v"(sb), "n"(LO), "n"(LO + 3), "n"(OA & 1), "n"(OB & 1), "n"(OA >> 1), "n"(OB >> 1));
+    else
+        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 a[%4:%5], %0, %1, a[%4:%5], %2, %3 op_sel:[%6,%7,0] op_sel_hi:[%8,%9,0] cbsz:4 blgp:4" ::"v"(a),
+                     "v"(b), "v"(sa), "v"(sb), "n"(LO), "n"(LO + 3), "n"(OA & 1), "n"(OB & 1), "n"(OA >> 1), "n"(OB >> 1));
+}
+template <int IDX>
+A8W8_DEV float acc_read()
+{
+    float x;
+    asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(x) : "n"(IDX));
+    return x;
+}
+
+template <int IDX>
+A8W8_DEV void acc_zero()
+{
+    asm volatile("v_accvgpr_write_b32 a[%0], 0" ::"n"(IDX));
 }
 
 }  // namespace a8w8

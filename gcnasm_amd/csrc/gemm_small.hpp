@@ -16,16 +16,19 @@
 
 namespace a8w8 {
 
-constexpr int SM_BM = 128, SM_BN = 128;               // SM_BN: the widest tile; the kernel also takes 64 columns
+constexpr int SM_BM = 128, SM_BN = 128;               // the usual tile; the kernel also takes 64 columns, or 256 rows
 constexpr int SM_THREADS = 256;
-constexpr int small_stage_bytes(int bn) { return (SM_BM + bn) * BK; }   // 32768 for 128 columns, 24576 for 64
+constexpr int small_stage_bytes(int bn, int bm = SM_BM) { return (bm + bn) * BK; }   // 128 x 128: 32768, 128 x 64: 24576, 256 x 128: 49152
 // Scale bytes per stage.  Block mode: 128 A-row scales, the B scale at +512 and +768.  Row-major MX: the step's
 // four E8M0 bytes of 128 A rows, then of 128 B rows.  Tiled MX: 1 KiB per wave, whose first half is the 512-byte
 // unit (64 rows x one pair of K steps) of the wave's row block.
 // Row-major MX scales of packed E2M1 operands (MODE_F4): a 128-byte K step is 256 elements, eight E8M0 bytes per row:
 // the rows' first dwords (128 A rows, then 128 B rows), then their second dwords.
-constexpr int small_scale_bytes(int mode)
+// 256-row tiles: row-major MX 256 A rows, then the 128 B rows (twice); MODE_F4 the same with A's second dwords behind A's first
+// and B's behind B's; tiled MX the six 512-byte units of the tile (four A blocks, two B blocks), two per wave.
+constexpr int small_scale_bytes(int mode, int bm = SM_BM)
 {
+    if (bm == 256) return mode == MODE_MX ? 2048 : mode == MODE_MXT || mode == MODE_F4T || mode == MODE_F4 ? 4096 : 0;
     return mode == MODE_MXT || mode == MODE_F4T ? 4096 : mode == MODE_F4 ? 2048 : (mode == MODE_BLOCK || mode == MODE_MX) ? 1024 : 0;
 }
 #ifndef A8W8_SMALL_PIPELINED
@@ -37,10 +40,9 @@ constexpr int small_scale_bytes(int mode)
 #ifndef A8W8_SMALL_LINES_BY_LANE
 #define A8W8_SMALL_LINES_BY_LANE 1      // 0: whole tiles are stored from the MFMA layout as they are (measurement)
 #endif
-constexpr int SM_TM = 4;                               // MFMA tiles per wave along M (along N: a quarter of the tile's columns / 8)
-constexpr int small_lds_bytes(int mode, int stages, int bn = SM_BN)
+constexpr int small_lds_bytes(int mode, int stages, int bn = SM_BN, int bm = SM_BM)
 {
-    return stages * (small_stage_bytes(bn) + small_scale_bytes(mode));
+    return stages * (small_stage_bytes(bn, bm) + small_scale_bytes(mode, bm));
 }
 
 // p.tiles_m / p.tiles_n count 128 x 128 tiles here; grid = (tiles, 1, batch).  The launch bound asks for a
@@ -63,15 +65,25 @@ constexpr int small_lds_bytes(int mode, int stages, int bn = SM_BN)
 // and the bf16 MFMA keeps fp32 sums (8e-8).  A K step is four quarters of 32 elements; the fragments of the next quarter
 // are converted between the MFMAs of this one.  Half the MFMA rate, and still bound by it.
 // 1000 x 3000 x 2000 row/col: 7545 us on the one-thread-per-element kernel, 21 us here; 4096 x 4096 x 4080: 1.2 PFLOP/s.
-template <int MODE, int CDT, int SM_STAGES, int BN_ = SM_BN, bool RAGGED = false>
-__global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
+// BM_ = 256: 256 x 128 tiles, a wave owns 128 x 64 (accumulators in named accumulation registers, one wave per SIMD, three stages
+// of 48 KiB), for grids that would need two workgroups per compute unit on 128 x 128 tiles but fit at one per compute unit here.
+// A 64 x 64 wave tile reads 16 KiB of LDS per 16 MFMAs and the loads write another 8: as many cycles as the MFMAs take, so
+// two workgroups on a compute unit queue for LDS.  128 x 64 reads 24 KiB per 32 MFMAs.  Not for block scales: their
+// multiply-adds need the accumulators where the VALU can read them, which 128 of them beside 192 fragment registers are not.
+template <int MODE, int CDT, int SM_STAGES, int BN_ = SM_BN, bool RAGGED = false, int BM_ = 128>
+__global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__((amdgpu_waves_per_eu(BM_ == 256 ? 1 : 2, BM_ == 256 ? 1 : 8))) gemm_a8w8_tile128(GemmParams p)
 {
+    constexpr bool TALL = BM_ == 256;
+    static_assert(BM_ == 128 || (TALL && SM_STAGES == 3 && BN_ == 128 && !RAGGED && MODE != MODE_BLOCK), "tile height");
     static_assert(!RAGGED || MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BF16, "partial K steps: no scales that change with K");
     constexpr bool BY_BF16 = RAGGED && MODE != MODE_BF16;      // FP8 operands converted to bf16
-    static_assert(SM_STAGES == 2 || SM_STAGES == 4 || SM_STAGES == 5 || SM_STAGES == 6, "two, four, five or six LDS stages");
+    static_assert(SM_STAGES == 2 || SM_STAGES == 3 || SM_STAGES == 4 || SM_STAGES == 5 || SM_STAGES == 6, "two to six LDS stages");
     static_assert(BN_ == 128 || BN_ == 64, "tile width");
     constexpr int SM_BN = BN_;
-    constexpr int SM_STAGE_BYTES = small_stage_bytes(SM_BN);
+    constexpr int SM_BM = BM_;
+    constexpr int SM_STAGE_BYTES = small_stage_bytes(SM_BN, SM_BM);
+    constexpr int SM_TM = SM_BM / 32;                  // MFMA tiles per wave along M
+    constexpr int A_LOADS = SM_BM / 32;                // 1 KiB chunks of A per wave and stage
     constexpr int SM_TN = SM_BN / 32;                  // MFMA tiles per wave along N
     constexpr int B_LOADS = SM_BN / 32;                // 1 KiB chunks of B per wave and stage
     static_assert(MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BLOCK || MODE == MODE_MX || MODE == MODE_MXT ||
@@ -82,7 +94,7 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
     constexpr bool TILED_SCALES = MODE == MODE_MXT || MODE == MODE_F4T;
     constexpr bool STEP_SCALES = MODE == MODE_BLOCK || MODE == MODE_MX || MODE == MODE_F4 || TILED_SCALES;      // scales that change with the K step
     constexpr bool IS_F4 = MODE == MODE_F4T || MODE == MODE_F4;      // packed E2M1 operands
-    constexpr int SM_SCALE_BYTES = small_scale_bytes(MODE);
+    constexpr int SM_SCALE_BYTES = small_scale_bytes(MODE, SM_BM);
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -103,24 +115,32 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
     const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(a_base, (uint32_t)(p.m - 1) * p.lda + p.k);
     const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(b_base, b_extent_bytes(p));
 
-    // ---- global -> LDS.  A stage holds 16 A chunks then 16 (or 8) B chunks of 1 KiB (8 rows x 128 B); wave w
+    // ---- global -> LDS.  A stage holds 16 (or 32) A chunks then 16 (or 8) B chunks of 1 KiB (8 rows x 128 B); wave w
     // fills chunks w, w+4, .. of each matrix.  Lane i of a load lands on row i/8, slot i%8 of its
     // chunk and therefore fetches K-piece slot ^ (row & 7) = (i%8) ^ (i/8).
     const int ld_row = wave * 8 + (lane >> 3);
     const int ld_piece16 = ((lane & 7) ^ (lane >> 3)) * 16;
-    int voff_a[4], voff_b[B_LOADS];
+    // (256-row tiles: one lane offset per operand, the 32 j rows are scalar; rows past the end read as zero or as another
+    // row inside the descriptor and only reach accumulators that are never stored)
+    int voff_a[TALL ? 1 : A_LOADS], voff_b[TALL ? 1 : B_LOADS];
+    if constexpr (TALL) {
+        voff_a[0] = (m0 + ld_row) * p.lda + ld_piece16;
+        voff_b[0] = b_lane_offset(p, n0 + ld_row, ld_piece16);
+    } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) voff_a[j] = min(m0 + ld_row + 32 * j, p.m - 1) * p.lda + ld_piece16;
+        for (int j = 0; j < A_LOADS; ++j) voff_a[j] = min(m0 + ld_row + 32 * j, p.m - 1) * p.lda + ld_piece16;
 #pragma unroll
-    for (int j = 0; j < B_LOADS; ++j) voff_b[j] = b_lane_offset(p, min(n0 + ld_row + 32 * j, p.n - 1), ld_piece16);
+        for (int j = 0; j < B_LOADS; ++j) voff_b[j] = b_lane_offset(p, min(n0 + ld_row + 32 * j, p.n - 1), ld_piece16);
+    }
     // the lane's piece of the last, partial K step lies past k: out of every descriptor's range (an extent is below 2^31)
     const int past_k = RAGGED && (nk - 1) * BK + ld_piece16 >= p.k ? (int)0x80000000u : 0;
     auto lane_offset = [&](int voff, int kstep) __attribute__((always_inline)) { return RAGGED ? voff | (kstep == nk - 1 ? past_k : 0) : voff; };
     // block mode: waves 0 and 1 fetch the step's 128 A-row scales (64 each), waves 2 and 3 the B scale
     // of the tile's 128 x 128 block (every lane the same dword: the stage's copy at +512 is the one read)
-    constexpr int LOADS_PER_STAGE = 4 + B_LOADS + (MODE == MODE_F4 ? 2 : STEP_SCALES ? 1 : 0);
-    __amdgpu_buffer_rsrc_t rsrc_sf = rsrc_a;
-    int voff_sf = 0, sf_step_bytes = 0;
+    constexpr int SF_LOADS = !STEP_SCALES ? 0 : TALL && !TILED_SCALES ? (MODE == MODE_F4 ? 4 : 2) : MODE == MODE_F4 ? 2 : 1;
+    constexpr int LOADS_PER_STAGE = A_LOADS + B_LOADS + SF_LOADS;
+    __amdgpu_buffer_rsrc_t rsrc_sf = rsrc_a, rsrc_sf_b = rsrc_a;      // (the second one: 256-row tiles, B's scales)
+    int voff_sf = 0, voff_sf_b = 0, sf_step_bytes = 0;
     if constexpr (MODE == MODE_BLOCK) {
         if (wave < 2) {
             rsrc_sf = make_rsrc(sfa_f, (uint32_t)((nk - 1) * p.stride_sfa + p.m) * 4u);
@@ -135,7 +155,15 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
     // MX: waves 0 and 1 fetch the step's dword (four E8M0 bytes, one per 32 of K) of 64 A rows each, waves 2
     // and 3 those of 64 B rows each
     // (packed E2M1 operands: p.k counts bytes, a row has p.k / 16 scale bytes, eight per K step, fetched as two dwords)
-    if constexpr (MODE == MODE_MX || MODE == MODE_F4) {
+    if constexpr (TALL && (MODE == MODE_MX || MODE == MODE_F4)) {
+        // 256-row tiles: every wave fetches those of 64 A rows, and of 64 B rows (waves 2 and 3 the same as 0 and 1)
+        const uint32_t row_bytes = MODE == MODE_F4 ? p.k >> 4 : p.k >> 5;
+        rsrc_sf = make_rsrc((const uint8_t*)p.sfa + (long long)batch * p.sfa_batch, (uint32_t)(p.m - 1) * p.stride_sfa + row_bytes);
+        rsrc_sf_b = make_rsrc((const uint8_t*)p.sfb + (long long)batch * p.sfb_batch, (uint32_t)(p.n - 1) * p.stride_sfb + row_bytes);
+        voff_sf = min(m0 + wave * 64 + lane, p.m - 1) * p.stride_sfa;
+        voff_sf_b = min(n0 + (wave & 1) * 64 + lane, p.n - 1) * p.stride_sfb;
+        sf_step_bytes = MODE == MODE_F4 ? 8 : 4;
+    } else if constexpr (MODE == MODE_MX || MODE == MODE_F4) {
         const bool is_b = wave >= 2;
         const int rows = is_b ? p.n : p.m;
         const int stride = is_b ? p.stride_sfb : p.stride_sfa;
@@ -157,26 +185,44 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
         voff_sf = lane * 16;
         mxt_nblk = (rows + 63) >> 6;
         // (a block past the last row: its rows are never stored; a 64-wide tile has one B block, wave 3 brings the next along unused)
-        mxt_blk = min(((is_b ? n0 : m0) >> 6) + (wave & 1), mxt_nblk - 1);
+        if constexpr (TALL) {
+            // 256-row tiles: waves 0 and 1 fetch two units of A each, wave 2 (and 3 once more) the two of B, one per 32 lanes
+            const int blk = min(((is_b ? n0 : m0) >> 6) + (is_b ? 0 : 2 * wave) + (lane >> 5), mxt_nblk - 1);
+            voff_sf = blk * 1024 + (lane & 31) * 16;
+            mxt_blk = 0;
+        } else
+            mxt_blk = min(((is_b ? n0 : m0) >> 6) + (wave & 1), mxt_nblk - 1);
     }
-    auto issue_stage = [&](int stage, int kstep) __attribute__((always_inline)) {
-        kstep = min(kstep, nk - 1);         // past the end: reload the last step into a stage nobody reads (fixed wait counts)
-        A8W8_LDS char* s = (A8W8_LDS char*)smem + stage * SM_STAGE_BYTES + wave * 1024;
-        const int koff = kstep * BK;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) load_to_lds_16(rsrc_a, s + j * 4096, lane_offset(voff_a[j], kstep), koff);
-#pragma unroll
-        for (int j = 0; j < B_LOADS; ++j) load_to_lds_16(rsrc_b, s + SM_BM * BK + j * 4096, lane_offset(voff_b[j], kstep), kstep << p.b_kshift);
+    // scale load n of a stage
+    auto load_scales = [&](int stage, int kstep, int n) __attribute__((always_inline)) {
         if constexpr (TILED_SCALES) {
             A8W8_LDS char* sc = (A8W8_LDS char*)smem + SM_STAGES * SM_STAGE_BYTES + stage * SM_SCALE_BYTES + wave * 1024;
             // the pair of 128-element K steps this step belongs to (FP8: two byte steps) or is (FP4: 256 elements)
             const int pair = MODE == MODE_F4T ? kstep : kstep >> 1;
             load_to_lds_16(rsrc_sf, sc, voff_sf, ((((pair >> 1) * mxt_nblk + mxt_blk) * 2 + (pair & 1)) * 512));
         } else if constexpr (STEP_SCALES) {
-            A8W8_LDS char* sc = (A8W8_LDS char*)smem + SM_STAGES * SM_STAGE_BYTES + stage * SM_SCALE_BYTES + wave * 256;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sf, sc, 4, voff_sf, kstep * sf_step_bytes, 0, 0);
-            if constexpr (MODE == MODE_F4) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sf, sc + 1024, 4, voff_sf, kstep * sf_step_bytes + 4, 0, 0);
+            A8W8_LDS char* sc = (A8W8_LDS char*)smem + SM_STAGES * SM_STAGE_BYTES + stage * SM_SCALE_BYTES + wave * 256 + n * 1024;
+            // n: 128-row tiles the step's first or second dword (A and B rows), 256-row tiles A's, then B's
+            const bool of_b = TALL && n >= SF_LOADS / 2;
+            const int dword = (TALL ? n % (SF_LOADS / 2) : n) * 4;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(of_b ? rsrc_sf_b : rsrc_sf, sc, 4, of_b ? voff_sf_b : voff_sf, kstep * sf_step_bytes + dword, 0, 0);
         }
+    };
+    auto load_a = [&](A8W8_LDS char* s, int j, int kstep) __attribute__((always_inline)) {
+        load_to_lds_16(rsrc_a, s, lane_offset(voff_a[TALL ? 0 : j], kstep), kstep * BK + (TALL ? 32 * j * p.lda : 0));
+    };
+    auto load_b = [&](A8W8_LDS char* s, int j, int kstep) __attribute__((always_inline)) {
+        load_to_lds_16(rsrc_b, s, lane_offset(voff_b[TALL ? 0 : j], kstep), (kstep << p.b_kshift) + (TALL ? 32 * j * p.ldb : 0));
+    };
+    auto issue_stage = [&](int stage, int kstep) __attribute__((always_inline)) {
+        kstep = min(kstep, nk - 1);         // past the end: reload the last step into a stage nobody reads (fixed wait counts)
+        A8W8_LDS char* s = (A8W8_LDS char*)smem + stage * SM_STAGE_BYTES + wave * 1024;
+#pragma unroll
+        for (int j = 0; j < A_LOADS; ++j) load_a(s + j * 4096, j, kstep);
+#pragma unroll
+        for (int j = 0; j < B_LOADS; ++j) load_b(s + SM_BM * BK + j * 4096, j, kstep);
+#pragma unroll
+        for (int n = 0; n < SF_LOADS; ++n) load_scales(stage, kstep, n);
     };
 
     // ---- LDS -> registers: a lane reads K-pieces g and g+4 of tile row r16; slot = piece ^ (row & 7), and
@@ -185,7 +231,7 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int slot = (g + 4 * h) ^ (lane & 7);
-        rd_a[h] = (wave_m * 64 + r16) * BK + (slot << 4);
+        rd_a[h] = (wave_m * (SM_BM / 2) + r16) * BK + (slot << 4);
         rd_b[h] = SM_BM * BK + (wave_n * (SM_BN / 2) + r16) * BK + (slot << 4);
     }
     auto read_frag = [&](int stage, const int (&base)[2], int t) __attribute__((always_inline)) -> v8i {
@@ -199,7 +245,10 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
     // block's unit, without s (see mx_tiled_index); the same for A tiles and B tiles
     // (a 64-wide tile lies inside one 64-row block of B: wave column 1 owns the block's MFMA tiles 2 and 3)
     int mxt_off[4], mxt_off_b[SM_TN];
-    const int mxt_unit_b = SM_BN == 128 ? (2 + wave_n) * 1024 : 2 * 1024;     // where the wave's B block lies in the stage's scale bytes
+    // where the unit of A tile t's 64-row block, and the wave's B block, lie in the stage's scale bytes
+    auto mxt_unit_a = [&](int t) __attribute__((always_inline)) { return TALL ? wave_m * 1024 + (t >> 2) * 512 : wave_m * 1024; };
+    const int mxt_unit_b = TALL ? 2048 + wave_n * 512 : SM_BN == 128 ? (2 + wave_n) * 1024 : 2 * 1024;
+    constexpr int SF_B_ROW0 = TALL ? (MODE == MODE_F4 ? 512 : 256) : 128;      // dword of B's first row in the row-major scale bytes
     if constexpr (TILED_SCALES) {
         auto unit_offset = [&](int t) __attribute__((always_inline)) {
             const int x = (2 * t + (r16 >> 3)) & 3, y = r16 & 3, par = (r16 >> 2) & 1;
@@ -211,14 +260,18 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
         for (int t = 0; t < SM_TN; ++t) mxt_off_b[t] = unit_offset(SM_BN == 128 ? t : 2 * wave_n + t);
     }
 
-    const int cm_base = m0 + wave_m * 64 + r16;          // + 16 * i
+    const int cm_base = m0 + wave_m * (SM_BM / 2) + r16;          // + 16 * i
     const int cn_base = n0 + wave_n * (SM_BN / 2) + 4 * g;        // + 16 * j + e
 
-    v4f acc[SM_TM][SM_TN];
+    v4f acc[SM_TM][SM_TN];      // (256-row tiles: filled from the accumulation registers behind the K loop)
+    if constexpr (!TALL) {
 #pragma unroll
-    for (int i = 0; i < SM_TM; ++i)
+        for (int i = 0; i < SM_TM; ++i)
 #pragma unroll
-        for (int j = 0; j < SM_TN; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < SM_TN; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    } else {
+        asm volatile("" ::: "a0", "a255");      // sizes the wave's register allocation: the compiler has no accumulation registers to itself
+    }
 
     // Deep staging: the step's three instruction streams overlap inside the one wave of a SIMD.  The fragments (and
     // scales) of step ks + 1 are read from LDS while the MFMAs of step ks run (two register sets, the loop unrolled by
@@ -231,7 +284,7 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
     // ks + 2) between them; the other workgroup's MFMAs run beside this one's LDS reads.
     constexpr bool TWO = SM_STAGES == 2;
     constexpr bool PIPELINED = TWO ? A8W8_SMALL_PIPELINED_TWO != 0 : A8W8_SMALL_PIPELINED != 0;
-    static_assert(PIPELINED || !RAGGED, "partial K steps exist in the overlapped loop only");
+    static_assert(PIPELINED || (!RAGGED && !TALL), "partial K steps and 256-row tiles exist in the overlapped loop only");
     if constexpr (PIPELINED) {
         constexpr int HALVES = BY_BF16 ? 4 : (IS_F4 || MODE == MODE_BF16) ? 2 : 1;      // MFMAs per pair of fragments
         constexpr int NFRAG = SM_TM + SM_TN, NSLOT = SM_TM * SM_TN * HALVES, NLOAD = LOADS_PER_STAGE;
@@ -255,9 +308,9 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
                 // lane (r16, g) scales K [32g, 32g+32) of its row: byte g of the row's dword
                 const unsigned* w = (const unsigned*)sc;
 #pragma unroll
-                for (int t = 0; t < SM_TM; ++t) sa[t] = (int)__builtin_amdgcn_ubfe(w[wave_m * 64 + 16 * t + r16], 8 * g, 8);
+                for (int t = 0; t < SM_TM; ++t) sa[t] = (int)__builtin_amdgcn_ubfe(w[wave_m * (SM_BM / 2) + 16 * t + r16], 8 * g, 8);
 #pragma unroll
-                for (int t = 0; t < SM_TN; ++t) sb[t] = (int)__builtin_amdgcn_ubfe(w[128 + wave_n * (SM_BN / 2) + 16 * t + r16], 8 * g, 8);
+                for (int t = 0; t < SM_TN; ++t) sb[t] = (int)__builtin_amdgcn_ubfe(w[SF_B_ROW0 + wave_n * (SM_BN / 2) + 16 * t + r16], 8 * g, 8);
             }
             if constexpr (MODE == MODE_F4) {
                 // lane (r16, g) scales 32-block g of each 128-element half of its row: byte g of the row's first and of
@@ -267,21 +320,21 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
                     return (int)(__builtin_amdgcn_ubfe(w[row], 8 * g, 8) | (__builtin_amdgcn_ubfe(w[256 + row], 8 * g, 8) << 8));
                 };
 #pragma unroll
-                for (int t = 0; t < SM_TM; ++t) sa[t] = two_bytes(wave_m * 64 + 16 * t + r16);
+                for (int t = 0; t < SM_TM; ++t) sa[t] = two_bytes(wave_m * (SM_BM / 2) + 16 * t + r16);
 #pragma unroll
-                for (int t = 0; t < SM_TN; ++t) sb[t] = two_bytes(128 + wave_n * (SM_BN / 2) + 16 * t + r16);
+                for (int t = 0; t < SM_TN; ++t) sb[t] = two_bytes(SF_B_ROW0 + wave_n * (SM_BN / 2) + 16 * t + r16);
             }
             if constexpr (MODE == MODE_F4T) {
                 // both halves' bytes sit side by side: one 16-bit read, the half is chosen by op_sel
 #pragma unroll
-                for (int t = 0; t < SM_TM; ++t) sa[t] = *(const unsigned short*)(sc + wave_m * 1024 + mxt_off[t]);
+                for (int t = 0; t < SM_TM; ++t) sa[t] = *(const unsigned short*)(sc + mxt_unit_a(t) + mxt_off[t & 3]);
 #pragma unroll
                 for (int t = 0; t < SM_TN; ++t) sb[t] = *(const unsigned short*)(sc + mxt_unit_b + mxt_off_b[t]);
             }
             if constexpr (MODE == MODE_MXT) {
                 const uint8_t* u = (const uint8_t*)sc + (ks & 1);
 #pragma unroll
-                for (int t = 0; t < SM_TM; ++t) sa[t] = u[wave_m * 1024 + mxt_off[t]];
+                for (int t = 0; t < SM_TM; ++t) sa[t] = u[mxt_unit_a(t) + mxt_off[t & 3]];
 #pragma unroll
                 for (int t = 0; t < SM_TN; ++t) sb[t] = u[mxt_unit_b + mxt_off_b[t]];
             }
@@ -294,23 +347,16 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
             const v2bf x3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)f[2 * h + 1], 1.0f, true);
             return v8bf{x0[0], x0[1], x1[0], x1[1], x2[0], x2[1], x3[0], x3[1]};
         };
-        // load n of a stage: four chunks of A, the chunks of B, then the step's scales
+        // load n of a stage: the chunks of A, the chunks of B, then the step's scales
         auto load_one = [&](int stage, int kstep, int n) __attribute__((always_inline)) {
             A8W8_LDS char* s = (A8W8_LDS char*)smem + stage * SM_STAGE_BYTES + wave * 1024;
-            if (n < 4) load_to_lds_16(rsrc_a, s + n * 4096, lane_offset(voff_a[n], kstep), kstep * BK);
-            else if (n < 4 + B_LOADS) load_to_lds_16(rsrc_b, s + SM_BM * BK + (n - 4) * 4096, lane_offset(voff_b[n - 4], kstep), kstep << p.b_kshift);
-            else if constexpr (TILED_SCALES) {
-                A8W8_LDS char* sc = (A8W8_LDS char*)smem + SM_STAGES * SM_STAGE_BYTES + stage * SM_SCALE_BYTES + wave * 1024;
-                const int pair = MODE == MODE_F4T ? kstep : kstep >> 1;
-                load_to_lds_16(rsrc_sf, sc, voff_sf, ((((pair >> 1) * mxt_nblk + mxt_blk) * 2 + (pair & 1)) * 512));
-            } else if constexpr (STEP_SCALES) {
-                A8W8_LDS char* sc = (A8W8_LDS char*)smem + SM_STAGES * SM_STAGE_BYTES + stage * SM_SCALE_BYTES + wave * 256;
-                if (n == 4 + B_LOADS) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sf, sc, 4, voff_sf, kstep * sf_step_bytes, 0, 0);
-                else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sf, sc + 1024, 4, voff_sf, kstep * sf_step_bytes + 4, 0, 0);
-            }
+            if (n < A_LOADS) load_a(s + n * 4096, n, kstep);
+            else if (n < A_LOADS + B_LOADS) load_b(s + SM_BM * BK + (n - A_LOADS) * 4096, n - A_LOADS, kstep);
+            else load_scales(stage, kstep, n - A_LOADS - B_LOADS);
         };
 #pragma unroll
         for (int st = 0; st < SM_STAGES; ++st) issue_stage(st, st);
+        if constexpr (TALL) static_for<SM_TM * SM_TN * 4>([&](auto I) { acc_zero<decltype(I)::value>(); });
         if constexpr (!TWO) {
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SM_STAGES - 1) * NLOAD) : "memory");
             A8W8_RAW_BARRIER();
@@ -337,6 +383,31 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             A8W8_RAW_BARRIER();
             const int kload = min(ks + SM_STAGES, nk - 1);      // past the end: the last step again, into a stage nobody reads
+            if constexpr (TALL) {
+                // the same order with the accumulators named: a column of eight tiles (two halves of it) at a time
+                static_for<NSLOT>([&](auto T) {
+                    constexpr int t = decltype(T)::value;
+                    constexpr int i = t % SM_TM, h = (t / SM_TM) % HALVES, j = t / (SM_TM * HALVES), lo = 4 * (i * SM_TN + j);
+                    const v8i& fb = have[SM_TM + j];
+                    const v8i& fa = have[i];
+                    if constexpr (IS_F4) {
+                        mfma_acc_f4<lo, false, h, h>(v4i{fb[4 * h], fb[4 * h + 1], fb[4 * h + 2], fb[4 * h + 3]},
+                                                     v4i{fa[4 * h], fa[4 * h + 1], fa[4 * h + 2], fa[4 * h + 3]}, sb[j], sa[i]);
+                    } else if constexpr (MODE == MODE_BF16) {
+                        mfma_acc_bf16<lo, false>(v4i{fb[4 * h], fb[4 * h + 1], fb[4 * h + 2], fb[4 * h + 3]},
+                                                 v4i{fa[4 * h], fa[4 * h + 1], fa[4 * h + 2], fa[4 * h + 3]});
+                    } else if constexpr (MODE == MODE_MX || MODE == MODE_MXT) {
+                        mfma_acc_mx<lo, false, 0, 0>(fb, fa, sb[j], sa[i]);
+                    } else {
+                        mfma_acc<lo, false>(fb, fa);
+                    }
+                    if constexpr (t % LOAD_EVERY == 0 && t / LOAD_EVERY < NLOAD) load_one(stage, kload, t / LOAD_EVERY);
+                    if constexpr (t % READ_EVERY == 0 && t / READ_EVERY < NFRAG) next[t / READ_EVERY] = read_one(next_stage, t / READ_EVERY);
+                    if constexpr (t == 0) read_scales(next_stage, ks + 1, next_sa, next_sb);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                return next_stage;
+            }
             v4f part[BLK_LAG + 1];
             v8bf quarter[BY_BF16 ? 2 : 1][NFRAG];
             if constexpr (BY_BF16) {
@@ -408,6 +479,13 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
             }
             if (ks < nk) step(ks, stage, fr[0], sc_a[0], sc_b[0], fr[1], sc_a[1], sc_b[1]);
         }
+        if constexpr (TALL) {
+            asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // last MFMA -> first accumulator read
+            static_for<SM_TM * SM_TN>([&](auto IJ) {
+                constexpr int ij = decltype(IJ)::value;
+                static_for<4>([&](auto E) { acc[ij / SM_TN][ij % SM_TN][decltype(E)::value] = acc_read<4 * ij + decltype(E)::value>(); });
+            });
+        }
     } else {
     issue_stage(0, 0);
     issue_stage(1, 1);
@@ -473,9 +551,9 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
                     return (int)(__builtin_amdgcn_ubfe(sc[row], 8 * g, 8) | (__builtin_amdgcn_ubfe(sc[256 + row], 8 * g, 8) << 8));
                 };
 #pragma unroll
-                for (int t = 0; t < SM_TM; ++t) mx_sa[t] = two_bytes(wave_m * 64 + 16 * t + r16);
+                for (int t = 0; t < SM_TM; ++t) mx_sa[t] = two_bytes(wave_m * (SM_BM / 2) + 16 * t + r16);
 #pragma unroll
-                for (int t = 0; t < SM_TN; ++t) mx_sb[t] = two_bytes(128 + wave_n * (SM_BN / 2) + 16 * t + r16);
+                for (int t = 0; t < SM_TN; ++t) mx_sb[t] = two_bytes(SF_B_ROW0 + wave_n * (SM_BN / 2) + 16 * t + r16);
             }
             if constexpr (MODE == MODE_F4T) {
                 // both halves' bytes sit side by side: one 16-bit read, the half is chosen by op_sel
@@ -579,7 +657,7 @@ __global__ void __launch_bounds__(SM_THREADS, 2) gemm_a8w8_tile128(GemmParams p)
         char* mine = smem + wave * (16 * (SM_BN / 2 * 4 + 16));
         const int wr = r16 * ROW_PITCH + 4 * g * ES;              // + 16 j ES: the lane's four values of MFMA tile j
         const int rd = (lane / LANES_PER_ROW) * ROW_PITCH + (lane % LANES_PER_ROW) * 16;      // + ROWS_PER_STORE rows per store
-        char* c_wave = c_base + ((long long)(m0 + wave_m * 64) * p.ldc + n0 + wave_n * (SM_BN / 2)) * ES;
+        char* c_wave = c_base + ((long long)(m0 + wave_m * (SM_BM / 2)) * p.ldc + n0 + wave_n * (SM_BN / 2)) * ES;
         const long long row_bytes = (long long)p.ldc * ES;
         float sb_all[SM_TN][4];
         if constexpr (MODE == MODE_ROWCOL) {

@@ -78,67 +78,6 @@ constexpr int wide_lds_bytes(int mode)
     return GEMM_LDS_BYTES + ((mode == MODE_MXT || mode == MODE_F4T || mode == MODE_F4) ? 4 * MX_GROUP_BYTES : mode == MODE_ROWCOL ? 2 * ROWCOL_SCALE_BYTES : 0);
 }
 
-// The 64 accumulator tiles of a wave live in accumulator registers a[0:255], tile (i, j) in
-// a[4 (8i + j) : +3].  They are named in assembly statements only and never appear as variables: the
-// compiler allocates nothing there (its own registers stay below 256, which the build checks), so no
-// copy, spill or re-materialisation can come between two MFMAs of one tile.  The statements keep
-// their order; the compiler does not see the MFMAs' latency, so the code that reads an accumulator
-// makes sure that enough instructions separate it from the last MFMA into that tile.
-template <int N, class F, int... I>
-A8W8_DEV void static_for_impl(F&& f, std::integer_sequence<int, I...>)
-{
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-A8W8_DEV void static_for(F&& f)
-{
-    static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
-}
-
-// tile LO/4 += a . b, or = a . b when ZC (the tile's first K step)
-template <int LO, bool ZC>
-A8W8_DEV void mfma_acc(const v8i& a, const v8i& b)
-{
-    if constexpr (ZC) asm volatile("v_mfma_f32_16x16x128_f8f6f4 a[%2:%3], %0, %1, 0" ::"v"(a), "v"(b), "n"(LO), "n"(LO + 3));
-    else asm volatile("v_mfma_f32_16x16x128_f8f6f4 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(a), "v"(b), "n"(LO), "n"(LO + 3));
-}
-// the same with E8M0 block scales: byte OA of sa scales a's K block of the lane, byte OB of sb b's
-template <int LO, bool ZC, int OA, int OB>
-A8W8_DEV void mfma_acc_mx(const v8i& a, const v8i& b, int sa, int sb)
-{
-    if constexpr (ZC)
-        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 a[%4:%5], %0, %1, 0, %2, %3 op_sel:[%6,%7,0] op_sel_hi:[%8,%9,0]" ::"v"(a),
-                     "v"(b), "v"(sa), "v"(sb), "n"(LO), "n"(LO + 3), "n"(OA & 1), "n"(OB & 1), "n"(OA >> 1), "n"(OB >> 1));
-    else
-        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 a[%4:%5], %0, %1, a[%4:%5], %2, %3 op_sel:[%6,%7,0] op_sel_hi:[%8,%9,0]" ::"v"(a),
-                     "v"(b), "v"(sa), "v"(sb), "n"(LO), "n"(LO + 3), "n"(OA & 1), "n"(OB & 1), "n"(OA >> 1), "n"(OB >> 1));
-}
-// bf16 operands: one 16 x 16 x 32 MFMA per 16-byte half of a fragment
-template <int LO, bool ZC>
-A8W8_DEV void mfma_acc_bf16(const v4i& a, const v4i& b)
-{
-    if constexpr (ZC) asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, 0" ::"v"(a), "v"(b), "n"(LO), "n"(LO + 3));
-    else asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(a), "v"(b), "n"(LO), "n"(LO + 3));
-}
-// packed E2M1 operands (format 4 for both): one 16 x 16 x 128 MFMA per 16-byte half of a fragment
-template <int LO, bool ZC, int OA, int OB>
-A8W8_DEV void mfma_acc_f4(const v4i& a, const v4i& b, int sa, int sb)
-{
-    if constexpr (ZC)
-        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 a[%4:%5], %0, %1, 0, %2, %3 op_sel:[%6,%7,0] op_sel_hi:[%8,%9,0] cbsz:4 blgp:4" ::"v"(a),
-                     "v"(b), "v"(sa), "v"(sb), "n"(LO), "n"(LO + 3), "n"(OA & 1), "n"(OB & 1), "n"(OA >> 1), "n"(OB >> 1));
-    else
-        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 a[%4:%5], %0, %1, a[%4:%5], %2, %3 op_sel:[%6,%7,0] op_sel_hi:[%8,%9,0] cbsz:4 blgp:4" ::"v"(a),
-                     "v"(b), "v"(sa), "v"(sb), "n"(LO), "n"(LO + 3), "n"(OA & 1), "n"(OB & 1), "n"(OA >> 1), "n"(OB >> 1));
-}
-template <int IDX>
-A8W8_DEV float acc_read()
-{
-    float x;
-    asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(x) : "n"(IDX));
-    return x;
-}
-
 template <int MODE, int CDT>
 __global__ void __launch_bounds__(WIDE_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gemm_a8w8_wide(PersistParams pp)
