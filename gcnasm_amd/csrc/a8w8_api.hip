@@ -216,7 +216,7 @@ bool tiled_ok(const a8w8_gemm_args* g)
 // Rows of whole 16-byte pieces whose length is no multiple of the 128-byte K step: the 128-tile kernel with a partial last
 // step (scales that do not change with K; k in bytes here).  It is the faster one at any size, since the one-thread-per-element
 // kernel takes 86 ns per K element however small the problem (128 x 256 x 240: 20.9 us against 5.4, 1000 x 3000 x 2000: 7545
-// against 21, 4096 x 4096 x 4080: 84 ms against 0.116); problems of a few rows, columns and K elements, where that is no more
+// against 18.5, 4096 x 4096 x 4080: 84 ms against 0.116); problems of a few rows, columns and K elements, where that is no more
 // than a launch or two, stay there, in the order of operations of the CPU reference.
 constexpr int RAGGED_MIN_K_BYTES = 256;
 constexpr long long RAGGED_MIN_MACS = 1ll << 19;

@@ -62,9 +62,10 @@ constexpr int small_lds_bytes(int mode, int stages, int bn = SM_BN, int bm = SM_
 // operands then run on the bf16 MFMA: the one-thread-per-element kernel that took these shapes before adds products in
 // fp32 one after the other, and the FP8 MFMA, which aligns its products to the largest one, is about 40 times less
 // precise than that (1.4e-5 against 8e-8 of the result in norm over K = 4096 normal data), while E4M3 -> bf16 is exact
-// and the bf16 MFMA keeps fp32 sums (8e-8).  A K step is four quarters of 32 elements; the fragments of the next quarter
-// are converted between the MFMAs of this one.  Half the MFMA rate, and still bound by it.
-// 1000 x 3000 x 2000 row/col: 7545 us on the one-thread-per-element kernel, 21 us here; 4096 x 4096 x 4080: 1.2 PFLOP/s.
+// and the bf16 MFMA keeps fp32 sums (8e-8).  A K step is four quarters of 32 elements; the fragments of the next quarter,
+// behind the last one those of the next step's first, are converted two instructions per MFMA (in bursts, with the first
+// quarter in front of the step's MFMAs: 1024 x 3072 x 2000 19.6 us, 16.9 this way).  Half the MFMA rate, and still bound by it.
+// 1000 x 3000 x 2000 row/col: 7545 us on the one-thread-per-element kernel, 18.5 us here; 4096 x 4096 x 4080: 1.2 PFLOP/s.
 // BM_ = 256: 256 x 128 tiles, a wave owns 128 x 64 (accumulators in named accumulation registers, one wave per SIMD, three stages
 // of 48 KiB), for grids that would need two workgroups per compute unit on 128 x 128 tiles but fit at one per compute unit here.
 // A 64 x 64 wave tile reads 16 KiB of LDS per 16 MFMAs and the loads write another 8: as many cycles as the MFMAs take, so
@@ -288,7 +289,9 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
     if constexpr (PIPELINED) {
         constexpr int HALVES = BY_BF16 ? 4 : (IS_F4 || MODE == MODE_BF16) ? 2 : 1;      // MFMAs per pair of fragments
         constexpr int NFRAG = SM_TM + SM_TN, NSLOT = SM_TM * SM_TN * HALVES, NLOAD = LOADS_PER_STAGE;
-        constexpr int LOAD_EVERY = NSLOT / NLOAD, READ_EVERY = NSLOT / NFRAG;
+        constexpr int LOAD_EVERY = NSLOT / NLOAD;
+        // converted operands: the next step's first quarter is converted behind this step's last MFMAs, so its fragments come in the first half
+        constexpr int READ_EVERY = BY_BF16 && !TWO ? NSLOT / (2 * NFRAG) : NSLOT / NFRAG;
         constexpr int BLK_LAG = MODE == MODE_BLOCK ? 4 : 0;
         static_assert(LOAD_EVERY >= 1 && READ_EVERY >= 1 && (SM_STAGES - 1) * NLOAD < 64, "the wait count is a 6-bit field");
         v8i fr[TWO ? 1 : 2][NFRAG];       // A tiles, then B tiles
@@ -347,6 +350,13 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
             const v2bf x3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)f[2 * h + 1], 1.0f, true);
             return v8bf{x0[0], x0[1], x1[0], x1[1], x2[0], x2[1], x3[0], x3[1]};
         };
+        // half `part` (two of the four conversions) of the same
+        auto half_quarter = [&](v8bf& q, const v8i& f, int h, int part) __attribute__((always_inline)) {
+            const v2bf x0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)f[2 * h + part], 1.0f, false);
+            const v2bf x1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((unsigned)f[2 * h + part], 1.0f, true);
+            q[4 * part] = x0[0]; q[4 * part + 1] = x0[1]; q[4 * part + 2] = x1[0]; q[4 * part + 3] = x1[1];
+        };
+        v8bf quarter[BY_BF16 ? 2 : 1][NFRAG];      // converted operands: the quarter in use and the next one
         // load n of a stage: the chunks of A, the chunks of B, then the step's scales
         auto load_one = [&](int stage, int kstep, int n) __attribute__((always_inline)) {
             A8W8_LDS char* s = (A8W8_LDS char*)smem + stage * SM_STAGE_BYTES + wave * 1024;
@@ -363,6 +373,10 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
 #pragma unroll
             for (int t = 0; t < NFRAG; ++t) fr[0][t] = read_one(0, t);
             read_scales(0, 0, sc_a[0], sc_b[0]);
+            if constexpr (BY_BF16) {
+#pragma unroll
+                for (int n = 0; n < NFRAG; ++n) quarter[0][n] = quarter_to_bf16(fr[0][n], 0);
+            }
         }
         // one K step: `have`, `sa`, `sb` hold its fragments and scales, the `next_` ones receive those of the step after it
         auto step = [&](int ks, int stage, v8i (&have)[NFRAG], int (&sa)[SM_TM], int (&sb)[SM_TN], v8i (&next)[NFRAG],
@@ -409,8 +423,7 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
                 return next_stage;
             }
             v4f part[BLK_LAG + 1];
-            v8bf quarter[BY_BF16 ? 2 : 1][NFRAG];
-            if constexpr (BY_BF16) {
+            if constexpr (BY_BF16 && TWO) {
 #pragma unroll
                 for (int n = 0; n < NFRAG; ++n) quarter[0][n] = quarter_to_bf16(have[n], 0);
             }
@@ -442,7 +455,15 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
                         acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb, fa, acc[i][j], 0, 0, 0, sb[j], 0, sa[i]);
                     } else if constexpr (BY_BF16) {
                         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(quarter[h & 1][SM_TM + j], quarter[h & 1][i], acc[i][j], 0, 0, 0);
-                        if (t % TILES < NFRAG && h + 1 < HALVES) quarter[(h + 1) & 1][t % TILES] = quarter_to_bf16(have[t % TILES], h + 1);
+                        // conversions of the next quarter, spread over this one's MFMAs: one half fragment per MFMA (16 tiles) or two
+                        // (8); behind the last quarter those of the next step's first one
+                        constexpr int CONV = (2 * NFRAG + TILES - 1) / TILES;
+#pragma unroll
+                        for (int u = (t % TILES) * CONV; u < (t % TILES + 1) * CONV; ++u) {
+                            if (u >= 2 * NFRAG) continue;
+                            if (h + 1 < HALVES) half_quarter(quarter[(h + 1) & 1][u >> 1], have[u >> 1], h + 1, u & 1);
+                            else if (!TWO) half_quarter(quarter[0][u >> 1], next[u >> 1], 0, u & 1);
+                        }
                     } else if constexpr (MODE == MODE_BF16) {
                         // a 128-byte row is 64 bf16: the fragment's two 16-byte halves feed one 16x16x32 MFMA each
                         const v4i bh = {fb[4 * h], fb[4 * h + 1], fb[4 * h + 2], fb[4 * h + 3]};
