@@ -479,9 +479,6 @@ int validate_flat(const a8w8_gemm_args* g)
     return A8W8_OK;
 }
 
-// Weight tiles (16 rows of B) per workgroup: the activation fragment of a K block is re-used by all of them, but
-// the grid shrinks by the same factor: the largest of 4, 2, 1 that still gives every compute unit a workgroup
-// (16 x 4096 x 4096: 8.6 us with 4 tiles per workgroup on 64 compute units, 5.4 us with 1 on 256).
 template <int NT, int MT, int CDT, int MODE, bool BROW>
 int launch_flat_nt(const GemmParams& p, int batch, hipStream_t stream)
 {
@@ -490,40 +487,44 @@ int launch_flat_nt(const GemmParams& p, int batch, hipStream_t stream)
     return launch(flatmm_a8w8<NT, MT, CDT, MODE, BROW>, grid, dim3(FLAT_THREADS), 0, stream, p);
 }
 
-// Up to four groups of 16 activation rows share one pass over the weights; as many weight tiles per workgroup as
-// still leave every compute unit a workgroup (every workgroup reads all rows of A once, so more weight tiles per
-// workgroup also means fewer reads of A: 16384 x 7168 at M = 48, 30 us with two tiles, 24 us with four).
+// Weight tiles (NT) and groups of 16 activation rows (MT) per workgroup: the smallest NT x MT whose workgroups all fit the chip
+// at once.  Every workgroup is eight waves and a chain of K pairs, reduction and store whose length grows with NT x MT, so a
+// layer of few weight tiles goes out in small pieces (row groups then read the weights once each, all but the first from L2), and
+// one of many in pieces large enough for a single round.  us, row/col / MXFP8, NT x MT before -> now:
+//   64 x 1024 x 4096     2 x 4  8.7 / 9.9   -> 1 x 1  5.2 / 6.1       100 x 1024 x 4096   2 x 8, 2 x 4  13.2 / 9.8 -> 1 x 2  5.2 / 6.0
+//   64 x 4096 x 4096     2 x 4  9.2 / 10.5  -> 2 x 2  7.1 / 8.0       100 x 4096 x 4096   2 x 8, 2 x 4  14.2 / 10.6 -> 2 x 4  9.3 / 10.6
+//   64 x 9216 x 3584     2 x 4  14.6 / 17.8 -> 4 x 4  12.8 / 13.1     128 x 8192 x 8192   2 x 8, 2 x 4  25.9 / 33.4 -> 4 x 4  23.3 / 24.2
+//   128 x 12288 x 2560   2 x 8  20.7 -> 2 x 4 in three rounds 16.2 (MXFP8: 2 x 4 17.9 before and now, 4 x 4 19.0)
+//   16 x 5120 x 5120     1 x 1  9.9 / 11.4  -> 2 x 1  8.0 / 8.7       16 x 10240 x 8192   2 x 1  19.9 / 22.5 -> 4 x 1  17.4 / 18.6
+// Four row groups share a pass at most, six where their registers allow it (MX scales do not: 4 x 4 on two passes is faster,
+// 80 x 7168 x 4096 14.6 -> 13.4).  Layers of at least four weight tiles per compute unit take four, and an even split of the row
+// groups over one or two passes (16384 x 7168 at M = 48, 30 us with two tiles, 24 us with four).
 template <int CDT, int MODE, bool BROW = false>
 int launch_flat(const GemmParams& p, int batch, hipStream_t stream)
 {
+    constexpr bool MX = MODE == MODE_MXT || MODE == MODE_F4T;
     const long long tiles = (long long)(p.n / 16) * batch;
-    const int cus = num_cus();
-    // row groups per workgroup: all of them up to four, an even split over two passes beyond
+    const long long cus = num_cus();
     const int groups = (p.m + 15) / 16, passes = (groups + 3) / 4;
     const int mt = (groups + passes - 1) / passes;
-    if (groups > 4 && tiles < 4ll * cus) {
-        // too few weight tiles for four per workgroup: two passes would run two tiles per workgroup anyway, and one
-        // pass with six or eight row groups on two tiles reads the weights once (8192 x 8192, M = 128: 30 -> 25 us)
-        if (groups <= 6) return launch_flat_nt<2, 6, CDT, MODE, BROW>(p, batch, stream);
-        // eight groups + scales would spill; with row-major weights their staging does not fit LDS
-        if constexpr (MODE != MODE_BLOCK && MODE != MODE_MXT && MODE != MODE_F4T && !BROW)
-            return launch_flat_nt<2, 8, CDT, MODE, BROW>(p, batch, stream);
+    if (tiles < 4 * cus) {
+        const auto fits = [&](int nt, int m) { return ((p.n / 16 + nt - 1) / nt) * (long long)batch * ((groups + m - 1) / m) <= cus; };
+        if (fits(1, 1)) return launch_flat_nt<1, 1, CDT, MODE, BROW>(p, batch, stream);
+        if (groups == 1 && fits(2, 1)) return launch_flat_nt<2, 1, CDT, MODE, BROW>(p, batch, stream);
+        if (groups > 1 && fits(1, 2)) return launch_flat_nt<1, 2, CDT, MODE, BROW>(p, batch, stream);
+        if (groups > 1 && fits(2, 2)) return launch_flat_nt<2, 2, CDT, MODE, BROW>(p, batch, stream);
+        if (groups > 2 && fits(2, 3)) return launch_flat_nt<2, 3, CDT, MODE, BROW>(p, batch, stream);
+        if (groups > 2 && (fits(2, 4) || (groups > 6 && !fits(4, 4)))) return launch_flat_nt<2, 4, CDT, MODE, BROW>(p, batch, stream);
+        if constexpr (!MX) {
+            if (groups > 4 && groups <= 6) return launch_flat_nt<2, 6, CDT, MODE, BROW>(p, batch, stream);
+        }
+        if (groups > 4) return launch_flat_nt<4, 4, CDT, MODE, BROW>(p, batch, stream);
+        // up to four groups, more than two and less than four weight tiles per compute unit: four tiles below
     }
-    if (mt == 4) {
-        if (tiles >= 4ll * cus) return launch_flat_nt<4, 4, CDT, MODE, BROW>(p, batch, stream);
-        return launch_flat_nt<2, 4, CDT, MODE, BROW>(p, batch, stream);
-    }
-    if (mt == 3) {
-        if (tiles >= 4ll * cus) return launch_flat_nt<4, 3, CDT, MODE, BROW>(p, batch, stream);
-        return launch_flat_nt<2, 3, CDT, MODE, BROW>(p, batch, stream);
-    }
-    if (mt == 2) {
-        if (tiles >= 4ll * cus) return launch_flat_nt<4, 2, CDT, MODE, BROW>(p, batch, stream);
-        return launch_flat_nt<2, 2, CDT, MODE, BROW>(p, batch, stream);
-    }
-    if (tiles >= 4ll * cus) return launch_flat_nt<4, 1, CDT, MODE, BROW>(p, batch, stream);
-    if (tiles >= 2ll * cus) return launch_flat_nt<2, 1, CDT, MODE, BROW>(p, batch, stream);
-    return launch_flat_nt<1, 1, CDT, MODE, BROW>(p, batch, stream);
+    if (mt == 4) return launch_flat_nt<4, 4, CDT, MODE, BROW>(p, batch, stream);
+    if (mt == 3) return launch_flat_nt<4, 3, CDT, MODE, BROW>(p, batch, stream);
+    if (mt == 2) return launch_flat_nt<4, 2, CDT, MODE, BROW>(p, batch, stream);
+    return launch_flat_nt<4, 1, CDT, MODE, BROW>(p, batch, stream);
 }
 
 // On shuffled weights both the flat GEMM and the MFMA kernels can run a skinny problem; the entry points take the
@@ -538,9 +539,9 @@ int launch_flat(const GemmParams& p, int batch, hipStream_t stream)
 // Weights of at most 32 MiB always go flat.  Measured on MI355X, shuffled FP8 weights, M = 16 / 32 / 48 / 64 / 80 / 96 /
 // 128, flat against dense:
 //   16384 x 7168   20 / 21 / 23 / 24 / 35 / 36 / 41  against  30 / 27 / 27 / 28 / 30 / 31 / 33   (MXFP8 about 10% more on both sides)
-//   8192 x 8192    13 / 14 / 16 / 18 / 20 / 21 / 26  against  26 / 26 / 26 / 27 / 28 / 29 / 31
+//   8192 x 8192    13 / 14 / 16 / 18 / 21 / 22 / 23  against  26 / 26 / 26 / 27 / 28 / 29 / 31
 //   28672 x 4096   20 / 23 / 25 / 28 / 39 / 41 / 47  against  26 / 26 / 27 / 28 / 29 / 30 / 31
-//   4096 x 14336   13 / 19 / 23 / 26 / 31 / 32 / 38  against  41 throughout
+//   4096 x 14336   13 / .. / .. / 19 / 23 / .. / 27  against  41 throughout
 // (tests/test_zz_gpu_routing.py times both sides of such cells through a8w8_route_override and checks the choice).
 // Row-major weights (a8w8_gemm without b_preshuffled; the flat kernel stages the weight rows through LDS, whole lines
 // per load): as fast as shuffled ones unless the rows are a large power of two apart, where the 16 rows of a tile fall
@@ -548,7 +549,7 @@ int launch_flat(const GemmParams& p, int batch, hipStream_t stream)
 // (13 / 14 / 18 shuffled).
 int g_route = A8W8_ROUTE_MODEL;      // a8w8_route_override
 
-bool prefer_flat(int m, int n, long long row_bytes, bool scaled_in_loop, double layout_factor = 1.0)
+bool prefer_flat(int m, int n, long long row_bytes, double layout_factor = 1.0)
 {
     if (g_route != A8W8_ROUTE_MODEL) return g_route == A8W8_ROUTE_FLAT;
     const double w = (double)n * (double)row_bytes;
@@ -561,11 +562,11 @@ bool prefer_flat(int m, int n, long long row_bytes, bool scaled_in_loop, double 
     // workgroup reads again for its NT weight tiles (n * row_bytes / NT bytes from L2) and their MFMAs; nearly twice
     // that where the workgroups do not fit the chip at once
     const long long tiles = n / 16;
-    const int nt = tiles >= 4ll * cus ? 4 : tiles >= 2ll * cus ? 2 : 1;
+    const int nt = tiles >= 4ll * cus || (groups <= 4 && tiles > 2ll * cus) ? 4 : tiles > cus ? 2 : 1;      // (as launch_flat chooses)
     const double per_group = w / nt / 21.0e6 * (tiles / nt > cus ? 1.9 : 1.0);
     double flat = 1.5 + w / 6.4e6;
-    if (groups > 4 && tiles < 4ll * cus && (groups <= 6 || !scaled_in_loop)) {
-        flat += per_group * (groups - 1);      // one pass with six or eight row groups (see launch_flat)
+    if (groups > 4 && tiles < 4ll * cus) {
+        flat += per_group * (groups - 1);      // six row groups in one pass, or four weight tiles per workgroup (see launch_flat)
     } else {
         flat += per_group * (mt - 1);
         if (passes == 2) flat *= 1.55;      // the second pass reads the weights from L2
@@ -581,10 +582,10 @@ bool prefer_flat(int m, int n, long long row_bytes, bool scaled_in_loop, double 
 
 bool prefer_flat_fp8(const a8w8_gemm_args* g)
 {
-    const bool scaled_in_loop = g->scale_mode == A8W8_SCALE_MX_E8M0_TILED;      // no kernel with eight row groups
+    const bool mx = g->scale_mode == A8W8_SCALE_MX_E8M0_TILED;
     const double layout_factor = g->b_preshuffled ? 1.0 : g->stride_b % 4096 == 0 ? 1.3 : 1.05;
     // (the flat kernel's MX scale bytes, one byte load per weight tile and K pair, cost it about a tenth)
-    return prefer_flat(g->m, g->n, g->k, scaled_in_loop, layout_factor * (scaled_in_loop ? 1.1 : 1.0));
+    return prefer_flat(g->m, g->n, g->k, layout_factor * (mx ? 1.1 : 1.0));
 }
 
 template <bool BROW>
@@ -715,7 +716,7 @@ static int a16w16_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allo
 {
     if (!g) return A8W8_ERR_NULL_POINTER;
     // a skinny problem on shuffled weights: the flat kernel where it is the faster one (and can run it)
-    if (allow_flat && g->b_preshuffled && g->m > 0 && g->m <= FLAT_MAX_M && prefer_flat(g->m, g->n, 2ll * g->k, false) &&
+    if (allow_flat && g->b_preshuffled && g->m > 0 && g->m <= FLAT_MAX_M && prefer_flat(g->m, g->n, 2ll * g->k) &&
         a16w16_flat_impl(g, hip_stream, false) == A8W8_OK)
         return A8W8_OK;
     if (!g->a || !g->b || !g->c) return A8W8_ERR_NULL_POINTER;
@@ -733,7 +734,7 @@ static int a16w16_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allo
     bytes.stride_a_batch = g->stride_a_batch * 2; bytes.stride_b_batch = g->stride_b_batch * 2;
     bytes.scale_mode = A8W8_SCALE_TENSOR;
     const bool fits = (long long)g->stride_a_batch * 2 < (1ll << 31) && (long long)g->stride_b_batch * 2 < (1ll << 31);
-    const bool flat_rows = fits && flat_rowmajor_ok(&bytes) && prefer_flat(g->m, g->n, bytes.k, false, bytes.stride_b % 4096 == 0 ? 1.3 : 1.05);
+    const bool flat_rows = fits && flat_rowmajor_ok(&bytes) && prefer_flat(g->m, g->n, bytes.k, bytes.stride_b % 4096 == 0 ? 1.3 : 1.05);
     if (!flat_rows && fits && c_stride_too_large(g, &bytes)) return A8W8_ERR_TOO_LARGE;
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     hipStream_t s = (hipStream_t)hip_stream;
@@ -784,7 +785,7 @@ static int a4w4_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
 {
     if (!g) return A8W8_ERR_NULL_POINTER;
     // a skinny problem on shuffled weights: the flat kernel where it is the faster one (and can run it)
-    if (allow_flat && g->b_preshuffled && g->m > 0 && g->m <= FLAT_MAX_M && prefer_flat(g->m, g->n, g->k / 2, false) &&
+    if (allow_flat && g->b_preshuffled && g->m > 0 && g->m <= FLAT_MAX_M && prefer_flat(g->m, g->n, g->k / 2) &&
         a4w4_flat_impl(g, hip_stream, false) == A8W8_OK)
         return A8W8_OK;
     if (!g->a || !g->b || !g->c || !g->sfa || !g->sfb) return A8W8_ERR_NULL_POINTER;
@@ -809,7 +810,7 @@ static int a4w4_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
     bytes.stride_a = g->stride_a / 2; bytes.stride_b = g->b_preshuffled ? bytes.k : g->stride_b / 2;
     bytes.stride_a_batch = g->stride_a_batch / 2; bytes.stride_b_batch = g->stride_b_batch / 2;
     bytes.scale_mode = A8W8_SCALE_MX_E8M0_TILED;
-    const bool flat_rows = tiled && flat_rowmajor_ok(&bytes) && prefer_flat(g->m, g->n, bytes.k, false, bytes.stride_b % 4096 == 0 ? 1.3 : 1.05);
+    const bool flat_rows = tiled && flat_rowmajor_ok(&bytes) && prefer_flat(g->m, g->n, bytes.k, bytes.stride_b % 4096 == 0 ? 1.3 : 1.05);
     if (!flat_rows && tiled && g->k % 256 == 0 && c_stride_too_large(g, &bytes)) return A8W8_ERR_TOO_LARGE;
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     hipStream_t s = (hipStream_t)hip_stream;
@@ -882,7 +883,7 @@ static int a4w4_flat_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
     if ((long long)g->n * g->k / 2 >= (1ll << 31) || g->batch > 65535) return A8W8_ERR_TOO_LARGE;
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     // several groups of 16 rows over weights too large to stay in cache: the MFMA kernels read the same weights
-    if (allow_dense && !prefer_flat(g->m, g->n, g->k / 2, false) && a4w4_gemm_impl(g, hip_stream, false) == A8W8_OK)
+    if (allow_dense && !prefer_flat(g->m, g->n, g->k / 2) && a4w4_gemm_impl(g, hip_stream, false) == A8W8_OK)
         return A8W8_OK;
     a8w8_gemm_args bytes = *g;      // packed rows as byte rows of k/2 columns
     bytes.k = g->k / 2;
@@ -930,7 +931,7 @@ static int a16w16_flat_impl(const a8w8_gemm_args* g, void* hip_stream, bool allo
         return A8W8_ERR_TOO_LARGE;
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     // several groups of 16 rows over weights too large to stay in cache: the MFMA kernels read the same weights
-    if (allow_dense && !prefer_flat(g->m, g->n, 2ll * g->k, false) && a16w16_gemm_impl(g, hip_stream, false) == A8W8_OK)
+    if (allow_dense && !prefer_flat(g->m, g->n, 2ll * g->k) && a16w16_gemm_impl(g, hip_stream, false) == A8W8_OK)
         return A8W8_OK;
     a8w8_gemm_args bytes = *g;      // bf16 rows as byte rows of 2k columns
     bytes.k = g->k * 2;

@@ -194,7 +194,8 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
     // of groups 0 and 2 for both steps s, those of (x + 2, kq) groups 1 and 3: two 8-byte loads instead of four 1- or 2-byte
     // ones (a load of a byte per lane takes its turn in the memory pipeline like one of 16 bytes: 64 x 16384 x 7168 26.9 -> 25.3 us,
     // MXFP4 16.4 -> 15.5; 16 x 28672 x 4096 22.1 -> 21.1).
-    constexpr bool MX_WIDE_A = (MODE == MODE_MXT || MODE == MODE_F4T) && MT == 4, MX_WIDE_B = (MODE == MODE_MXT || MODE == MODE_F4T) && NT == 4;
+    // (not for MXFP8 on two weight tiles: the registers would pass 128, and two workgroups no longer share a compute unit)
+    constexpr bool MX_WIDE_A = MT == 4 && ((MODE == MODE_MXT && NT == 4) || MODE == MODE_F4T), MX_WIDE_B = (MODE == MODE_MXT || MODE == MODE_F4T) && NT == 4;
     const int mx_par = (r16 >> 2) & 1;
     uint32_t mx_a[MT], mx_b[NT];
     auto load_unit = [&](__amdgpu_buffer_rsrc_t rs, uint32_t lane_offset, int unit, int (&s)[4]) {
@@ -212,7 +213,7 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
             const int mt = min(m_tile_ * MT + g, ((p.m + 15) >> 4) - 1);
             // four groups are one 64-row block: constant distances from group 0 (rows past m stay inside the block)
             // (the distance goes into the scalar offset of the load: one lane offset for the four groups)
-            mx_a[g] = MT == 4 ? (uint32_t)m_tile_ * 1024u + lane_off(0) - 2 * mx_par : (uint32_t)(mt >> 2) * 1024u + lane_off(mt & 3);
+            mx_a[g] = MT == 4 ? (uint32_t)m_tile_ * 1024u + lane_off(0) - (MX_WIDE_A ? 2 * mx_par : 0) : (uint32_t)(mt >> 2) * 1024u + lane_off(mt & 3);
         }
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
@@ -313,7 +314,7 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
             if constexpr (MX_WIDE_A) load_unit(rs_sa, mx_a[0], unit_a, f.sa);
             else {
 #pragma unroll
-                for (int g = 0; g < MT; ++g) f.sa[g] = __builtin_amdgcn_raw_buffer_load_b8(rs_sa, mx_a[g], unit_a + (pp & 1), 0);
+                for (int g = 0; g < MT; ++g) f.sa[g] = __builtin_amdgcn_raw_buffer_load_b8(rs_sa, mx_a[MT == 4 ? 0 : g], unit_a + (pp & 1) + (MT == 4 ? (int)MX_DELTA[g & 3] : 0), 0);
             }
         }
         if constexpr (MODE == MODE_F4T) {
