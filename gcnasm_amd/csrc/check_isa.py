@@ -9,7 +9,8 @@ The four-wave GEMM kernels, and the 256 x 128 variants of the 128-tile kernel (w
 
 Those kernels keep their accumulators in registers a[0:255] that only their own assembly statements
 name.  That is sound as long as the compiler places nothing of its own there and spills nothing:
-this script reads the device assembly of the library and fails the build otherwise.
+this script reads the device assembly of the library and fails the build otherwise, as it does when a
+vector instruction writes an MFMA's operand in the two slots in front of it.
 Usage: check_isa.py <device .s file> [--no-stores-ok]     (the option: for measurement builds that leave the stores out)
 """
 import re
@@ -68,6 +69,15 @@ def main(path, no_stores_ok=False):
         if "gemm_a8w8_wide" not in name and not tall:
             continue
         checked += 1
+        # their MFMAs are assembly statements, for which the compiler keeps no distance to a vector instruction that writes an
+        # operand: none may stand in the two slots in front
+        for i, ins in enumerate(seq):
+            if not ins.startswith("v_mfma"):
+                continue
+            sources = set().union(*(registers(o) for o in re.split(r" (?:op_sel|cbsz)", ins.split(None, 1)[1])[0].split(",")[1:]))
+            for before in seq[max(i - 2, 0):i]:
+                if before.startswith("v_") and not before.startswith("v_mfma") and registers(before.split(None, 1)[1].split(",")[0]) & sources:
+                    sys.exit(f"{name}: an operand of an MFMA is written directly in front of it: {before} / {ins}")
         mfma = reads = 0
         for line in f.split("\n"):
             ins = line.split(";", 1)[0].strip()
