@@ -133,9 +133,10 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
 #pragma unroll
         for (int j = 0; j < B_LOADS; ++j) voff_b[j] = b_lane_offset(p, min(n0 + ld_row + 32 * j, p.n - 1), ld_piece16);
     }
-    // the lane's piece of the last, partial K step lies past k: out of every descriptor's range (an extent is below 2^31)
-    const int past_k = RAGGED && (nk - 1) * BK + ld_piece16 >= p.k ? (int)0x80000000u : 0;
-    auto lane_offset = [&](int voff, int kstep) __attribute__((always_inline)) { return RAGGED ? voff | (kstep == nk - 1 ? past_k : 0) : voff; };
+    // the lane's piece of the last, partial K step lies past k: out of every descriptor's range (an extent is below 2^31; 2^31 in
+    // place of the lane's offset, not on top of it: together with the scalar offset that could pass 2^32, and wrap into the matrix)
+    const bool past_k = RAGGED && (nk - 1) * BK + ld_piece16 >= p.k;
+    auto lane_offset = [&](int voff, int kstep) __attribute__((always_inline)) { return RAGGED && past_k && kstep == nk - 1 ? (int)0x80000000u : voff; };
     // block mode: waves 0 and 1 fetch the step's 128 A-row scales (64 each), waves 2 and 3 the B scale
     // of the tile's 128 x 128 block (every lane the same dword: the stage's copy at +512 is the one read)
     constexpr int SF_LOADS = !STEP_SCALES ? 0 : TALL && !TILED_SCALES ? (MODE == MODE_F4 ? 4 : 2) : MODE == MODE_F4 ? 2 : 1;

@@ -57,3 +57,27 @@ def test_partial_last_step_keeps_fp32_sums(orc):
     got = g.gemm(*(torch.from_numpy(x).cuda() for x in (a, b, sa, sb)), g.ROWCOL, c_dtype=g.FP32).cpu().numpy()
     exact, mag = exact64(orc, a, b, sa, sb, g.ROWCOL)
     assert (np.abs(got - exact) <= 1e-7 * mag).all()
+
+
+@pytest.mark.parametrize("side", ["a", "b"])
+def test_partial_last_step_at_the_end_of_two_gigabytes(side):
+    """A matrix that ends 16 bytes below 2 GiB: the pieces past K of its last row lie beyond 2^31, where a lane offset with bit 31
+    on top, plus the step's scalar offset, would wrap to the matrix's first bytes.  Those are NaN codes here: row 0 is NaN, and
+    no other row may be."""
+    rows, stride, k, other = 3, 1073741680, 272, 64
+    assert (rows - 1) * stride + k == 2 ** 31 - 16
+    r = np.random.default_rng(9)
+    x, y = (r.integers(-4, 5, (m, k)).astype(np.float32) for m in (rows, other))
+    whole = torch.empty(2 ** 31, dtype=torch.uint8, device="cuda")
+    long = whole.as_strided((rows, k), (stride, 1))
+    long.copy_(torch.from_numpy(oracle.encode(x)))
+    long[0, :16] = 0x7F
+    short = torch.from_numpy(oracle.encode(y)).cuda()
+    one = torch.ones(1, device="cuda")
+    a, b = (long, short) if side == "a" else (short, long)
+    assert g.kernel_name(g.raw_gemm_args(a.data_ptr(), b.data_ptr(), 1 << 12, 1 << 12, 1 << 12, a.shape[0], b.shape[0], k, g.TENSOR,
+                                         stride_a=a.stride(0), stride_b=b.stride(0))) == "gemm_a8w8_tile128"
+    got = g.gemm(a, b, one, one, g.TENSOR, c_dtype=g.FP32)
+    got = (got if side == "a" else got.T).cpu().numpy()
+    assert np.isnan(got[0]).all()
+    assert (got[1:] == x[1:] @ y.T).all()
