@@ -167,7 +167,8 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
                            // rows past m lie beyond the descriptor's extent and read as zero: no clamp
                            : (uint32_t)(m0 + g * 16 + ld_row) * (uint32_t)p.lda + ld_piece * 16;
     v4i* stage = smem + wave * (STAGED * FLAT_STAGE_SLOTS);
-    const uint32_t kill_second = ld_piece >= 4 ? 0x80000000u : 0u;
+    constexpr uint32_t PAST_K = 0x80000000u;             // beyond every descriptor's extent
+    const bool second_past_k = ld_piece >= 4;            // the lane's piece lies in the second K block of a pair
     const int st_write = ld_piece * 18 + ld_row;         // row + 8 is 8 slots on
     const int st_read = kq * 18 + r16;                   // piece kq, the second K block's is 4 * 18 slots on
 
@@ -261,7 +262,8 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
     auto load_rows = [&](int pp) {
         // pieces 4 .. 7 are the second K block of the pair: past the end of K (an odd number of blocks) they get an
         // offset beyond the descriptor's extent instead of a branch, which reads as zero and touches no memory
-        const uint32_t off = a_off[0] | (2 * pp + 1 < k_tiles ? 0u : kill_second);
+        // (2^31 in place of the lane's offset, not on top of it: with the scalar offset that could pass 2^32 and wrap into the matrix)
+        const uint32_t off = second_past_k && 2 * pp + 1 >= k_tiles ? PAST_K : a_off[0];
 #pragma unroll
         for (int g = 0; g < MT; ++g) {
             // (group g is 16 g rows on: a scalar offset, so that one lane offset serves every group)
@@ -270,7 +272,7 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
         }
     };
     auto load_weight_rows = [&](int pp) {
-        const uint32_t off = b_off[0] | (2 * pp + 1 < k_tiles ? 0u : kill_second);
+        const uint32_t off = second_past_k && 2 * pp + 1 >= k_tiles ? PAST_K : b_off[0];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             // (tile t is 16 t rows on: a scalar offset, one lane offset for every tile)
@@ -301,10 +303,10 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
     };
     auto load = [&](int pp, Frag& f) {
         const int kt0 = 2 * pp, kt1 = 2 * pp + 1;
-        const uint32_t kill1 = kt1 < k_tiles ? 0u : 0x80000000u;      // reads as zero, see load_rows
+        const bool past1 = kt1 >= k_tiles;      // the second K block reads as zero, see load_rows
         if constexpr (MT == 1) {
             f.a[0] = ld16(rs_a, a_off[0], kt0 * 64);
-            f.a[1] = ld16(rs_a, a_off[0] | kill1, kt1 * 64);
+            f.a[1] = ld16(rs_a, past1 ? PAST_K : a_off[0], kt1 * 64);
         }
         int unit_a = 0, unit_b = 0;
         if constexpr (MODE == MODE_MXT) {
@@ -346,7 +348,7 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
         for (int t = 0; t < NT; ++t) {
             if constexpr (!BROW) {
                 f.b[t][0] = ld16_nt(rs_b, lane16, b_off[t] + kt0 * 1024);
-                f.b[t][1] = ld16_nt(rs_b, lane16 | kill1, b_off[t] + kt1 * 1024);
+                f.b[t][1] = ld16_nt(rs_b, past1 ? PAST_K : lane16, b_off[t] + kt1 * 1024);
             }
         }
     };

@@ -197,3 +197,28 @@ def test_row_major_weights_on_the_flat_kernel(orc, mode, m, many_tiles):
     n, k = (144, 320) if mode in (g.ROWCOL, g.TENSOR) else (384, 256)
     batch = (1024 * 16 + n - 1) // n if many_tiles else 2
     _row_group_case(orc, mode, m, n, k, batch, 8800 + m, rowmajor=True)
+
+
+@pytest.mark.parametrize("side,rows,stride,k,other", [("a", 3, 1073741712, 192, 64), ("a", 20, 113025424, 576, 64), ("a", 64, 34087024, 1088, 80),
+                                                      ("b", 16, 143165552, 320, 5), ("b", 48, 45691120, 960, 40), ("b", 64, 34087024, 1088, 64)])
+def test_odd_block_count_at_the_end_of_two_gigabytes(orc, side, rows, stride, k, other):
+    """A matrix that ends less than 64 bytes below 2 GiB, K an odd number of 64-wide blocks: the second block of the last pair lies
+    beyond 2^31 on the last row, where a lane offset with bit 31 on top, plus the scalar offset, would wrap to the matrix's first
+    bytes.  Those are NaN codes here: row 0 is NaN, and no other row may be."""
+    import torch
+    assert (rows - 1) * stride + k in (2 ** 31 - 16, 2 ** 31 - 32, 2 ** 31 - 48)
+    r = np.random.default_rng(rows)
+    x, y = (r.integers(-4, 5, (m, k)).astype(np.float32) for m in (rows, other))
+    whole = torch.empty(2 ** 31, dtype=torch.uint8, device="cuda")
+    long = whole.as_strided((rows, k), (stride, 1))
+    long.copy_(torch.from_numpy(orc.encode(x)))
+    long[0, :64] = 0x7F
+    short = torch.from_numpy(orc.encode(y)).cuda()
+    one = torch.ones(1, device="cuda")
+    a, b = (long, short) if side == "a" else (short, long)
+    args, _ = g.api._args_from_tensors(a, b, one, one, g.TENSOR, None, g.FP32, 0)
+    assert g.kernel_name(args) == "flatmm_a8w8"
+    got = g.gemm(a, b, one, one, g.TENSOR, c_dtype=g.FP32)
+    got = (got if side == "a" else got.T).cpu().numpy()
+    assert np.isnan(got[0]).all()
+    assert (got[1:] == x[1:] @ y.T).all()
