@@ -1072,7 +1072,8 @@ int a8w8_quantize(const float* src, int rows, int k, int ld, uint8_t* q, void* s
                     return launch(quant_tensor_one_kernel, dim3(1), dim3(1024), 0, s, (const float4*)src, (int)units, (uint32_t*)q, (float*)scale);
                 const unsigned parts = (unsigned)std::min<size_t>((units + 1023) / 1024, QUANT_TENSOR_PARTS);
                 const size_t apply = (units + 256 * QUANT_TENSOR_UNITS - 1) / (256 * QUANT_TENSOR_UNITS);
-                if (apply < (1u << 31)) {
+                // (a launch has less than 2^32 threads along a dimension; the kernels below walk an array of any size with a fixed grid)
+                if (apply * 256 < (1ull << 32)) {
                     A8W8_LAUNCH_OR_RETURN(quant_tensor_amax_vec_kernel, dim3(parts), dim3(256), 0, s, (const float4*)src, units, (float*)q);
                     A8W8_LAUNCH_OR_RETURN(quant_tensor_fold_kernel, dim3(1), dim3(256), 0, s, (const float*)q, (int)parts, (float*)scale);
                     return launch(quant_tensor_apply_vec_kernel, dim3((unsigned)apply), dim3(256), 0, s, (const float4*)src, units, (uint32_t*)q,

@@ -206,3 +206,20 @@ def test_rowwise_at_every_row_length(orc, k):
     qr, sr = orc.quantize(x, orc.ROWCOL)
     q, s = _run(x, g.ROWCOL)
     assert (q == qr).all() and (s == sr).all()
+
+
+def test_per_tensor_beyond_the_threads_of_one_launch():
+    """2^35 elements, 128 GiB of them: one thread per eight elements would be 2^32 threads, more than a launch takes."""
+    rows, k = 1 << 20, 1 << 15
+    if torch.cuda.mem_get_info()[0] < 180 << 30:
+        pytest.skip("needs 160 GiB of free memory")
+    x = torch.empty((rows, k), device="cuda")
+    x.uniform_(-1.0, 1.0)
+    x[rows - 1, k - 3] = -896.0
+    q, s = g.quantize(x, g.TENSOR)
+    assert float(s) == 2.0
+    for first in (0, 1, rows // 2, rows - 3):
+        want = g.cvt_f32_to_e4m3(x[first:first + 3] / 2.0)
+        assert torch.equal(q[first:first + 3], want), first
+    del x, q
+    torch.cuda.empty_cache()
