@@ -16,6 +16,7 @@
 #include "gemm_small.hpp"
 #include "gemm_wide.hpp"
 #include "hbm_probe.hpp"
+#include "routes.hpp"
 
 using namespace a8w8;
 
@@ -662,16 +663,15 @@ int fill_mx_tiled(int rows, int k, uint8_t* scale, hipStream_t s)
 }
 
 // The vectorised MX quantisers: as many chunks per wave as the array fills the chip with (quant_mx_vec_kernel), over the padded
-// array where its elements can be counted with 31 bits.
+// array where mx_padding_in_launch says so.
 template <bool FP4, bool TILED>
 int launch_quant_mx(const float* src, int rows, int k, int ld, uint8_t* q, uint8_t* scale, hipStream_t s)
 {
     int rows_p = rows, k_p = k;
     if constexpr (TILED) {
-        const long long rp = (rows + 63ll) / 64 * 64, kp = (k + 511ll) / 512 * 512;
-        if (rp * kp < (1ll << 31)) {
-            rows_p = (int)rp;
-            k_p = (int)kp;
+        if (mx_padding_in_launch(rows, k)) {
+            rows_p = (rows + 63) / 64 * 64;
+            k_p = (k + 511) / 512 * 512;
         } else if (const int st = fill_mx_tiled(rows, k, scale, s); st != A8W8_OK) {
             return st;
         }

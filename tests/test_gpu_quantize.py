@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import gcnasm_amd as g
+import routes
 from gpu_util import dev
 
 pytestmark = pytest.mark.gpu
@@ -223,3 +224,12 @@ def test_per_tensor_beyond_the_threads_of_one_launch():
         assert torch.equal(q[first:first + 3], want), first
     del x, q
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("rows,k", [(1, 131072), (3, 140000 // 32 * 32), (16384, 32), (16385, 96), (9000, 544)])
+def test_tiled_scales_with_much_padding(orc, rows, k):
+    """More than three million padding elements: their scales come from a fill launch, the others from a quantiser over the real ones."""
+    assert not routes.mx_padding_in_launch(rows, k)
+    x = np.random.default_rng(rows + k).standard_normal((rows, k)).astype(np.float32)
+    for q, s, qr, sr in [(*g.quantize(dev(x), g.MX_TILED), *orc.quantize(x, orc.MX)), (*g.quantize_mxfp4(dev(x), tiled=True), *orc.quantize_mxfp4(x))]:
+        assert (q.cpu().numpy() == qr).all() and (s.cpu().numpy() == orc.mx_tile_scales(sr)).all()
