@@ -261,14 +261,15 @@ bool small_ok(const a8w8_gemm_args* g);
 
 // MXFP4 with row-major scales on the four-wave kernel (`g`: byte view, k in bytes, row-major scale mode).  It fetches 16 scale
 // bytes of a row at a time (two K steps: an even number of them) with 32-bit offsets that run up to 256 rows past the end of
-// the matrix.  The line to the 128-tile kernel is the one every other mode has (small_ok): above it 256-tiles are the
-// faster ones (4096^3 57 us on the 128-tile kernel, 36.5 here; 8192^3 393 and 244).
+// the matrix.  Up to two 128-tiles per compute unit (small_ok, the line of every other mode) and where
+// f4_row_scales_on_256_tiles says so the 128-tile kernel is the faster one.
 bool wide_row_scales_ok(const a8w8_gemm_args* g)
 {
     const auto rows_ok = [&](const void* s, long long stride, long long batch_stride, long long rows) {
         return aligned16(s) && stride % 16 == 0 && (g->batch == 1 || batch_stride % 16 == 0) && (rows + BM) * stride < (1ll << 31);
     };
-    return !small_ok(g) && persist_ok(g) && (g->k / BK) % 2 == 0 && rows_ok(g->sfa, g->stride_sfa, g->stride_sfa_batch, g->m) &&
+    return !small_ok(g) && f4_row_scales_on_256_tiles(g->m, g->n, g->k / BK, g->batch, g->c_dtype == A8W8_C_FP32, num_cus()) &&
+           persist_ok(g) && (g->k / BK) % 2 == 0 && rows_ok(g->sfa, g->stride_sfa, g->stride_sfa_batch, g->m) &&
            rows_ok(g->sfb, g->stride_sfb, g->stride_sfb_batch, g->n) && c_tile_fits(g->stride_c, g->c_dtype == A8W8_C_BF16 ? 2 : 4);
 }
 

@@ -18,4 +18,22 @@ inline bool mx_padding_in_launch(long long rows, long long k)
            (padded <= 4ll << 20 || padded - rows * k <= 3ll << 20);
 }
 
+// MXFP4 on row-major scales, more than two 128-tiles per compute unit: the four-wave kernel (256-tiles, one workgroup per compute
+// unit) or the two-stage 128-tile kernel.  Both run in rounds: a round of 256-tiles (one per compute unit) is worth about three
+// rounds of one 128-tile per compute unit, three and a half where K is short and a prologue and a tile's stores, longer with fp32
+// C, weigh more; below four K steps of 256 elements (fp32 C: eight) they weigh too much.  us, 128-tiles / 256-tiles, bf16 C:
+//   4096 x 4096 (4 rounds of one 128-tile per compute unit, 1 of 256-tiles)   K 512 13.8 / 14.7, 1024 19.4 / 18.1, 2048 28.4 / 25.4, 4096 50 / 39
+//   4096 x 7168 (7, 2)    512 20.9 / 22.1, 1024 30.0 / 28.7, 2048 45.0 / 41.8, 4096 86 / 70
+//   3000 x 8192 (6, 2)    512 18.8 / 21.9, 1024 26.0 / 27.6, 2048 38.2 / 39.5, 3072 54.9 / 53.3, 4096 72 / 66
+//   8192 x 2560 (5, 2)    512 16.3 / 21.9, 1024 22.0 / 27.5, 2048 32.3 / 39.5, 4096 60 / 65, 8192 112 / 116
+// fp32 C: 4096 x 4096 1024 23.0 / 22.6, 2048 31.7 / 29.5; 4096 x 7168 1024 34.1 / 36.6, 2048 49.0 / 49.9, 3072 66.8 / 63.7;
+// 3000 x 8192 2048 42.5 / 49.0, 3072 56.8 / 61.0, 4096 77 / 75; 8192 x 2560 512 20.0 / 30.1, 4096 63 / 73.
+inline bool f4_row_scales_on_256_tiles(long long m, long long n, long long k_steps, long long batch, bool fp32_c, long long cus)
+{
+    const long long rounds128 = (batch * ((m + 127) / 128) * ((n + 127) / 128) + cus - 1) / cus;
+    const long long rounds256 = (batch * ((m + 255) / 256) * ((n + 255) / 256) + cus - 1) / cus;
+    if (k_steps < (fp32_c ? 8 : 4)) return false;
+    return 2 * rounds128 >= (k_steps >= (fp32_c ? 16 : 12) ? 6 : 7) * rounds256;
+}
+
 }  // namespace a8w8

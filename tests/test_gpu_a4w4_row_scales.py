@@ -1,5 +1,5 @@
 """MXFP4 with row-major scales past two 128-tiles per compute unit: the four-wave kernel where the scale rows take its 16-byte
-loads, the 128-tile kernel elsewhere.  Values in {0, +-0.5, +-1, +-2}, scales 2^-2 .. 2^1: products are multiples of 2^-6 and at
+loads and its rounds pay (f4_row_scales_on_256_tiles of routes.hpp), the 128-tile kernel elsewhere.  Values in {0, +-0.5, +-1, +-2}, scales 2^-2 .. 2^1: products are multiples of 2^-6 and at
 most 16, so a sum over K <= 2048 stays below 2^15 and is exact in fp32 (21 bits): the result has to be equal."""
 import ctypes
 
@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import gcnasm_amd as g
+import routes
 from gpu_util import dev
 
 pytestmark = pytest.mark.gpu
@@ -26,7 +27,7 @@ def _value(orc, q, s):
     return torch.from_numpy(orc.e2m1_decode_packed(q).astype(np.float64) * np.exp2(s.astype(np.float64) - 127).repeat(32, axis=1)).cuda()
 
 
-# whole tiles, ragged edges in both directions, one to four pairs of K steps (the scale batches hold two)
+# whole tiles, ragged edges in both directions
 @pytest.mark.parametrize("m,n,k", [(4096, 4096, 512), (4350, 2311, 1024), (2049, 4097, 1536), (6145, 2050, 2048), (4200, 4100, 768)])
 @pytest.mark.parametrize("pad", [0, 16, 4])                  # bytes between scale rows; 4 (and k = 768): the 128-tile kernel
 def test_exact_against_float64(orc, m, n, k, pad):
@@ -47,7 +48,10 @@ def test_exact_against_float64(orc, m, n, k, pad):
 
 def test_batch_with_padded_scale_sets(orc):
     """Three problems in one launch, scale sets 48 bytes apart more than they need."""
-    m, n, k, batch = 2100, 2100, 1024, 3
+    _batch_with_padded_scale_sets(orc, 2100, 2100, 1024, 3)
+
+
+def _batch_with_padded_scale_sets(orc, m, n, k, batch):
     rng = np.random.Generator(np.random.Philox(5))
     ops = [(_operand(rng, m, k), _operand(rng, n, k)) for _ in range(batch)]
     a, b = (torch.stack([dev(o[i][0]) for o in ops]) for i in range(2))
@@ -62,3 +66,18 @@ def test_batch_with_padded_scale_sets(orc):
     assert g.lib().a4w4_gemm(ctypes.byref(args), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
     for e, o in enumerate(ops):
         assert torch.equal(c[e], (_value(orc, *o[0]) @ _value(orc, *o[1]).T).float())
+
+
+# the four-wave kernel: two to nine pairs of K steps (the scale batches hold two), whole and ragged tiles, one round and two
+@pytest.mark.parametrize("m,n,k,fp32", [(4096, 4096, 1024, False), (3900, 3850, 1536, False), (3900, 3850, 2048, True), (6145, 2050, 2560, True),
+                                        (3001, 7000, 3072, False), (2049, 4097, 4096, True), (2049, 4097, 4608, False)])
+@pytest.mark.parametrize("pad", [0, 16])
+def test_four_wave_kernel_is_exact(orc, m, n, k, fp32, pad):
+    assert routes.f4_row_scales_on_256_tiles(m, n, k, fp32=fp32)
+    test_exact_against_float64(orc, m, n, k, pad)
+
+
+def test_four_wave_kernel_batch(orc):
+    m, n, k, batch = 2100, 2100, 2048, 3
+    assert routes.f4_row_scales_on_256_tiles(m, n, k, batch, fp32=True)
+    _batch_with_padded_scale_sets(orc, m, n, k, batch)

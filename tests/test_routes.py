@@ -12,3 +12,13 @@ def test_padding_of_tiled_mx_scales(rows, k, in_launch):
     """Padded in the quantiser's own launch up to four million elements in all or three million of padding; arrays without padding always (the grid is the same)
     as long as their elements can be counted with 31 bits."""
     assert routes.mx_padding_in_launch(rows, k) is in_launch
+
+
+@pytest.mark.parametrize("m,n,k,bf16,fp32", [(4096, 4096, 512, False, False), (4096, 4096, 1024, True, False), (4096, 4096, 2048, True, True),
+                                             (8192, 8192, 8192, True, True), (4096, 7168, 1024, True, False), (4096, 7168, 3072, True, True),
+                                             (3000, 8192, 2048, False, False), (3000, 8192, 3072, True, False), (3000, 8192, 4096, True, True),
+                                             (8192, 2560, 512, False, False), (8192, 2560, 8192, False, False), (4096, 2560, 2048, False, False),
+                                             (4096, 2560, 4096, True, True)])
+def test_mxfp4_row_major_scales_past_two_tiles_per_compute_unit(m, n, k, bf16, fp32):
+    assert routes.f4_row_scales_on_256_tiles(m, n, k) is bf16
+    assert routes.f4_row_scales_on_256_tiles(m, n, k, fp32=True) is fp32
