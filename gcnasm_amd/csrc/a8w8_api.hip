@@ -1102,7 +1102,12 @@ int a8w8_quantize(const float* src, int rows, int k, int ld, uint8_t* q, void* s
                 if (const int ds = device_status(); ds != A8W8_OK) return ds;
                 const long long waves = (long long)rows * (k / 128);
                 const unsigned groups = (unsigned)(k / 128);
-                if (quant_vec_ok(src, rows, k, ld, q, 4) && waves <= QUANT_1X128_FEW)
+                if (quant_vec_ok(src, rows, k, ld, q, 4) && quant_1x128_along_rows(rows, k))
+                    return waves > QUANT_1X128_FEW ? launch(quant_1x128_along_rows_kernel<4>, dim3((unsigned)((waves + 31) / 32)), dim3(256), 0, s, src,
+                                                            rows, k, ld, q, (float*)scale)
+                                                   : launch(quant_1x128_along_rows_kernel<1>, dim3((unsigned)((waves + 7) / 8)), dim3(256), 0, s, src,
+                                                            rows, k, ld, q, (float*)scale);
+                if (quant_vec_ok(src, rows, k, ld, q, 4) && (waves <= QUANT_1X128_FEW || rows < 32))
                     A8W8_LAUNCH_OR_RETURN(quant_1x128_vec_kernel<8>, dim3(groups * ((rows + 7) / 8)), dim3(256), 0, s, src, rows, k, ld, q,
                                        (float*)scale);
                 else if (quant_vec_ok(src, rows, k, ld, q, 4))

@@ -551,6 +551,37 @@ __global__ void __launch_bounds__(256) quant_1x128_vec_kernel(const float* __res
     if (threadIdx.x < ROWS && row0 + (int)threadIdx.x < rows) scale[(size_t)g * rows + row0 + threadIdx.x] = tile_scale[threadIdx.x];
 }
 
+// The same for few rows (quant_1x128_along_rows of routes.hpp): half waves take (row, group) pairs counted along the rows, so that none
+// is without a row and memory is read in one run; of few rows the scales of neighbouring groups share their lines all the same.
+// G pairs per half wave, all loads first: four where there are enough of them to fill the chip
+// (17 x 2^20 21.0 -> 19.2 us, 65 x 2^20 71 -> 66), else one.
+template <int G>
+__global__ void __launch_bounds__(256) quant_1x128_along_rows_kernel(const float* __restrict__ src, int rows, int k, int ld,
+                                                                     uint8_t* __restrict__ q, float* __restrict__ scale)
+{
+    const unsigned groups = (unsigned)(k >> 7), i0 = blockIdx.x * (8u * G) + (threadIdx.x >> 5), l = threadIdx.x & 31;
+    unsigned row[G], g[G];
+    float4 v[G];
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+        row[u] = (i0 + 8 * u) / groups;
+        g[u] = (i0 + 8 * u) % groups;
+        v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (row[u] < (unsigned)rows) v[u] = load_once4(src + (size_t)row[u] * ld + g[u] * 128 + 4 * l);
+    }
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+        float amax = fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w)));
+#pragma unroll
+        for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+        const float s = amax > 0.f ? __fdiv_rn(amax, 448.0f) : 1.0f;   // an all-zero group keeps scale 1
+        if (row[u] >= (unsigned)rows) continue;
+        if (l == 0) scale[(size_t)g[u] * rows + row[u]] = s;
+        *(uint32_t*)(q + (size_t)row[u] * k + g[u] * 128 + 4 * l) =
+            pack4_e4m3(__fdiv_rn(v[u].x, s), __fdiv_rn(v[u].y, s), __fdiv_rn(v[u].z, s), __fdiv_rn(v[u].w, s));
+    }
+}
+
 // 128 x 128 blocks, one workgroup per block; the block stays in registers between the amax and the quantisation (one read
 // of the input: 8192 x 8192 149 -> 55 us, 2560 x 2560 39.7 -> 8.3).  Scale stored [rows/128][k/128].
 __global__ void __launch_bounds__(256) quant_128x128_vec_kernel(const float* __restrict__ src, int k, int ld, uint8_t* __restrict__ q,

@@ -18,6 +18,14 @@ inline bool mx_padding_in_launch(long long rows, long long k)
            (padded <= 4ll << 20 || padded - rows * k <= 3ll << 20);
 }
 
+// The 1 x 128 quantiser's workgroups take 8 or 32 rows of one group, for the sake of the scales' lines.  With fewer than eight rows part
+// of every workgroup has none (1 x 2^20 7.3 us, 3 x 2^20 11.8, against 3.3 and 5.5 along the rows), and over long rows the 512 bytes
+// they read of each lie far apart (12 x 2^20 17.2, 17 x 2^20 24.3, 33 x 2^21 75, against 14.7, 19.2 and 69 along the rows).
+inline bool quant_1x128_along_rows(long long rows, long long k)
+{
+    return rows < 8 || (rows < 96 && k >= 1 << 19);
+}
+
 // MXFP4 on row-major scales, more than two 128-tiles per compute unit: the four-wave kernel (256-tiles, one workgroup per compute
 // unit) or the two-stage 128-tile kernel.  Both run in rounds: a round of 256-tiles (one per compute unit) is worth about three
 // rounds of one 128-tile per compute unit, three and a half where K is short and a prologue and a tile's stores, longer with fp32

@@ -25,6 +25,10 @@ def mx_padding_in_launch(rows, k):
     return bool(lib().route_mx_padding_in_launch(_ll(rows), _ll(k)))
 
 
+def quant_1x128_along_rows(rows, k):
+    return bool(lib().route_quant_1x128_along_rows(_ll(rows), _ll(k)))
+
+
 def f4_row_scales_on_256_tiles(m, n, k, batch=1, fp32=False, cus=256):
     """k in elements; for problems of more than two 128-tiles per compute unit whose K and scale rows the four-wave kernel takes."""
     return bool(lib().route_f4_row_scales_on_256_tiles(_ll(m), _ll(n), _ll(k // 256), _ll(batch), int(fp32), _ll(cus)))

@@ -233,3 +233,17 @@ def test_tiled_scales_with_much_padding(orc, rows, k):
     x = np.random.default_rng(rows + k).standard_normal((rows, k)).astype(np.float32)
     for q, s, qr, sr in [(*g.quantize(dev(x), g.MX_TILED), *orc.quantize(x, orc.MX)), (*g.quantize_mxfp4(dev(x), tiled=True), *orc.quantize_mxfp4(x))]:
         assert (q.cpu().numpy() == qr).all() and (s.cpu().numpy() == orc.mx_tile_scales(sr)).all()
+
+
+@pytest.mark.parametrize("rows,k", [(1, 128), (1, 1152), (2, 128), (3, 1152), (5, 70016), (7, 1152), (8, 1152), (9, 1 << 19), (31, 70016), (33, (1 << 19) + 128)])
+def test_1x128_few_rows(orc, rows, k):
+    """Along the rows (fewer than eight of them, or long ones), eight rows per workgroup, and the lines between; an all-zero group, a
+    padded input."""
+    assert routes.quant_1x128_along_rows(rows, k) is (rows < 8 or k >= 1 << 19)
+    x = np.random.default_rng(rows * k).standard_normal((rows, k)).astype(np.float32)
+    x[rows - 1, k - 128:] = 0
+    whole = torch.full((rows, k + 8), 1e30, device="cuda")
+    whole[:, :k] = dev(x)
+    q, s = g.quantize(whole[:, :k], g.BLOCK)
+    qr, sr = orc.quantize(x, orc.BLOCK, 1)
+    assert (q.cpu().numpy() == qr).all() and (s.cpu().numpy() == sr).all()

@@ -14,6 +14,12 @@ def test_padding_of_tiled_mx_scales(rows, k, in_launch):
     assert routes.mx_padding_in_launch(rows, k) is in_launch
 
 
+@pytest.mark.parametrize("rows,k,along", [(1, 128, True), (1, 1 << 20, True), (3, 1 << 20, True), (7, 4096, True), (8, 4096, False), (17, 1 << 20, True),
+                                          (65, 1 << 20, True), (65, 65536, False), (128, 1 << 20, False), (8192, 8192, False)])
+def test_1x128_quantiser(rows, k, along):
+    assert routes.quant_1x128_along_rows(rows, k) is along
+
+
 @pytest.mark.parametrize("m,n,k,bf16,fp32", [(4096, 4096, 512, False, False), (4096, 4096, 1024, True, False), (4096, 4096, 2048, True, True),
                                              (8192, 8192, 8192, True, True), (4096, 7168, 1024, True, False), (4096, 7168, 3072, True, True),
                                              (3000, 8192, 2048, False, False), (3000, 8192, 3072, True, False), (3000, 8192, 4096, True, True),
