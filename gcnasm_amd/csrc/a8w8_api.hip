@@ -1021,7 +1021,7 @@ int a8w8_cvt_f32_to_e4m3(const float* src, uint8_t* dst, size_t n, int dialect, 
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     hipStream_t s = (hipStream_t)hip_stream;
     const dim3 block(256);
-    if (aligned16(src) && ((uintptr_t)dst & 3) == 0) {
+    if (aligned16(src) && ((uintptr_t)dst & 3) == 0 && !(dialect == A8W8_E4M3_FNUZ && cvt_fnuz_few(n))) {
         const dim3 grid((unsigned)((n / 4 + 256 * CVT_UNITS) / (256 * CVT_UNITS)));      // (one thread at least, for the last n % 4)
         if (dialect == A8W8_E4M3_OCP)
             return clamp240 ? launch(cvt_f32_to_e4m3_vec_kernel<0, 1>, grid, block, 0, s, src, dst, n)
@@ -1046,7 +1046,7 @@ int a8w8_cvt_e4m3_to_f32(const uint8_t* src, float* dst, size_t n, int dialect, 
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     hipStream_t s = (hipStream_t)hip_stream;
     const dim3 block(256);
-    if (((uintptr_t)src & 3) == 0 && aligned16(dst)) {
+    if (((uintptr_t)src & 3) == 0 && aligned16(dst) && !(dialect == A8W8_E4M3_FNUZ && cvt_fnuz_few(n))) {
         const dim3 grid((unsigned)((n / 4 + 256 * CVT_UNITS) / (256 * CVT_UNITS)));
         return dialect == A8W8_E4M3_OCP ? launch(cvt_e4m3_to_f32_vec_kernel<0>, grid, block, 0, s, src, dst, n)
                                         : launch(cvt_e4m3_to_f32_vec_kernel<1>, grid, block, 0, s, src, dst, n);

@@ -18,6 +18,15 @@ inline bool mx_padding_in_launch(long long rows, long long k)
            (padded <= 4ll << 20 || padded - rows * k <= 3ll << 20);
 }
 
+// FNUZ conversions are 30 to 40 integer operations per value: eight values per thread (the vectorised kernels) are a longer chain than
+// the launch, and below two million values there are enough threads without them.  us, eight per thread / four (encode) and
+// one (decode) per thread: encode 65536 3.4 / 2.7, 2^19 3.5 / 3.1, 7 x 2^18 4.7 / 4.5; decode 65536 3.0 / 2.2, 2^19 3.3 / 2.5, 7 x 2^18 4.7 / 4.4;
+// equal at 2^21.  The OCP dialect, one hardware instruction per pair, is as fast either way.
+inline bool cvt_fnuz_few(unsigned long long n)
+{
+    return n < 1ull << 21;
+}
+
 // The 1 x 128 quantiser's workgroups take 8 or 32 rows of one group, for the sake of the scales' lines.  With fewer than eight rows part
 // of every workgroup has none (1 x 2^20 7.3 us, 3 x 2^20 11.8, against 3.3 and 5.5 along the rows), and over long rows the 512 bytes
 // they read of each lie far apart (12 x 2^20 17.2, 17 x 2^20 24.3, 33 x 2^21 75, against 14.7, 19.2 and 69 along the rows).

@@ -25,6 +25,10 @@ def mx_padding_in_launch(rows, k):
     return bool(lib().route_mx_padding_in_launch(_ll(rows), _ll(k)))
 
 
+def cvt_fnuz_few(n):
+    return bool(lib().route_cvt_fnuz_few(ctypes.c_ulonglong(n)))
+
+
 def quant_1x128_along_rows(rows, k):
     return bool(lib().route_quant_1x128_along_rows(_ll(rows), _ll(k)))
 

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import gcnasm_amd as g
+import routes
 from gpu_util import dev
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +96,17 @@ def test_vectorised_and_unaligned_conversions_agree(orc, dialect, n):
         assert (codes[shift: shift + n].cpu().numpy() == want).all()
         assert (back[shift: shift + n].cpu().numpy() == want_back).all()
         assert (codes[shift + n:] == 0x55).all() and (back[shift + n:] == 7.0).all()
+
+
+@pytest.mark.parametrize("n", [(1 << 21) - 1, 1 << 21, (1 << 21) + 1, (1 << 21) + 2, (1 << 21) + 2051])
+def test_fnuz_on_both_sides_of_its_line(orc, n):
+    """FNUZ conversions take the vectorised kernels from two million values on; every remainder of 4 there."""
+    assert routes.cvt_fnuz_few(n) is (n < 1 << 21)
+    x = np.random.default_rng(n).standard_normal(n).astype(np.float32) * 100
+    want = orc.encode(x, orc.FNUZ, clamp240=True)
+    src, codes, back = dev(x), torch.full((n + 8,), 0x55, dtype=torch.uint8, device="cuda"), torch.full((n + 8,), 7.0, device="cuda")
+    L, s = g.lib(), g.api._stream()
+    assert L.a8w8_cvt_f32_to_e4m3(src.data_ptr(), codes.data_ptr(), n, orc.FNUZ, 1, s) == 0
+    assert L.a8w8_cvt_e4m3_to_f32(codes.data_ptr(), back.data_ptr(), n, orc.FNUZ, s) == 0
+    assert (codes[:n].cpu().numpy() == want).all() and (back[:n].cpu().numpy() == orc.decode(want, orc.FNUZ)).all()
+    assert (codes[n:] == 0x55).all() and (back[n:] == 7.0).all()

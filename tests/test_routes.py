@@ -14,6 +14,11 @@ def test_padding_of_tiled_mx_scales(rows, k, in_launch):
     assert routes.mx_padding_in_launch(rows, k) is in_launch
 
 
+@pytest.mark.parametrize("n,few", [(1, True), (65536, True), ((1 << 20) + 3, True), ((1 << 21) - 1, True), (1 << 21, False), (1 << 25, False), (1 << 40, False)])
+def test_fnuz_conversions(n, few):
+    assert routes.cvt_fnuz_few(n) is few
+
+
 @pytest.mark.parametrize("rows,k,along", [(1, 128, True), (1, 1 << 20, True), (3, 1 << 20, True), (7, 4096, True), (8, 4096, False), (17, 1 << 20, True),
                                           (65, 1 << 20, True), (65, 65536, False), (128, 1 << 20, False), (8192, 8192, False)])
 def test_1x128_quantiser(rows, k, along):
