@@ -214,18 +214,12 @@ bool tiled_ok(const a8w8_gemm_args* g)
     return g->k % BK == 0 && rows_aligned(g) && (long long)((g->m + BM - 1) / BM) * ((g->n + BN - 1) / BN) < (1ll << 31);
 }
 
-// Rows of whole 16-byte pieces whose length is no multiple of the 128-byte K step: the 128-tile kernel with a partial last
-// step (scales that do not change with K; k in bytes here).  It is the faster one at any size, since the one-thread-per-element
-// kernel takes 86 ns per K element however small the problem (128 x 256 x 240: 20.9 us against 5.4, 1000 x 3000 x 2000: 7545
-// against 18.5, 4096 x 4096 x 4080: 84 ms against 0.116); problems of a few rows, columns and K elements, where that is no more
-// than a launch or two, stay there, in the order of operations of the CPU reference.
-constexpr int RAGGED_MIN_K_BYTES = 256;
-constexpr long long RAGGED_MIN_MACS = 1ll << 19;
+// The 128-tile kernel with a partial last K step: rows of whole 16-byte pieces, scales that do not change with K (k in bytes here).
 bool ragged_ok(const a8w8_gemm_args* g)
 {
     return (g->scale_mode == A8W8_SCALE_TENSOR || g->scale_mode == A8W8_SCALE_ROWCOL) && !g->b_preshuffled && g->k % BK != 0 &&
            g->k % 16 == 0 && rows_aligned(g) && (long long)((g->m + SM_BM - 1) / SM_BM) * ((g->n + 63) / 64) < (1ll << 31) &&
-           (g->k >= RAGGED_MIN_K_BYTES || (double)g->batch * g->m * g->n * g->k >= (double)RAGGED_MIN_MACS);
+           partial_steps_on_tiles(g->m, g->n, g->k, g->batch);
 }
 
 // B in the a8w8_preshuffle_b layout is read by the MFMA kernels only (the one-thread-per-element kernel reads

@@ -18,6 +18,19 @@ inline bool mx_padding_in_launch(long long rows, long long k)
            (padded <= 4ll << 20 || padded - rows * k <= 3ll << 20);
 }
 
+// Rows of whole 16-byte pieces whose length is no multiple of the 128-byte K step (scales that do not change with K): the 128-tile kernel
+// with a partial last step, 4.6 to 8 us at the least, or the one-thread-per-element kernel, 2.2 us and 60 to 85 ns per K element while
+// its outputs fit the chip at once.  us, one thread per element / tiles, row/col scales, K in bytes:
+//   128 x 512 x 16  3.4 / 4.8    129 x 1000 x 16  4.4 / 5.0    256 x 1024 x 16  7.0 / 5.5    128 x 260 x 48  5.7 / 6.8    128 x 512 x 32  6.5 / 5.4
+//   64 x 260 x 80   9.1 / 7.2    300 x 391 x 240   38 / 11.5   1000 x 3000 x 2000  7540 / 21   4096 x 4096 x 4080  84 ms / 116
+// so that K below 64 bytes stays with the former up to 2^21 multiply-adds.  Problems of less than 2^19 with K below 256 bytes stay there
+// too, although tiles would be faster (46 x 46 x 240: 21 us): a few thousand outputs in the order of operations of the CPU
+// reference, bit for bit, which is what callers compare small problems with.
+inline bool partial_steps_on_tiles(long long m, long long n, long long k_bytes, long long batch)
+{
+    return k_bytes >= 256 || (double)batch * m * n * k_bytes >= (double)(1ll << (k_bytes < 64 ? 21 : 19));
+}
+
 // FNUZ conversions are 30 to 40 integer operations per value: eight values per thread (the vectorised kernels) are a longer chain than
 // the launch, and below two million values there are enough threads without them.  us, eight per thread / four (encode) and
 // one (decode) per thread: encode 65536 3.4 / 2.7, 2^19 3.5 / 3.1, 7 x 2^18 4.7 / 4.5; decode 65536 3.0 / 2.2, 2^19 3.3 / 2.5, 7 x 2^18 4.7 / 4.4;

@@ -3,6 +3,10 @@
 
 extern "C" {
 int route_mx_padding_in_launch(long long rows, long long k) { return a8w8::mx_padding_in_launch(rows, k); }
+int route_partial_steps_on_tiles(long long m, long long n, long long k_bytes, long long batch)
+{
+    return a8w8::partial_steps_on_tiles(m, n, k_bytes, batch);
+}
 int route_cvt_fnuz_few(unsigned long long n) { return a8w8::cvt_fnuz_few(n); }
 int route_quant_1x128_along_rows(long long rows, long long k) { return a8w8::quant_1x128_along_rows(rows, k); }
 int route_f4_row_scales_on_256_tiles(long long m, long long n, long long k_steps, long long batch, int fp32_c, long long cus)

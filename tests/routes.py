@@ -25,6 +25,10 @@ def mx_padding_in_launch(rows, k):
     return bool(lib().route_mx_padding_in_launch(_ll(rows), _ll(k)))
 
 
+def partial_steps_on_tiles(m, n, k_bytes, batch=1):
+    return bool(lib().route_partial_steps_on_tiles(_ll(m), _ll(n), _ll(k_bytes), _ll(batch)))
+
+
 def cvt_fnuz_few(n):
     return bool(lib().route_cvt_fnuz_few(ctypes.c_ulonglong(n)))
 

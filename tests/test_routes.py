@@ -1,6 +1,7 @@
 """The size rules of the dispatch, at sizes where the variants on their two sides were measured to differ."""
 import pytest
 
+import gcnasm_amd as g
 import routes
 
 
@@ -12,6 +13,16 @@ def test_padding_of_tiled_mx_scales(rows, k, in_launch):
     """Padded in the quantiser's own launch up to four million elements in all or three million of padding; arrays without padding always (the grid is the same)
     as long as their elements can be counted with 31 bits."""
     assert routes.mx_padding_in_launch(rows, k) is in_launch
+
+
+@pytest.mark.parametrize("m,n,k,tiles", [(128, 260, 16, False), (128, 512, 16, False), (129, 1000, 16, False), (256, 1024, 16, True), (64, 260, 48, False),
+                                         (128, 260, 48, False), (128, 512, 32, True), (64, 260, 80, True), (37, 53, 96, False), (46, 46, 240, False),
+                                         (300, 391, 240, True), (1, 16, 272, True), (1000, 3000, 2000, True)])
+def test_partial_k_steps(m, n, k, tiles):
+    """On the tiles from 256 bytes of K on, below by the multiply-adds: the library's own choice, too."""
+    assert routes.partial_steps_on_tiles(m, n, k) is tiles
+    args = g.raw_gemm_args(1 << 12, 1 << 12, 1 << 12, 1 << 12, 1 << 12, m, n, k, g.ROWCOL)
+    assert g.kernel_name(args) == ("gemm_a8w8_tile128" if tiles else "gemm_a8w8_general")
 
 
 @pytest.mark.parametrize("n,few", [(1, True), (65536, True), ((1 << 20) + 3, True), ((1 << 21) - 1, True), (1 << 21, False), (1 << 25, False), (1 << 40, False)])
