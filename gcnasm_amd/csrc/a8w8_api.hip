@@ -299,17 +299,6 @@ bool small_ok(const a8w8_gemm_args* g)
     return items128 <= (long long)A8W8_SMALL_TILES_PER_CU * num_cus();
 }
 
-// 128 x 64 tiles instead of 128 x 128: when the wide tiles would occupy at most half of the compute units and the K
-// loop is long enough for the deeper staging to matter (a problem of a few K steps is bound by launch and store latency,
-// which narrower tiles do not change).
-#ifndef A8W8_NARROW_MIN_KSTEPS
-#define A8W8_NARROW_MIN_KSTEPS 16
-#endif
-bool narrow_tiles_pay(long long items128, int n, int k)
-{
-    return 2 * items128 <= num_cus() && n > 64 && k / BK >= A8W8_NARROW_MIN_KSTEPS;
-}
-
 // 256 x 128 tiles where 128 x 128 ones would put two workgroups on a compute unit, 256 x 128 ones would not, and the K loop is
 // long enough to make up for a prologue and a tile's stores that no second workgroup hides.  us per launch, bf16 C, two-stage
 // 128-tiles -> 256 x 128 (row/col, row-major MX, tiled MX, MXFP4 row-major / tiled, bf16):
@@ -339,7 +328,7 @@ int launch_small(const GemmParams& p, int batch, hipStream_t stream)
         q.tiles_m = (p.m + SM_BM - 1) / SM_BM;
         q.tiles_n = (p.n + SM_BN - 1) / SM_BN;
         const long long items = (long long)q.tiles_m * q.tiles_n * batch;
-        if (narrow_tiles_pay(items, p.n, p.k)) {
+        if (narrow_tiles_pay(items, p.n, p.k, num_cus())) {
             // short and wide: 128 x 64 tiles give every compute unit a workgroup, deep staging keeps its share of the
             // weights in flight
             q.tiles_n = (p.n + 63) / 64;
@@ -483,62 +472,31 @@ int launch_flat_nt(const GemmParams& p, int batch, hipStream_t stream)
     return launch(flatmm_a8w8<NT, MT, CDT, MODE, BROW>, grid, dim3(FLAT_THREADS), 0, stream, p);
 }
 
-// Weight tiles (NT) and groups of 16 activation rows (MT) per workgroup: the smallest NT x MT whose workgroups all fit the chip
-// at once.  Every workgroup is eight waves and a chain of K pairs, reduction and store whose length grows with NT x MT, so a
-// layer of few weight tiles goes out in small pieces (row groups then read the weights once each, all but the first from L2), and
-// one of many in pieces large enough for a single round.  us, row/col / MXFP8, NT x MT before -> now:
-//   64 x 1024 x 4096     2 x 4  8.7 / 9.9   -> 1 x 1  5.2 / 6.1       100 x 1024 x 4096   2 x 8, 2 x 4  13.2 / 9.8 -> 1 x 2  5.2 / 6.0
-//   64 x 4096 x 4096     2 x 4  9.2 / 10.5  -> 2 x 2  7.1 / 8.0       100 x 4096 x 4096   2 x 8, 2 x 4  14.2 / 10.6 -> 2 x 4  9.3 / 10.6
-//   64 x 9216 x 3584     2 x 4  14.6 / 17.8 -> 4 x 4  12.8 / 13.1     128 x 8192 x 8192   2 x 8, 2 x 4  25.9 / 33.4 -> 4 x 4  23.3 / 24.2
-//   128 x 12288 x 2560   2 x 8  20.7 -> 2 x 4 in three rounds 16.2 (MXFP8: 2 x 4 17.9 before and now, 4 x 4 19.0)
-//   16 x 5120 x 5120     1 x 1  9.9 / 11.4  -> 2 x 1  8.0 / 8.7       16 x 10240 x 8192   2 x 1  19.9 / 22.5 -> 4 x 1  17.4 / 18.6
-// Four row groups share a pass at most, six where their registers allow it (MX scales do not: 4 x 4 on two passes is faster,
-// 80 x 7168 x 4096 14.6 -> 13.4).  Layers of at least four weight tiles per compute unit take four, and an even split of the row
-// groups over one or two passes (16384 x 7168 at M = 48, 30 us with two tiles, 24 us with four).
+// The split of weight tiles and row groups is flat_split's.
 template <int CDT, int MODE, bool BROW = false>
 int launch_flat(const GemmParams& p, int batch, hipStream_t stream)
 {
-    constexpr bool MX = MODE == MODE_MXT || MODE == MODE_F4T;
-    const long long tiles = (long long)(p.n / 16) * batch;
-    const long long cus = num_cus();
-    const int groups = (p.m + 15) / 16, passes = (groups + 3) / 4;
-    const int mt = (groups + passes - 1) / passes;
-    if (tiles < 4 * cus) {
-        const auto fits = [&](int nt, int m) { return ((p.n / 16 + nt - 1) / nt) * (long long)batch * ((groups + m - 1) / m) <= cus; };
-        if (fits(1, 1)) return launch_flat_nt<1, 1, CDT, MODE, BROW>(p, batch, stream);
-        if (groups == 1 && fits(2, 1)) return launch_flat_nt<2, 1, CDT, MODE, BROW>(p, batch, stream);
-        if (groups > 1 && fits(1, 2)) return launch_flat_nt<1, 2, CDT, MODE, BROW>(p, batch, stream);
-        if (groups > 1 && fits(2, 2)) return launch_flat_nt<2, 2, CDT, MODE, BROW>(p, batch, stream);
-        if (groups > 2 && fits(2, 3)) return launch_flat_nt<2, 3, CDT, MODE, BROW>(p, batch, stream);
-        if (groups > 2 && (fits(2, 4) || (groups > 6 && !fits(4, 4)))) return launch_flat_nt<2, 4, CDT, MODE, BROW>(p, batch, stream);
-        if constexpr (!MX) {
-            if (groups > 4 && groups <= 6) return launch_flat_nt<2, 6, CDT, MODE, BROW>(p, batch, stream);
-        }
-        if (groups > 4) return launch_flat_nt<4, 4, CDT, MODE, BROW>(p, batch, stream);
-        // up to four groups, more than two and less than four weight tiles per compute unit: four tiles below
+    constexpr FlatKind KIND = MODE == MODE_MXT ? FLAT_MXFP8 : MODE == MODE_F4T ? FLAT_MXFP4 : MODE == MODE_BLOCK ? FLAT_BLOCK
+                              : MODE == MODE_BF16 ? FLAT_BF16 : FLAT_FP8;
+    const FlatSplit split = flat_split(KIND, BROW, p.m, p.n, p.k, batch, num_cus());
+    switch (10 * split.nt + split.mt) {
+        case 11: return launch_flat_nt<1, 1, CDT, MODE, BROW>(p, batch, stream);
+        case 12: return launch_flat_nt<1, 2, CDT, MODE, BROW>(p, batch, stream);
+        case 21: return launch_flat_nt<2, 1, CDT, MODE, BROW>(p, batch, stream);
+        case 22: return launch_flat_nt<2, 2, CDT, MODE, BROW>(p, batch, stream);
+        case 23: return launch_flat_nt<2, 3, CDT, MODE, BROW>(p, batch, stream);
+        case 24: return launch_flat_nt<2, 4, CDT, MODE, BROW>(p, batch, stream);
+        case 26: return launch_flat_nt<2, 6, CDT, MODE, BROW>(p, batch, stream);
+        case 41: return launch_flat_nt<4, 1, CDT, MODE, BROW>(p, batch, stream);
+        case 42: return launch_flat_nt<4, 2, CDT, MODE, BROW>(p, batch, stream);
+        case 43: return launch_flat_nt<4, 3, CDT, MODE, BROW>(p, batch, stream);
+        case 44: return launch_flat_nt<4, 4, CDT, MODE, BROW>(p, batch, stream);
+        default: return A8W8_ERR_BAD_MODE;
     }
-    if (mt == 4) return launch_flat_nt<4, 4, CDT, MODE, BROW>(p, batch, stream);
-    if (mt == 3) return launch_flat_nt<4, 3, CDT, MODE, BROW>(p, batch, stream);
-    if (mt == 2) return launch_flat_nt<4, 2, CDT, MODE, BROW>(p, batch, stream);
-    return launch_flat_nt<4, 1, CDT, MODE, BROW>(p, batch, stream);
 }
 
-// On shuffled weights both the flat GEMM and the MFMA kernels can run a skinny problem; the entry points take the
-// one a small cost model calls faster.  Times in microseconds, W = weight bytes, row_bytes = bytes of one weight row:
-//   flat:  one pass over the weights at ~6.4 TB/s; every further group of 16 activation rows adds the activation rows
-//          that each workgroup reads again for its weight tiles, W / NT bytes at ~21 TB/s (1.4 us on 16384 x 7168), and
-//          the scale bytes of MXFP8 about a tenth; a second pass (more than 64 rows over at least four weight tiles
-//          per compute unit) reads the weights from L2 and costs 55% more.
-//   dense: the 128-tile kernel pulls the weights with one workgroup per 128 weight rows at ~28 GB/s each, or, where
-//          128 x 128 tiles would occupy at most half of the compute units, per 64 rows at ~22 GB/s each (its 128 x 64
-//          tiles), ~5 TB/s at best over the chip; 20% more at 128 activation rows than at a few.
-// Weights of at most 32 MiB always go flat.  Measured on MI355X, shuffled FP8 weights, M = 16 / 32 / 48 / 64 / 80 / 96 /
-// 128, flat against dense:
-//   16384 x 7168   20 / 21 / 23 / 24 / 35 / 36 / 41  against  30 / 27 / 27 / 28 / 30 / 31 / 33   (MXFP8 about 10% more on both sides)
-//   8192 x 8192    13 / 14 / 16 / 18 / 21 / 22 / 23  against  26 / 26 / 26 / 27 / 28 / 29 / 31
-//   28672 x 4096   20 / 23 / 25 / 28 / 39 / 41 / 47  against  26 / 26 / 27 / 28 / 29 / 30 / 31
-//   4096 x 14336   13 / .. / .. / 19 / 23 / .. / 27  against  41 throughout
-// (tests/test_zz_gpu_routing.py times both sides of such cells through a8w8_route_override and checks the choice).
+// On shuffled weights both the flat GEMM and the MFMA kernels can run a skinny problem; the entry points take the one that the cost
+// model of flat_is_faster calls faster.
 // Row-major weights (a8w8_gemm without b_preshuffled; the flat kernel stages the weight rows through LDS, whole lines
 // per load): as fast as shuffled ones unless the rows are a large power of two apart, where the 16 rows of a tile fall
 // on the same memory channels -- 16384 x 7168 FP8 M = 16 / 32 / 64: 20 / 21 / 25 us, 8192 x 8192: 17 / 17 / 20 us
@@ -548,39 +506,14 @@ int g_route = A8W8_ROUTE_MODEL;      // a8w8_route_override
 bool prefer_flat(int m, int n, long long row_bytes, double layout_factor = 1.0)
 {
     if (g_route != A8W8_ROUTE_MODEL) return g_route == A8W8_ROUTE_FLAT;
-    const double w = (double)n * (double)row_bytes;
-    if (w <= (double)(32ll << 20)) return true;
-    const int groups = (m + 15) / 16, passes = (groups + 3) / 4;
-    const int mt = (groups + passes - 1) / passes;
-    const int cus = num_cus();
-    const int rounds = ((n + 127) / 128 + cus - 1) / cus;
-    // one pass over the weights, plus, for every further group of 16 activation rows, the activation rows each
-    // workgroup reads again for its NT weight tiles (n * row_bytes / NT bytes from L2) and their MFMAs; nearly twice
-    // that where the workgroups do not fit the chip at once
-    const long long tiles = n / 16;
-    const int nt = tiles >= 4ll * cus || (groups <= 4 && tiles > 2ll * cus) ? 4 : tiles > cus ? 2 : 1;      // (as launch_flat chooses)
-    const double per_group = w / nt / 21.0e6 * (tiles / nt > cus ? 1.9 : 1.0);
-    double flat = 1.5 + w / 6.4e6;
-    if (groups > 4 && tiles < 4ll * cus) {
-        flat += per_group * (groups - 1);      // six row groups in one pass, or four weight tiles per workgroup (see launch_flat)
-    } else {
-        flat += per_group * (mt - 1);
-        if (passes == 2) flat *= 1.55;      // the second pass reads the weights from L2
-    }
-    flat *= layout_factor;      // row-major weights: rows staged through LDS, rows a power of two apart share channels
-    // (the 128-tile kernel's own choice of tile width, narrow_tiles_pay, for one row of 128-row tiles)
-    const bool narrow = narrow_tiles_pay((n + 127) / 128, n, (int)std::min<long long>(row_bytes, 1 << 30));
-    const double per_workgroup = narrow ? 64.0 * (double)row_bytes / 22.0e3 : rounds * 128.0 * (double)row_bytes / 28.0e3;
-    double dense = 4.0 + std::max(per_workgroup, w / 5.0e6);
-    dense *= 1.0 + 0.2 * m / 128.0;
-    return flat <= dense;
+    return flat_is_faster(m, n, row_bytes, layout_factor, num_cus());
 }
 
 bool prefer_flat_fp8(const a8w8_gemm_args* g)
 {
     const bool mx = g->scale_mode == A8W8_SCALE_MX_E8M0_TILED;
     const double layout_factor = g->b_preshuffled ? 1.0 : g->stride_b % 4096 == 0 ? 1.3 : 1.05;
-    // (the flat kernel's MX scale bytes, one byte load per weight tile and K pair, cost it about a tenth)
+    // (MXFP8 costs the flat kernel more than the dense one: 1.0, 1.05 and 1.1 fit the measured cells equally well)
     return prefer_flat(g->m, g->n, g->k, layout_factor * (mx ? 1.1 : 1.0));
 }
 

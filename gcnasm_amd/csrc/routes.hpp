@@ -2,6 +2,7 @@
 // units, without the HIP runtime, so that they can be checked without a GPU.  Times in the comments: MI355X, 256 compute units,
 // us per launch inside a graph.
 #pragma once
+#include <algorithm>
 
 namespace a8w8 {
 
@@ -64,6 +65,118 @@ inline bool f4_row_scales_on_256_tiles(long long m, long long n, long long k_ste
     const long long rounds256 = (batch * ((m + 255) / 256) * ((n + 255) / 256) + cus - 1) / cus;
     if (k_steps < (fp32_c ? 8 : 4)) return false;
     return 2 * rounds128 >= (k_steps >= (fp32_c ? 16 : 12) ? 6 : 7) * rounds256;
+}
+
+// 128 x 64 tiles instead of 128 x 128: when the wide tiles would occupy at most half of the compute units and the K loop is long
+// enough for the deeper staging to matter (a problem of a few K steps is bound by launch and store latency, which narrower tiles
+// do not change).
+#ifndef A8W8_NARROW_MIN_KSTEPS
+#define A8W8_NARROW_MIN_KSTEPS 16
+#endif
+inline bool narrow_tiles_pay(long long items128, long long n, long long k_bytes, long long cus)
+{
+    return 2 * items128 <= cus && n > 64 && k_bytes / 128 >= A8W8_NARROW_MIN_KSTEPS;
+}
+
+// ---------------------------------------------------------------- flat GEMM (up to 128 activation rows)
+// Weight tiles (nt) and groups of 16 activation rows (mt) per workgroup of the flat GEMM.
+//
+// Below four weight tiles per compute unit: the smallest nt x mt whose workgroups all fit the chip at once.  Every workgroup is
+// eight waves and a chain of K pairs, reduction and store whose length grows with nt x mt, so a layer of few weight tiles goes out in
+// small pieces (row groups then read the weights once each, all but the first from L2), and one of many in pieces large enough for
+// a single round.  us, row/col / MXFP8, fixed splits -> these:
+//   64 x 1024 x 4096     2 x 4  8.7 / 9.9   -> 1 x 1  5.2 / 6.1       100 x 1024 x 4096   2 x 8, 2 x 4  13.2 / 9.8 -> 1 x 2  5.2 / 6.0
+//   64 x 4096 x 4096     2 x 4  9.2 / 10.5  -> 2 x 2  7.1 / 8.0       100 x 4096 x 4096   2 x 8, 2 x 4  14.2 / 10.6 -> 2 x 4  9.3 / 10.6
+//   64 x 9216 x 3584     2 x 4  14.6 / 17.8 -> 4 x 4  12.8 / 13.1     128 x 8192 x 8192   2 x 8, 2 x 4  25.9 / 33.4 -> 4 x 4  23.3 / 24.2
+//   128 x 12288 x 2560   2 x 8  20.7 -> 2 x 4 in three rounds 16.2 (MXFP8: 2 x 4 17.9 before and now, 4 x 4 19.0)
+//   16 x 5120 x 5120     1 x 1  9.9 / 11.4  -> 2 x 1  8.0 / 8.7       16 x 10240 x 8192   2 x 1  19.9 / 22.5 -> 4 x 1  17.4 / 18.6
+// Four row groups share a pass at most, six where their registers allow it (MX scales: only over a few K pairs; otherwise 4 x 4 on two
+// passes is faster, 80 x 7168 x 4096 14.6 -> 13.4).
+//
+// Two weight tiles stay two, in up to two rounds, where four would make the chain longer than they save:
+//  - rows of at most 1024 bytes (MX formats 512), one K pair or less per wave: four tiles only lengthen reduction and stores
+//    (four / two tiles: 32 x 14336 x 1024 6.1 / 5.5, block scales 48 x 14336 x 1024 7.4 / 6.7, MXFP4 64 x 12288 x 1024 6.1 / 5.8).  Not
+//    where a workgroup stages row-major weights beside three or four row groups (tensor 64 x 10240 x 512 two tiles 29% slower), nor
+//    for block scales with four groups (64 x 12288 x 512 18% slower);
+//  - up to eight activation rows over at least 3.25 tiles per compute unit, where two rounds of two tiles are nearly full and there
+//    are few activation bytes to share (four / two: 1 x 14336 x 8192 20.1 / 18.9, bf16 1 x 15360 x 4096 22.0 / 20.5); on row-major weights,
+//    whose rows a workgroup stages through LDS, for rows of up to 2048 bytes, without MX scales from two tiles on (1 x 12288 x 2048
+//    7.6 / 7.2, 16 x 15360 x 2048 8.8 / 8.4; beyond 2048 bytes four are 8 to 11% faster: bf16 8 x 13312 x 8192).
+// One tile stays one for up to four rows over row-major weights with per-tensor, row/col or no scales and rows of up to 8192 bytes
+// (two / one: 1 x 7168 x 8192 11.7 / 10.7, bf16 1 x 6144 x 4096 11.1 / 10.4; bf16 4 x 6144 x 8192 the other way, 8%).
+//
+// Layers of at least four weight tiles per compute unit take four, and an even split of the row groups over one or two passes (16384 x
+// 7168 at M = 48, 30 us with two tiles, 24 us with four).
+enum FlatKind { FLAT_FP8, FLAT_BLOCK, FLAT_BF16, FLAT_MXFP8, FLAT_MXFP4 };      // (FLAT_FP8: per-tensor and row/col scales)
+struct FlatSplit { int nt, mt; };
+inline FlatSplit flat_split(FlatKind kind, bool row_major, long long m, long long n, long long row_bytes, long long batch, long long cus)
+{
+    const bool mx = kind == FLAT_MXFP8 || kind == FLAT_MXFP4;
+    const long long tiles = n / 16 * batch;
+    const int groups = (int)((m + 15) / 16), passes = (groups + 3) / 4, mt = (groups + passes - 1) / passes;
+    if (tiles >= 4 * cus) return {4, mt};
+    const auto fits = [&](int nt, int g) { return (n / 16 + nt - 1) / nt * batch * ((groups + g - 1) / g) <= cus; };
+    const bool short_rows = row_bytes <= (mx ? 512 : 1024);
+    if (fits(1, 1)) return {1, 1};
+    if (groups == 1) {
+        if (fits(2, 1)) return row_major && (kind == FLAT_FP8 || kind == FLAT_BF16) && m <= 4 && row_bytes <= 8192 ? FlatSplit{1, 1} : FlatSplit{2, 1};
+        const bool two_rounds_full = m <= 8 && 4 * tiles >= 13 * cus;
+        return short_rows || (row_major ? row_bytes <= 2048 && (!mx || two_rounds_full) : two_rounds_full) ? FlatSplit{2, 1} : FlatSplit{4, 1};
+    }
+    if (fits(1, 2)) return {1, 2};
+    if (fits(2, 2)) return {2, 2};
+    if (groups > 2 && fits(2, 3)) return {2, 3};
+    if (groups > 2 && fits(2, 4)) return {2, 4};
+    if (groups <= 4) return {short_rows && (groups == 2 || (!row_major && !(kind == FLAT_BLOCK && groups == 4))) ? 2 : 4, mt};
+    if (groups <= 6) return !mx || short_rows ? FlatSplit{2, 6} : FlatSplit{4, 4};
+    if (!fits(4, 4) || (kind == FLAT_MXFP4 && !row_major && short_rows)) return {2, 4};
+    return {4, 4};
+}
+
+// The flat GEMM against the 128-tile kernel on problems of at most 128 activation rows: true where this cost model calls the flat one
+// faster.  Times in microseconds, W = weight bytes, row_bytes = bytes of one weight row:
+//   flat:  one pass over the weights at ~6.4 TB/s; every further group of 16 activation rows adds the activation rows
+//          that each workgroup reads again for its weight tiles, W / NT bytes at ~21 TB/s (1.4 us on 16384 x 7168), nearly twice
+//          that where the workgroups do not fit the chip at once; a second pass (more than 64 rows over at least four weight
+//          tiles per compute unit) reads the weights from L2 and costs 55% more; MXFP8 a tenth (layout_factor).
+//   dense: the 128-tile kernel pulls the weights with one workgroup per 128 weight rows at ~28 GB/s each, or, where
+//          128 x 128 tiles would occupy at most half of the compute units, per 64 rows at ~22 GB/s each (its 128 x 64
+//          tiles), ~5 TB/s at best over the chip; 20% more at 128 activation rows than at a few.
+// Weights of at most 32 MiB (per batch entry) always go flat.  Measured, shuffled FP8 weights, M = 16 / 32 / 48 / 64 / 80 / 96 / 128, flat
+// against dense:
+//   16384 x 7168   20 / 21 / 23 / 24 / 35 / 36 / 41  against  30 / 27 / 27 / 28 / 30 / 31 / 33   (MXFP8 about 10% more on both sides)
+//   8192 x 8192    13 / 14 / 16 / 18 / 21 / 22 / 23  against  26 / 26 / 26 / 27 / 28 / 29 / 31
+//   28672 x 4096   20 / 23 / 25 / 28 / 39 / 41 / 47  against  26 / 26 / 27 / 28 / 29 / 30 / 31
+//   4096 x 14336   13 / .. / .. / 19 / 23 / .. / 27  against  41 throughout
+// (tests/test_zz_gpu_routing.py times both sides of such cells through a8w8_route_override and checks the choice).
+// NT here is what the fit was made with, not what flat_split takes today: four for one to four groups past two tiles per compute
+// unit, but two for five to eight groups there, whose 2 x 6 or 4 x 4 on two passes costs per group as two tiles do (four in the
+// formula: 21% of 3936 cells more than 10% off, two: 7%).
+inline bool flat_is_faster(long long m, long long n, long long row_bytes, double layout_factor, long long cus)
+{
+    const double w_entry = (double)n * (double)row_bytes;
+    if (w_entry <= (double)(32ll << 20)) return true;
+    const int groups = (int)((m + 15) / 16), passes = (groups + 3) / 4, mt = (groups + passes - 1) / passes;
+    const long long entries = 1;
+    const double w = w_entry * (double)entries;
+    const long long tiles = n / 16 * entries, tiles128 = (n + 127) / 128 * entries;
+    const int nt = tiles >= 4 * cus || (groups <= 4 && tiles > 2 * cus) ? 4 : tiles > cus ? 2 : 1;
+    const double per_group = w / nt / 21.0e6 * (tiles / nt > cus ? 1.9 : 1.0);
+    double flat = 1.5 + w / 6.4e6;
+    if (groups > 4 && tiles < 4 * cus) {
+        flat += per_group * (groups - 1);      // six row groups in one pass, or two passes of workgroups of four (see flat_split)
+    } else {
+        flat += per_group * (mt - 1);
+        if (passes == 2) flat *= 1.55;         // the second pass reads the weights from L2
+    }
+    flat *= layout_factor;      // row-major weights: rows staged through LDS, rows a power of two apart share channels
+    // (the 128-tile kernel's own choice of tile width for one row of 128-row tiles)
+    const bool narrow = narrow_tiles_pay(tiles128, n, row_bytes, cus);
+    const long long rounds = (tiles128 + cus - 1) / cus;
+    const double per_workgroup = narrow ? 64.0 * (double)row_bytes / 22.0e3 : (double)rounds * 128.0 * (double)row_bytes / 28.0e3;
+    double dense = 4.0 + std::max(per_workgroup, w / 5.0e6);
+    dense *= 1.0 + 0.2 * (double)m / 128.0;
+    return flat <= dense;
 }
 
 }  // namespace a8w8

@@ -13,4 +13,10 @@ int route_f4_row_scales_on_256_tiles(long long m, long long n, long long k_steps
 {
     return a8w8::f4_row_scales_on_256_tiles(m, n, k_steps, batch, fp32_c != 0, cus);
 }
+// 10 nt + mt
+int route_flat_split(int kind, int row_major, long long m, long long n, long long row_bytes, long long batch, long long cus)
+{
+    const a8w8::FlatSplit f = a8w8::flat_split((a8w8::FlatKind)kind, row_major != 0, m, n, row_bytes, batch, cus);
+    return 10 * f.nt + f.mt;
+}
 }

@@ -40,3 +40,13 @@ def quant_1x128_along_rows(rows, k):
 def f4_row_scales_on_256_tiles(m, n, k, batch=1, fp32=False, cus=256):
     """k in elements; for problems of more than two 128-tiles per compute unit whose K and scale rows the four-wave kernel takes."""
     return bool(lib().route_f4_row_scales_on_256_tiles(_ll(m), _ll(n), _ll(k // 256), _ll(batch), int(fp32), _ll(cus)))
+
+
+KINDS = ("fp8", "block", "bf16", "mxfp8", "mxfp4")          # enum FlatKind
+BYTES = {"bf16": 2.0, "mxfp4": 0.5}                          # per element of a weight row, else 1
+
+
+def flat_split(kind, row_major, m, n, k, batch=1, cus=256):
+    """(weight tiles, row groups) per workgroup of the flat GEMM; k in elements."""
+    split = lib().route_flat_split(KINDS.index(kind), int(row_major), _ll(m), _ll(n), _ll(int(k * BYTES.get(kind, 1))), _ll(batch), _ll(cus))
+    return split // 10, split % 10

@@ -44,3 +44,18 @@ def test_1x128_quantiser(rows, k, along):
 def test_mxfp4_row_major_scales_past_two_tiles_per_compute_unit(m, n, k, bf16, fp32):
     assert routes.f4_row_scales_on_256_tiles(m, n, k) is bf16
     assert routes.f4_row_scales_on_256_tiles(m, n, k, fp32=True) is fp32
+
+
+# the flat GEMM's splits on both sides of their lines, 256 compute units; (weight tiles, row groups) per workgroup
+@pytest.mark.parametrize("kind,row_major,m,n,k,split", [
+    ("fp8", False, 16, 4096, 4096, (1, 1)), ("fp8", False, 16, 5120, 8192, (2, 1)), ("fp8", True, 16, 5120, 8192, (2, 1)),
+    ("fp8", True, 1, 7168, 8192, (1, 1)), ("bf16", True, 4, 6144, 4096, (1, 1)), ("bf16", True, 4, 6144, 8192, (2, 1)), ("block", True, 1, 7168, 8192, (2, 1)),
+    ("mxfp8", True, 1, 7168, 8192, (2, 1)), ("fp8", False, 16, 10240, 8192, (4, 1)), ("fp8", False, 1, 14336, 8192, (2, 1)), ("fp8", False, 16, 14336, 8192, (4, 1)),
+    ("bf16", False, 8, 15360, 4096, (2, 1)), ("fp8", True, 1, 12288, 2048, (2, 1)), ("fp8", True, 8, 13312, 8192, (4, 1)), ("mxfp8", True, 1, 14336, 2048, (2, 1)),
+    ("mxfp8", True, 16, 14336, 2048, (4, 1)), ("fp8", False, 32, 14336, 1024, (2, 2)), ("fp8", False, 32, 14336, 4096, (4, 2)),
+    ("block", False, 48, 14336, 1024, (2, 3)), ("block", False, 64, 14336, 1024, (4, 4)), ("fp8", True, 64, 14336, 512, (4, 4)), ("fp8", False, 64, 14336, 512, (2, 4)),
+    ("mxfp4", False, 64, 12288, 1024, (2, 4)), ("mxfp4", False, 64, 12288, 4096, (4, 4)), ("mxfp8", False, 48, 14336, 1024, (4, 3)), ("fp8", False, 96, 8192, 8192, (2, 6)),
+    ("mxfp8", False, 96, 8192, 8192, (4, 4)), ("mxfp4", False, 80, 5120, 1024, (2, 6)), ("fp8", False, 128, 8192, 8192, (4, 4)), ("fp8", False, 128, 12288, 2560, (2, 4)),
+    ("fp8", False, 100, 1024, 4096, (1, 2)), ("fp8", False, 48, 16384, 7168, (4, 3)), ("fp8", False, 80, 16384, 7168, (4, 3)), ("fp8", False, 128, 16384, 7168, (4, 4))])
+def test_flat_splits(kind, row_major, m, n, k, split):
+    assert routes.flat_split(kind, row_major, m, n, k) == split
