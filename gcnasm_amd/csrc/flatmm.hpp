@@ -168,6 +168,7 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
                            : (uint32_t)(m0 + g * 16 + ld_row) * (uint32_t)p.lda + ld_piece * 16;
     v4i* stage = smem + wave * (STAGED * FLAT_STAGE_SLOTS);
     constexpr uint32_t PAST_K = 0x80000000u;             // beyond every descriptor's extent
+    constexpr bool ODD_BLOCKS = MODE != MODE_BLOCK;      // K may be an odd number of 64-wide blocks (block scales: whole 128-wide groups)
     const bool second_past_k = ld_piece >= 4;            // the lane's piece lies in the second K block of a pair
     const int st_write = ld_piece * 18 + ld_row;         // row + 8 is 8 slots on
     const int st_read = kq * 18 + r16;                   // piece kq, the second K block's is 4 * 18 slots on
@@ -263,7 +264,7 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
         // pieces 4 .. 7 are the second K block of the pair: past the end of K (an odd number of blocks) they get an
         // offset beyond the descriptor's extent instead of a branch, which reads as zero and touches no memory
         // (2^31 in place of the lane's offset, not on top of it: with the scalar offset that could pass 2^32 and wrap into the matrix)
-        const uint32_t off = second_past_k && 2 * pp + 1 >= k_tiles ? PAST_K : a_off[0];
+        const uint32_t off = ODD_BLOCKS && second_past_k && 2 * pp + 1 >= k_tiles ? PAST_K : a_off[0];
 #pragma unroll
         for (int g = 0; g < MT; ++g) {
             // (group g is 16 g rows on: a scalar offset, so that one lane offset serves every group)
@@ -272,7 +273,7 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
         }
     };
     auto load_weight_rows = [&](int pp) {
-        const uint32_t off = second_past_k && 2 * pp + 1 >= k_tiles ? PAST_K : b_off[0];
+        const uint32_t off = ODD_BLOCKS && second_past_k && 2 * pp + 1 >= k_tiles ? PAST_K : b_off[0];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             // (tile t is 16 t rows on: a scalar offset, one lane offset for every tile)
@@ -303,7 +304,7 @@ __global__ void __launch_bounds__(FLAT_THREADS) flatmm_a8w8(GemmParams p)
     };
     auto load = [&](int pp, Frag& f) {
         const int kt0 = 2 * pp, kt1 = 2 * pp + 1;
-        const bool past1 = kt1 >= k_tiles;      // the second K block reads as zero, see load_rows
+        const bool past1 = ODD_BLOCKS && kt1 >= k_tiles;      // the second K block reads as zero, see load_rows
         if constexpr (MT == 1) {
             f.a[0] = ld16(rs_a, a_off[0], kt0 * 64);
             f.a[1] = ld16(rs_a, past1 ? PAST_K : a_off[0], kt1 * 64);
