@@ -97,7 +97,8 @@ inline bool narrow_tiles_pay(long long items128, long long n, long long k_bytes,
 //  - rows of at most 1024 bytes (MX formats 512), one K pair or less per wave: four tiles only lengthen reduction and stores
 //    (four / two tiles: 32 x 14336 x 1024 6.1 / 5.5, block scales 48 x 14336 x 1024 7.4 / 6.7, MXFP4 64 x 12288 x 1024 6.1 / 5.8).  Not
 //    where a workgroup stages row-major weights beside three or four row groups (tensor 64 x 10240 x 512 two tiles 29% slower), nor
-//    for block scales with four groups (64 x 12288 x 512 18% slower);
+//    for block scales with four groups (64 x 12288 x 512 18% slower), nor for nine to sixteen rows over rows of more than 512 bytes
+//    and less than 3.25 tiles per compute unit (16 x 10240 x 1024 4% slower);
 //  - up to eight activation rows over at least 3.25 tiles per compute unit, where two rounds of two tiles are nearly full and there
 //    are few activation bytes to share (four / two: 1 x 14336 x 8192 20.1 / 18.9, bf16 1 x 15360 x 4096 22.0 / 20.5); on row-major weights,
 //    whose rows a workgroup stages through LDS, for rows of up to 2048 bytes, without MX scales from two tiles on (1 x 12288 x 2048
@@ -120,7 +121,8 @@ inline FlatSplit flat_split(FlatKind kind, bool row_major, long long m, long lon
     if (fits(1, 1)) return {1, 1};
     if (groups == 1) {
         if (fits(2, 1)) return row_major && (kind == FLAT_FP8 || kind == FLAT_BF16) && m <= 4 && row_bytes <= 8192 ? FlatSplit{1, 1} : FlatSplit{2, 1};
-        const bool two_rounds_full = m <= 8 && 4 * tiles >= 13 * cus;
+        const bool full = 4 * tiles >= 13 * cus, two_rounds_full = m <= 8 && full;
+        if (m > 8 && !full && row_bytes > 512) return {4, 1};
         return short_rows || (row_major ? row_bytes <= 2048 && (!mx || two_rounds_full) : two_rounds_full) ? FlatSplit{2, 1} : FlatSplit{4, 1};
     }
     if (fits(1, 2)) return {1, 2};

@@ -85,7 +85,7 @@ def _split_cases(kind, row_major):
         cases += [((2, 3), 48, two, short)] + ([] if kind == "block" else [((2, 4), 64, two, short)])
         cases += [((2, 1), 8, 13312, long), ((4, 1), 9, 13312, long)]
     elif kind in ("fp8", "bf16"):
-        cases += [((1, 1), 4, odd, 640), ((2, 1), 16, two, 1024)]
+        cases += [((1, 1), 4, odd, 640), ((2, 1), 8, two, 1024)]
     return cases
 
 

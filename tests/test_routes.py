@@ -50,7 +50,8 @@ def test_mxfp4_row_major_scales_past_two_tiles_per_compute_unit(m, n, k, bf16, f
 @pytest.mark.parametrize("kind,row_major,m,n,k,split", [
     ("fp8", False, 16, 4096, 4096, (1, 1)), ("fp8", False, 16, 5120, 8192, (2, 1)), ("fp8", True, 16, 5120, 8192, (2, 1)),
     ("fp8", True, 1, 7168, 8192, (1, 1)), ("bf16", True, 4, 6144, 4096, (1, 1)), ("bf16", True, 4, 6144, 8192, (2, 1)), ("block", True, 1, 7168, 8192, (2, 1)),
-    ("mxfp8", True, 1, 7168, 8192, (2, 1)), ("fp8", False, 16, 10240, 8192, (4, 1)), ("fp8", False, 1, 14336, 8192, (2, 1)), ("fp8", False, 16, 14336, 8192, (4, 1)),
+    ("mxfp8", True, 1, 7168, 8192, (2, 1)), ("fp8", False, 16, 10240, 8192, (4, 1)), ("fp8", False, 16, 10240, 1024, (4, 1)), ("fp8", False, 8, 10240, 1024, (2, 1)), ("fp8", False, 16, 14336, 1024, (2, 1)),
+    ("fp8", True, 16, 9216, 512, (2, 1)), ("fp8", False, 1, 14336, 8192, (2, 1)), ("fp8", False, 16, 14336, 8192, (4, 1)),
     ("bf16", False, 8, 15360, 4096, (2, 1)), ("fp8", True, 1, 12288, 2048, (2, 1)), ("fp8", True, 8, 13312, 8192, (4, 1)), ("mxfp8", True, 1, 14336, 2048, (2, 1)),
     ("mxfp8", True, 16, 14336, 2048, (4, 1)), ("fp8", False, 32, 14336, 1024, (2, 2)), ("fp8", False, 32, 14336, 4096, (4, 2)),
     ("block", False, 48, 14336, 1024, (2, 3)), ("block", False, 64, 14336, 1024, (4, 4)), ("fp8", True, 64, 14336, 512, (4, 4)), ("fp8", False, 64, 14336, 512, (2, 4)),
