@@ -503,10 +503,10 @@ int launch_flat(const GemmParams& p, int batch, hipStream_t stream)
 // (13 / 14 / 18 shuffled).
 int g_route = A8W8_ROUTE_MODEL;      // a8w8_route_override
 
-bool prefer_flat(int m, int n, long long row_bytes, double layout_factor = 1.0)
+bool prefer_flat(int m, int n, long long row_bytes, int batch, double layout_factor = 1.0)
 {
     if (g_route != A8W8_ROUTE_MODEL) return g_route == A8W8_ROUTE_FLAT;
-    return flat_is_faster(m, n, row_bytes, layout_factor, num_cus());
+    return flat_is_faster(m, n, row_bytes, batch, layout_factor, num_cus());
 }
 
 bool prefer_flat_fp8(const a8w8_gemm_args* g)
@@ -514,7 +514,7 @@ bool prefer_flat_fp8(const a8w8_gemm_args* g)
     const bool mx = g->scale_mode == A8W8_SCALE_MX_E8M0_TILED;
     const double layout_factor = g->b_preshuffled ? 1.0 : g->stride_b % 4096 == 0 ? 1.3 : 1.05;
     // (MXFP8 costs the flat kernel more than the dense one: 1.0, 1.05 and 1.1 fit the measured cells equally well)
-    return prefer_flat(g->m, g->n, g->k, layout_factor * (mx ? 1.1 : 1.0));
+    return prefer_flat(g->m, g->n, g->k, g->batch, layout_factor * (mx ? 1.1 : 1.0));
 }
 
 template <bool BROW>
@@ -644,7 +644,7 @@ static int a16w16_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allo
 {
     if (!g) return A8W8_ERR_NULL_POINTER;
     // a skinny problem on shuffled weights: the flat kernel where it is the faster one (and can run it)
-    if (allow_flat && g->b_preshuffled && g->m > 0 && g->m <= FLAT_MAX_M && prefer_flat(g->m, g->n, 2ll * g->k) &&
+    if (allow_flat && g->b_preshuffled && g->m > 0 && g->m <= FLAT_MAX_M && prefer_flat(g->m, g->n, 2ll * g->k, g->batch) &&
         a16w16_flat_impl(g, hip_stream, false) == A8W8_OK)
         return A8W8_OK;
     if (!g->a || !g->b || !g->c) return A8W8_ERR_NULL_POINTER;
@@ -662,7 +662,7 @@ static int a16w16_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allo
     bytes.stride_a_batch = g->stride_a_batch * 2; bytes.stride_b_batch = g->stride_b_batch * 2;
     bytes.scale_mode = A8W8_SCALE_TENSOR;
     const bool fits = (long long)g->stride_a_batch * 2 < (1ll << 31) && (long long)g->stride_b_batch * 2 < (1ll << 31);
-    const bool flat_rows = fits && flat_rowmajor_ok(&bytes) && prefer_flat(g->m, g->n, bytes.k, bytes.stride_b % 4096 == 0 ? 1.3 : 1.05);
+    const bool flat_rows = fits && flat_rowmajor_ok(&bytes) && prefer_flat(g->m, g->n, bytes.k, g->batch, bytes.stride_b % 4096 == 0 ? 1.3 : 1.05);
     if (!flat_rows && fits && c_stride_too_large(g, &bytes)) return A8W8_ERR_TOO_LARGE;
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     hipStream_t s = (hipStream_t)hip_stream;
@@ -713,7 +713,7 @@ static int a4w4_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
 {
     if (!g) return A8W8_ERR_NULL_POINTER;
     // a skinny problem on shuffled weights: the flat kernel where it is the faster one (and can run it)
-    if (allow_flat && g->b_preshuffled && g->m > 0 && g->m <= FLAT_MAX_M && prefer_flat(g->m, g->n, g->k / 2) &&
+    if (allow_flat && g->b_preshuffled && g->m > 0 && g->m <= FLAT_MAX_M && prefer_flat(g->m, g->n, g->k / 2, g->batch) &&
         a4w4_flat_impl(g, hip_stream, false) == A8W8_OK)
         return A8W8_OK;
     if (!g->a || !g->b || !g->c || !g->sfa || !g->sfb) return A8W8_ERR_NULL_POINTER;
@@ -738,7 +738,7 @@ static int a4w4_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
     bytes.stride_a = g->stride_a / 2; bytes.stride_b = g->b_preshuffled ? bytes.k : g->stride_b / 2;
     bytes.stride_a_batch = g->stride_a_batch / 2; bytes.stride_b_batch = g->stride_b_batch / 2;
     bytes.scale_mode = A8W8_SCALE_MX_E8M0_TILED;
-    const bool flat_rows = tiled && flat_rowmajor_ok(&bytes) && prefer_flat(g->m, g->n, bytes.k, bytes.stride_b % 4096 == 0 ? 1.3 : 1.05);
+    const bool flat_rows = tiled && flat_rowmajor_ok(&bytes) && prefer_flat(g->m, g->n, bytes.k, g->batch, bytes.stride_b % 4096 == 0 ? 1.3 : 1.05);
     if (!flat_rows && tiled && g->k % 256 == 0 && c_stride_too_large(g, &bytes)) return A8W8_ERR_TOO_LARGE;
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     hipStream_t s = (hipStream_t)hip_stream;
@@ -811,7 +811,7 @@ static int a4w4_flat_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
     if ((long long)g->n * g->k / 2 >= (1ll << 31) || g->batch > 65535) return A8W8_ERR_TOO_LARGE;
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     // several groups of 16 rows over weights too large to stay in cache: the MFMA kernels read the same weights
-    if (allow_dense && !prefer_flat(g->m, g->n, g->k / 2) && a4w4_gemm_impl(g, hip_stream, false) == A8W8_OK)
+    if (allow_dense && !prefer_flat(g->m, g->n, g->k / 2, g->batch) && a4w4_gemm_impl(g, hip_stream, false) == A8W8_OK)
         return A8W8_OK;
     a8w8_gemm_args bytes = *g;      // packed rows as byte rows of k/2 columns
     bytes.k = g->k / 2;
@@ -859,7 +859,7 @@ static int a16w16_flat_impl(const a8w8_gemm_args* g, void* hip_stream, bool allo
         return A8W8_ERR_TOO_LARGE;
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     // several groups of 16 rows over weights too large to stay in cache: the MFMA kernels read the same weights
-    if (allow_dense && !prefer_flat(g->m, g->n, 2ll * g->k) && a16w16_gemm_impl(g, hip_stream, false) == A8W8_OK)
+    if (allow_dense && !prefer_flat(g->m, g->n, 2ll * g->k, g->batch) && a16w16_gemm_impl(g, hip_stream, false) == A8W8_OK)
         return A8W8_OK;
     a8w8_gemm_args bytes = *g;      // bf16 rows as byte rows of 2k columns
     bytes.k = g->k * 2;

@@ -150,19 +150,25 @@ inline FlatSplit flat_split(FlatKind kind, bool row_major, long long m, long lon
 //   8192 x 8192    13 / 14 / 16 / 18 / 21 / 22 / 23  against  26 / 26 / 26 / 27 / 28 / 29 / 31
 //   28672 x 4096   20 / 23 / 25 / 28 / 39 / 41 / 47  against  26 / 26 / 27 / 28 / 29 / 30 / 31
 //   4096 x 14336   13 / .. / .. / 19 / 23 / .. / 27  against  41 throughout
-// (tests/test_zz_gpu_routing.py times both sides of such cells through a8w8_route_override and checks the choice).
+// (tests/test_zz_gpu_routing.py times both sides of such cells through a8w8_route_override and checks the choice).  Over 3936 cells (six kinds
+// of operands, both layouts, M = 16 .. 128, 2048 .. 28672 columns, batches of 1, 2 and 4) the choice costs 1.0% over the better
+// side in the mean and is more than 10% off in 4% of them.
 // NT here is what the fit was made with, not what flat_split takes today: four for one to four groups past two tiles per compute
 // unit, but two for five to eight groups there, whose 2 x 6 or 4 x 4 on two passes costs per group as two tiles do (four in the
-// formula: 21% of 3936 cells more than 10% off, two: 7%).
-inline bool flat_is_faster(long long m, long long n, long long row_bytes, double layout_factor, long long cus)
+// formula: 17% of the cells more than 10% off).
+// The batch: more than four groups are priced over all entries together (128 x 8192 x 8192 MXFP8, four entries: flat 99, dense 66).  Up to
+// four are priced by the entry, which is within 5% except between two and four tiles per compute unit on more than 128 MiB of weights
+// in all (64 x 14336 x 14336, two entries: flat 88, dense 78; 64 x 14336 x 4096, two: 28, 31): two tiles there, as for large grids.
+inline bool flat_is_faster(long long m, long long n, long long row_bytes, long long batch, double layout_factor, long long cus)
 {
     const double w_entry = (double)n * (double)row_bytes;
     if (w_entry <= (double)(32ll << 20)) return true;
     const int groups = (int)((m + 15) / 16), passes = (groups + 3) / 4, mt = (groups + passes - 1) / passes;
-    const long long entries = 1;
+    const long long entries = groups > 4 ? std::max(batch, 1ll) : 1;
     const double w = w_entry * (double)entries;
     const long long tiles = n / 16 * entries, tiles128 = (n + 127) / 128 * entries;
-    const int nt = tiles >= 4 * cus || (groups <= 4 && tiles > 2 * cus) ? 4 : tiles > cus ? 2 : 1;
+    const bool small_batch = batch <= 1 || w_entry * (double)batch <= (double)(128ll << 20);
+    const int nt = tiles >= 4 * cus || (groups <= 4 && tiles > 2 * cus && small_batch) ? 4 : tiles > cus ? 2 : 1;
     const double per_group = w / nt / 21.0e6 * (tiles / nt > cus ? 1.9 : 1.0);
     double flat = 1.5 + w / 6.4e6;
     if (groups > 4 && tiles < 4 * cus) {

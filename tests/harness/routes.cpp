@@ -19,4 +19,8 @@ int route_flat_split(int kind, int row_major, long long m, long long n, long lon
     const a8w8::FlatSplit f = a8w8::flat_split((a8w8::FlatKind)kind, row_major != 0, m, n, row_bytes, batch, cus);
     return 10 * f.nt + f.mt;
 }
+int route_flat_is_faster(long long m, long long n, long long row_bytes, long long batch, double layout_factor, long long cus)
+{
+    return a8w8::flat_is_faster(m, n, row_bytes, batch, layout_factor, cus);
+}
 }

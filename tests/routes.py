@@ -50,3 +50,10 @@ def flat_split(kind, row_major, m, n, k, batch=1, cus=256):
     """(weight tiles, row groups) per workgroup of the flat GEMM; k in elements."""
     split = lib().route_flat_split(KINDS.index(kind), int(row_major), _ll(m), _ll(n), _ll(int(k * BYTES.get(kind, 1))), _ll(batch), _ll(cus))
     return split // 10, split % 10
+
+
+def flat_is_faster(kind, row_major, m, n, k, batch=1, cus=256):
+    """The flat GEMM's side of the cost model, with the layout factors of the entry points; k in elements."""
+    row_bytes = int(k * BYTES.get(kind, 1))
+    factor = (1.1 if kind == "mxfp8" else 1.0) * ((1.3 if row_bytes % 4096 == 0 else 1.05) if row_major else 1.0)
+    return bool(lib().route_flat_is_faster(_ll(m), _ll(n), _ll(row_bytes), _ll(batch), ctypes.c_double(factor), _ll(cus)))

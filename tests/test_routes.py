@@ -60,3 +60,19 @@ def test_mxfp4_row_major_scales_past_two_tiles_per_compute_unit(m, n, k, bf16, f
     ("fp8", False, 100, 1024, 4096, (1, 2)), ("fp8", False, 48, 16384, 7168, (4, 3)), ("fp8", False, 80, 16384, 7168, (4, 3)), ("fp8", False, 128, 16384, 7168, (4, 4))])
 def test_flat_splits(kind, row_major, m, n, k, split):
     assert routes.flat_split(kind, row_major, m, n, k) == split
+
+
+@pytest.mark.parametrize("kind,row_major,m,n,k,batch,flat", [
+    ("fp8", False, 16, 16384, 7168, 1, True), ("fp8", False, 128, 16384, 7168, 1, False), ("fp8", False, 128, 8192, 8192, 1, True),
+    ("mxfp8", True, 128, 8192, 8192, 4, False), ("mxfp8", True, 128, 8192, 8192, 2, False), ("bf16", False, 96, 8192, 8192, 2, False),
+    ("fp8", True, 64, 14336, 14336, 2, False), ("fp8", True, 64, 14336, 4096, 2, True), ("mxfp4", True, 64, 14336, 14336, 4, False),
+    ("block", False, 64, 14336, 4096, 4, False), ("fp8", True, 64, 8192, 8192, 4, True), ("bf16", True, 64, 8192, 8192, 4, True),
+    ("fp8", False, 96, 4096, 4096, 16, True)])
+def test_flat_against_dense(kind, row_major, m, n, k, batch, flat):
+    """The side of cells whose two sides were measured to be more than 5% apart; a batch counts where more than four row groups share
+    the weights of an entry, and past 128 MiB of weights between two and four weight tiles per compute unit."""
+    assert routes.flat_is_faster(kind, row_major, m, n, k, batch) is flat
+    if kind in ("fp8", "mxfp8", "block"):
+        mode = {"fp8": g.ROWCOL, "mxfp8": g.MX_TILED, "block": g.BLOCK}[kind]
+        args = g.raw_gemm_args(1 << 12, 1 << 12, 1 << 12, 1 << 12, 1 << 12, m, n, k, mode, batch=batch, b_preshuffled=int(not row_major))
+        assert (g.kernel_name(args) == "flatmm_a8w8") is flat
