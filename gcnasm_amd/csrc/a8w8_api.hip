@@ -278,37 +278,14 @@ int num_cus()
     return g_dev[dev].num_cus > 0 ? g_dev[dev].num_cus : 256;
 }
 
-// 128 x 128 tiles when all of them fit on the chip at once, two workgroups per compute unit: a problem of that
-// size leaves 256 x 256 tiles with at most half of the compute units.  Measured on 256 compute units against the
-// 256-tile kernels (block / row-col / tiled MX): 2.2x / 1.7x / 1.6x at 64 workgroups, 1.9x / 1.6x / 1.5x at 256,
-// +45% / +21% / +15% at 400, +37% / +17% / +9% at 512; beyond that the second round of workgroups costs more than
-// the idle compute units did (-9% for row/col at 576).
-// (the bound as a switch, for measurement: with 8 instead of 2, 4096 x 7168 x 2048 and 4096^3 take 12-30% longer in every scale mode)
-#ifndef A8W8_SMALL_TILES_PER_CU
-#define A8W8_SMALL_TILES_PER_CU 2
-#endif
-#ifndef A8W8_SMALL_DEEP_UP_TO
-#define A8W8_SMALL_DEEP_UP_TO 1         // four LDS stages up to this many 128-tiles per compute unit, two stages beyond
-#endif
+// Two 128-tiles per compute unit at most (fits_128_tiles).
 bool small_ok(const a8w8_gemm_args* g)
 {
     const bool mxt = g->scale_mode == A8W8_SCALE_MX_E8M0_TILED;
     // tiled MX scales with an odd number of K steps have no 256-tile kernel: any size runs here
     if (mxt && (g->k / BK) % 2 != 0) return true;
-    const long long items128 = (long long)g->batch * ((g->m + SM_BM - 1) / SM_BM) * ((g->n + SM_BN - 1) / SM_BN);
-    return items128 <= (long long)A8W8_SMALL_TILES_PER_CU * num_cus();
+    return fits_128_tiles(g->m, g->n, g->batch, num_cus());
 }
-
-// 256 x 128 tiles where 128 x 128 ones would put two workgroups on a compute unit, 256 x 128 ones would not, and the K loop is
-// long enough to make up for a prologue and a tile's stores that no second workgroup hides.  us per launch, bf16 C, two-stage
-// 128-tiles -> 256 x 128 (row/col, row-major MX, tiled MX, MXFP4 row-major / tiled, bf16):
-//   2560^3            22.2 -> 20.3, 26.1 -> 23.5, 23.3 -> 20.3, 16.8 / 13.9 -> 16.7 / 14.1, 41.3 -> 36.5
-//   2049x3584x4096    34.6 -> 28.5, 45.1 -> 36.0, 35.7 -> 30.2, 29.0 / 21.7 -> 24.6 / 19.8, 66.4 -> 51.5
-//   512x16384x7168    67.3 -> 57.1, 88.6 -> 81.5, 71.1 -> 60.2, 42.7 / 33.3 -> 39.1 / 29.5, 126.4 -> 112.5
-//   2048x4096x2048    18.0 -> 18.1, 21.3 -> 20.2, 19.4 -> 18.6, 15.2 / 12.7 -> 15.8 / 13.5, 31.1 -> 30.1
-//   1000x8192x1024    14.2 -> 14.7, 14.9 -> 15.2, 14.3 -> 14.4, 11.8 / 10.7 -> 13.3 / 12.1, 19.1 -> 20.1
-// i.e. the line lies at 16 steps of 128 bytes, and where a step's scales cost next to nothing beside its short MFMAs at 24.
-constexpr int tall_min_ksteps(int mode) { return mode == MODE_BF16 || mode == MODE_F4T ? 24 : 16; }
 
 template <int MODE, int CDT, int STAGES, bool RAGGED>
 int launch_small_stages(const GemmParams& q, int batch, hipStream_t stream)
@@ -317,40 +294,33 @@ int launch_small_stages(const GemmParams& q, int batch, hipStream_t stream)
     return launch(gemm_a8w8_tile128<MODE, CDT, STAGES, SM_BN, RAGGED>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, STAGES), stream, q);
 }
 
-// Up to one workgroup per compute unit: four LDS stages (deep prefetch, one workgroup per compute unit).  More: two
-// stages, so that two workgroups share a compute unit and hide each other's waits.
+// The tile shape and depth of staging are tile128_variant's.
 template <int MODE, int CDT, bool RAGGED = false>
 int launch_small(const GemmParams& p, int batch, hipStream_t stream)
 {
-    if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BLOCK || MODE == MODE_MX || MODE == MODE_MXT ||
-                  MODE == MODE_BF16 || MODE == MODE_F4T || MODE == MODE_F4) {
-        GemmParams q = p;
-        q.tiles_m = (p.m + SM_BM - 1) / SM_BM;
-        q.tiles_n = (p.n + SM_BN - 1) / SM_BN;
-        const long long items = (long long)q.tiles_m * q.tiles_n * batch;
-        if (narrow_tiles_pay(items, p.n, p.k, num_cus())) {
-            // short and wide: 128 x 64 tiles give every compute unit a workgroup, deep staging keeps its share of the
-            // weights in flight
+    GemmParams q = p;
+    q.tiles_m = (p.m + SM_BM - 1) / SM_BM;
+    q.tiles_n = (p.n + SM_BN - 1) / SM_BN;
+    // (256 x 128 tiles leave rows past the end to the buffer descriptors: the 32-bit offsets of a whole tile must not wrap)
+    const bool tall = MODE != MODE_BLOCK && !RAGGED && (p.m + 256ll) * p.lda + p.k < (1ll << 32) && (p.n + 128ll) * p.ldb + p.k < (1ll << 32);
+    switch (tile128_variant(p.m, p.n, p.k, batch, tall, MODE == MODE_BF16 || MODE == MODE_F4T, num_cus())) {
+        case TILES_128x64: {
             q.tiles_n = (p.n + 63) / 64;
             dim3 grid((unsigned)(q.tiles_m * q.tiles_n), 1, (unsigned)batch);
             constexpr int ST = narrow_stages(MODE);
             return launch(gemm_a8w8_tile128<MODE, CDT, ST, 64, RAGGED>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, ST, 64), stream, q);
         }
-        if (items <= (long long)A8W8_SMALL_DEEP_UP_TO * num_cus())
+        case TILES_128_FOUR_STAGES:
             return launch_small_stages<MODE, CDT, 4, RAGGED>(q, batch, stream);
-        if constexpr (MODE != MODE_BLOCK && !RAGGED) {
-            const int tall_m = (p.m + 255) / 256;
-            // (its rows past the end are left to the buffer descriptors: the 32-bit offsets of a whole tile must not wrap)
-            const bool offsets_fit = (p.m + 256ll) * p.lda + p.k < (1ll << 32) && (p.n + 128ll) * p.ldb + p.k < (1ll << 32);
-            if (offsets_fit && (long long)tall_m * q.tiles_n * batch <= num_cus() && p.k / BK >= tall_min_ksteps(MODE)) {
-                q.tiles_m = tall_m;
+        case TILES_256x128:
+            if constexpr (MODE != MODE_BLOCK && !RAGGED) {
+                q.tiles_m = (p.m + 255) / 256;
                 dim3 grid((unsigned)(q.tiles_m * q.tiles_n), 1, (unsigned)batch);
                 return launch(gemm_a8w8_tile128<MODE, CDT, 3, SM_BN, false, 256>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, 3, SM_BN, 256), stream, q);
             }
-        }
-        return launch_small_stages<MODE, CDT, 2, RAGGED>(q, batch, stream);
-    } else {
-        return A8W8_ERR_BAD_MODE;
+            [[fallthrough]];
+        default:
+            return launch_small_stages<MODE, CDT, 2, RAGGED>(q, batch, stream);
     }
 }
 

@@ -67,6 +67,24 @@ inline bool f4_row_scales_on_256_tiles(long long m, long long n, long long k_ste
     return 2 * rounds128 >= (k_steps >= (fp32_c ? 16 : 12) ? 6 : 7) * rounds256;
 }
 
+// ---------------------------------------------------------------- 128-tile kernel
+// 128 x 128 tiles when all of them fit on the chip at once, two workgroups per compute unit: a problem of that
+// size leaves 256 x 256 tiles with at most half of the compute units.  Measured on 256 compute units against the
+// 256-tile kernels (block / row-col / tiled MX): 2.2x / 1.7x / 1.6x at 64 workgroups, 1.9x / 1.6x / 1.5x at 256,
+// +45% / +21% / +15% at 400, +37% / +17% / +9% at 512; beyond that the second round of workgroups costs more than
+// the idle compute units did (-9% for row/col at 576).
+// (the bound as a switch, for measurement: with 8 instead of 2, 4096 x 7168 x 2048 and 4096^3 take 12-30% longer in every scale mode)
+#ifndef A8W8_SMALL_TILES_PER_CU
+#define A8W8_SMALL_TILES_PER_CU 2
+#endif
+#ifndef A8W8_SMALL_DEEP_UP_TO
+#define A8W8_SMALL_DEEP_UP_TO 1         // four LDS stages up to this many 128-tiles per compute unit, two stages beyond
+#endif
+inline bool fits_128_tiles(long long m, long long n, long long batch, long long cus)
+{
+    return batch * ((m + 127) / 128) * ((n + 127) / 128) <= A8W8_SMALL_TILES_PER_CU * cus;
+}
+
 // 128 x 64 tiles instead of 128 x 128: when the wide tiles would occupy at most half of the compute units and the K loop is long
 // enough for the deeper staging to matter (a problem of a few K steps is bound by launch and store latency, which narrower tiles
 // do not change).
@@ -76,6 +94,31 @@ inline bool f4_row_scales_on_256_tiles(long long m, long long n, long long k_ste
 inline bool narrow_tiles_pay(long long items128, long long n, long long k_bytes, long long cus)
 {
     return 2 * items128 <= cus && n > 64 && k_bytes / 128 >= A8W8_NARROW_MIN_KSTEPS;
+}
+
+// 256 x 128 tiles where 128 x 128 ones would put two workgroups on a compute unit, 256 x 128 ones would not, and the K loop is
+// long enough to make up for a prologue and a tile's stores that no second workgroup hides.  us per launch, bf16 C, two-stage
+// 128-tiles -> 256 x 128 (row/col, row-major MX, tiled MX, MXFP4 row-major / tiled, bf16):
+//   2560^3            22.2 -> 20.3, 26.1 -> 23.5, 23.3 -> 20.3, 16.8 / 13.9 -> 16.7 / 14.1, 41.3 -> 36.5
+//   2049x3584x4096    34.6 -> 28.5, 45.1 -> 36.0, 35.7 -> 30.2, 29.0 / 21.7 -> 24.6 / 19.8, 66.4 -> 51.5
+//   512x16384x7168    67.3 -> 57.1, 88.6 -> 81.5, 71.1 -> 60.2, 42.7 / 33.3 -> 39.1 / 29.5, 126.4 -> 112.5
+//   2048x4096x2048    18.0 -> 18.1, 21.3 -> 20.2, 19.4 -> 18.6, 15.2 / 12.7 -> 15.8 / 13.5, 31.1 -> 30.1
+//   1000x8192x1024    14.2 -> 14.7, 14.9 -> 15.2, 14.3 -> 14.4, 11.8 / 10.7 -> 13.3 / 12.1, 19.1 -> 20.1
+// i.e. the line lies at 16 steps of 128 bytes, and where a step's scales cost next to nothing beside its short MFMAs at 24.
+constexpr int tall_min_ksteps(bool cheap_steps) { return cheap_steps ? 24 : 16; }
+
+// The variant of the 128-tile kernel.  128 x 64 tiles (short and wide problems): every compute unit gets a workgroup, deep staging keeps
+// its share of the weights in flight.  Up to one workgroup per compute unit: four LDS stages (deep prefetch).  More: 256 x 128 tiles
+// where they pay (has_tall: the variant exists for the operands), else two stages, so that two workgroups share a compute unit and
+// hide each other's waits.  cheap_steps: bf16, and MXFP4 on tiled scales.
+enum Tile128 { TILES_128x64, TILES_128_FOUR_STAGES, TILES_256x128, TILES_128_TWO_STAGES };
+inline Tile128 tile128_variant(long long m, long long n, long long k_bytes, long long batch, bool has_tall, bool cheap_steps, long long cus)
+{
+    const long long tiles_n = (n + 127) / 128, items = batch * ((m + 127) / 128) * tiles_n;
+    if (narrow_tiles_pay(items, n, k_bytes, cus)) return TILES_128x64;
+    if (items <= A8W8_SMALL_DEEP_UP_TO * cus) return TILES_128_FOUR_STAGES;
+    if (has_tall && batch * ((m + 255) / 256) * tiles_n <= cus && k_bytes / 128 >= tall_min_ksteps(cheap_steps)) return TILES_256x128;
+    return TILES_128_TWO_STAGES;
 }
 
 // ---------------------------------------------------------------- flat GEMM (up to 128 activation rows)

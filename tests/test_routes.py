@@ -76,3 +76,13 @@ def test_flat_against_dense(kind, row_major, m, n, k, batch, flat):
         mode = {"fp8": g.ROWCOL, "mxfp8": g.MX_TILED, "block": g.BLOCK}[kind]
         args = g.raw_gemm_args(1 << 12, 1 << 12, 1 << 12, 1 << 12, 1 << 12, m, n, k, mode, batch=batch, b_preshuffled=int(not row_major))
         assert (g.kernel_name(args) == "flatmm_a8w8") is flat
+
+
+@pytest.mark.parametrize("kind,m,n,k_bytes,batch,variant", [
+    ("fp8", 256, 8192, 8192, 1, "128x64"), ("fp8", 256, 8192, 1920, 1, "128, four stages"), ("fp8", 2048, 2048, 2048, 1, "128, four stages"),
+    ("fp8", 2560, 2560, 2560, 1, "256x128"), ("fp8", 2560, 2560, 1920, 1, "128, two stages"), ("block", 2560, 2560, 2560, 1, "128, two stages"),
+    ("bf16", 2560, 2560, 3072, 1, "256x128"), ("bf16", 2560, 2560, 2944, 1, "128, two stages"), ("mxfp4_tiled", 2560, 2560, 2048, 1, "128, two stages"),
+    ("mxfp4", 2560, 2560, 2048, 1, "256x128"), ("fp8", 512, 16384, 7168, 1, "256x128"), ("fp8", 129, 16400, 2048, 1, "256x128"),
+    ("fp8", 129, 16400, 2048, 2, None), ("fp8", 4096, 4096, 4096, 1, None)])
+def test_128_tile_kernel(kind, m, n, k_bytes, batch, variant):
+    assert routes.tile128_variant(kind, m, n, k_bytes, batch) == variant
