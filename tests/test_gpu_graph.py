@@ -57,17 +57,22 @@ def test_quantise_reorder_gemm_replays(m, n, k):
         assert (got.float() - ref).abs().max() <= 0.08 * ref.abs().max()      # FP8 quantisation error, not a parity bound
 
 
-def test_per_tensor_quantiser_replays():
-    """The per-tensor quantiser is four launches around one device-side maximum: replays must start from a clean one."""
-    rows, k = 300, 1024
-    x = _fresh((rows, k), 3)
+@pytest.mark.parametrize("rows,k,ld,shift", [(4, 1024, 1024, 0), (300, 1024, 1024, 0), (300, 1024, 1040, 0), (300, 1024, 1024, 1)],
+                         ids=["one launch", "three launches", "four launches: padded rows", "four launches: off 16 bytes"])
+def test_per_tensor_quantiser_replays(rows, k, ld, shift):
+    """Up to 16384 contiguous aligned elements one launch, beyond three (partial maxima in the output, folded, applied), other arrays four
+    around one device-side maximum (cleared, raised, applied, turned into the scale).  Replays must see the maximum of their own
+    input only: a smaller one after a larger one, with other values in the output and the scale beforehand."""
+    whole = torch.zeros(rows * ld + 8, device="cuda")
+    x = whole[shift: shift + rows * ld].view(rows, ld)[:, :k]
     q = torch.empty((rows, k), dtype=torch.uint8, device="cuda")
     s = torch.empty(1, dtype=torch.float32, device="cuda")
     L = g.lib()
 
     def run():
-        assert L.a8w8_quantize(x.data_ptr(), rows, k, k, q.data_ptr(), s.data_ptr(), g.TENSOR, 1, g.api._stream()) == 0
+        assert L.a8w8_quantize(x.data_ptr(), rows, k, ld, q.data_ptr(), s.data_ptr(), g.TENSOR, 1, g.api._stream()) == 0
 
+    x.copy_(_fresh((rows, k), 3))
     run()
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
@@ -76,8 +81,10 @@ def test_per_tensor_quantiser_replays():
         with torch.cuda.graph(graph, stream=side):
             run()
     torch.cuda.synchronize()
-    for rep in range(3):
-        x.copy_(_fresh((rows, k), 30 + rep) * (0.25 if rep == 1 else 4.0))      # a smaller maximum after a larger one
+    for rep in range(4):
+        x.copy_(_fresh((rows, k), 30 + rep) * (0.25 if rep % 2 else 4.0))      # a smaller maximum after a larger one
+        q.fill_(0x7E)                                                          # (as floats, partial maxima: 8e37)
+        s.fill_(1e30)
         graph.replay()
         torch.cuda.synchronize()
         got_q, got_s = q.clone(), s.clone()
@@ -85,6 +92,7 @@ def test_per_tensor_quantiser_replays():
         torch.cuda.synchronize()
         assert torch.equal(got_q, q) and torch.equal(got_s, s)
         assert np.isclose(float(got_s[0]), float(x.abs().max()) / 448.0, rtol=1e-6)
+        assert torch.equal(got_q, g.cvt_f32_to_e4m3(x / got_s))
 
 
 @pytest.mark.parametrize("m", [16, 48, 128])      # fragments gathered from memory / rows staged through LDS / two row-group sets
