@@ -1,6 +1,6 @@
-"""How the flat GEMM deals weight tiles and row groups to workgroups: every split its rule can choose (layers from a few
-weight tiles to more than two per compute unit, two to eight groups of 16 rows, ragged last ones), against exact products, on
-pre-shuffled and on row-major weights."""
+"""How the flat GEMM deals weight tiles and row groups to workgroups, against exact products, on pre-shuffled and on row-major weights:
+layers from a few weight tiles to more than two per compute unit with two to eight groups of 16 rows, ragged last ones (test_fp8,
+test_mxfp4_and_bf16), and every split that its rule can choose, for every kind of operands (test_every_split_is_exact)."""
 import pytest
 import torch
 

@@ -172,7 +172,7 @@ def _row_group_case(orc, mode, m, n, k, batch, seed, rowmajor=False):
 @pytest.mark.parametrize("m", [17, 32, 33, 47, 48, 49, 63, 64, 65, 80, 97, 128])
 @pytest.mark.parametrize("mode", [g.ROWCOL, g.TENSOR, g.MX_TILED, g.BLOCK])
 def test_row_groups_two_weight_tiles(orc, mode, m):
-    """Few weight tiles: two per workgroup, 2 / 3 / 4 row groups; 9 tiles leave the last workgroup half empty."""
+    """Few weight tiles, two batch entries: a workgroup each per weight tile and row group (every split of larger layers: test_gpu_flat_splits.py)."""
     n, k = (144, 320) if mode in (g.ROWCOL, g.TENSOR) else (256, 384)      # 320 = an odd number of 64-wide K blocks
     _row_group_case(orc, mode, m, n, k, 2, 8500 + m)
 
@@ -180,9 +180,8 @@ def test_row_groups_two_weight_tiles(orc, mode, m):
 @pytest.mark.parametrize("m", [17, 32, 33, 48, 49, 64, 81, 96, 113, 128])
 @pytest.mark.parametrize("mode", [g.ROWCOL, g.TENSOR, g.MX_TILED, g.BLOCK])
 def test_row_groups_four_weight_tiles(orc, mode, m):
-    """At least four weight tiles per compute unit over all batch entries: four per workgroup (two for MX and block
-    scales past 48 rows); 18 or 24 tiles per entry are not a multiple of four or leave the id remap without its
-    multiple of eight."""
+    """At least four weight tiles per compute unit over all batch entries: four per workgroup; 18 or 24 tiles per entry are not a
+    multiple of four or leave the id remap without its multiple of eight."""
     n, k = (288, 192) if mode in (g.ROWCOL, g.TENSOR) else (384, 256)
     batch = (1024 * 16 + n - 1) // n
     _row_group_case(orc, mode, m, n, k, batch, 8600 + m)
@@ -192,8 +191,8 @@ def test_row_groups_four_weight_tiles(orc, mode, m):
 @pytest.mark.parametrize("mode", [g.ROWCOL, g.TENSOR, g.MX_TILED, g.BLOCK])
 @pytest.mark.parametrize("many_tiles", [False, True])
 def test_row_major_weights_on_the_flat_kernel(orc, mode, m, many_tiles):
-    """a8w8_gemm with row-major B and at most 128 rows: the flat kernel stages the weight rows through LDS.  Two or
-    four weight tiles per workgroup, every count of row groups, ragged tile counts, an odd number of K blocks."""
+    """a8w8_gemm with row-major B and at most 128 rows: the flat kernel stages the weight rows through LDS.  One weight tile and row
+    group per workgroup (few tiles) or four tiles and up to four groups, ragged tile counts, an odd number of K blocks."""
     n, k = (144, 320) if mode in (g.ROWCOL, g.TENSOR) else (384, 256)
     batch = (1024 * 16 + n - 1) // n if many_tiles else 2
     _row_group_case(orc, mode, m, n, k, batch, 8800 + m, rowmajor=True)
