@@ -10,7 +10,8 @@ The four-wave GEMM kernels, and the 256 x 128 variants of the 128-tile kernel (w
 Those kernels keep their accumulators in registers a[0:255] that only their own assembly statements
 name.  That is sound as long as the compiler places nothing of its own there and spills nothing:
 this script reads the device assembly of the library and fails the build otherwise, as it does when a
-vector instruction writes an MFMA's operand in the two slots in front of it.
+vector instruction writes an MFMA's operand in the two slots in front of it, along every path: past a label the
+instructions in front of the branches to it count as well as those in front of the label.
 Usage: check_isa.py <device .s file> [--no-stores-ok]     (the option: for measurement builds that leave the stores out)
 """
 import re
@@ -22,6 +23,35 @@ def instructions(func):
         ins = line.split(";", 1)[0].strip()
         if ins and not ins.startswith(".") and not ins.endswith(":"):
             yield ins
+
+
+def predecessors(func):
+    """For every instruction (as instructions() counts them) the indexes of those that can issue directly before it."""
+    labels, targets, at, fall = {}, [], 0, []
+    for line in func.split("\n"):
+        ins = line.split(";", 1)[0].strip()
+        if re.fullmatch(r"[.\w$]+:", ins):
+            labels[ins[:-1]] = at
+        elif ins and not ins.startswith(".") and not ins.endswith(":"):
+            op = ins.split()[0]
+            if op.startswith(("s_branch", "s_cbranch")):
+                targets.append((at, ins.split()[1]))
+            fall.append(not op.startswith(("s_branch", "s_endpgm", "s_setpc")))
+            at += 1
+    before = [[i - 1] if i and fall[i - 1] else [] for i in range(at)]
+    for branch, label in targets:
+        if labels.get(label, at) < at:
+            before[labels[label]].append(branch)
+    return before
+
+
+def in_front(before, i, slots):
+    """The instructions in the `slots` issue slots in front of instruction i, along every path."""
+    found, edge = set(), {i}
+    for _ in range(slots):
+        edge = {j for k in edge for j in before[k]}
+        found |= edge
+    return found
 
 
 def registers(operand):
@@ -71,11 +101,12 @@ def main(path, no_stores_ok=False):
         checked += 1
         # their MFMAs are assembly statements, for which the compiler keeps no distance to a vector instruction that writes an
         # operand: none may stand in the two slots in front
+        issued_before = predecessors(f)
         for i, ins in enumerate(seq):
             if not ins.startswith("v_mfma"):
                 continue
             sources = set().union(*(registers(o) for o in re.split(r" (?:op_sel|cbsz)", ins.split(None, 1)[1])[0].split(",")[1:]))
-            for before in seq[max(i - 2, 0):i]:
+            for before in (seq[j] for j in in_front(issued_before, i, 2)):
                 if before.startswith("v_") and not before.startswith("v_mfma") and registers(before.split(None, 1)[1].split(",")[0]) & sources:
                     sys.exit(f"{name}: an operand of an MFMA is written directly in front of it: {before} / {ins}")
         mfma = reads = 0
