@@ -78,7 +78,8 @@ A8W8_DEV uint32_t cvt_four_to_e4m3(float a, float b, float c, float d)
            ((uint32_t)f32_to_e4m3_fnuz_sw(d) << 24);
 }
 
-// One thread converts four consecutive floats: arrays that do not start on 16 bytes (floats) or 4 bytes (codes).
+// One thread converts four consecutive floats (decode: one code): arrays that do not start on 16 bytes (floats) or 4 bytes (codes),
+// and FNUZ arrays that do not fill the chip (cvt_fnuz_few of routes.hpp).
 template <int DIALECT, int CLAMP>
 __global__ void __launch_bounds__(256) cvt_f32_to_e4m3_kernel(const float* src, uint8_t* dst, size_t n)
 {
@@ -379,7 +380,7 @@ A8W8_DEV float4 load_once4(const float* p)
 // 2.7; 16 x 7168: 3.7 / 2.6 / 2.3).
 // TILED: the grid covers the padded [rows_p, k_p] array of the tiled layout (rows_p % 64 == 0, k_p % 512 == 0), so that the
 // positions no (row, block) owns get their 127 here instead of from a launch of their own before this one (2.3 us).  Otherwise,
-// and where the caller filled the scales beforehand, rows_p = rows and k_p = k.
+// and where that launch precedes this one (much padding: mx_padding_in_launch of routes.hpp), rows_p = rows and k_p = k.
 // FP4: packed E2M1, two bytes per lane and chunk; the hardware convert instead of seven comparisons per element (8192 x 8192
 // 62.6 -> 50.3 us, 4096 x 4096 16.8 -> 13.6).
 template <bool FP4, bool TILED, int CHUNKS>
@@ -518,7 +519,7 @@ __global__ void __launch_bounds__(THREADS) quant_rowwise_vec_kernel(const float*
 // 1 x 128 blocks: 32 lanes per (row, 128-group) (bound: HBM).  A workgroup takes one group of ROWS rows (8 or 32: a half wave
 // takes every eighth row, all loads first), so that the scales, stored [k/128][rows], leave as one run of the group's row:
 // taken along a row instead, every scale is a 4-byte write into a cache line of its own, which the workgroups of eight L2s
-// share.  8192 x 8192: 82.3 -> 55.9 us (6.0 TB/s), 4096 x 2048: 11.3 -> 9.4.  Eight rows per workgroup where few blocks leave
+// share (few rows, whose scales lie together, are taken along the row: quant_1x128_along_rows_kernel below).  8192 x 8192: 82.3 -> 55.9 us (6.0 TB/s), 4096 x 2048: 11.3 -> 9.4.  Eight rows per workgroup where few blocks leave
 // the latency of one workgroup: 512 x 4096 3.5 us against 4.0 with 32 rows, 16 x 7168 2.3 against 3.0 (4.3 along the rows);
 // 2560 x 2560 8.5 against 8.3, 8192 x 8192 65 against 58.
 constexpr int QUANT_1X128_FEW = 1 << 14;      // blocks up to which a workgroup takes eight rows

@@ -670,8 +670,8 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
     // operations complete in order, so neither step needs a barrier.  Every direct-to-LDS load has landed by then (the
     // loop's last loads re-fill stages nobody reads).
     // Tiles on the edge of the matrix too, as long as the matrix ends on one of the 16-byte pieces: a lane stores its piece or
-    // not.  (From the MFMA layout, with checks per element, they ended after all others: row/col 1000 x 3000, K = 512: 7.5 us against 5.8
-    // on 1024 x 3072, 6.4 this way; K = 2048 12.0 -> 10.8.)
+    // not.  (From the MFMA layout, with checks per element, they ended after all others: row/col 1000 x 3000, K = 512: 8.2 us against 6.3
+    // on 1024 x 3072, 6.7 this way; K = 2048 12.4 -> 10.9, 10.4 on 1024 x 3072.)
     constexpr int ES = CDT == C_BF16 ? 2 : 4;
     auto write_lines = [&](auto CHECKED) __attribute__((always_inline)) {
         constexpr bool checked = decltype(CHECKED)::value != 0;

@@ -1,5 +1,5 @@
 """Kernel choice for skinny problems (M <= 128) on shuffled weights: the entry points pick between the flat GEMM
-and the MFMA tile kernels with a cost model (prefer_flat in the library).  For cells of the table that model was
+and the MFMA tile kernels with a cost model (flat_is_faster in routes.hpp).  For cells of the table that model was
 fitted to, both sides are timed through a8w8_route_override and the model's own choice has to be within 10% of
 the faster one.  The two sides must also agree on the result."""
 import pytest
