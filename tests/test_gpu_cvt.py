@@ -80,7 +80,8 @@ def test_device_preshuffle(orc):
 @pytest.mark.parametrize("n", [4, 7, 2047, 2048, 2049, 2051, 4095, 6151])
 def test_vectorised_and_unaligned_conversions_agree(orc, dialect, n):
     """Lengths around a workgroup's 2048 elements with every remainder of 4; arrays that start on and off the 16 (floats)
-    and 4 (codes) bytes the vectorised kernels need; nothing is written behind the end."""
+    and 4 (codes) bytes the vectorised kernels need (the FNUZ dialect takes them from two million values on: below); nothing is
+    written behind the end."""
     x = np.random.default_rng(n).standard_normal(n).astype(np.float32) * 100
     want = orc.encode(x, dialect, clamp240=True)
     want_back = orc.decode(want, dialect)

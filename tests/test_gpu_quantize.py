@@ -142,7 +142,8 @@ def test_vector_and_scalar_kernels_agree_with_the_oracle_on_views(orc):
 @pytest.mark.parametrize("rows", [1, 7, 8, 9, 31, 33, 1025])
 @pytest.mark.parametrize("k", [128, 2176])
 def test_1x128_row_tiles(orc, rows, k):
-    """Tiles of 8 rows (few blocks) and of 32 (1025 x 2176: more than 2^14 blocks), whole and ragged; rows in a wider buffer."""
+    """Tiles of 8 rows (few blocks) and of 32 (1025 x 2176: more than 2^14 blocks), whole and ragged, and fewer than eight rows, which are
+    taken along the rows; rows in a wider buffer."""
     x = np.random.default_rng(rows + k).standard_normal((rows, k)).astype(np.float32)
     x[0, :128] = 0
     whole = torch.full((rows, k + 4), 1e30, device="cuda")
