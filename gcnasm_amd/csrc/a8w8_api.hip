@@ -233,37 +233,54 @@ int validate_shuffled_b(const a8w8_gemm_args* g)
     return tiled_ok(&rows) ? A8W8_OK : A8W8_ERR_MISALIGNED;
 }
 
-// The persistent kernel pipelines two K steps ahead and indexes work items with an int.
-bool persist_ok(const a8w8_gemm_args* g)
+int num_cus();
+
+// What the pipelined kernels count with an int: two K steps at least, the work items.
+bool items_ok(const a8w8_gemm_args* g)
 {
-    // tiled MX scales come in pairs of K steps (one dword serves two steps)
-    if (g->scale_mode == A8W8_SCALE_MX_E8M0_TILED && (g->k / BK) % 2 != 0) return false;
-    return g->k >= 2 * BK &&
-           (long long)g->batch * ((g->m + BM - 1) / BM) * ((g->n + BN - 1) / BN) < (1ll << 30);
+    return g->k >= 2 * BK && (long long)g->batch * ((g->m + BM - 1) / BM) * ((g->n + BN - 1) / BN) < (1ll << 30);
 }
 
-// The four-wave kernel walks K in pairs of steps and has the per-tensor, row/col and tiled-MX scale modes.
+// Whether the four-wave kernel takes the number of K steps: any even one, odd ones where odd_steps_on_four_waves and
+// odd_tiled_mx_on_four_waves say so.  (Tiled scales with an odd number and C rows too far apart for its 32-bit offsets stay with the 128-tile
+// kernel, which takes any distance.)  `fp4`: the byte view of packed E2M1 operands.
+bool steps_on_four_waves(const a8w8_gemm_args* g, bool fp4)
+{
+    const int steps = g->k / BK;
+    if (steps % 2 == 0) return true;
+    if (g->scale_mode != A8W8_SCALE_MX_E8M0_TILED) return odd_steps_on_four_waves(steps);
+    const bool fp32 = g->c_dtype == A8W8_C_FP32;
+    return odd_tiled_mx_on_four_waves(fp4, g->m, g->n, steps, g->batch, fp32, num_cus()) && c_tile_fits(g->stride_c, fp32 ? 4 : 2) && items_ok(g);
+}
+
+// The persistent kernels; tiled MX scales exist on the four-wave one only.
+bool persist_ok(const a8w8_gemm_args* g, bool fp4 = false)
+{
+    return items_ok(g) && (g->scale_mode != A8W8_SCALE_MX_E8M0_TILED || steps_on_four_waves(g, fp4));
+}
+
+// The four-wave kernel has the per-tensor, row/col and tiled-MX scale modes.
 bool wide_ok(const a8w8_gemm_args* g)
 {
     if (g->scale_mode != A8W8_SCALE_TENSOR && g->scale_mode != A8W8_SCALE_ROWCOL && g->scale_mode != A8W8_SCALE_MX_E8M0_TILED)
         return false;
-    return persist_ok(g) && (g->k / BK) % 2 == 0;
+    return items_ok(g) && steps_on_four_waves(g, false);
 }
 
-int num_cus();
-bool small_ok(const a8w8_gemm_args* g);
+bool small_ok(const a8w8_gemm_args* g, bool fp4 = false);
 
 // MXFP4 with row-major scales on the four-wave kernel (`g`: byte view, k in bytes, row-major scale mode).  It fetches 16 scale
-// bytes of a row at a time (two K steps: an even number of them) with 32-bit offsets that run up to 256 rows past the end of
-// the matrix.  Up to two 128-tiles per compute unit (small_ok, the line of every other mode) and where
-// f4_row_scales_on_256_tiles says so the 128-tile kernel is the faster one.
+// bytes of a row at a time (two K steps) with 32-bit offsets that run up to 256 rows past the end of the matrix.  Scale rows of an odd number of
+// steps are eight bytes more than a multiple of 16, and its loads then start on dwords, as the caller has checked.  Up to two 128-tiles per
+// compute unit (small_ok, the line of every other mode) and where f4_row_scales_on_256_tiles says so the 128-tile kernel is the faster one.
 bool wide_row_scales_ok(const a8w8_gemm_args* g)
 {
+    const bool odd = (g->k / BK) % 2 != 0;
     const auto rows_ok = [&](const void* s, long long stride, long long batch_stride, long long rows) {
-        return aligned16(s) && stride % 16 == 0 && (g->batch == 1 || batch_stride % 16 == 0) && (rows + BM) * stride < (1ll << 31);
+        return (odd || (aligned16(s) && stride % 16 == 0 && (g->batch == 1 || batch_stride % 16 == 0))) && (rows + BM) * stride < (1ll << 31);
     };
     return !small_ok(g) && f4_row_scales_on_256_tiles(g->m, g->n, g->k / BK, g->batch, g->c_dtype == A8W8_C_FP32, num_cus()) &&
-           persist_ok(g) && (g->k / BK) % 2 == 0 && rows_ok(g->sfa, g->stride_sfa, g->stride_sfa_batch, g->m) &&
+           items_ok(g) && rows_ok(g->sfa, g->stride_sfa, g->stride_sfa_batch, g->m) &&
            rows_ok(g->sfb, g->stride_sfb, g->stride_sfb_batch, g->n) && c_tile_fits(g->stride_c, g->c_dtype == A8W8_C_BF16 ? 2 : 4);
 }
 
@@ -279,11 +296,11 @@ int num_cus()
 }
 
 // Two 128-tiles per compute unit at most (fits_128_tiles).
-bool small_ok(const a8w8_gemm_args* g)
+bool small_ok(const a8w8_gemm_args* g, bool fp4)
 {
     const bool mxt = g->scale_mode == A8W8_SCALE_MX_E8M0_TILED;
-    // tiled MX scales with an odd number of K steps have no 256-tile kernel: any size runs here
-    if (mxt && (g->k / BK) % 2 != 0) return true;
+    // tiled MX scales on a number of K steps that the four-wave kernel does not take have no other kernel: any size runs here
+    if (mxt && !steps_on_four_waves(g, fp4)) return true;
     return fits_128_tiles(g->m, g->n, g->batch, num_cus());
 }
 
@@ -524,13 +541,13 @@ bool flat_rowmajor_ok(const a8w8_gemm_args* g)
 
 // Whether launch_dense_fp8 (and the bf16 / MXFP4 entry points on their byte views) would take one of the two 256-tile
 // kernels: their C tiles must fit 32-bit offsets (c_tile_fits), which the entry points check before any device call.
-bool takes_tile256(const a8w8_gemm_args* g)
+bool takes_tile256(const a8w8_gemm_args* g, bool fp4)
 {
-    return tiled_ok(g) && !small_ok(g) && (wide_ok(g) || persist_ok(g));
+    return tiled_ok(g) && !small_ok(g, fp4) && persist_ok(g, fp4);
 }
-bool c_stride_too_large(const a8w8_gemm_args* g, const a8w8_gemm_args* byte_view)
+bool c_stride_too_large(const a8w8_gemm_args* g, const a8w8_gemm_args* byte_view, bool fp4 = false)
 {
-    return takes_tile256(byte_view) && !c_tile_fits(g->stride_c, g->c_dtype == A8W8_C_BF16 ? 2 : 4);
+    return takes_tile256(byte_view, fp4) && !c_tile_fits(g->stride_c, g->c_dtype == A8W8_C_BF16 ? 2 : 4);
 }
 
 int launch_dense_fp8(const a8w8_gemm_args* g, hipStream_t s)
@@ -651,7 +668,7 @@ static int a16w16_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allo
         if (small_ok(&bytes))            // few tiles: 128 x 128 ones
             return g->c_dtype == A8W8_C_BF16 ? launch_small<MODE_BF16, C_BF16>(p, g->batch, s)
                                              : launch_small<MODE_BF16, C_FP32>(p, g->batch, s);
-        if ((bytes.k / BK) % 2 == 0)     // an even number of K steps: the four-wave kernel
+        if (steps_on_four_waves(&bytes, false))
             return g->c_dtype == A8W8_C_BF16 ? launch_wide<MODE_BF16, C_BF16>(p, g->batch, s)
                                              : launch_wide<MODE_BF16, C_FP32>(p, g->batch, s);
         return g->c_dtype == A8W8_C_BF16 ? launch_persist<MODE_BF16, C_BF16>(p, g->batch, s)
@@ -709,7 +726,7 @@ static int a4w4_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
     bytes.stride_a_batch = g->stride_a_batch / 2; bytes.stride_b_batch = g->stride_b_batch / 2;
     bytes.scale_mode = A8W8_SCALE_MX_E8M0_TILED;
     const bool flat_rows = tiled && flat_rowmajor_ok(&bytes) && prefer_flat(g->m, g->n, bytes.k, g->batch, bytes.stride_b % 4096 == 0 ? 1.3 : 1.05);
-    if (!flat_rows && tiled && g->k % 256 == 0 && c_stride_too_large(g, &bytes)) return A8W8_ERR_TOO_LARGE;
+    if (!flat_rows && tiled && g->k % 256 == 0 && c_stride_too_large(g, &bytes, true)) return A8W8_ERR_TOO_LARGE;
     if (const int ds = device_status(); ds != A8W8_OK) return ds;
     hipStream_t s = (hipStream_t)hip_stream;
     // a skinny problem on row-major weights: the flat kernel where it is the faster one
@@ -720,7 +737,7 @@ static int a4w4_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
     }
     // weights shuffled as bytes (a4w4_flatmm's): MFMA kernels only
     if (g->b_preshuffled && (!tiled || g->k % 256 != 0 || validate_shuffled_b(&bytes) != A8W8_OK ||
-                             (!small_ok(&bytes) && !persist_ok(&bytes))))
+                             (!small_ok(&bytes, true) && !persist_ok(&bytes, true))))
         return A8W8_ERR_BAD_GROUP;
     // row-major scales: the 128-tile kernel at any size (it stages the step's eight scale bytes per row as two dwords:
     // scale rows have to start on dwords), the four-wave kernel where the problem fills the chip with 256-tiles and the
@@ -739,10 +756,10 @@ static int a4w4_gemm_impl(const a8w8_gemm_args* g, void* hip_stream, bool allow_
     }
     if (tiled && g->k % 256 == 0 && tiled_ok(&bytes)) {
         const GemmParams p = make_params(&bytes);
-        if (small_ok(&bytes))       // few tiles, or an odd number of 128-byte K steps
+        if (small_ok(&bytes, true))       // few tiles, or few K steps, an odd number
             return g->c_dtype == A8W8_C_BF16 ? launch_small<MODE_F4T, C_BF16>(p, g->batch, s)
                                              : launch_small<MODE_F4T, C_FP32>(p, g->batch, s);
-        if (persist_ok(&bytes))
+        if (persist_ok(&bytes, true))
             return g->c_dtype == A8W8_C_BF16 ? launch_wide<MODE_F4T, C_BF16>(p, g->batch, s)
                                              : launch_wide<MODE_F4T, C_FP32>(p, g->batch, s);
     }

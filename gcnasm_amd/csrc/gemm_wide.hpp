@@ -107,7 +107,11 @@ gemm_a8w8_wide(PersistParams pp)
     const int wave = wave_uniform(tid >> 6);
     const int wave_m = wave >> 1, wave_n = wave & 1;
     const int r16 = lane & 15, g = lane >> 4;
-    const int nk = p.k / BK;                       // >= 2 (checked by the host)
+    // K steps, >= 2 (checked by the host).  Stages, fragment sets and scales alternate in pairs of steps, so an odd number is walked
+    // as one more: the step that is not there issues its loads (of bytes behind the rows' K, or none: inside the descriptors) and
+    // reads the next tile's first fragments like any other, without MFMAs.
+    const int nk_real = p.k / BK, nk = (nk_real + 1) & ~1;
+    const bool odd = (nk_real & 1) != 0;
 
     // LDS: [A of stage 0][A of stage 1][B of stage 0][B of stage 1], 32 KiB each.  A lane's read
     // addresses are its row and K-piece offset inside an operand (below 32 KiB) plus the stage and the
@@ -485,8 +489,9 @@ gemm_a8w8_wide(PersistParams pp)
     // accumulator quadrant EQ is written out meanwhile, one piece per two MFMAs (EQA: that quadrant's
     // MFMAs ran A-major).
     bool have_prev = false;                         // a quadrant of the tile before is still to be written out
+    // IDLE: no MFMAs (the step behind an odd last one).
     auto quad = [&](auto IA, auto JB, auto REF, auto RS, auto LQ, auto LS, auto AOUTER, auto SPAR, auto SCREAD, auto ZC, auto EQ,
-                    auto EQA) __attribute__((always_inline)) {
+                    auto EQA, auto IDLE) __attribute__((always_inline)) {
         constexpr bool a_outer = decltype(AOUTER)::value != 0;
         constexpr int sp = decltype(SPAR)::value;            // the step's parity: scale byte inside a pair
         constexpr bool SCR = decltype(SCREAD)::value != 0;   // this quadrant also fetches the next pair's scales
@@ -511,7 +516,8 @@ gemm_a8w8_wide(PersistParams pp)
             constexpr int j = jb + (a_outer ? inner : (t >> 2)), i = ia + (a_outer ? (t >> 2) : inner);
             constexpr int lo = (i * 8 + j) * 4;
             constexpr bool z = zc && hf == 0;
-            if constexpr (IS_F4) {
+            if constexpr (decltype(IDLE)::value != 0) {
+            } else if constexpr (IS_F4) {
                 const v4i bh = hf ? v4i{fb[j][4], fb[j][5], fb[j][6], fb[j][7]} : v4i{fb[j][0], fb[j][1], fb[j][2], fb[j][3]};
                 const v4i ah = hf ? v4i{fa[i][4], fa[i][5], fa[i][6], fa[i][7]} : v4i{fa[i][0], fa[i][1], fa[i][2], fa[i][3]};
                 mfma_acc_f4<lo, z, 2 * (j & 1) + hf, 2 * (i & 1) + hf>(bh, ah, sc_b[j >> 2][(j >> 1) & 1], sc_a[i >> 2][(i >> 1) & 1]);
@@ -611,10 +617,13 @@ gemm_a8w8_wide(PersistParams pp)
     // A K step.  FIRST: the tile's first step (even): accumulators start from zero, and the previous
     // tile's last quadrant is written out behind the first 16 MFMAs.  LAST: the tile's last step
     // (odd): each accumulator quadrant is written out behind the MFMAs of the quadrant after it.
-    auto step = [&](auto parity, auto first, auto last) __attribute__((always_inline)) {
+    // IDLE: the step behind the last one of an odd number (odd).
+    auto step = [&](auto parity, auto first, auto last, auto idle) __attribute__((always_inline)) {
+        using ID = decltype(idle);
         constexpr int P = decltype(parity)::value;
         constexpr bool FIRST = decltype(first)::value != 0, LAST = decltype(last)::value != 0;
         static_assert(!(FIRST && P == 1) && !(LAST && P == 0), "tiles start on even steps and end on odd ones");
+        static_assert(!ID::value || (P == 1 && !LAST), "the idle step is an odd one");
         // keeps the 32 LDS addresses of the loads from being computed once and parked in registers
         // (always wave * 1024, but tied to a value that changes with the step)
         wave_lds = wave * 1024 + (ld_ks >> 30);
@@ -623,9 +632,9 @@ gemm_a8w8_wide(PersistParams pp)
         using Z = std::integral_constant<int, FIRST ? 1 : 0>;
         if constexpr (P == 0) {
             // aL x bL | read bH of this step | load aL            (| write out aH x bH of the previous tile)
-            quad(I0{}, I0{}, I3{}, SP{}, I0{}, SP{}, I0{}, SP{}, I0{}, Z{}, std::integral_constant<int, FIRST && !BURST ? 4 : 0>{}, I0{});
+            quad(I0{}, I0{}, I3{}, SP{}, I0{}, SP{}, I0{}, SP{}, I0{}, Z{}, std::integral_constant<int, FIRST && !BURST ? 4 : 0>{}, I0{}, ID{});
             // aL x bH | read aH of this step | load bL
-            quad(I0{}, I4{}, I1{}, SP{}, I2{}, SP{}, I0{}, SP{}, I0{}, Z{}, I0{}, I0{});
+            quad(I0{}, I4{}, I1{}, SP{}, I2{}, SP{}, I0{}, SP{}, I0{}, Z{}, I0{}, I0{}, ID{});
             if constexpr (FIRST) {
                 if (have_prev) handover(std::conditional_t<BURST, SALL, S24>{});
                 else handover(S0{});
@@ -633,9 +642,9 @@ gemm_a8w8_wide(PersistParams pp)
                 handover(S0{});
             }
             // aH x bH | read aL of the next step | load bH
-            quad(I4{}, I4{}, I0{}, SN{}, I3{}, SP{}, I1{}, SP{}, I0{}, Z{}, I0{}, I0{});
+            quad(I4{}, I4{}, I0{}, SN{}, I3{}, SP{}, I1{}, SP{}, I0{}, Z{}, I0{}, I0{}, ID{});
             // aH x bL | read bH of the next step | load aH
-            quad(I4{}, I0{}, I3{}, SN{}, I1{}, SP{}, I0{}, SP{}, std::integral_constant<int, PAIR_STEPS == 1 ? 1 : 0>{}, Z{}, I0{}, I0{});
+            quad(I4{}, I0{}, I3{}, SN{}, I1{}, SP{}, I0{}, SP{}, std::integral_constant<int, PAIR_STEPS == 1 ? 1 : 0>{}, Z{}, I0{}, I0{}, ID{});
             advance_ld();
             if constexpr (IS_MXT && PAIR_STEPS == 1) {
 #pragma unroll
@@ -652,15 +661,15 @@ gemm_a8w8_wide(PersistParams pp)
             }
         } else {
             // aL x bH | read bL of this step | load aL
-            quad(I0{}, I4{}, I2{}, SP{}, I0{}, SP{}, I0{}, SP{}, I0{}, I0{}, I0{}, I0{});
+            quad(I0{}, I4{}, I2{}, SP{}, I0{}, SP{}, I0{}, SP{}, I0{}, I0{}, I0{}, I0{}, ID{});
             // aL x bL | read aH of this step | load bH             (| write out aL x bH)
-            quad(I0{}, I0{}, I1{}, SP{}, I3{}, SP{}, I0{}, SP{}, I0{}, I0{}, std::integral_constant<int, LAST ? 2 : 0>{}, I0{});
+            quad(I0{}, I0{}, I1{}, SP{}, I3{}, SP{}, I0{}, SP{}, I0{}, I0{}, std::integral_constant<int, LAST ? 2 : 0>{}, I0{}, ID{});
             if constexpr (LAST) handover(S8{});
             else handover(S0{});
             // aH x bL | read aL of the next step | load bL         (| write out aL x bL)
-            quad(I4{}, I0{}, I0{}, SN{}, I2{}, SP{}, I1{}, SP{}, I0{}, I0{}, std::integral_constant<int, LAST ? 1 : 0>{}, I0{});
+            quad(I4{}, I0{}, I0{}, SN{}, I2{}, SP{}, I1{}, SP{}, I0{}, I0{}, std::integral_constant<int, LAST ? 1 : 0>{}, I0{}, ID{});
             // aH x bH | read bL of the next step | load aH         (| write out aH x bL, whose MFMAs ran A-major)
-            quad(I4{}, I4{}, I2{}, SN{}, I1{}, SP{}, I0{}, SP{}, I1{}, I0{}, std::integral_constant<int, LAST ? 3 : 0>{}, I1{});
+            quad(I4{}, I4{}, I2{}, SN{}, I1{}, SP{}, I0{}, SP{}, I1{}, I0{}, std::integral_constant<int, LAST ? 3 : 0>{}, I1{}, ID{});
             advance_ld();
             if constexpr (IS_MXT) {
 #pragma unroll
@@ -676,8 +685,8 @@ gemm_a8w8_wide(PersistParams pp)
     using F = std::integral_constant<int, 0>;
     using T = std::integral_constant<int, 1>;
 
-    // The K loop of a tile is an even number of steps (checked by the host), so every tile starts on
-    // an even step; loads and fragment reads run on across the tile boundary.
+    // The K loop of a tile is an even number of steps, so every tile starts on an even step; loads and fragment
+    // reads run on across the tile boundary.
     for (int it = 0; it < my_items; ++it) {
         issue_rowcol_scales(cur_batch, m0, n0, tile_seq & 1);
         for (int ks = 0; ks < nk; ks += 2) {
@@ -707,10 +716,11 @@ gemm_a8w8_wide(PersistParams pp)
                 }
             };
             point_scale_read_at(PAIR_STEPS == 1 ? ks + 1 : ks + 2);
-            if (ks == 0) step(F{}, T{}, F{});
-            else step(F{}, F{}, F{});
+            if (ks == 0) step(F{}, T{}, F{}, F{});
+            else step(F{}, F{}, F{}, F{});
             point_scale_read_at(ks + 2);
-            if (ks + 2 == nk) {
+            const bool last = ks + 2 == nk;
+            if (last) {
                 // from here on the accumulators are written out under this tile's coordinates
                 ep_batch = cur_batch;
                 ep_m0 = m0;
@@ -720,8 +730,6 @@ gemm_a8w8_wide(PersistParams pp)
                     ep_ts = ((const float*)p.sfa + (long long)cur_batch * p.sfa_batch)[0] * ((const float*)p.sfb + (long long)cur_batch * p.sfb_batch)[0];
                 const uintptr_t c_addr = (uintptr_t)p.c + (uintptr_t)((long long)cur_batch * p.c_batch * (CDT == C_BF16 ? 2 : 4));
                 ep_vec_ok = (p.ldc & (CDT == C_BF16 ? 7 : 3)) == 0 && (c_addr & 15) == 0;
-                // pieces are written without checks: only for whole tiles with aligned rows
-                const bool fast = ep_vec_ok && m0 + BM <= p.m && n0 + BN <= p.n;
                 {
                     constexpr int ES = CDT == C_BF16 ? 2 : 4;
                     ep_rs = make_rsrc((const char*)c_addr + ((long long)m0 * p.ldc + n0) * ES, (uint32_t)((BM - 1) * p.ldc + BN) * ES);
@@ -734,30 +742,29 @@ gemm_a8w8_wide(PersistParams pp)
                                                                 (int)((uint32_t)(wave_m * 128 + row_of(c_line_row<BL>(lane) + 8)) * (uint32_t)ep_row_bytes),
                                                                 wave_n * 128 * ES, ep_line_low, ep_line_high);
                 }
-                if (fast && BURST) {
+            }
+            // pieces are written without checks: only for whole tiles with aligned rows
+            const bool fast = ep_vec_ok && m0 + BM <= p.m && n0 + BN <= p.n;
+            if (last && odd) step(T{}, F{}, F{}, T{});
+            else if (!BURST && last && fast) step(T{}, F{}, T{}, F{});
+            else step(T{}, F{}, F{}, F{});
+            if (last) {
+                have_prev = fast;
+                if (fast && (BURST || odd)) {
                     // The whole tile in one burst between its last step and the next tile's first: a store among the
                     // MFMAs makes its wave wait for a place in the memory pipeline, which the loads of the next steps
                     // share, and the K steps around a tile boundary then take three times as long as the others;
                     // written back to back the 32 stores of a wave cost less than they stretched those steps by.
                     // The next tile's first step lets them stay in flight (have_prev).
-                    step(T{}, F{}, F{});
                     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // last MFMA -> first accumulator read
                     if constexpr (CDT == C_BF16 && A8W8_WIDE_LINE_PAIRS)
                         static_for<WIDE_T / 4>([&](auto JPP) { static_for<WIDE_T>([&](auto I) { store_line_pair(I, JPP); }); });
                     else
                         static_for<WIDE_T / 2>([&](auto JP) { static_for<WIDE_T>([&](auto I) { store_piece(I, JP, false); }); });
-                    have_prev = true;
-                } else if (fast) {
-                    step(T{}, F{}, T{});
-                    have_prev = true;
-                } else {
-                    step(T{}, F{}, F{});
+                } else if (!fast) {
                     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // last MFMA -> first accumulator read
                     store_tile_checked();
-                    have_prev = false;
                 }
-            } else {
-                step(T{}, F{}, F{});
             }
         }
         cur_bbase += batches_per_tile;

@@ -59,12 +59,41 @@ inline bool quant_1x128_along_rows(long long rows, long long k)
 //   8192 x 2560 (5, 2)    512 16.3 / 21.9, 1024 22.0 / 27.5, 2048 32.3 / 39.5, 4096 60 / 65, 8192 112 / 116
 // fp32 C: 4096 x 4096 1024 23.0 / 22.6, 2048 31.7 / 29.5; 4096 x 7168 1024 34.1 / 36.6, 2048 49.0 / 49.9, 3072 66.8 / 63.7;
 // 3000 x 8192 2048 42.5 / 49.0, 3072 56.8 / 61.0, 4096 77 / 75; 8192 x 2560 512 20.0 / 30.1, 4096 63 / 73.
+// An odd number of K steps costs the four-wave kernel the idle step behind it and has to be longer: bf16 seven, fp32 thirteen
+// (2816 x 5120 bf16 5 steps 21.2 / 21.6, 7 25.6 / 25.4, fp32 9 33.4 / 35.2, 17 63.5 / 53.1; 8192 x 8192 41 steps bf16 518 / 349).
+struct Rounds { long long of128, of256; };
+inline Rounds tile_rounds(long long m, long long n, long long batch, long long cus)
+{
+    return {(batch * ((m + 127) / 128) * ((n + 127) / 128) + cus - 1) / cus, (batch * ((m + 255) / 256) * ((n + 255) / 256) + cus - 1) / cus};
+}
 inline bool f4_row_scales_on_256_tiles(long long m, long long n, long long k_steps, long long batch, bool fp32_c, long long cus)
 {
-    const long long rounds128 = (batch * ((m + 127) / 128) * ((n + 127) / 128) + cus - 1) / cus;
-    const long long rounds256 = (batch * ((m + 255) / 256) * ((n + 255) / 256) + cus - 1) / cus;
-    if (k_steps < (fp32_c ? 8 : 4)) return false;
-    return 2 * rounds128 >= (k_steps >= (fp32_c ? 16 : 12) ? 6 : 7) * rounds256;
+    const Rounds rounds = tile_rounds(m, n, batch, cus);
+    if (k_steps < (k_steps % 2 ? (fp32_c ? 13 : 7) : (fp32_c ? 8 : 4))) return false;
+    return 2 * rounds.of128 >= (k_steps >= (fp32_c ? 16 : 12) ? 6 : 7) * rounds.of256;
+}
+
+// An odd number of K steps on the four-wave kernel, which walks them in pairs: one step more, without MFMAs (about 0.4 us of the 1.2
+// to 1.4 a step takes), more than two 128-tiles per compute unit.
+// Per-tensor and row/col scales and bf16: instead of the eight-wave kernel, from 33 steps on (us, eight waves / four: 2816 x 5120 17 steps
+// 32.1 / 32.3, 41 64.1 / 62.9; 8192 x 8192 33 208.1 / 202.6, 49 298.4 / 288.5; fp32 C 3000 x 8192 17 65.6 / 67.9, 41 124.5 / 121.5).
+inline bool odd_steps_on_four_waves(long long k_steps)
+{
+    return k_steps >= 33;
+}
+// Tiled MX scales: instead of the 128-tile kernel, whose rounds compare as above.  us, 128-tiles / 256-tiles, MXFP8 bf16 C, MXFP8 fp32, MXFP4
+// bf16, MXFP4 fp32 (K steps of 128 bytes):
+//   2816 x 5120 (4 rounds, 1)   5 steps 19.5 / 18.0, 22.3 / 24.5, 19.9 / 19.1, 23.1 / 25.0   17: 41.0 / 33.9, 43.6 / 39.8, 41.8 / 37.8, 44.5 / 43.8
+//   8192 x 8192 (16, 4)         5  83.0 / 66.5, 107.8 / 92.7, 84.6 / 69.7, 109.6 / 95.3      41: 358 / 257, 374 / 278, 378 / 296, 402 / 315
+//   2560 x 4352 (3, 1)          13 27.2 / 26.9, 29.2 / 31.0, 27.9 / 29.6, 30.4 / 33.6        33: 56.0 / 50.5, 58.2 / 54.5, 60.0 / 57.3, 62.5 / 60.9
+//   3000 x 8192 (6, 2)          17 63.0 / 60.2, 69.6 / 70.5, 65.4 / 67.2, 70.5 / 77.0        41: 133 / 118, 143 / 130, 137 / 134, 148 / 147
+//   8192 x 2560 (5, 2)          25 73.0 / 74.4, 83.6 / 84.4, 75.8 / 84.3, 85.4 / 94.0        41: 114 / 111, 127 / 120, 123 / 128, 133 / 138
+inline bool odd_tiled_mx_on_four_waves(bool fp4, long long m, long long n, long long k_steps, long long batch, bool fp32_c, long long cus)
+{
+    const Rounds rounds = tile_rounds(m, n, batch, cus);
+    if (2 * rounds.of128 >= 7 * rounds.of256) return k_steps >= (!fp32_c ? 5 : fp4 ? 13 : 11);
+    if (rounds.of128 >= 3 * rounds.of256) return k_steps >= (fp4 ? (fp32_c ? 33 : 25) : fp32_c ? 21 : 13);
+    return !fp4 && k_steps >= 33;
 }
 
 // ---------------------------------------------------------------- 128-tile kernel

@@ -128,7 +128,7 @@ A8W8_API int a16w16_flatmm(const a8w8_gemm_args* args, void* hip_stream);
  * B [batch, n, k/2 bytes]; m, n, k and every stride count ELEMENTS (strides even); scale_mode is
  * MX_E8M0_1x32 (row-major scales, as a4w4_quantize_mx writes them by default) or MX_E8M0_TILED.  The MFMA kernels
  * take either when k % 256 == 0 and rows are 16-byte aligned (row-major scales: scale pointers and strides
- * multiples of 4; the four-wave kernel takes large problems whose tiles fill it, with k % 512 == 0 and 16-byte aligned scale rows, 17% slower
+ * multiples of 4; the four-wave kernel takes large problems whose tiles fill it, with k % 512 == 256 or 16-byte aligned scale rows, 17% slower
  * than on tiled scales, the 128 x 128-tile kernel the others);
  * everything else runs on the one-thread-per-element kernel. */
 A8W8_API int a4w4_gemm(const a8w8_gemm_args* args, void* hip_stream);

@@ -42,6 +42,15 @@ def f4_row_scales_on_256_tiles(m, n, k, batch=1, fp32=False, cus=256):
     return bool(lib().route_f4_row_scales_on_256_tiles(_ll(m), _ll(n), _ll(k // 256), _ll(batch), int(fp32), _ll(cus)))
 
 
+def odd_steps_on_four_waves(steps):
+    """Per-tensor and row/col scales and bf16; K steps of 128 bytes."""
+    return bool(lib().route_odd_steps_on_four_waves(_ll(steps)))
+
+
+def odd_tiled_mx_on_four_waves(m, n, steps, fp4=False, batch=1, fp32=False, cus=256):
+    return bool(lib().route_odd_tiled_mx_on_four_waves(int(fp4), _ll(m), _ll(n), _ll(steps), _ll(batch), int(fp32), _ll(cus)))
+
+
 KINDS = ("fp8", "block", "bf16", "mxfp8", "mxfp4")          # enum FlatKind
 BYTES = {"bf16": 2.0, "mxfp4": 0.5}                          # per element of a weight row, else 1
 
