@@ -56,7 +56,7 @@ bool raise_lds_limits_of_mode()
     if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BLOCK || MODE == MODE_MX || MODE == MODE_BF16)
         ok = ok && raise_lds_limit(gemm_a8w8_persist<MODE, C_BF16>, persist_lds_bytes(MODE)) &&
              raise_lds_limit(gemm_a8w8_persist<MODE, C_FP32>, persist_lds_bytes(MODE));
-    if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16 || MODE == MODE_F4T || MODE == MODE_F4)
+    if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_MX || MODE == MODE_BF16 || MODE == MODE_F4T || MODE == MODE_F4)
         ok = ok && raise_lds_limit(gemm_a8w8_wide<MODE, C_BF16>, wide_lds_bytes(MODE)) &&
              raise_lds_limit(gemm_a8w8_wide<MODE, C_FP32>, wide_lds_bytes(MODE));
     {
@@ -259,11 +259,14 @@ bool persist_ok(const a8w8_gemm_args* g, bool fp4 = false)
     return items_ok(g) && (g->scale_mode != A8W8_SCALE_MX_E8M0_TILED || steps_on_four_waves(g, fp4));
 }
 
-// The four-wave kernel has the per-tensor, row/col and tiled-MX scale modes.
+// The four-wave kernel has every scale mode but block scales.  Row-major MX scales: 32-bit offsets that run up to 256 rows past the end of the
+// matrix.
 bool wide_ok(const a8w8_gemm_args* g)
 {
-    if (g->scale_mode != A8W8_SCALE_TENSOR && g->scale_mode != A8W8_SCALE_ROWCOL && g->scale_mode != A8W8_SCALE_MX_E8M0_TILED)
-        return false;
+    if (g->scale_mode == A8W8_SCALE_BLOCK_1x128_128x128) return false;
+    if (g->scale_mode == A8W8_SCALE_MX_E8M0_1x32)
+        return items_ok(g) && mx_row_scales_on_four_waves(g->k / BK) && (g->m + (long long)BM) * g->stride_sfa < (1ll << 31) &&
+               (g->n + (long long)BM) * g->stride_sfb < (1ll << 31);
     return items_ok(g) && steps_on_four_waves(g, false);
 }
 
@@ -367,7 +370,7 @@ int launch_persist(const GemmParams& p, int batch, hipStream_t stream)
 template <int MODE, int CDT>
 int launch_wide(const GemmParams& p, int batch, hipStream_t stream)
 {
-    if constexpr (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16 || MODE == MODE_F4T || MODE == MODE_F4) {
+    if constexpr (MODE != MODE_BLOCK) {
         if (!c_tile_fits(p.ldc, CDT == C_BF16 ? 2 : 4)) return A8W8_ERR_TOO_LARGE;
         PersistParams pp;
         pp.g = p;

@@ -75,25 +75,24 @@ constexpr int WIDE_T = 8;                            // 8 x 8 MFMA tiles per wav
 constexpr int wide_lds_bytes(int mode)
 {
     // MX scales: two buffers of two scale groups each, i.e. all of the 160 KiB
-    return GEMM_LDS_BYTES + ((mode == MODE_MXT || mode == MODE_F4T || mode == MODE_F4) ? 4 * MX_GROUP_BYTES : mode == MODE_ROWCOL ? 2 * ROWCOL_SCALE_BYTES : 0);
+    return GEMM_LDS_BYTES + ((mode == MODE_MXT || mode == MODE_MX || mode == MODE_F4T || mode == MODE_F4) ? 4 * MX_GROUP_BYTES : mode == MODE_ROWCOL ? 2 * ROWCOL_SCALE_BYTES : 0);
 }
 
 template <int MODE, int CDT>
 __global__ void __launch_bounds__(WIDE_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gemm_a8w8_wide(PersistParams pp)
 {
-    static_assert(MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16 || MODE == MODE_F4T || MODE == MODE_F4,
-                  "modes of the four-wave kernel");
+    static_assert(MODE != MODE_BLOCK, "block scales need their accumulators where the VALU can read them");
     // MODE_F4T (packed E2M1 operands): a 128-byte K step holds 256 elements = eight scale blocks = one
     // "pair of K steps" of the tiled scale layout: the tiled-MX plumbing serves it with a scale fetch
     // every step and two 16 x 16 x 128 FP4 MFMAs per fragment pair.  MODE_BF16: a step is 64 elements,
     // two 16 x 16 x 32 MFMAs per fragment pair, no scales.
-    // MODE_F4 (the same operands, row-major scales): a scale group in LDS is 16 bytes of each of the tile's 512 rows, two
-    // K steps of eight bytes, where the tiled layout has the same bytes in the order the lanes want them.  Everything but
-    // the fetch (one row per lane) and the read (two bytes of a row put in place by v_perm) is shared.
+    // MODE_F4 and MODE_MX (the operands of MODE_F4T and MODE_MXT, row-major scales): a scale group in LDS is 16 bytes of each of the
+    // tile's 512 rows, two "pairs of K steps" of eight bytes, where the tiled layout has the same bytes in the order the lanes want
+    // them.  Everything but the fetch (one row per lane) and the read (two bytes of a row put in place by v_perm) is shared.
     constexpr bool IS_F4 = MODE == MODE_F4T || MODE == MODE_F4;
-    constexpr bool ROW_SCALES = MODE == MODE_F4;
-    constexpr bool IS_MXT = MODE == MODE_MXT || IS_F4;               // E8M0 scales
+    constexpr bool ROW_SCALES = MODE == MODE_F4 || MODE == MODE_MX;
+    constexpr bool IS_MXT = MODE == MODE_MXT || MODE == MODE_MX || IS_F4;               // E8M0 scales
     constexpr int MPF = (MODE == MODE_BF16 || IS_F4) ? 2 : 1;        // MFMAs per fragment pair
     constexpr int PAIR_STEPS = IS_F4 ? 1 : 2;                        // K steps served by one fetch of scales
     // tiled MX scales are laid out for A tiles whose rows are dealt like the B tiles' rows
@@ -176,8 +175,8 @@ gemm_a8w8_wide(PersistParams pp)
     };
     ScaleTile sf_cur = {}, sf_next = {};
     const int sf_nblk[2] = {(p.m + 63) >> 6, (p.n + 63) >> 6};
-    const uint32_t sf_bytes[2] = {ROW_SCALES ? (uint32_t)(p.m - 1) * p.stride_sfa + (p.k >> 4) : (uint32_t)mx_tiled_bytes(p.m, IS_F4 ? 2 * p.k : p.k),
-                                  ROW_SCALES ? (uint32_t)(p.n - 1) * p.stride_sfb + (p.k >> 4) : (uint32_t)mx_tiled_bytes(p.n, IS_F4 ? 2 * p.k : p.k)};
+    const uint32_t sf_bytes[2] = {ROW_SCALES ? (uint32_t)(p.m - 1) * p.stride_sfa + (p.k >> (IS_F4 ? 4 : 5)) : (uint32_t)mx_tiled_bytes(p.m, IS_F4 ? 2 * p.k : p.k),
+                                  ROW_SCALES ? (uint32_t)(p.n - 1) * p.stride_sfb + (p.k >> (IS_F4 ? 4 : 5)) : (uint32_t)mx_tiled_bytes(p.n, IS_F4 ? 2 * p.k : p.k)};
     auto point_scales_at = [&](ScaleTile& t, int item) __attribute__((always_inline)) {
         if constexpr (IS_MXT) {
             item = min(item, pp.items - 1);
@@ -202,12 +201,17 @@ gemm_a8w8_wide(PersistParams pp)
 #pragma unroll
                 for (int side = 0; side < 2; ++side) {
                     const __amdgpu_buffer_rsrc_t rs = make_rsrc(t.base[side], sf_bytes[side]);   // past the end: reads 0
-                    A8W8_LDS char* s =
-                        (A8W8_LDS char*)smem + GEMM_LDS_BYTES + buf * BATCH_BYTES + gi * MX_GROUP_BYTES + side * 4096 + wave_lds;
-                    if constexpr (ROW_SCALES)      // one row per lane, the 16 bytes of the group's two K steps
-                        load_to_lds_16(rs, s, ((t.blk[side] + wave) * 64 + lane) * (side ? p.stride_sfb : p.stride_sfa), (batch * GPB + gi) * 16);
-                    else
+                    A8W8_LDS char* s = (A8W8_LDS char*)smem + GEMM_LDS_BYTES + buf * BATCH_BYTES;
+                    if constexpr (ROW_SCALES) {
+                        // half gi of the block's rows, a row's 32 bytes of the batch by two lanes: half as many lines as a group at a time, a
+                        // row per lane (MXFP4, 4096 x 4096 x 4096: 44.7 -> 42.1 us; 2816 x 5120 x 4096 42.8 -> 40.9, fp32 C 48.5 -> 46.6)
+                        s += side * 8192 + 2 * wave_lds + gi * 1024;
+                        load_to_lds_16(rs, s, ((t.blk[side] + wave) * 64 + 32 * gi + (lane >> 1)) * (side ? p.stride_sfb : p.stride_sfa) + (lane & 1) * 16,
+                                       batch * (16 * GPB));
+                    } else {
+                        s += gi * MX_GROUP_BYTES + side * 4096 + wave_lds;
                         load_to_lds_16(rs, s, lane16, ((batch * GPB + gi) * sf_nblk[side] + t.blk[side] + wave) * 1024);
+                    }
                 }
         }
     };
@@ -260,16 +264,17 @@ gemm_a8w8_wide(PersistParams pp)
     // pair, whose byte 2 (tile parity) + (step parity) belongs to the MFMA; they serve two K steps.
     const int lane_rg = r16 * 4 + g;
     // (row-major: the row this lane scales in MFMA tile 0 of the wave's first block; tile parity adds 4 rows, the pair 32, the block 64)
-    const int sf_lane = ROW_SCALES ? (8 * (r16 >> 2) + (r16 & 3)) * 16 : lane_rg * 8;
-    const int rd_sfa = GEMM_LDS_BYTES + wave_m * 2048 + sf_lane;
-    const int rd_sfb = GEMM_LDS_BYTES + 4096 + wave_n * 2048 + sf_lane;
-    // Row-major scales: of the step's eight bytes of a row the lane needs g (first half of the step) and 4 + g (second
-    // half); tile parity 0's two go into the low half of the dword, parity 1's into the high half.
+    constexpr int SF_BLOCK = ROW_SCALES ? 2048 : 1024;      // bytes of a 64-row block in its side's share of a batch
+    const int sf_lane = ROW_SCALES ? (8 * (r16 >> 2) + (r16 & 3)) * 32 : lane_rg * 8;
+    const int rd_sfa = GEMM_LDS_BYTES + wave_m * (2 * SF_BLOCK) + sf_lane;
+    const int rd_sfb = GEMM_LDS_BYTES + 4 * SF_BLOCK + wave_n * (2 * SF_BLOCK) + sf_lane;
+    // Row-major scales: of the pair's eight bytes of a row the lane needs g (its first step; MXFP4: first half of the step) and 4 + g
+    // (second); tile parity 0's two go into the low half of the dword, parity 1's into the high half.
     const unsigned sf_sel_even = (unsigned)g | (unsigned)(4 + g) << 8 | 0x0c0c0000u;      // 0x0c: a zero byte
     const unsigned sf_sel_odd = (unsigned)g << 16 | (unsigned)(4 + g) << 24 | 0x0c0cu;
     auto read_row_scales = [&](int at, v2i (&raw)[4]) __attribute__((always_inline)) {      // [pair][parity]
 #pragma unroll
-        for (int e = 0; e < 4; ++e) raw[e] = *(const v2i*)(smem + at + (e >> 1) * 512 + (e & 1) * 64);
+        for (int e = 0; e < 4; ++e) raw[e] = *(const v2i*)(smem + at + (e >> 1) * 1024 + (e & 1) * 128);
     };
     auto place_row_scales = [&](const v2i (&raw)[4]) __attribute__((always_inline)) -> v2i {
         v2i v;
@@ -469,9 +474,9 @@ gemm_a8w8_wide(PersistParams pp)
         for (int u = 0; u < 2; ++u) {
             if constexpr (ROW_SCALES) {
                 v2i raw[4];
-                read_row_scales(rd_sfa + u * 1024, raw);
+                read_row_scales(rd_sfa + u * SF_BLOCK, raw);
                 sc_a[u] = place_row_scales(raw);
-                read_row_scales(rd_sfb + u * 1024, raw);
+                read_row_scales(rd_sfb + u * SF_BLOCK, raw);
                 sc_b[u] = place_row_scales(raw);
             } else {
                 sc_a[u] = *(const v2i*)(smem + rd_sfa + u * 1024);
@@ -555,13 +560,13 @@ gemm_a8w8_wide(PersistParams pp)
                 constexpr int u = sl / (4 * MPF);
                 if constexpr (ROW_SCALES) {
                     // row-major: four reads, put in place when the next four have been issued (the last ones behind the quadrant)
-                    read_row_scales(sc_rd_off + (u < 2 ? rd_sfa : rd_sfb) + (u & 1) * 1024, sf_raw[u & 1]);
+                    read_row_scales(sc_rd_off + (u < 2 ? rd_sfa : rd_sfb) + (u & 1) * SF_BLOCK, sf_raw[u & 1]);
                     if constexpr (u > 0) (u <= 2 ? sc_a_next[(u - 1) & 1] : sc_b_next[0]) = place_row_scales(sf_raw[(u & 1) ^ 1]);
                 } else {
 #ifdef A8W8_ABLATE_SCALE_READS
                 const v2i v = u < 2 ? sc_a[u] : sc_b[u - 2];
 #else
-                const v2i v = *(const v2i*)(smem + sc_rd_off + (u < 2 ? rd_sfa : rd_sfb) + (u & 1) * 1024);
+                const v2i v = *(const v2i*)(smem + sc_rd_off + (u < 2 ? rd_sfa : rd_sfb) + (u & 1) * SF_BLOCK);
 #endif
                 if constexpr (u < 2) sc_a_next[u] = v;
                 else sc_b_next[u - 2] = v;
@@ -712,7 +717,7 @@ gemm_a8w8_wide(PersistParams pp)
                     const int q = first / PAIR_STEPS;          // pair; two pairs per scale group, GPB groups per batch
                     const bool same = first < nk;
                     const int buf = same ? (cur_bbase + (q >> 2)) & 1 : (cur_bbase + batches_per_tile) & 1;
-                    sc_rd_off = buf * BATCH_BYTES + (same ? ((q >> 1) & 1) * MX_GROUP_BYTES + (q & 1) * (ROW_SCALES ? 8 : 512) : 0);
+                    sc_rd_off = buf * BATCH_BYTES + (same ? ((q >> 1) & 1) * (ROW_SCALES ? 16 : MX_GROUP_BYTES) + (q & 1) * (ROW_SCALES ? 8 : 512) : 0);
                 }
             };
             point_scale_read_at(PAIR_STEPS == 1 ? ks + 1 : ks + 2);

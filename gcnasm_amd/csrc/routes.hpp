@@ -81,6 +81,17 @@ inline bool odd_steps_on_four_waves(long long k_steps)
 {
     return k_steps >= 33;
 }
+// MXFP8 on row-major scales, more than two 128-tiles per compute unit: the four-wave kernel instead of the eight-wave one from 32 steps on.
+// Below, the four-wave kernel's scale loads, a line for every two lanes in front of the operands' in one queue, cost what its fewer LDS reads save.
+// us, eight waves / four, 8192 x 8192, 2816 x 5120, 8192 x 2560 (a second round of 64 tiles):
+//   bf16   9 steps 90.0 / 91.9, 24.2 / 24.9, 38.8 / 41.0    16 134 / 128, 35.0 / 34.1, 58.5 / 58.1    33 245 / 228, 62.1 / 61.9, 104 / 104
+//          64 433 / 409, 111 / 105, 191 / 182
+//   fp32   9 118 / 116, 30.3 / 30.3, 46.9 / 47.2            16 163 / 149, 41.1 / 39.9, 65.5 / 66.8    33 264 / 250, 67.6 / 65.5, 112 / 112
+//          64 456 / 425, 115 / 111, 200 / 190
+inline bool mx_row_scales_on_four_waves(long long k_steps)
+{
+    return k_steps >= 32;
+}
 // Tiled MX scales: instead of the 128-tile kernel, whose rounds compare as above.  us, 128-tiles / 256-tiles, MXFP8 bf16 C, MXFP8 fp32, MXFP4
 // bf16, MXFP4 fp32 (K steps of 128 bytes):
 //   2816 x 5120 (4 rounds, 1)   5 steps 19.5 / 18.0, 22.3 / 24.5, 19.9 / 19.1, 23.1 / 25.0   17: 41.0 / 33.9, 43.6 / 39.8, 41.8 / 37.8, 44.5 / 43.8

@@ -14,6 +14,7 @@ int route_f4_row_scales_on_256_tiles(long long m, long long n, long long k_steps
     return a8w8::f4_row_scales_on_256_tiles(m, n, k_steps, batch, fp32_c != 0, cus);
 }
 int route_odd_steps_on_four_waves(long long k_steps) { return a8w8::odd_steps_on_four_waves(k_steps); }
+int route_mx_row_scales_on_four_waves(long long k_steps) { return a8w8::mx_row_scales_on_four_waves(k_steps); }
 int route_odd_tiled_mx_on_four_waves(int fp4, long long m, long long n, long long k_steps, long long batch, int fp32_c, long long cus)
 {
     return a8w8::odd_tiled_mx_on_four_waves(fp4 != 0, m, n, k_steps, batch, fp32_c != 0, cus);

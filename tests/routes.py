@@ -47,6 +47,10 @@ def odd_steps_on_four_waves(steps):
     return bool(lib().route_odd_steps_on_four_waves(_ll(steps)))
 
 
+def mx_row_scales_on_four_waves(steps):
+    return bool(lib().route_mx_row_scales_on_four_waves(_ll(steps)))
+
+
 def odd_tiled_mx_on_four_waves(m, n, steps, fp4=False, batch=1, fp32=False, cus=256):
     return bool(lib().route_odd_tiled_mx_on_four_waves(int(fp4), _ll(m), _ll(n), _ll(steps), _ll(batch), int(fp32), _ll(cus)))
 

@@ -1,6 +1,6 @@
 """An odd number of K steps (of 128 bytes) on the four-wave kernel, which walks them in pairs: the step behind the last one must add nothing,
-whatever the bytes behind K hold.  Values in {0, +-0.5, +-1, +-2} and scales 2^-2 .. 2^1 (per-row scales powers of two): products are multiples
-of 2^-6 and at most 16, so a sum over K <= 4352 stays below 2^17 and is exact in fp32 (23 bits): the result has to be equal to float64's.
+whatever the bytes behind K hold; and row-major MX scales there, which it fetches 16 bytes of a row at a time.  Values in {0, +-0.5, +-1, +-2} and scales 2^-2 .. 2^1 (per-row scales powers of two): products are multiples
+of 2^-6 and at most 16, so a sum over K <= 4480 stays below 2^17 and is exact in fp32 (23 bits): the result has to be equal to float64's.
 Behind every row of A and B lie NaN codes (FP8, bf16) or sixes (FP4), behind its scales, and at the positions of the tiled layout that no block owns,
 the NaN scale."""
 import ctypes
@@ -93,6 +93,30 @@ def test_tiled_scales_of_a_batch(kind):
 def test_mxfp4_on_row_major_scales(m, n, steps, pad):
     assert routes.f4_row_scales_on_256_tiles(m, n, steps * 256)
     _check("fp4", g.MX, m, n, steps * 256, pad=pad)
+
+
+# scale rows of 4 bytes a step that start at every dword of a 16-byte piece (128, 132, 136, 140 bytes and four more); one round and two
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,steps", [(2300, 4099, 32), (2816, 5120, 33), (4350, 4200, 34), (4090, 7100, 33), (2300, 4099, 35)])
+@pytest.mark.parametrize("pad", [0, 4])
+def test_mxfp8_on_row_major_scales(m, n, steps, pad):
+    assert routes.mx_row_scales_on_four_waves(steps)
+    _check("fp8", g.MX, m, n, steps * 128, pad=pad)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("steps", [32, 33])
+def test_mxfp8_on_row_major_scales_of_a_batch(steps):
+    _check("fp8", g.MX, 2100, 2100, steps * 128, batch=3, pad=4)
+
+
+def test_rule_for_mxfp8_on_row_major_scales():
+    for steps, wide in ((31, False), (32, True), (33, True)):
+        assert routes.mx_row_scales_on_four_waves(steps) is wide
+        args = g.raw_gemm_args(1 << 12, 1 << 12, 1 << 12, 1 << 12, 1 << 12, 4096, 4096, steps * 128, g.MX)
+        assert g.kernel_name(args) == ("gemm_a8w8_wide" if wide else "gemm_a8w8_persist")
+        args.stride_sfa = (1 << 31) // 4096      # scale rows too far apart for 32-bit offsets past the end: still taken
+        assert g.kernel_name(args) == "gemm_a8w8_persist"
 
 
 @pytest.mark.gpu
