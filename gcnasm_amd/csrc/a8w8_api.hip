@@ -580,8 +580,8 @@ int fill_mx_tiled(int rows, int k, uint8_t* scale, hipStream_t s)
     return launch(mx_tiled_fill_kernel, dim3((unsigned)((dwords + 255) / 256)), dim3(256), 0, s, (uint32_t*)scale, dwords);
 }
 
-// The vectorised MX quantisers: as many chunks per wave as the array fills the chip with (quant_mx_vec_kernel), over the padded
-// array where mx_padding_in_launch says so.
+// The vectorised MX quantisers: by lines of the tiled scales or as many chunks per wave as the array fills the chip with (quant_mx_lines_kernel,
+// quant_mx_vec_kernel), over the padded array where mx_padding_in_launch says so.
 template <bool FP4, bool TILED>
 int launch_quant_mx(const float* src, int rows, int k, int ld, uint8_t* q, uint8_t* scale, hipStream_t s)
 {
@@ -590,6 +590,12 @@ int launch_quant_mx(const float* src, int rows, int k, int ld, uint8_t* q, uint8
         if (mx_padding_in_launch(rows, k)) {
             rows_p = (rows + 63) / 64 * 64;
             k_p = (k + 511) / 512 * 512;
+            const MxLines lines = quant_mx_by_lines(FP4, rows, k);
+            if (lines != MX_NOT_BY_LINES) {
+                const unsigned col_groups = (unsigned)(k_p / 256);
+                return launch(lines == MX_LINES_FOUR_WAVES ? quant_mx_lines_kernel<FP4, 4> : quant_mx_lines_kernel<FP4, 8>, dim3((unsigned)(rows_p / 16) * col_groups),
+                              dim3(lines == MX_LINES_FOUR_WAVES ? 256 : 512), 0, s, src, rows, k, ld, q, scale, col_groups);
+            }
         } else if (const int st = fill_mx_tiled(rows, k, scale, s); st != A8W8_OK) {
             return st;
         }
@@ -1006,6 +1012,8 @@ int a8w8_quantize(const float* src, int rows, int k, int ld, uint8_t* q, void* s
         }
         case A8W8_SCALE_ROWCOL:
             if (const int ds = device_status(); ds != A8W8_OK) return ds;
+            if (quant_vec_ok(src, rows, k, ld, q, 4) && quant_rows_by_wave(rows, k))
+                return launch(quant_rowwise_wave_kernel, dim3((unsigned)((rows + 3ll) / 4)), dim3(256), 0, s, src, rows, k, ld, q, (float*)scale);
             if (quant_vec_ok(src, rows, k, ld, q, 4))
                 return launch(k <= 4096 ? quant_rowwise_vec_kernel<256, true> : k <= 8192 ? quant_rowwise_vec_kernel<512, true>
                               : k <= 16384 ? quant_rowwise_vec_kernel<1024, true> : quant_rowwise_vec_kernel<256, false>,

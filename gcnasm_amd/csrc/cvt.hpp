@@ -377,7 +377,7 @@ A8W8_DEV float4 load_once4(const float* p)
 // store instruction of a wave covers one contiguous run of memory; all loads are issued before any chunk is processed.
 // Four chunks are what large arrays want (8192 x 8192 E4M3, tiled scales: 56.3 us, two 58.3, one 64.9), fewer where there are
 // not enough of them to fill the chip and a wave's own latency is the time (2560 x 2560: 8.2 / 7.4 / 8.5; 64 x 7168: 3.8 / 2.7 /
-// 2.7; 16 x 7168: 3.7 / 2.6 / 2.3).
+// 2.7; 16 x 7168: 3.7 / 2.6 / 2.3).  Tiled scales of arrays past a million elements: quant_mx_lines_kernel below.
 // TILED: the grid covers the padded [rows_p, k_p] array of the tiled layout (rows_p % 64 == 0, k_p % 512 == 0), so that the
 // positions no (row, block) owns get their 127 here instead of from a launch of their own before this one (2.3 us).  Otherwise,
 // and where that launch precedes this one (much padding: mx_padding_in_launch of routes.hpp), rows_p = rows and k_p = k.
@@ -459,8 +459,64 @@ __global__ void __launch_bounds__(256) quant_mxfp4_few_kernel(const float* __res
     *(uint32_t*)(q + (((size_t)row * k + col) >> 1)) =
         e2m1_pair<3>(e2m1_pair<2>(e2m1_pair<1>(e2m1_pair<0>(0u, a.x, a.y, s), a.z, a.w, s), b.x, b.y, s), b.z, b.w, s);
 }
-// elements from which the chip is full
-constexpr long long QUANT_MX_FULL = 1ll << 23, QUANT_MX_FEW = 1ll << 18;
+
+// The same for tiled scales, by lines of the scale array (bound: HBM).  A workgroup takes the 16 rows and 256 columns whose scales are one
+// 128-byte line of the tiled layout (rows 8x .. 8x + 7 and 32 + 8x .. of a 64-row block, one "pair"), a wave 16 / WAVES of the rows, 256
+// columns per load; the scale bytes meet in LDS and leave as the line.  Written straight from the blocks, as above, they are single bytes of lines
+// that a dozen workgroups on several L2s share.  Padding, rows and columns alike, is in the lines (127) and costs no element.
+// us, E4M3 / MXFP4, above -> here: 8192 x 8192 55.8 -> 50.0 / 52.7 -> 45.7 (6.7 TB/s), 4096 x 4096 17.2 -> 15.0 / 16.2 -> 13.3, 5248 x 2688 15.8 -> 14.1 /
+// 15.1 -> 13.0, 2560 x 2560 8.2 -> 7.4 / 7.5 -> 6.8, 256 x 8192 4.2 -> 3.9 / 3.8 -> 3.7 (of which a launch is 2.4).
+// Four waves a workgroup between 5 and 15 million elements, eight otherwise (us, four / eight: 1012 x 4096 5.5 / 5.0, 3000 x 2048 6.8 / 7.0, 5831 x 2304 12.9 / 14.1,
+// 4200 x 4096 15.8 / 15.3, 8192 x 4096 27.8 / 26.5).
+template <bool FP4, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) quant_mx_lines_kernel(const float* __restrict__ src, int rows, int k, int ld, uint8_t* __restrict__ q,
+                                                                    uint8_t* __restrict__ scale, unsigned col_groups)
+{
+    constexpr int R = 16 / WAVES;
+    __shared__ __attribute__((aligned(16))) uint8_t line[128];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int cg = (int)(blockIdx.x % col_groups), rg = (int)(blockIdx.x / col_groups);      // 256 columns; block rg / 4, x = rg % 4
+    const int col = cg * 256 + lane * 4;
+    const bool col_owned = col < k;
+    int row[R];
+    float4 v[R];
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+        const int r = wave * R + u;      // row r & 7 of the lower eight, or of the upper ones
+        row[u] = (rg >> 2) * 64 + (rg & 3) * 8 + (r & 7) + (r >> 3) * 32;
+        v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (col_owned && row[u] < rows) v[u] = load_once4(src + (size_t)row[u] * ld + col);
+    }
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+        const int r = wave * R + u;
+        const bool owned = col_owned && row[u] < rows;
+        float amax = fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w)));
+#pragma unroll
+        for (int off = 4; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+        const int e = FP4 ? mx_exponent_e2m1(amax) : mx_exponent_e4m3(amax);
+        // (mx_tiled_index within the line: y = row % 4, g = block % 4, jp = upper eight, par = row / 4 % 2, s = block / 4)
+        if ((lane & 7) == 0) line[((r & 3) * 4 + ((lane >> 3) & 3)) * 8 + (r >> 3) * 4 + ((r >> 2) & 1) * 2 + (lane >> 5)] = (uint8_t)((owned ? e : 0) + 127);
+        if (!owned) continue;
+        if constexpr (FP4) {
+            const float s = __uint_as_float((unsigned)(e + 127) << 23);
+            *(uint16_t*)(q + (((size_t)row[u] * k + col) >> 1)) = (uint16_t)e2m1_pair<1>(e2m1_pair<0>(0u, v[u].x, v[u].y, s), v[u].z, v[u].w, s);
+        } else {
+            *(uint32_t*)(q + (size_t)row[u] * k + col) =
+                pack4_e4m3(ldexpf(v[u].x, -e), ldexpf(v[u].y, -e), ldexpf(v[u].z, -e), ldexpf(v[u].w, -e));
+        }
+    }
+    __syncthreads();
+    // (the array is on a dword at least)
+    if (threadIdx.x < 32) {
+        const size_t at = (((size_t)(cg >> 1) * ((rows + 63) >> 6) + (rg >> 2)) * 2 + (cg & 1)) * 512 + (rg & 3) * 128;
+        ((uint32_t*)(scale + at))[threadIdx.x] = ((const uint32_t*)line)[threadIdx.x];
+    }
+}
+
+// elements from which the chip is full; elements up to which a chunk per wave is the fastest (64 x 7168 row-major 2.93 us with two, 2.68 with one, 128 x 8192
+// 3.05 / 2.97, 512 x 4096 3.87 / 3.97)
+constexpr long long QUANT_MX_FULL = 1ll << 23, QUANT_MX_FEW = 1ll << 20;
 
 // per-row scale, one workgroup per row.  HOLD: the row (at most 16 THREADS elements) stays in registers between the amax pass
 // and the quantisation, four 16-byte loads per thread (one read of the input); otherwise it is read twice.  256 threads up to
@@ -513,6 +569,35 @@ __global__ void __launch_bounds__(THREADS) quant_rowwise_vec_kernel(const float*
             *(uint32_t*)(q + (size_t)row * k + i) =
                 pack4_e4m3(__fdiv_rn(v.x, s), __fdiv_rn(v.y, s), __fdiv_rn(v.z, s), __fdiv_rn(v.w, s));
         }
+    }
+}
+
+// Many short rows (k <= 1024): a wave per row, four to a workgroup, no barrier and no thread without elements: 2306 x 768 4.7 -> 4.1 us, 8192 x 1024
+// 11.0 -> 9.0, 8192 x 512 9.1 -> 5.5, 65536 x 128 44.9 -> 17.5; 1000 rows as fast either way, 300 x 1024 3.2 against 3.5.
+__global__ void __launch_bounds__(256) quant_rowwise_wave_kernel(const float* __restrict__ src, int rows, int k, int ld, uint8_t* __restrict__ q,
+                                                                 float* __restrict__ scale)
+{
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    const float* x = src + (size_t)row * ld;
+    float4 held[4];
+    float amax = 0.f;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int i = lane * 4 + 256 * u;
+        held[u] = i < k ? load_once4(x + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        amax = fmaxf(amax, fmaxf(fmaxf(fabsf(held[u].x), fabsf(held[u].y)), fmaxf(fabsf(held[u].z), fabsf(held[u].w))));
+    amax = wave_max(amax);
+    const float s = amax > 0.f ? __fdiv_rn(amax, 448.0f) : 1.0f;   // an all-zero group keeps scale 1
+    if (lane == 0) scale[row] = s;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int i = lane * 4 + 256 * u;
+        if (i < k)
+            *(uint32_t*)(q + (size_t)row * k + i) = pack4_e4m3(__fdiv_rn(held[u].x, s), __fdiv_rn(held[u].y, s), __fdiv_rn(held[u].z, s), __fdiv_rn(held[u].w, s));
     }
 }
 

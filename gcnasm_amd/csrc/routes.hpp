@@ -19,6 +19,23 @@ inline bool mx_padding_in_launch(long long rows, long long k)
            (padded <= 4ll << 20 || padded - rows * k <= 3ll << 20);
 }
 
+// Tiled MX scales whose padding is in the launch: by lines of the scale array past a million elements, padding counted for E4M3 (1 x 65536 4.5 -> 3.6 us,
+// 8192 x 32 4.9 -> 3.9) and not for MXFP4 (3.4 / 3.6, 3.7 / 3.8), whose kernel for few elements is the faster one there (128 x 8192 3.32 / 3.34,
+// 300 x 5632 3.75 / 3.66).  At half a million E4M3 takes 3.0 us with one chunk per wave, 3.3 by lines.
+enum MxLines { MX_NOT_BY_LINES, MX_LINES_FOUR_WAVES, MX_LINES_EIGHT_WAVES };
+inline MxLines quant_mx_by_lines(bool fp4, long long rows, long long k)
+{
+    const long long elements = rows * k, padded = ((rows + 63) / 64 * 64) * ((k + 511) / 512 * 512);
+    if ((fp4 ? elements : padded) <= 1ll << 20) return MX_NOT_BY_LINES;
+    return elements >= 5000000 && elements < 15000000 ? MX_LINES_FOUR_WAVES : MX_LINES_EIGHT_WAVES;
+}
+
+// The per-row quantiser: a wave per row for more than a thousand rows of at most 1024 elements, else a workgroup (quant_rowwise_wave_kernel).
+inline bool quant_rows_by_wave(long long rows, long long k)
+{
+    return k <= 1024 && rows > 1024;
+}
+
 // Rows of whole 16-byte pieces whose length is no multiple of the 128-byte K step (scales that do not change with K): the 128-tile kernel
 // with a partial last step, 4.6 to 8 us at the least, or the one-thread-per-element kernel, 2.2 us and 60 to 85 ns per K element while
 // its outputs fit the chip at once.  us, one thread per element / tiles, row/col scales, K in bytes:

@@ -3,6 +3,8 @@
 
 extern "C" {
 int route_mx_padding_in_launch(long long rows, long long k) { return a8w8::mx_padding_in_launch(rows, k); }
+int route_quant_mx_by_lines(int fp4, long long rows, long long k) { return a8w8::quant_mx_by_lines(fp4 != 0, rows, k); }
+int route_quant_rows_by_wave(long long rows, long long k) { return a8w8::quant_rows_by_wave(rows, k); }
 int route_partial_steps_on_tiles(long long m, long long n, long long k_bytes, long long batch)
 {
     return a8w8::partial_steps_on_tiles(m, n, k_bytes, batch);

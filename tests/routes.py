@@ -25,6 +25,15 @@ def mx_padding_in_launch(rows, k):
     return bool(lib().route_mx_padding_in_launch(_ll(rows), _ll(k)))
 
 
+def quant_mx_by_lines(rows, k, fp4=False):
+    """Waves per workgroup of the quantiser by lines of the tiled scales (padding in the launch), or None."""
+    return (None, 4, 8)[lib().route_quant_mx_by_lines(int(fp4), _ll(rows), _ll(k))]
+
+
+def quant_rows_by_wave(rows, k):
+    return bool(lib().route_quant_rows_by_wave(_ll(rows), _ll(k)))
+
+
 def partial_steps_on_tiles(m, n, k_bytes, batch=1):
     return bool(lib().route_partial_steps_on_tiles(_ll(m), _ll(n), _ll(k_bytes), _ll(batch)))
 
