@@ -46,8 +46,12 @@ constexpr int persist_lds_bytes(int mode)
     return mode == MODE_MX ? PERSIST_LDS_BYTES_MX : mode == MODE_ROWCOL ? PERSIST_LDS_BYTES_ROWCOL : PERSIST_LDS_BYTES;
 }
 
-// LDS stages of the 128 x 64 variant of the 128-tile kernel: as many as fit 160 KiB
-constexpr int narrow_stages(int mode) { return mode == MODE_MXT || mode == MODE_F4T ? 5 : 6; }
+// LDS stages of the 128 x 64 variant of the 128-tile kernel: three, and as many as fit 160 KiB for the modes that narrow_tiles_deep is for
+constexpr int NARROW_STAGES = 3, SHORT_STAGES = 4;      // (64 x 64 tiles: four; six and eight are 2 to 10% slower)
+constexpr int narrow_deep_stages(int mode, bool ragged)
+{
+    return ragged ? 0 : mode == MODE_MXT ? 5 : mode == MODE_TENSOR || mode == MODE_ROWCOL || mode == MODE_BF16 ? 6 : 0;
+}
 
 template <int MODE>
 bool raise_lds_limits_of_mode()
@@ -64,9 +68,14 @@ bool raise_lds_limits_of_mode()
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 2>, small_lds_bytes(MODE, 2)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, 4>, small_lds_bytes(MODE, 4)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 4>, small_lds_bytes(MODE, 4)) &&
-             raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, narrow_stages(MODE), 64>, small_lds_bytes(MODE, narrow_stages(MODE), 64)) &&
-             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, narrow_stages(MODE), 64>, small_lds_bytes(MODE, narrow_stages(MODE), 64));
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, NARROW_STAGES, 64>, small_lds_bytes(MODE, NARROW_STAGES, 64)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, NARROW_STAGES, 64>, small_lds_bytes(MODE, NARROW_STAGES, 64)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, SHORT_STAGES, 64, false, 64>, small_lds_bytes(MODE, SHORT_STAGES, 64, 64)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, SHORT_STAGES, 64, false, 64>, small_lds_bytes(MODE, SHORT_STAGES, 64, 64));
     }
+    if constexpr (constexpr int deep = narrow_deep_stages(MODE, false); deep != 0)
+        ok = ok && raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, deep, 64>, small_lds_bytes(MODE, deep, 64)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, deep, 64>, small_lds_bytes(MODE, deep, 64));
     if constexpr (MODE != MODE_BLOCK)
         ok = ok && raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, 3, SM_BN, false, 256>, small_lds_bytes(MODE, 3, SM_BN, 256)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 3, SM_BN, false, 256>, small_lds_bytes(MODE, 3, SM_BN, 256));
@@ -75,8 +84,10 @@ bool raise_lds_limits_of_mode()
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 2, SM_BN, true>, small_lds_bytes(MODE, 2)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, 4, SM_BN, true>, small_lds_bytes(MODE, 4)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 4, SM_BN, true>, small_lds_bytes(MODE, 4)) &&
-             raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, narrow_stages(MODE), 64, true>, small_lds_bytes(MODE, narrow_stages(MODE), 64)) &&
-             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, narrow_stages(MODE), 64, true>, small_lds_bytes(MODE, narrow_stages(MODE), 64));
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, NARROW_STAGES, 64, true>, small_lds_bytes(MODE, NARROW_STAGES, 64)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, NARROW_STAGES, 64, true>, small_lds_bytes(MODE, NARROW_STAGES, 64)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, SHORT_STAGES, 64, true, 64>, small_lds_bytes(MODE, SHORT_STAGES, 64, 64)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, SHORT_STAGES, 64, true, 64>, small_lds_bytes(MODE, SHORT_STAGES, 64, 64));
     return ok;
 }
 
@@ -189,6 +200,7 @@ GemmParams make_params(const a8w8_gemm_args* g)
     p.stride_sfa = g->stride_sfa; p.stride_sfb = g->stride_sfb;
     p.tiles_m = (g->m + BM - 1) / BM;
     p.tiles_n = (g->n + BN - 1) / BN;
+    p.inv_per_group = p.inv_rem = 0;
     return p;
 }
 
@@ -307,40 +319,36 @@ bool small_ok(const a8w8_gemm_args* g, bool fp4)
     return fits_128_tiles(g->m, g->n, g->batch, num_cus());
 }
 
-template <int MODE, int CDT, int STAGES, bool RAGGED>
-int launch_small_stages(const GemmParams& q, int batch, hipStream_t stream)
+// One variant of the 128-tile kernel: stages, tile columns, partial K steps, tile rows.
+template <int MODE, int CDT, int STAGES, int BN_, bool RAGGED, int BM_>
+int launch_tiles(const GemmParams& p, int batch, hipStream_t stream)
 {
-    dim3 grid((unsigned)(q.tiles_m * q.tiles_n), 1, (unsigned)batch);
-    return launch(gemm_a8w8_tile128<MODE, CDT, STAGES, SM_BN, RAGGED>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, STAGES), stream, q);
+    GemmParams q = p;
+    q.tiles_m = (p.m + BM_ - 1) / BM_;
+    q.tiles_n = (p.n + BN_ - 1) / BN_;
+    q.inv_per_group = tile_map_inverse(8 * q.tiles_n);
+    q.inv_rem = tile_map_inverse(q.tiles_m % 8);
+    const dim3 grid((unsigned)(q.tiles_m * q.tiles_n), 1, (unsigned)batch);
+    return launch(gemm_a8w8_tile128<MODE, CDT, STAGES, BN_, RAGGED, BM_>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, STAGES, BN_, BM_), stream, q);
 }
 
 // The tile shape and depth of staging are tile128_variant's.
 template <int MODE, int CDT, bool RAGGED = false>
 int launch_small(const GemmParams& p, int batch, hipStream_t stream)
 {
-    GemmParams q = p;
-    q.tiles_m = (p.m + SM_BM - 1) / SM_BM;
-    q.tiles_n = (p.n + SM_BN - 1) / SM_BN;
     // (256 x 128 tiles leave rows past the end to the buffer descriptors: the 32-bit offsets of a whole tile must not wrap)
     const bool tall = MODE != MODE_BLOCK && !RAGGED && (p.m + 256ll) * p.lda + p.k < (1ll << 32) && (p.n + 128ll) * p.ldb + p.k < (1ll << 32);
-    switch (tile128_variant(p.m, p.n, p.k, batch, tall, MODE == MODE_BF16 || MODE == MODE_F4T, num_cus())) {
-        case TILES_128x64: {
-            q.tiles_n = (p.n + 63) / 64;
-            dim3 grid((unsigned)(q.tiles_m * q.tiles_n), 1, (unsigned)batch);
-            constexpr int ST = narrow_stages(MODE);
-            return launch(gemm_a8w8_tile128<MODE, CDT, ST, 64, RAGGED>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, ST, 64), stream, q);
-        }
-        case TILES_128_FOUR_STAGES:
-            return launch_small_stages<MODE, CDT, 4, RAGGED>(q, batch, stream);
+    switch (tile128_variant(p.m, p.n, p.k, batch, tall, MODE == MODE_BF16 || MODE == MODE_F4T, num_cus(), MODE == MODE_BLOCK)) {
+        case TILES_64x64: return launch_tiles<MODE, CDT, SHORT_STAGES, 64, RAGGED, 64>(p, batch, stream);
+        case TILES_128x64:
+            if constexpr (constexpr int deep = narrow_deep_stages(MODE, RAGGED); deep != 0)
+                if (narrow_tiles_deep(p.k)) return launch_tiles<MODE, CDT, deep, 64, false, 128>(p, batch, stream);
+            return launch_tiles<MODE, CDT, NARROW_STAGES, 64, RAGGED, 128>(p, batch, stream);
+        case TILES_128_FOUR_STAGES: return launch_tiles<MODE, CDT, 4, 128, RAGGED, 128>(p, batch, stream);
         case TILES_256x128:
-            if constexpr (MODE != MODE_BLOCK && !RAGGED) {
-                q.tiles_m = (p.m + 255) / 256;
-                dim3 grid((unsigned)(q.tiles_m * q.tiles_n), 1, (unsigned)batch);
-                return launch(gemm_a8w8_tile128<MODE, CDT, 3, SM_BN, false, 256>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, 3, SM_BN, 256), stream, q);
-            }
+            if constexpr (MODE != MODE_BLOCK && !RAGGED) return launch_tiles<MODE, CDT, 3, 128, false, 256>(p, batch, stream);
             [[fallthrough]];
-        default:
-            return launch_small_stages<MODE, CDT, 2, RAGGED>(q, batch, stream);
+        default: return launch_tiles<MODE, CDT, 2, 128, RAGGED, 128>(p, batch, stream);
     }
 }
 

@@ -30,27 +30,11 @@ constexpr int GEMM_LDS_BYTES_MX = GEMM_LDS_BYTES + 2 * MX_GROUP_BYTES;
 constexpr int WAVE_M = 64, WAVE_N = 128;
 constexpr int TM = WAVE_M / 16, TN = WAVE_N / 16;    // 4 x 8 MFMA tiles per wave
 
-// Workgroup id -> tile.  Consecutive workgroup ids land on different XCDs (round-robin over
+// Workgroup id -> tile (tile_of_block).  Consecutive workgroup ids land on different XCDs (round-robin over
 // 8), each with its own L2, so ids are first regrouped so that one XCD works on a
-// contiguous run of tiles; inside the run, tiles are walked down 8 tile-rows before moving
+// contiguous run of tiles (without it, on tile counts that 8 does not divide, 210 tiles of 64 x 64 with K = 3072 took 10.8 us instead of 7.8); inside the run, tiles are walked down 8 tile-rows before moving
 // to the next tile-column so that concurrently resident tiles share A rows and B rows.
-A8W8_DEV void tile_of_block(int bid, int tiles_m, int tiles_n, int& tm, int& tn)
-{
-    const int nt = tiles_m * tiles_n;
-    int id = bid;
-    if ((nt & 7) == 0) id = (bid & 7) * (nt >> 3) + (bid >> 3);
-    constexpr int GROUP = 8;
-    const int per_group = GROUP * tiles_n;
-    const int group = id / per_group;
-    const int first_m = group * GROUP;
-    const int gsz = min(tiles_m - first_m, GROUP);
-    const int in_group = id - group * per_group;
-    tm = first_m + in_group % gsz;
-    tn = in_group / gsz;
-}
-
-// The same mapping for the persistent kernels, which look tiles up at every tile change, where nothing hides the
-// lookup: every division is by a value the host knows, so the host passes floor(2^32 / d) for each of them and the
+// Nothing hides the lookup (the persistent kernels look tiles up at every tile change, the 128-tile kernel in front of its first load): every division is by a value the host knows, so the host passes floor(2^32 / d) for each of them and the
 // kernel divides with one multiply and one correction (exact for 0 <= n < 2^31 and any d >= 1: the estimate
 // mulhi(n, floor(2^32 / d)) is the quotient or one less).  Measured against run-time divisors: 0.25% of the MXFP8 8192^3
 // launch (four tiles per workgroup), 1-2% of block-scale 4096 x 7168 x 2048 (two tiles of 16 K steps).
@@ -82,6 +66,21 @@ A8W8_DEV int div_by_known(int n, int d, uint32_t inv)
     int q = (int)__umulhi((uint32_t)n, inv);
     if (n - q * d >= d) ++q;
     return q;
+}
+A8W8_DEV void tile_of_block(const GemmParams& p, int bid, int& tm, int& tn)
+{
+    const int nt = p.tiles_m * p.tiles_n;
+    // (runs of nt / 8 tiles, the first nt % 8 of them one longer)
+    const int id = (bid & 7) * (nt >> 3) + min(bid & 7, nt & 7) + (bid >> 3);
+    const int per_group = 8 * p.tiles_n, group = div_by_known(id, per_group, p.inv_per_group), first_m = group * 8, in_group = id - group * per_group;
+    if (p.tiles_m - first_m >= 8) {
+        tn = in_group >> 3;
+        tm = first_m + (in_group & 7);
+    } else {
+        const int rem = p.tiles_m & 7;
+        tn = div_by_known(in_group, rem, p.inv_rem);
+        tm = first_m + in_group - tn * rem;
+    }
 }
 // work item (batch entry, tile) -> batch entry and tile coordinates
 A8W8_DEV void tile_of_item(const TileMap& t, int item, int& batch, int& tm, int& tn)

@@ -16,7 +16,7 @@
 
 namespace a8w8 {
 
-constexpr int SM_BM = 128, SM_BN = 128;               // the usual tile; the kernel also takes 64 columns, or 256 rows
+constexpr int SM_BM = 128, SM_BN = 128;               // the usual tile; the kernel also takes 64 columns, 64 x 64, or 256 rows
 constexpr int SM_THREADS = 256;
 constexpr int small_stage_bytes(int bn, int bm = SM_BM) { return (bm + bn) * BK; }   // 128 x 128: 32768, 128 x 64: 24576, 256 x 128: 49152
 // Scale bytes per stage.  Block mode: 128 A-row scales, the B scale at +512 and +768.  Row-major MX: the step's
@@ -56,7 +56,12 @@ constexpr int small_lds_bytes(int mode, int stages, int bn = SM_BN, int bm = SM_
 // of many megabytes -- where 128 x 128 tiles would leave half of the compute units without a workgroup.  A workgroup
 // alone on its compute unit streams its share of the weights through a long K loop: SM_STAGES = 6 there (five K
 // steps of loads ahead, 144-154 KiB of LDS; 5 with tiled MX scales, whose 4 KiB per stage would not fit six; measured,
-// five and six stages run alike, and so does a separate ring of ten stages for the weights).
+// five and six stages run alike, and so does a separate ring of ten stages for the weights); three where steps are few or
+// more than their operands (narrow_tiles_deep).
+// BM_ = 64: tiles of 64 x 64 (a wave owns 32 x 32), four stages of 16 KiB, for problems of at most one of them per compute unit, where the time
+// is one workgroup's K loop: half the operand bytes of a 128 x 64 tile per step (bound: L2 -> LDS, about 90 GB/s per compute unit at any tile size;
+// 1024 x 1024 x 1024 5.6 -> 4.5 us, 512 x 2048 x 8192 19.1 -> 14.6).  Splitting K over workgroups instead costs 2.5 to 9 us for the exchange of
+// the partial tiles (134 x 1984 x 6912: 16.1 unsplit, 13.4 in three parts, 12.7 on 64 x 64 tiles; 256 x 4096 x 4096 11.5, 13.7, 9.0).
 // RAGGED: k is no multiple of 128 (bytes).  The last K step is a partial one: the 16-byte pieces past k are fetched with a
 // lane offset beyond the buffer descriptor and read as zero on both sides (k % 16 == 0, so a piece is never split).  FP8
 // operands then run on the bf16 MFMA: the one-thread-per-element kernel that took these shapes before adds products in
@@ -75,10 +80,11 @@ template <int MODE, int CDT, int SM_STAGES, int BN_ = SM_BN, bool RAGGED = false
 __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__((amdgpu_waves_per_eu(BM_ == 256 ? 1 : 2, BM_ == 256 ? 1 : 8))) gemm_a8w8_tile128(GemmParams p)
 {
     constexpr bool TALL = BM_ == 256;
-    static_assert(BM_ == 128 || (TALL && SM_STAGES == 3 && BN_ == 128 && !RAGGED && MODE != MODE_BLOCK), "tile height");
+    constexpr bool SHORT = BM_ == 64;
+    static_assert(BM_ == 128 || (SHORT && BN_ == 64 && SM_STAGES > 2) || (TALL && SM_STAGES == 3 && BN_ == 128 && !RAGGED && MODE != MODE_BLOCK), "tile height");
     static_assert(!RAGGED || MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BF16, "partial K steps: no scales that change with K");
     constexpr bool BY_BF16 = RAGGED && MODE != MODE_BF16;      // FP8 operands converted to bf16
-    static_assert(SM_STAGES == 2 || SM_STAGES == 3 || SM_STAGES == 4 || SM_STAGES == 5 || SM_STAGES == 6, "two to six LDS stages");
+    static_assert(SM_STAGES == 2 || SM_STAGES == 3 || SM_STAGES == 4 || SM_STAGES == 5 || SM_STAGES == 6 || SM_STAGES == 8, "LDS stages");
     static_assert(BN_ == 128 || BN_ == 64, "tile width");
     constexpr int SM_BN = BN_;
     constexpr int SM_BM = BM_;
@@ -104,8 +110,12 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
     const int batch = blockIdx.z;
     const int r16 = lane & 15, g = lane >> 4;
 
+    // What the first loads' addresses need of the arguments is fetched here, with the tile counts: fetched where it is used, it is a second wait for
+    // the argument block in front of the first load.
+    asm volatile("" ::"s"(p.a), "s"(p.b), "s"(p.sfa), "s"(p.sfb), "s"(p.m), "s"(p.n), "s"(p.k), "s"(p.lda), "s"(p.ldb), "s"(p.a_batch), "s"(p.b_batch),
+                 "s"(p.sfa_batch), "s"(p.sfb_batch), "s"(p.stride_sfa), "s"(p.stride_sfb), "s"(p.b_kshift));
     int tile_m, tile_n;
-    tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    tile_of_block(p, blockIdx.x, tile_m, tile_n);
     const int m0 = tile_m * SM_BM, n0 = tile_n * SM_BN;
     const int nk = RAGGED ? (p.k + BK - 1) / BK : p.k / BK;
 
@@ -248,7 +258,7 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
     // (a 64-wide tile lies inside one 64-row block of B: wave column 1 owns the block's MFMA tiles 2 and 3)
     int mxt_off[4], mxt_off_b[SM_TN];
     // where the unit of A tile t's 64-row block, and the wave's B block, lie in the stage's scale bytes
-    auto mxt_unit_a = [&](int t) __attribute__((always_inline)) { return TALL ? wave_m * 1024 + (t >> 2) * 512 : wave_m * 1024; };
+    auto mxt_unit_a = [&](int t) __attribute__((always_inline)) { return TALL ? wave_m * 1024 + (t >> 2) * 512 : SHORT ? 0 : wave_m * 1024; };
     const int mxt_unit_b = TALL ? 2048 + wave_n * 512 : SM_BN == 128 ? (2 + wave_n) * 1024 : 2 * 1024;
     constexpr int SF_B_ROW0 = TALL ? (MODE == MODE_F4 ? 512 : 256) : 128;      // dword of B's first row in the row-major scale bytes
     if constexpr (TILED_SCALES) {
@@ -257,7 +267,7 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
             return ((4 * x + y) * 4 + g) * 8 + (t >> 1) * 4 + par * 2;
         };
 #pragma unroll
-        for (int t = 0; t < 4; ++t) mxt_off[t] = unit_offset(t);
+        for (int t = 0; t < 4; ++t) mxt_off[t] = unit_offset(SHORT ? (2 * wave_m + t) & 3 : t);
 #pragma unroll
         for (int t = 0; t < SM_TN; ++t) mxt_off_b[t] = unit_offset(SM_BN == 128 ? t : 2 * wave_n + t);
     }
@@ -286,11 +296,11 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
     // ks + 2) between them; the other workgroup's MFMAs run beside this one's LDS reads.
     constexpr bool TWO = SM_STAGES == 2;
     constexpr bool PIPELINED = TWO ? A8W8_SMALL_PIPELINED_TWO != 0 : A8W8_SMALL_PIPELINED != 0;
-    static_assert(PIPELINED || (!RAGGED && !TALL), "partial K steps and 256-row tiles exist in the overlapped loop only");
+    static_assert(PIPELINED || (!RAGGED && !TALL && !SHORT), "partial K steps, 256- and 64-row tiles exist in the overlapped loop only");
     if constexpr (PIPELINED) {
         constexpr int HALVES = BY_BF16 ? 4 : (IS_F4 || MODE == MODE_BF16) ? 2 : 1;      // MFMAs per pair of fragments
         constexpr int NFRAG = SM_TM + SM_TN, NSLOT = SM_TM * SM_TN * HALVES, NLOAD = LOADS_PER_STAGE;
-        constexpr int LOAD_EVERY = NSLOT / NLOAD;
+        constexpr int LOADS_PER_SLOT = (NLOAD + NSLOT - 1) / NSLOT, LOAD_EVERY = LOADS_PER_SLOT > 1 ? 1 : NSLOT / NLOAD;      // (64 x 64 tiles have fewer MFMAs than loads)
         // converted operands: the next step's first quarter is converted behind this step's last MFMAs, so its fragments come in the first half
         constexpr int READ_EVERY = BY_BF16 && !TWO ? NSLOT / (2 * NFRAG) : NSLOT / NFRAG;
         constexpr int BLK_LAG = MODE == MODE_BLOCK ? 4 : 0;
@@ -306,7 +316,7 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
                 const float* f = (const float*)sc;
                 const float b = f[128];
 #pragma unroll
-                for (int t = 0; t < SM_TM; ++t) sa[t] = __builtin_bit_cast(int, f[wave_m * 64 + 16 * t + r16] * b);
+                for (int t = 0; t < SM_TM; ++t) sa[t] = __builtin_bit_cast(int, f[wave_m * (SM_BM / 2) + 16 * t + r16] * b);
             }
             if constexpr (MODE == MODE_MX) {
                 // lane (r16, g) scales K [32g, 32g+32) of its row: byte g of the row's dword
@@ -473,7 +483,9 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
                     } else {
                         acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb, fa, acc[i][j], 0, 0, 0, 0, 0, 0);
                     }
-                    if (t % LOAD_EVERY == 0 && t / LOAD_EVERY < NLOAD) load_one(stage, kload, t / LOAD_EVERY);
+#pragma unroll
+                    for (int n = t / LOAD_EVERY * LOADS_PER_SLOT; n < (t / LOAD_EVERY + 1) * LOADS_PER_SLOT; ++n)
+                        if (t % LOAD_EVERY == 0 && n < NLOAD) load_one(stage, kload, n);
                     if constexpr (!TWO) {
                         if (t % READ_EVERY == 0 && t / READ_EVERY < NFRAG) next[t / READ_EVERY] = read_one(next_stage, t / READ_EVERY);
                         if (t == 0) read_scales(next_stage, ks + 1, next_sa, next_sb);

@@ -142,7 +142,7 @@ inline bool fits_128_tiles(long long m, long long n, long long batch, long long 
     return batch * ((m + 127) / 128) * ((n + 127) / 128) <= A8W8_SMALL_TILES_PER_CU * cus;
 }
 
-// 128 x 64 tiles instead of 128 x 128: when the wide tiles would occupy at most half of the compute units and the K loop is long
+// Up to 128 activation rows, 128 x 64 tiles instead of 128 x 128: when the wide tiles would occupy at most half of the compute units and the K loop is long
 // enough for the deeper staging to matter (a problem of a few K steps is bound by launch and store latency, which narrower tiles
 // do not change).
 #ifndef A8W8_NARROW_MIN_KSTEPS
@@ -162,17 +162,39 @@ inline bool narrow_tiles_pay(long long items128, long long n, long long k_bytes,
 //   2048x4096x2048    18.0 -> 18.1, 21.3 -> 20.2, 19.4 -> 18.6, 15.2 / 12.7 -> 15.8 / 13.5, 31.1 -> 30.1
 //   1000x8192x1024    14.2 -> 14.7, 14.9 -> 15.2, 14.3 -> 14.4, 11.8 / 10.7 -> 13.3 / 12.1, 19.1 -> 20.1
 // i.e. the line lies at 16 steps of 128 bytes, and where a step's scales cost next to nothing beside its short MFMAs at 24.
+// LDS stages of 128 x 64 tiles: three, or as many as fit 160 KiB from 28 steps on where a step is little more than its operands (per-tensor, row/col and
+// tiled MXFP8 scales, bf16).  us, three / six: 1000 x 1536 x 1024 5.9 / 6.3, 402 x 1920 x 3072 10.3 / 10.5, 1024 x 2048 x 4096 13.7 / 13.0, 1495 x 1344 x 7168
+// 20.6 / 19.8; tiled MXFP8 11.0 / 11.4 at 24 steps, 14.5 / 14.2 at 32.  Others: block scales 1024 x 2048 x 4096 14.9 / 15.4, row-major MX 20.8 / 22.2, MXFP4 23.5 /
+// 24.9, tiled 14.7 / 14.9; partial steps 800 x 2000 x 2000 12.8 / 14.2.
+inline bool narrow_tiles_deep(long long k_bytes) { return k_bytes / 128 >= 28; }
+
 constexpr int tall_min_ksteps(bool cheap_steps) { return cheap_steps ? 24 : 16; }
 
-// The variant of the 128-tile kernel.  128 x 64 tiles (short and wide problems): every compute unit gets a workgroup, deep staging keeps
-// its share of the weights in flight.  Up to one workgroup per compute unit: four LDS stages (deep prefetch).  More: 256 x 128 tiles
+// The variant of the 128-tile kernel: the smallest tile whose workgroups do not outnumber the compute units, since a workgroup alone on its
+// compute unit takes as long as its own K loop, and that as long as its tile's rows take from L2 (16, 24, 32 KiB a step: 0.18, 0.27, 0.36 us).
+// Beyond 128 activation rows (up to there the flat GEMM's cost model goes by the tiles of narrow_tiles_pay):
+//  64 x 64: us, row/col scales, 128 x 128 / 128 x 64 / 64 x 64: 1024 x 1024 x 1024 6.7 / 5.6 / 4.5, 200 x 512 x 512 5.6 / 4.7 / 3.7, 300 x 3072 x 3072
+//   12.5 / 10.3 / 7.9, 512 x 2048 x 8192 23.7 / 19.1 / 14.6, bf16 4 x 162 x 384 x 3840 23.9 / 19.4 / 15.1; block scales 1024 x 1024 x 4096 18.1 / 13.8 / 11.1;
+//   row-major MX 512 x 512 x 1024 7.4 / 6.3 / 5.0; K = 2000 (a partial step) 1000 x 1000 16.8 / 12.4 / 9.8.  Not for two workgroups per compute unit (700 x
+//   2048 x 2048, 352 tiles of 64 x 64 9.7 / 8.3 / 9.2).
+//  128 x 64: 1000 x 1536 x 1024 7.3 / 5.9, 1437 x 1280 x 1152 7.6 / 6.4, 1495 x 1344 x 7168 23.3 / 19.8, 512 x 4096 x 1024 on row-major MXFP4 8.9 / 7.5; with block
+//   scales also where 128 x 128 ones fill more than three quarters of the chip (two workgroups per compute unit hide each other's multiply-adds:
+//   2048 x 2048 x 1024 fp32 C 11.3 / 10.9; row/col 8.5 / 9.3).  Fewer than 16 steps: up to seven eighths of the compute units.
+// Then, up to one workgroup per compute unit: four LDS stages (deep prefetch).  More: 256 x 128 tiles
 // where they pay (has_tall: the variant exists for the operands), else two stages, so that two workgroups share a compute unit and
 // hide each other's waits.  cheap_steps: bf16, and MXFP4 on tiled scales.
-enum Tile128 { TILES_128x64, TILES_128_FOUR_STAGES, TILES_256x128, TILES_128_TWO_STAGES };
-inline Tile128 tile128_variant(long long m, long long n, long long k_bytes, long long batch, bool has_tall, bool cheap_steps, long long cus)
+enum Tile128 { TILES_128x64, TILES_128_FOUR_STAGES, TILES_256x128, TILES_128_TWO_STAGES, TILES_64x64 };
+inline Tile128 tile128_variant(long long m, long long n, long long k_bytes, long long batch, bool has_tall, bool cheap_steps, long long cus, bool block = false)
 {
     const long long tiles_n = (n + 127) / 128, items = batch * ((m + 127) / 128) * tiles_n;
-    if (narrow_tiles_pay(items, n, k_bytes, cus)) return TILES_128x64;
+    if (m <= 128) {
+        if (narrow_tiles_pay(items, n, k_bytes, cus)) return TILES_128x64;
+    } else {
+        const long long columns64 = (n + 63) / 64, items64 = batch * ((m + 127) / 128) * columns64;
+        if (batch * ((m + 63) / 64) * columns64 <= cus) return TILES_64x64;
+        if (8 * items64 <= (k_bytes / 128 >= A8W8_NARROW_MIN_KSTEPS ? 8 : 7) * cus) return TILES_128x64;
+        if (block && 4 * items > 3 * cus && items <= cus) return TILES_128x64;
+    }
     if (items <= A8W8_SMALL_DEEP_UP_TO * cus) return TILES_128_FOUR_STAGES;
     if (has_tall && batch * ((m + 255) / 256) * tiles_n <= cus && k_bytes / 128 >= tall_min_ksteps(cheap_steps)) return TILES_256x128;
     return TILES_128_TWO_STAGES;

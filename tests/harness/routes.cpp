@@ -32,8 +32,8 @@ int route_flat_is_faster(long long m, long long n, long long row_bytes, long lon
     return a8w8::flat_is_faster(m, n, row_bytes, batch, layout_factor, cus);
 }
 int route_fits_128_tiles(long long m, long long n, long long batch, long long cus) { return a8w8::fits_128_tiles(m, n, batch, cus); }
-int route_tile128_variant(long long m, long long n, long long k_bytes, long long batch, int has_tall, int cheap_steps, long long cus)
+int route_tile128_variant(long long m, long long n, long long k_bytes, long long batch, int has_tall, int cheap_steps, long long cus, int block)
 {
-    return a8w8::tile128_variant(m, n, k_bytes, batch, has_tall != 0, cheap_steps != 0, cus);
+    return a8w8::tile128_variant(m, n, k_bytes, batch, has_tall != 0, cheap_steps != 0, cus, block != 0);
 }
 }

@@ -81,7 +81,7 @@ def flat_is_faster(kind, row_major, m, n, k, batch=1, cus=256):
     return bool(lib().route_flat_is_faster(_ll(m), _ll(n), _ll(row_bytes), _ll(batch), ctypes.c_double(factor), _ll(cus)))
 
 
-TILE128 = ("128x64", "128, four stages", "256x128", "128, two stages")     # enum Tile128
+TILE128 = ("128x64", "128, four stages", "256x128", "128, two stages", "64x64")     # enum Tile128
 
 
 def tile128_variant(kind, m, n, k_bytes, batch=1, cus=256):
@@ -89,4 +89,4 @@ def tile128_variant(kind, m, n, k_bytes, batch=1, cus=256):
     "bf16", "mxfp4" (row-major scales), "mxfp4_tiled"; whole K steps."""
     if not lib().route_fits_128_tiles(_ll(m), _ll(n), _ll(batch), _ll(cus)):
         return None
-    return TILE128[lib().route_tile128_variant(_ll(m), _ll(n), _ll(k_bytes), _ll(batch), int(kind != "block"), int(kind in ("bf16", "mxfp4_tiled")), _ll(cus))]
+    return TILE128[lib().route_tile128_variant(_ll(m), _ll(n), _ll(k_bytes), _ll(batch), int(kind != "block"), int(kind in ("bf16", "mxfp4_tiled")), _ll(cus), int(kind == "block"))]
