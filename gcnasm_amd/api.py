@@ -50,7 +50,7 @@ def library_path():
 
 
 def build_library(verbose=False):
-    """Compile the HIP sources for gfx950 with hipcc (cross-compiles without a GPU)."""
+    """Compile the HIP sources for gfx950 with hipcc (cross-compiles without a GPU) and the host's binding."""
     subprocess.check_call(["make", "-C", os.path.join(_HERE, "csrc"), "-B"],
                           stdout=None if verbose else subprocess.DEVNULL,
                           stderr=None if verbose else subprocess.DEVNULL)
@@ -119,9 +119,60 @@ def status_string(status):
 
 
 # The host's part of a call is what a decoding step of a small layer waits for (1 x 4096 x 4096 with its quantiser: the two
-# launches take 8 us of device time).  Hence below: shapes and strides are read from a tensor once, the argument block is
-# filled by its constructor, the stream comes as the raw handle: quantize 10.3 -> 8.3 us per call, flatmm 12.8 -> 8.5 (of which the
-# library and its launch are 3.5, each allocation 1.8).
+# launches take 8 us of device time).  Hence the compiled path (csrc/binding.cpp) for ordinary tensors: the functions below try it first, and
+# go through their own statements where it answers None -- to name what is wrong with the arguments, or for tensor subclasses and active modes.
+_OPS = ("a8w8_gemm", "a8w8_gemm_blockscale", "a8w8_flatmm", "a16w16_gemm", "a16w16_flatmm", "a4w4_gemm", "a4w4_flatmm")
+_GEMM, _BLOCKSCALE, _FLATMM, _GEMM16, _FLATMM16, _GEMM4, _FLATMM4 = range(7)
+
+
+def _connect():
+    """Load csrc/binding.cpp's module on the first call that takes tensors and hand it the library's entry points."""
+    global _fast_gemm, _fast_quantize, _fast_quantize_mxfp4, _fast_encode, _fast_decode
+    _need_torch()
+    L = lib()
+    try:
+        from . import _binding
+    except ImportError as e:
+        raise FileNotFoundError(f"{os.path.join(_HERE, '_binding.so')} is missing or was built for another torch: build it with "
+                                f"gcnasm_amd.build_library() or `make -C gcnasm_amd/csrc` ({e})") from e
+    _binding.connect(*(ctypes.cast(getattr(L, f), ctypes.c_void_p).value
+                       for f in _OPS + ("a8w8_quantize", "a4w4_quantize_mx", "a8w8_cvt_f32_to_e4m3", "a8w8_cvt_e4m3_to_f32")))
+    _fast_gemm, _fast_quantize, _fast_quantize_mxfp4 = _binding.gemm, _binding.quantize, _binding.quantize_mxfp4
+    _fast_encode, _fast_decode = _binding.encode, _binding.decode
+
+
+def _fast_gemm(*args):
+    _connect()
+    return _fast_gemm(*args)
+
+
+def _fast_quantize(*args):
+    _connect()
+    return _fast_quantize(*args)
+
+
+def _fast_quantize_mxfp4(*args):
+    _connect()
+    return _fast_quantize_mxfp4(*args)
+
+
+def _fast_encode(*args):
+    _connect()
+    return _fast_encode(*args)
+
+
+def _fast_decode(*args):
+    _connect()
+    return _fast_decode(*args)
+
+
+def _done(result, where):
+    """What the compiled path returned: the outputs, or the status of a call that the library refused."""
+    if type(result) is int:
+        raise A8W8Error(result, where)
+    return result
+
+
 def _stream():
     """The current stream's handle (what torch.cuda.current_stream().cuda_stream holds, without the object around it)."""
     _need_torch()
@@ -280,6 +331,9 @@ def _args_from_tensors(a, b, sfa, sfb, scale_mode, c, c_dtype, b_preshuffled, n=
 def gemm(a, b, sfa, sfb, scale_mode, c=None, c_dtype=BF16, n=None):
     """C = dequant(A) @ dequant(B)^T through a8w8_gemm.  a [.., M, K] u8, b [.., N, K] u8 on the GPU; with `n` given,
     b is the flat pre-shuffled weight (preshuffle_b_device) of n rows."""
+    r = _fast_gemm(_GEMM, a, b, sfa, sfb, scale_mode, c, c_dtype, n)
+    if r is not None:
+        return _done(r, "a8w8_gemm")
     g, c = _args_from_tensors(a, b, sfa, sfb, scale_mode, c, c_dtype, 0 if n is None else 1, n=n)
     _check(lib().a8w8_gemm(ctypes.byref(g), _stream()), "a8w8_gemm")
     return c
@@ -288,6 +342,9 @@ def gemm(a, b, sfa, sfb, scale_mode, c=None, c_dtype=BF16, n=None):
 def gemm_a16w16(a, b, c=None, c_dtype=BF16, n=None):
     """C = A @ B^T for bf16 a [.., M, K] and b [.., N, K] (torch.bfloat16 on the GPU) through a16w16_gemm; with `n`
     given, b is the flat pre-shuffled weight of n rows (preshuffle_b_bf16_device)."""
+    r = _fast_gemm(_GEMM16, a, b, a, b, TENSOR, c, c_dtype, n)
+    if r is not None:
+        return _done(r, "a16w16_gemm")
     g, c = _args_from_tensors(a, b, a, b, TENSOR, c, c_dtype, 0 if n is None else 1, n=n, scaled=False)
     _check(lib().a16w16_gemm(ctypes.byref(g), _stream()), "a16w16_gemm")
     return c
@@ -302,6 +359,9 @@ def preshuffle_b_bf16_device(b):
 
 def flatmm_a16w16(a, b_shuffled, n, c=None, c_dtype=BF16):
     """Skinny-M bf16 GEMM over weights from preshuffle_b_bf16_device."""
+    r = None if n is None else _fast_gemm(_FLATMM16, a, b_shuffled, a, a, TENSOR, c, c_dtype, n)
+    if r is not None:
+        return _done(r, "a16w16_flatmm")
     g, c = _args_from_tensors(a, b_shuffled, a, a, TENSOR, c, c_dtype, 1, n=n, scaled=False)
     _check(lib().a16w16_flatmm(ctypes.byref(g), _stream()), "a16w16_flatmm")
     return c
@@ -309,6 +369,9 @@ def flatmm_a16w16(a, b_shuffled, n, c=None, c_dtype=BF16):
 
 def quantize_mxfp4(x, tiled=False):
     """fp32 [rows, K] -> (packed E2M1 bytes [rows, K/2], E8M0 scales row-major [rows, K/32] or tiled)."""
+    r = _fast_quantize_mxfp4(x, tiled)
+    if r is not None:
+        return _done(r, "a4w4_quantize_mx")
     _need_torch()
     rows, k = x.shape
     q = torch.empty((rows, k // 2), dtype=torch.uint8, device=x.device)
@@ -321,6 +384,9 @@ def quantize_mxfp4(x, tiled=False):
 def gemm_a4w4(a, b, sfa, sfb, scale_mode=MX_TILED, c=None, c_dtype=BF16, n=None):
     """MXFP4 GEMM through a4w4_gemm: a [M, K/2], b [N, K/2] packed E2M1 (uint8 on the GPU); with `n` given, b is the
     flat pre-shuffled weight of n rows (preshuffle_b_device on the packed bytes)."""
+    r = _fast_gemm(_GEMM4, a, b, sfa, sfb, scale_mode, c, c_dtype, n)
+    if r is not None:
+        return _done(r, "a4w4_gemm")
     _need_torch()
     m, k = a.shape[-2], a.shape[-1] * 2
     shuffled = n is not None
@@ -337,6 +403,9 @@ def gemm_a4w4(a, b, sfa, sfb, scale_mode=MX_TILED, c=None, c_dtype=BF16, n=None)
 def flatmm_a4w4(a, b_shuffled, sfa_tiled, sfb_tiled, n, c=None, c_dtype=BF16):
     """MXFP4 skinny-M GEMM through a4w4_flatmm: a [M, K/2] packed E2M1 with M <= 128, b_shuffled from
     preshuffle_b_device on the packed weight bytes [N, K/2], both scale arrays in the MX_TILED layout."""
+    r = None if n is None else _fast_gemm(_FLATMM4, a, b_shuffled, sfa_tiled, sfb_tiled, MX_TILED, c, c_dtype, n)
+    if r is not None:
+        return _done(r, "a4w4_flatmm")
     _need_torch()
     m, k = a.shape[-2], a.shape[-1] * 2
     c, c_dtype = _out(c, (m, n), c_dtype, a.device)
@@ -348,6 +417,9 @@ def flatmm_a4w4(a, b_shuffled, sfa_tiled, sfb_tiled, n, c=None, c_dtype=BF16):
 
 def gemm_blockscale(a, b, sfa, sfb, c=None, c_dtype=FP32):
     """The reference's block-scale GEMM (1x128 / 128x128 scales), fp32 C by default as there."""
+    r = _fast_gemm(_BLOCKSCALE, a, b, sfa, sfb, BLOCK, c, c_dtype, None)
+    if r is not None:
+        return _done(r, "a8w8_gemm_blockscale")
     g, c = _args_from_tensors(a, b, sfa, sfb, BLOCK, c, c_dtype, 0)
     _check(lib().a8w8_gemm_blockscale(ctypes.byref(g), _stream()), "a8w8_gemm_blockscale")
     return c
@@ -356,6 +428,9 @@ def gemm_blockscale(a, b, sfa, sfb, c=None, c_dtype=FP32):
 def flatmm(a, b_shuffled, sfa, sfb, n, scale_mode=ROWCOL, c=None, c_dtype=BF16):
     """Skinny-M GEMM over weights in the a8w8_preshuffle_b layout (flat u8 tensor of n*k bytes); scale_mode ROWCOL,
     TENSOR or MX_TILED (MXFP8: both scale arrays in the tiled layout)."""
+    r = None if n is None else _fast_gemm(_FLATMM, a, b_shuffled, sfa, sfb, scale_mode, c, c_dtype, n)
+    if r is not None:
+        return _done(r, "a8w8_flatmm")
     g, c = _args_from_tensors(a, b_shuffled, sfa, sfb, scale_mode, c, c_dtype, 1, n=n)
     _check(lib().a8w8_flatmm(ctypes.byref(g), _stream()), "a8w8_flatmm")
     return c
@@ -388,6 +463,9 @@ def preshuffle_b_device(b):
 
 
 def cvt_f32_to_e4m3(x, dialect=OCP, clamp240=False):
+    r = _fast_encode(x, dialect, clamp240)
+    if r is not None:
+        return _done(r, "a8w8_cvt_f32_to_e4m3")
     _need_torch()
     x = x.contiguous()
     out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
@@ -397,6 +475,9 @@ def cvt_f32_to_e4m3(x, dialect=OCP, clamp240=False):
 
 
 def cvt_e4m3_to_f32(codes, dialect=OCP):
+    r = _fast_decode(codes, dialect)
+    if r is not None:
+        return _done(r, "a8w8_cvt_e4m3_to_f32")
     _need_torch()
     codes = codes.contiguous()
     out = torch.empty(codes.shape, dtype=torch.float32, device=codes.device)
@@ -407,6 +488,9 @@ def cvt_e4m3_to_f32(codes, dialect=OCP):
 
 def quantize(x, scale_mode, group_rows=1):
     """fp32 [rows, K] -> (E4M3 bytes [rows, K], scales in the layout a8w8_gemm reads)."""
+    r = _fast_quantize(x, scale_mode, group_rows)
+    if r is not None:
+        return _done(r, "a8w8_quantize")
     _need_torch()
     rows, k = x.shape
     q = torch.empty((rows, k), dtype=torch.uint8, device=x.device)
