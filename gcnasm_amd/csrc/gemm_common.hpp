@@ -87,8 +87,8 @@ A8W8_DEV void tile_of_item(const TileMap& t, int item, int& batch, int& tm, int&
 {
     batch = div_by_known(item, t.tiles, t.inv_tiles);
     const int bid = item - batch * t.tiles;
-    int id = bid;
-    if ((t.tiles & 7) == 0) id = (bid & 7) * (t.tiles >> 3) + (bid >> 3);
+    // (220 tiles, 2816 x 5120 x 5120: 59.0 -> 58.0 us; 209, 2700 x 4736 x 5120: 63.5 -> 61.3)
+    const int id = (bid & 7) * (t.tiles >> 3) + min(bid & 7, t.tiles & 7) + (bid >> 3);
     const int group = div_by_known(id, t.per_group, t.inv_per_group);
     const int first_m = group * 8;
     const int in_group = id - group * t.per_group;
