@@ -142,7 +142,8 @@ A8W8_DEV int from_lane_8_apart(int v)
 //     (about 30 ns per store and compute unit either way), does not, and leaves step 2 out.
 // upper: the lane's row index within the 16 is 8 or more; source_low / _high: c_line_source of the lane for the two stores;
 // lane_offset_low / _high: the lane's place in the first / second store (c_line_offsets, per tile).
-template <bool BY_LANE>
+// WRITE_THROUGH: as in store_c_16; not where rows start inside a 64-byte piece of a line, whose halves would go to memory one by one.
+template <bool BY_LANE, bool WRITE_THROUGH = true>
 A8W8_DEV void store_c_lines(__amdgpu_buffer_rsrc_t rsrc, v4i lo, v4i hi, bool upper, int source_low, int source_high,
                             int lane_offset_low, int lane_offset_high, int scalar_offset)
 {
@@ -155,8 +156,8 @@ A8W8_DEV void store_c_lines(__amdgpu_buffer_rsrc_t rsrc, v4i lo, v4i hi, bool up
             second[e] = __builtin_amdgcn_ds_bpermute(source_high, second[e]);
         }
     }
-    store_c_16<true>(rsrc, first, lane_offset_low, scalar_offset);
-    store_c_16<true>(rsrc, second, lane_offset_high, scalar_offset);
+    store_c_16<WRITE_THROUGH>(rsrc, first, lane_offset_low, scalar_offset);
+    store_c_16<WRITE_THROUGH>(rsrc, second, lane_offset_high, scalar_offset);
 }
 // After step 1 lane 16 g + r16 holds, of row r16 % 8 of each store, a 16-byte piece of the row's line: in the first
 // store piece 4 u + g (bf16 pairs, DISTANCE 64: the line is two 64-byte halves of four pieces) or 2 g + u (fp32, DISTANCE

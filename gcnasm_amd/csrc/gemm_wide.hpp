@@ -306,7 +306,8 @@ gemm_a8w8_wide(PersistParams pp)
     int ep_batch = 0, ep_m0 = 0, ep_n0 = 0, ep_seq = 0;
     int tile_seq = 0;                               // tiles this workgroup has started: picks the row/col scale buffer
     float ep_ts = 1.f;
-    bool ep_vec_ok = false;                         // C rows of this batch entry take 16-byte stores
+    bool ep_vec_ok = false;                         // C rows of this batch entry start on dwords: 16-byte stores
+    bool ep_lines_ok = false;                       // ... and on 64-byte pieces of a line: written through
     // whole tiles go out through a buffer descriptor over the tile's own rows (store_c_16)
     __amdgpu_buffer_rsrc_t ep_rs;
     int ep_lane_off = 0, ep_row_bytes = 0;
@@ -343,7 +344,7 @@ gemm_a8w8_wide(PersistParams pp)
     // bf16, whole tiles: the pieces of tile pairs 2 jpp and 2 jpp + 1 of one MFMA tile row lie 64 bytes apart in every row;
     // the lanes of rows r and r + 8 exchange them (store_c_lines), and each of the two stores then writes eight whole
     // 128-byte lines instead of 64-byte halves of sixteen (a compute unit writes whole lines nearly twice as fast)
-    auto store_line_pair = [&](auto I, auto JPP) __attribute__((always_inline)) {
+    auto store_line_pair = [&](auto I, auto JPP, auto WT) __attribute__((always_inline)) {
         constexpr int i = decltype(I)::value, jpp = decltype(JPP)::value;
         float v0[8], v1[8];
         piece_values(I, std::integral_constant<int, 2 * jpp>{}, v0);
@@ -359,9 +360,9 @@ gemm_a8w8_wide(PersistParams pp)
             w1[e] = bf16x2_bits(v1[2 * e], v1[2 * e + 1]);
         }
         constexpr int row = PERM_A ? 32 * (i >> 1) + 4 * (i & 1) : 16 * i;
-        store_c_lines<A8W8_WIDE_LINES_BY_LANE != 0>(ep_rs, w0, w1, r16 >= 8, ep_line_src_low, ep_line_src_high, ep_line_low + 128 * jpp, ep_line_high + 128 * jpp, (int)((uint32_t)row * (uint32_t)ep_row_bytes));
+        store_c_lines<A8W8_WIDE_LINES_BY_LANE != 0, decltype(WT)::value != 0>(ep_rs, w0, w1, r16 >= 8, ep_line_src_low, ep_line_src_high, ep_line_low + 128 * jpp, ep_line_high + 128 * jpp, (int)((uint32_t)row * (uint32_t)ep_row_bytes));
     };
-    auto store_piece = [&](auto I, auto JP, bool checked) __attribute__((always_inline)) {
+    auto store_piece = [&](auto I, auto JP, bool checked, auto WT) __attribute__((always_inline)) {
         constexpr int i = decltype(I)::value, jp = decltype(JP)::value;
         const int cm = ep_m0 + wave_m * 128 + (PERM_A ? 8 * (r16 >> 2) + (r16 & 3) + 32 * (i >> 1) + 4 * (i & 1) : r16 + 16 * i);
         const int cn = ep_n0 + wave_n * 128 + 8 * g + 32 * jp;
@@ -369,7 +370,7 @@ gemm_a8w8_wide(PersistParams pp)
         float v[8];
         piece_values(I, JP, v);
         if (!checked) {
-            // a whole tile: through the tile's buffer descriptor
+            // through the tile's buffer descriptor
             constexpr int ES = CDT == C_BF16 ? 2 : 4;
             constexpr int row = PERM_A ? 32 * (i >> 1) + 4 * (i & 1) : 16 * i;
             const int voff = ep_lane_off + 32 * jp * ES, soff = (int)((uint32_t)row * (uint32_t)ep_row_bytes);
@@ -381,16 +382,16 @@ gemm_a8w8_wide(PersistParams pp)
                 v4i w;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) w[e] = bf16x2_bits(v[2 * e], v[2 * e + 1]);
-                store_c_16<A8W8_WIDE_WRITE_THROUGH != 0>(ep_rs, w, voff, soff);
+                store_c_16<A8W8_WIDE_WRITE_THROUGH != 0 && decltype(WT)::value != 0>(ep_rs, w, voff, soff);
             } else {
                 (void)voff;
-                store_c_lines<A8W8_WIDE_LINES_BY_LANE != 0>(ep_rs, __builtin_bit_cast(v4i, v4f{v[0], v[1], v[2], v[3]}), __builtin_bit_cast(v4i, v4f{v[4], v[5], v[6], v[7]}),
+                store_c_lines<A8W8_WIDE_LINES_BY_LANE != 0, decltype(WT)::value != 0>(ep_rs, __builtin_bit_cast(v4i, v4f{v[0], v[1], v[2], v[3]}), __builtin_bit_cast(v4i, v4f{v[4], v[5], v[6], v[7]}),
                               r16 >= 8, ep_line_src_low, ep_line_src_high, ep_line_low + 32 * jp * 4, ep_line_high + 32 * jp * 4, soff);
             }
             return;
         }
         if (cm >= p.m) return;
-        const bool vec = ep_vec_ok && cn + 7 < p.n;
+        const bool vec = ep_vec_ok && cn + 7 < p.n;      // (ordinary stores, which take any dword)
         if constexpr (CDT == C_BF16) {
             unsigned short* dst = (unsigned short*)c_base + (long long)cm * p.ldc + cn;
             if (vec) {
@@ -424,11 +425,26 @@ gemm_a8w8_wide(PersistParams pp)
         constexpr bool a_outer = decltype(AO)::value != 0;
         constexpr int i = (eq >> 1) * 4 + (a_outer ? (gq >> 1) : (gq & 3));
         constexpr int jp = (eq & 1) * 2 + (a_outer ? (gq & 1) : (gq >> 2));
-        store_piece(std::integral_constant<int, i>{}, std::integral_constant<int, jp>{}, false);
+        store_piece(std::integral_constant<int, i>{}, std::integral_constant<int, jp>{}, false, std::integral_constant<int, 1>{});
     };
     // the whole tile with every bounds and alignment check, for tiles the pieces cannot serve
     auto store_tile_checked = [&]() __attribute__((always_inline)) {
-        static_for<WIDE_T / 2>([&](auto JP) { static_for<WIDE_T>([&](auto I) { store_piece(I, JP, true); }); });
+        static_for<WIDE_T / 2>([&](auto JP) {
+            if (ep_n0 + wave_n * 128 + 32 * decltype(JP)::value < p.n)
+                static_for<WIDE_T>([&](auto I) { store_piece(I, JP, true, std::integral_constant<int, 0>{}); });
+        });
+    };
+    // The tile through its descriptor, which ends with the matrix's last row; columns past n are left out by whole groups (of 64, fp32 32).
+    auto store_tile = [&](auto WT) __attribute__((always_inline)) {
+        const int cols = p.n - ep_n0 - wave_n * 128;
+        if constexpr (CDT == C_BF16 && A8W8_WIDE_LINE_PAIRS)
+            static_for<WIDE_T / 4>([&](auto JPP) {
+                if (64 * decltype(JPP)::value < cols) static_for<WIDE_T>([&](auto I) { store_line_pair(I, JPP, WT); });
+            });
+        else
+            static_for<WIDE_T / 2>([&](auto JP) {
+                if (32 * decltype(JP)::value < cols) static_for<WIDE_T>([&](auto I) { store_piece(I, JP, false, WT); });
+            });
     };
     constexpr int STORES_PER_PIECE = CDT == C_BF16 ? 1 : 2;
 
@@ -734,10 +750,11 @@ gemm_a8w8_wide(PersistParams pp)
                 if constexpr (MODE == MODE_TENSOR)
                     ep_ts = ((const float*)p.sfa + (long long)cur_batch * p.sfa_batch)[0] * ((const float*)p.sfb + (long long)cur_batch * p.sfb_batch)[0];
                 const uintptr_t c_addr = (uintptr_t)p.c + (uintptr_t)((long long)cur_batch * p.c_batch * (CDT == C_BF16 ? 2 : 4));
-                ep_vec_ok = (p.ldc & (CDT == C_BF16 ? 7 : 3)) == 0 && (c_addr & 15) == 0;
+                ep_vec_ok = (CDT == C_FP32 || (p.ldc & 1) == 0) && (c_addr & 3) == 0;
+                ep_lines_ok = (p.ldc & (CDT == C_BF16 ? 31 : 15)) == 0 && (c_addr & 63) == 0;
                 {
                     constexpr int ES = CDT == C_BF16 ? 2 : 4;
-                    ep_rs = make_rsrc((const char*)c_addr + ((long long)m0 * p.ldc + n0) * ES, (uint32_t)((BM - 1) * p.ldc + BN) * ES);
+                    ep_rs = make_rsrc((const char*)c_addr + ((long long)m0 * p.ldc + n0) * ES, ((uint32_t)(min(p.m - m0, BM) - 1) * (uint32_t)p.ldc + (uint32_t)min(p.n - n0, BN)) * ES);
                     ep_row_bytes = p.ldc * ES;
                     auto row_of = [&](int r) __attribute__((always_inline)) { return PERM_A ? 8 * (r >> 2) + (r & 3) : r; };
                     // (unsigned arithmetic: with stride_c in the millions these byte offsets pass 2^31; the hardware takes them as unsigned)
@@ -748,13 +765,17 @@ gemm_a8w8_wide(PersistParams pp)
                                                                 wave_n * 128 * ES, ep_line_low, ep_line_high);
                 }
             }
-            // pieces are written without checks: only for whole tiles with aligned rows
-            const bool fast = ep_vec_ok && m0 + BM <= p.m && n0 + BN <= p.n;
+            // Pieces are written without checks where rows start on dwords and the matrix ends with a group of columns.  (With checks, an edge tile's
+            // stores ended 5 us after the others': 2816 x 4736 x 1024 bf16 C 25.5 us, 19.6 this way, 2816 x 5120 19.8; 4350 x 4224 x 1024 38.9, 33.3; rows
+            // on dwords only, 2816 x 4700 x 1024, element by element 45.0, 22.6; rows inside 64-byte pieces written through, 5000 x 5000 x 1024 fp32 C 63.8, 60.6.)
+            const bool columns_whole = n0 + BN <= p.n;
+            const bool fast = ep_vec_ok && (columns_whole || p.n % (CDT == C_BF16 && A8W8_WIDE_LINE_PAIRS ? 64 : 32) == 0) &&
+                              (BURST || odd || (columns_whole && m0 + BM <= p.m));
             if (last && odd) step(T{}, F{}, F{}, T{});
             else if (!BURST && last && fast) step(T{}, F{}, T{}, F{});
             else step(T{}, F{}, F{}, F{});
             if (last) {
-                have_prev = fast;
+                have_prev = fast && columns_whole;      // (the stores that the next tile's first step lets fly: all of them, or none)
                 if (fast && (BURST || odd)) {
                     // The whole tile in one burst between its last step and the next tile's first: a store among the
                     // MFMAs makes its wave wait for a place in the memory pipeline, which the loads of the next steps
@@ -762,10 +783,8 @@ gemm_a8w8_wide(PersistParams pp)
                     // written back to back the 32 stores of a wave cost less than they stretched those steps by.
                     // The next tile's first step lets them stay in flight (have_prev).
                     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // last MFMA -> first accumulator read
-                    if constexpr (CDT == C_BF16 && A8W8_WIDE_LINE_PAIRS)
-                        static_for<WIDE_T / 4>([&](auto JPP) { static_for<WIDE_T>([&](auto I) { store_line_pair(I, JPP); }); });
-                    else
-                        static_for<WIDE_T / 2>([&](auto JP) { static_for<WIDE_T>([&](auto I) { store_piece(I, JP, false); }); });
+                    if (ep_lines_ok) store_tile(T{});
+                    else store_tile(F{});
                 } else if (!fast) {
                     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // last MFMA -> first accumulator read
                     store_tile_checked();

@@ -42,7 +42,8 @@ def _mx_scales(rows, k, tiled, pad):
     return g.mx_tile_scales(whole), 0, value
 
 
-def check(kind, mode, m, n, k, batch=1, pad=0, shuffled=False):
+def check(kind, mode, m, n, k, batch=1, pad=0, shuffled=False, c_pad=0, c_shift=0):
+    """c_pad: elements between C's rows, c_shift: in front of its first one; neither may be written."""
     rng = np.random.Generator(np.random.Philox(m + n + k))
     per_byte = {"fp4": 2, "bf16": 0.5}.get(kind, 1)
     a, b = [[_operand(rng, rows, k, kind) for _ in range(batch)] for rows in (m, n)]
@@ -65,12 +66,14 @@ def check(kind, mode, m, n, k, batch=1, pad=0, shuffled=False):
         b_all = torch.stack([g.preshuffle_b_device(o[0][:, :row_bytes].contiguous()) for o in b])
         b_batch = n * k
     for c_dtype, dtype in ((g.FP32, torch.float32), (g.BF16, torch.bfloat16)):
-        c = torch.full((batch, m, n), float("nan"), dtype=dtype, device="cuda")
+        store = torch.full((c_shift + batch * m * (n + c_pad) + 64,), -7.0, dtype=dtype, device="cuda")
+        c = store[c_shift:c_shift + batch * m * (n + c_pad)].view(batch, m, n + c_pad)
         args = g.raw_gemm_args(a_all.data_ptr(), b_all.data_ptr(), c.data_ptr(), s_all[0].data_ptr(), s_all[1].data_ptr(), m, n, k, mode, c_dtype, batch,
-                               stride_a=stride, stride_b=stride, stride_sfa=sa[1], stride_sfb=sb[1],
-                               b_preshuffled=int(shuffled), batch_strides=(m * stride, b_batch, m * n, s_all[0].shape[1], s_all[1].shape[1]))
+                               stride_a=stride, stride_b=stride, stride_c=n + c_pad, stride_sfa=sa[1], stride_sfb=sb[1],
+                               b_preshuffled=int(shuffled), batch_strides=(m * stride, b_batch, m * (n + c_pad), s_all[0].shape[1], s_all[1].shape[1]))
         entry = {"fp4": g.lib().a4w4_gemm, "bf16": g.lib().a16w16_gemm}.get(kind, g.lib().a8w8_gemm)
         assert entry(ctypes.byref(args), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
         for e in range(batch):
             want = (a[e][1] * fa) @ (b[e][1] * fb).T
-            assert torch.equal(c[e], want.float().to(dtype)), (kind, mode, m, n, k, c_dtype, e)
+            assert torch.equal(c[e, :, :n], want.float().to(dtype)), (kind, mode, m, n, k, c_dtype, e)
+        assert bool((c[:, :, n:] == -7.0).all() and (store[:c_shift] == -7.0).all() and (store[c_shift + batch * m * (n + c_pad):] == -7.0).all())
