@@ -92,6 +92,9 @@ def lib():
         L.a8w8_cvt_e4m3_to_f32.argtypes = [vp, vp, ctypes.c_size_t, ctypes.c_int, vp]
         L.a8w8_quantize.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp, ctypes.c_int,
                                     ctypes.c_int, vp]
+        L.a8w8_quantize_ws.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp, ctypes.c_int, ctypes.c_int, vp, ctypes.c_size_t, vp]
+        L.a8w8_quantize_workspace_bytes.restype = ctypes.c_size_t
+        L.a8w8_quantize_workspace_bytes.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int]
         L.a8w8_mx_tile_scales.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp]
         L.a8w8_mx_tile_scales_ab.argtypes = [vp, ctypes.c_int, ctypes.c_int, vp, vp, ctypes.c_int, ctypes.c_int, vp,
                                              ctypes.c_int, vp]
@@ -136,7 +139,8 @@ def _connect():
         raise FileNotFoundError(f"{os.path.join(_HERE, '_binding.so')} is missing or was built for another torch: build it with "
                                 f"gcnasm_amd.build_library() or `make -C gcnasm_amd/csrc` ({e})") from e
     _binding.connect(*(ctypes.cast(getattr(L, f), ctypes.c_void_p).value
-                       for f in _OPS + ("a8w8_quantize", "a4w4_quantize_mx", "a8w8_cvt_f32_to_e4m3", "a8w8_cvt_e4m3_to_f32")))
+                       for f in _OPS + ("a8w8_quantize_ws", "a4w4_quantize_mx", "a8w8_cvt_f32_to_e4m3", "a8w8_cvt_e4m3_to_f32",
+                                        "a8w8_quantize_workspace_bytes")))
     _fast_gemm, _fast_quantize, _fast_quantize_mxfp4 = _binding.gemm, _binding.quantize, _binding.quantize_mxfp4
     _fast_encode, _fast_decode = _binding.encode, _binding.decode
 

@@ -990,6 +990,17 @@ int a8w8_cvt_e4m3_to_f32(const uint8_t* src, float* dst, size_t n, int dialect, 
 int a8w8_quantize(const float* src, int rows, int k, int ld, uint8_t* q, void* scale, int scale_mode, int group_rows,
                   void* hip_stream)
 {
+    return a8w8_quantize_ws(src, rows, k, ld, q, scale, scale_mode, group_rows, nullptr, 0, hip_stream);
+}
+
+size_t a8w8_quantize_workspace_bytes(int rows, int k, int scale_mode)
+{
+    return scale_mode == A8W8_SCALE_TENSOR && rows > 0 && k > 0 && (long long)rows * k > 4ll * QUANT_TENSOR_ONE ? sizeof(float) * QUANT_TENSOR_WS_PARTS : 0;
+}
+
+int a8w8_quantize_ws(const float* src, int rows, int k, int ld, uint8_t* q, void* scale, int scale_mode, int group_rows, void* workspace,
+                     size_t workspace_bytes, void* hip_stream)
+{
     if (!src || !q || !scale) return A8W8_ERR_NULL_POINTER;
     if (rows <= 0 || k <= 0) return A8W8_ERR_BAD_SHAPE;
     if (ld < k) return A8W8_ERR_BAD_STRIDE;
@@ -1006,6 +1017,12 @@ int a8w8_quantize(const float* src, int rows, int k, int ld, uint8_t* q, void* s
                 const size_t apply = (units + 256 * QUANT_TENSOR_UNITS - 1) / (256 * QUANT_TENSOR_UNITS);
                 // (a launch has less than 2^32 threads along a dimension; the kernels below walk an array of any size with a fixed grid)
                 if (apply * 256 < (1ull << 32)) {
+                    if (workspace && aligned16(workspace) && workspace_bytes >= sizeof(float) * QUANT_TENSOR_WS_PARTS) {
+                        const unsigned few = ((unsigned)std::min<size_t>((units + 1023) / 1024, QUANT_TENSOR_WS_PARTS) + 3) / 4 * 4;
+                        A8W8_LAUNCH_OR_RETURN(quant_tensor_amax_ws_kernel, dim3(few), dim3(512), 0, s, (const float4*)src, units, (float*)workspace);
+                        return launch(quant_tensor_apply_ws_kernel, dim3((unsigned)apply), dim3(256), 0, s, (const float4*)src, units, (uint32_t*)q, (float*)scale,
+                                      (const float*)workspace, (int)few);
+                    }
                     A8W8_LAUNCH_OR_RETURN(quant_tensor_amax_vec_kernel, dim3(parts), dim3(256), 0, s, (const float4*)src, units, (float*)q);
                     A8W8_LAUNCH_OR_RETURN(quant_tensor_fold_kernel, dim3(1), dim3(256), 0, s, (const float*)q, (int)parts, (float*)scale);
                     return launch(quant_tensor_apply_vec_kernel, dim3((unsigned)apply), dim3(256), 0, s, (const float4*)src, units, (uint32_t*)q,

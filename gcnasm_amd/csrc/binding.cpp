@@ -14,6 +14,7 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 
 #include "../../include/mi355_a8w8.h"
@@ -23,7 +24,8 @@ namespace {
 // the library's entry points, in the order of api.py's list (addresses: the library that api.py has loaded, whichever build it is)
 enum Op { GEMM, GEMM_BLOCKSCALE, FLATMM, GEMM_A16W16, FLATMM_A16W16, GEMM_A4W4, FLATMM_A4W4, GEMM_OPS };
 decltype(&a8w8_gemm) g_gemm[GEMM_OPS];
-decltype(&a8w8_quantize) g_quantize;
+decltype(&a8w8_quantize_ws) g_quantize;
+decltype(&a8w8_quantize_workspace_bytes) g_workspace_bytes;
 decltype(&a4w4_quantize_mx) g_quantize_mx;
 decltype(&a8w8_cvt_f32_to_e4m3) g_encode;
 decltype(&a8w8_cvt_e4m3_to_f32) g_decode;
@@ -93,9 +95,14 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t count)
     const void* src = x->data_ptr();
     void *qp = q.data_ptr(), *sp = s.data_ptr(), *st = stream();
     const int64_t ld = x->stride(0);
+    // (the workspace goes back to the allocator with this call: to be handed out again behind it on the stream that it was allocated on, which is the
+    // launches' own only on the current device)
+    const size_t ws_bytes = x->device().index() == c10::hip::current_device() ? g_workspace_bytes((int)rows, (int)k, (int)mode) : 0;
+    const at::Tensor ws = ws_bytes ? allocate({(int64_t)ws_bytes}, at::kByte, *x) : at::Tensor();
+    void* wp = ws_bytes ? ws.data_ptr() : nullptr;
     int status;
     Py_BEGIN_ALLOW_THREADS
-    status = g_quantize((const float*)src, (int)rows, (int)k, (int)ld, (uint8_t*)qp, sp, (int)mode, (int)group, st);
+    status = g_quantize((const float*)src, (int)rows, (int)k, (int)ld, (uint8_t*)qp, sp, (int)mode, (int)group, wp, ws_bytes, st);
     Py_END_ALLOW_THREADS
     return status ? PyLong_FromLong(status) : pair(q, s);
     END_HANDLE_TH_ERRORS
@@ -255,8 +262,8 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t count)
 // (address, ...) of the entry points, in the order of their variables above
 PyObject* connect(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
-    void* p[GEMM_OPS + 4];
-    if (count != GEMM_OPS + 4) {
+    void* p[GEMM_OPS + 5];
+    if (count != GEMM_OPS + 5) {
         PyErr_SetString(PyExc_TypeError, "one address per entry point");
         return nullptr;
     }
@@ -268,10 +275,11 @@ PyObject* connect(PyObject*, PyObject* const* args, Py_ssize_t count)
         }
     }
     for (int i = 0; i < GEMM_OPS; ++i) g_gemm[i] = (decltype(&a8w8_gemm))p[i];
-    g_quantize = (decltype(&a8w8_quantize))p[GEMM_OPS];
+    g_quantize = (decltype(&a8w8_quantize_ws))p[GEMM_OPS];
     g_quantize_mx = (decltype(&a4w4_quantize_mx))p[GEMM_OPS + 1];
     g_encode = (decltype(&a8w8_cvt_f32_to_e4m3))p[GEMM_OPS + 2];
     g_decode = (decltype(&a8w8_cvt_e4m3_to_f32))p[GEMM_OPS + 3];
+    g_workspace_bytes = (decltype(&a8w8_quantize_workspace_bytes))p[GEMM_OPS + 4];
     Py_RETURN_NONE;
 }
 

@@ -754,6 +754,56 @@ __global__ void __launch_bounds__(256) quant_tensor_apply_vec_kernel(const float
         if (i0 + 256 * u < units)
             q[i0 + 256 * u] = pack4_e4m3(__fdiv_rn(v[u].x, s), __fdiv_rn(v[u].y, s), __fdiv_rn(v[u].z, s), __fdiv_rn(v[u].w, s));
 }
+// The same in two launches, with memory of the caller's for the maxima: pass 1 over at most QUANT_TENSOR_WS_PARTS workgroups, whose maxima (a multiple of
+// four of them) every wave of pass 2 folds for itself, behind its own loads.  2560 x 2560 16.2 -> 14.7 us, 276 x 2880 6.9 -> 5.7, 163 x 1380 6.7 -> 5.2
+// (a launch is 2.4); 8192 x 8192 97.5 -> 97.0.  (1024 workgroups of 256 threads in pass 1 15.0 and 5.9, four units per thread in pass 2 14.9 and 6.2.)
+constexpr int QUANT_TENSOR_WS_PARTS = 512;
+__global__ void __launch_bounds__(512) quant_tensor_amax_ws_kernel(const float4* __restrict__ src, size_t units, float* __restrict__ parts)
+{
+    __shared__ float part[8];
+    float amax = 0.f;
+    const size_t stride = (size_t)gridDim.x * 512;
+    for (size_t i = (size_t)blockIdx.x * 512 + threadIdx.x; i < units; i += 4 * stride) {
+        float4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = i + u * stride < units ? src[i + u * stride] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
+    }
+    amax = wave_max(amax);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = amax;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < 8; ++w) amax = fmaxf(amax, part[w]);
+        parts[blockIdx.x] = amax;
+    }
+}
+__global__ void __launch_bounds__(256) quant_tensor_apply_ws_kernel(const float4* __restrict__ src, size_t units, uint32_t* __restrict__ q,
+                                                                    float* __restrict__ scale, const float* __restrict__ parts, int n)
+{
+    constexpr int U = QUANT_TENSOR_UNITS, P = QUANT_TENSOR_WS_PARTS / 256;
+    const size_t i0 = (size_t)(gridDim.x - 1 - blockIdx.x) * (256 * U) + threadIdx.x;
+    float4 m[P], v[U];
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+        const int i = (threadIdx.x & 63) * 4 + 256 * u;
+        m[u] = i < n ? *(const float4*)(parts + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = i0 + 256 * u < units ? load_once4((const float*)(src + i0 + 256 * u)) : make_float4(0.f, 0.f, 0.f, 0.f);
+    float amax = 0.f;
+#pragma unroll
+    for (int u = 0; u < P; ++u) amax = fmaxf(amax, fmaxf(fmaxf(m[u].x, m[u].y), fmaxf(m[u].z, m[u].w)));
+    amax = wave_max(amax);
+    const float s = amax > 0.f ? __fdiv_rn(amax, 448.0f) : 1.0f;   // an all-zero group keeps scale 1
+    if (blockIdx.x == 0 && threadIdx.x == 0) *scale = s;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (i0 + 256 * u < units)
+            q[i0 + 256 * u] = pack4_e4m3(__fdiv_rn(v[u].x, s), __fdiv_rn(v[u].y, s), __fdiv_rn(v[u].z, s), __fdiv_rn(v[u].w, s));
+}
 // Up to QUANT_TENSOR_ONE units: one workgroup, one launch, the array in its registers (1 x 4096 2.7 us against 6.1 in three
 // launches, 4 x 4096 4.0 against 6.2; with eight units per thread 8 x 4096 5.9 against 6.3, which one compute unit's loads bound).
 constexpr int QUANT_TENSOR_ONE = 4096;

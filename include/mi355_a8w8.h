@@ -206,6 +206,14 @@ A8W8_API int a8w8_cvt_e4m3_to_f32(const uint8_t* src_dev, float* dst_dev, size_t
 A8W8_API int a8w8_quantize(const float* src_dev, int rows, int k, int ld, uint8_t* q_dev, void* scale_dev,
                            int scale_mode, int group_rows, void* hip_stream);
 
+/* The same with memory of the caller's for intermediate values: a8w8_quantize_workspace_bytes(rows, k, scale_mode) bytes (0 where none is of use; a
+ * multiple of 16, at most 2 KiB) on the current device, 16-byte aligned, with any content, not used by anything else until the stream reaches the
+ * end of the call.  TENSOR then takes two launches instead of three.  The results are the same, bit for bit; a NULL, short or misaligned workspace
+ * is not used.  No counterpart in the reference. */
+A8W8_API size_t a8w8_quantize_workspace_bytes(int rows, int k, int scale_mode);
+A8W8_API int a8w8_quantize_ws(const float* src_dev, int rows, int k, int ld, uint8_t* q_dev, void* scale_dev, int scale_mode, int group_rows,
+                              void* workspace_dev, size_t workspace_bytes, void* hip_stream);
+
 /* E8M0 scales, row-major sf[r*stride + k/32] -> the MX_TILED layout, device buffers
  * (a8w8_mx_tiled_bytes(rows, k) bytes at out, 16-byte aligned).  No counterpart in the
  * reference, which has no MXFP8 program; weights' scales are converted once, activations'
