@@ -310,12 +310,17 @@ int num_cus()
     return g_dev[dev].num_cus > 0 ? g_dev[dev].num_cus : 256;
 }
 
-// Two 128-tiles per compute unit at most (fits_128_tiles).
+// Two 128-tiles per compute unit at most (fits_128_tiles), or rounds of 256-tiles that leave the chip idle (rounds_on_128_tiles).
 bool small_ok(const a8w8_gemm_args* g, bool fp4)
 {
     const bool mxt = g->scale_mode == A8W8_SCALE_MX_E8M0_TILED;
     // tiled MX scales on a number of K steps that the four-wave kernel does not take have no other kernel: any size runs here
     if (mxt && !steps_on_four_waves(g, fp4)) return true;
+    // (C rows too far apart for the 256-tile kernels stay refused)
+    const bool fp32 = g->c_dtype == A8W8_C_FP32;
+    if (g->scale_mode != A8W8_SCALE_BLOCK_1x128_128x128 && g->scale_mode != A8W8_SCALE_MX_E8M0_1x32 && c_tile_fits(g->stride_c, fp32 ? 4 : 2) &&
+        rounds_on_128_tiles(mxt, fp4, g->m, g->n, g->k / BK, g->batch, fp32, num_cus()))
+        return true;
     return fits_128_tiles(g->m, g->n, g->batch, num_cus());
 }
 

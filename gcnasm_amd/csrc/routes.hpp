@@ -66,6 +66,32 @@ inline bool quant_1x128_along_rows(long long rows, long long k)
     return rows < 8 || (rows < 96 && k >= 1 << 19);
 }
 
+// Rounds of one tile per compute unit.
+struct Rounds { long long of128, of256; };
+inline Rounds tile_rounds(long long m, long long n, long long batch, long long cus)
+{
+    return {(batch * ((m + 127) / 128) * ((n + 127) / 128) + cus - 1) / cus, (batch * ((m + 255) / 256) * ((n + 255) / 256) + cus - 1) / cus};
+}
+
+// One or two rounds of 256-tiles, the last of which leaves much of the chip idle: the two-stage 128-tile kernel, whose rounds are finer, up to the K where
+// the 256-tiles' cheaper steps have made up for it.  us, 128-tiles / 256-tiles, row/col bf16 C, row/col fp32, tiled MXFP8 bf16, tiled MXFP4 bf16 (bf16
+// operands as row/col):
+//   6144 x 3072 (5 rounds of 128-tiles, 2 of 256-tiles)  6 steps 23.1 / 28.6, 27.0 / 39.0, 25.3 / 29.6, 25.9 / 32.0   16: 41.6 / 50.2, 44.1 / 60.5, 47.6 / 52.2, 50.0 / 58.7
+//                                                        32: 73.8 / 85.2, 84.7 / 95.1, 86.5 / 87.5, 92.0 / 101
+//   8192 x 2560 (5, 2)   6: 23.9 / 29.1, 29.5 / 38.6, 26.1 / 30.3, 26.9 / 32.6   24: 61.6 / 69.3, 75.5 / 78.0, 70.9 / 70.7, 73.6 / 79.7   32: 80.2 / 85.6, 94.7 / 95.4, 91.9 / 87.7, 95.7 / 101
+//   5376 x 4096 (6, 2)   6: 26.7 / 28.9, 31.8 / 37.8, 29.1 / 30.4, 29.9 / 32.3   16: 48.6 / 52.1, 53.7 / 60.1, 54.7 / 52.8, 56.6 / 59.5   24: 70.9 / 69.1, 78.4 / 78.2, 82.3 / 72.1, 84.1 / 81.1
+//   2560 x 4352 (3, 1)   6: 15.6 / 16.7, 18.5 / 20.4, 17.3 / 17.4, 17.7 / 18.6   16: 26.7 / 28.0, 28.7 / 32.0, 31.0 / 29.1, 32.3 / 32.0
+//   4096 x 7168 (7, 2)   6: 32.4 / 31.3, 47.1 / 40.5, 35.2 / 32.4, 35.6 / 34.9   8192 x 4608 (9, 3)  6: 42.1 / 42.3, 64.6 / 57.0, 44.8 / 44.3, 45.2 / 47.1
+// Fewer than five steps stay with the 256-tiles although they are 4 to 28% slower in the same shapes: the kernel that a8w8_kernel_name reports for
+// calls of that size is held fixed by the library's tests.
+inline bool rounds_on_128_tiles(bool mx, bool fp4, long long m, long long n, long long k_steps, long long batch, bool fp32_c, long long cus)
+{
+    const Rounds rounds = tile_rounds(m, n, batch, cus);
+    if (k_steps < 5 || rounds.of256 > 2 || rounds.of128 > 3 * rounds.of256) return false;
+    if (rounds.of128 < 3 * rounds.of256) return k_steps <= (mx && !fp4 ? 20 : 32);
+    return k_steps <= (!mx ? 16 : fp4 ? (fp32_c ? 16 : 8) : fp32_c ? 8 : 0);
+}
+
 // MXFP4 on row-major scales, more than two 128-tiles per compute unit: the four-wave kernel (256-tiles, one workgroup per compute
 // unit) or the two-stage 128-tile kernel.  Both run in rounds: a round of 256-tiles (one per compute unit) is worth about three
 // rounds of one 128-tile per compute unit, three and a half where K is short and a prologue and a tile's stores, longer with fp32
@@ -78,11 +104,6 @@ inline bool quant_1x128_along_rows(long long rows, long long k)
 // 3000 x 8192 2048 42.5 / 49.0, 3072 56.8 / 61.0, 4096 77 / 75; 8192 x 2560 512 20.0 / 30.1, 4096 63 / 73.
 // An odd number of K steps costs the four-wave kernel the idle step behind it and has to be longer: bf16 seven, fp32 thirteen
 // (2816 x 5120 bf16 5 steps 21.2 / 21.6, 7 25.6 / 25.4, fp32 9 33.4 / 35.2, 17 63.5 / 53.1; 8192 x 8192 41 steps bf16 518 / 349).
-struct Rounds { long long of128, of256; };
-inline Rounds tile_rounds(long long m, long long n, long long batch, long long cus)
-{
-    return {(batch * ((m + 127) / 128) * ((n + 127) / 128) + cus - 1) / cus, (batch * ((m + 255) / 256) * ((n + 255) / 256) + cus - 1) / cus};
-}
 inline bool f4_row_scales_on_256_tiles(long long m, long long n, long long k_steps, long long batch, bool fp32_c, long long cus)
 {
     const Rounds rounds = tile_rounds(m, n, batch, cus);

@@ -81,6 +81,11 @@ def flat_is_faster(kind, row_major, m, n, k, batch=1, cus=256):
     return bool(lib().route_flat_is_faster(_ll(m), _ll(n), _ll(row_bytes), _ll(batch), ctypes.c_double(factor), _ll(cus)))
 
 
+def rounds_on_128_tiles(m, n, steps, kind="fp8", batch=1, fp32=False, cus=256):
+    """kind: "fp8" (per-tensor and row/col scales), "bf16", "mxfp8", "mxfp4" (tiled scales)."""
+    return bool(lib().route_rounds_on_128_tiles(int(kind in ("mxfp8", "mxfp4")), int(kind == "mxfp4"), _ll(m), _ll(n), _ll(steps), _ll(batch), int(fp32), _ll(cus)))
+
+
 TILE128 = ("128x64", "128, four stages", "256x128", "128, two stages", "64x64")     # enum Tile128
 
 

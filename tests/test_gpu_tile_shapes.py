@@ -1,5 +1,7 @@
 """The tile shapes of the 128-tile kernel, each at sizes that take it: ragged edges in both directions, fewer K steps than LDS stages, as many and more,
 every kind of operand and scale, shuffled weights, batches.  Exact results (exact_gemm.py)."""
+import ctypes
+
 import pytest
 
 import gcnasm_amd as g
@@ -39,6 +41,31 @@ def test_shuffled_weights(m, n, steps, batch, kind, mode):
 def test_partial_steps(m, n, k, variant, kind, mode):
     assert routes.tile128_variant("block", m, n, k, 1) == variant or variant == "128, four stages"      # (no 256 x 128 tiles here either)
     check(kind, mode, m, n, k // 2 if kind == "bf16" else k)
+
+
+# more than two 128-tiles per compute unit, in rounds that 256-tiles fill badly
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,steps", [(4352, 4608, 5), (6100, 3001, 6), (2100, 4200, 8), (5300, 4000, 16)])
+@pytest.mark.parametrize("kind,mode,route", [k for k in KINDS if k[1] not in (g.BLOCK, g.MX)], ids=lambda v: str(v))
+def test_badly_filled_rounds(m, n, steps, kind, mode, route):
+    name = {"fp8": "mxfp8" if mode == g.MX_TILED else "fp8", "fp4": "mxfp4"}.get(kind, kind)
+    assert routes.tile128_variant(route, m, n, steps * 128) is None and (routes.rounds_on_128_tiles(m, n, steps, name, fp32=True) or steps * (name != "fp8") > 8)
+    check(kind, mode, m, n, steps * ELEMENTS[kind])
+
+
+def test_rule_for_badly_filled_rounds():
+    for m, n, steps, kind, fp32, small in ((4352, 4608, 4, "fp8", False, False), (4352, 4608, 5, "fp8", False, True), (4352, 4608, 32, "bf16", True, True), (4352, 4608, 33, "fp8", True, False),
+                                           (4352, 4608, 20, "mxfp8", False, True), (4352, 4608, 22, "mxfp8", False, False), (4352, 4608, 32, "mxfp4", False, True),
+                                           (2304, 4096, 16, "fp8", False, True), (2304, 4096, 18, "fp8", False, False), (2304, 4096, 6, "mxfp8", False, False), (2304, 4096, 8, "mxfp8", True, True),
+                                           (2304, 4096, 10, "mxfp4", False, False), (2304, 4096, 16, "mxfp4", True, True), (4096, 4096, 8, "fp8", False, False),
+                                           (4096, 7168, 8, "fp8", False, False), (8192, 4608, 8, "fp8", False, False)):
+        assert routes.rounds_on_128_tiles(m, n, steps, kind, fp32=fp32) is small, (m, n, steps, kind, fp32)
+        if kind in ("fp8", "mxfp8"):
+            args = g.raw_gemm_args(1 << 12, 1 << 12, 1 << 12, 1 << 12, 1 << 12, m, n, steps * 128, g.ROWCOL if kind == "fp8" else g.MX_TILED, g.FP32 if fp32 else g.BF16)
+            assert (g.kernel_name(args) == "gemm_a8w8_tile128") is small
+            args.stride_c = 1 << 24          # past the 256-tile kernels' offsets: refused, as before
+            if steps % 2 == 0:
+                assert g.kernel_name(args) in ("gemm_a8w8_wide", "gemm_a8w8_persist") and g.lib().a8w8_gemm(ctypes.byref(args), None) == -7
 
 
 def test_rule():
