@@ -287,14 +287,14 @@ bool small_ok(const a8w8_gemm_args* g, bool fp4 = false);
 // MXFP4 with row-major scales on the four-wave kernel (`g`: byte view, k in bytes, row-major scale mode).  It fetches 16 scale
 // bytes of a row at a time (two K steps) with 32-bit offsets that run up to 256 rows past the end of the matrix.  Scale rows of an odd number of
 // steps are eight bytes more than a multiple of 16, and its loads then start on dwords, as the caller has checked.  Up to two 128-tiles per
-// compute unit (small_ok, the line of every other mode) and where f4_row_scales_on_256_tiles says so the 128-tile kernel is the faster one.
+// compute unit (fits_128_tiles, the line of every other mode) and where f4_row_scales_on_256_tiles says so the 128-tile kernel is the faster one.
 bool wide_row_scales_ok(const a8w8_gemm_args* g)
 {
     const bool odd = (g->k / BK) % 2 != 0;
     const auto rows_ok = [&](const void* s, long long stride, long long batch_stride, long long rows) {
         return (odd || (aligned16(s) && stride % 16 == 0 && (g->batch == 1 || batch_stride % 16 == 0))) && (rows + BM) * stride < (1ll << 31);
     };
-    return !small_ok(g) && f4_row_scales_on_256_tiles(g->m, g->n, g->k / BK, g->batch, g->c_dtype == A8W8_C_FP32, num_cus()) &&
+    return !fits_128_tiles(g->m, g->n, g->batch, num_cus()) && f4_row_scales_on_256_tiles(g->m, g->n, g->k / BK, g->batch, g->c_dtype == A8W8_C_FP32, num_cus()) &&
            items_ok(g) && rows_ok(g->sfa, g->stride_sfa, g->stride_sfa_batch, g->m) &&
            rows_ok(g->sfb, g->stride_sfb, g->stride_sfb_batch, g->n) && c_tile_fits(g->stride_c, g->c_dtype == A8W8_C_BF16 ? 2 : 4);
 }
@@ -318,9 +318,9 @@ bool small_ok(const a8w8_gemm_args* g, bool fp4)
     if (mxt && !steps_on_four_waves(g, fp4)) return true;
     // (C rows too far apart for the 256-tile kernels stay refused)
     const bool fp32 = g->c_dtype == A8W8_C_FP32;
-    if (g->scale_mode != A8W8_SCALE_BLOCK_1x128_128x128 && g->scale_mode != A8W8_SCALE_MX_E8M0_1x32 && c_tile_fits(g->stride_c, fp32 ? 4 : 2) &&
-        rounds_on_128_tiles(mxt, fp4, g->m, g->n, g->k / BK, g->batch, fp32, num_cus()))
-        return true;
+    const RoundsKind kind = mxt ? (fp4 ? ROUNDS_MXFP4_TILED : ROUNDS_MXFP8_TILED) : g->scale_mode == A8W8_SCALE_BLOCK_1x128_128x128 ? ROUNDS_BLOCK
+                            : g->scale_mode == A8W8_SCALE_MX_E8M0_1x32 ? ROUNDS_MXFP8_ROWS : ROUNDS_PLAIN;
+    if (c_tile_fits(g->stride_c, fp32 ? 4 : 2) && rounds_on_128_tiles(kind, g->m, g->n, g->k / BK, g->batch, fp32, num_cus())) return true;
     return fits_128_tiles(g->m, g->n, g->batch, num_cus());
 }
 

@@ -84,12 +84,23 @@ inline Rounds tile_rounds(long long m, long long n, long long batch, long long c
 //   4096 x 7168 (7, 2)   6: 32.4 / 31.3, 47.1 / 40.5, 35.2 / 32.4, 35.6 / 34.9   8192 x 4608 (9, 3)  6: 42.1 / 42.3, 64.6 / 57.0, 44.8 / 44.3, 45.2 / 47.1
 // Fewer than five steps stay with the 256-tiles although they are 4 to 28% slower in the same shapes: the kernel that a8w8_kernel_name reports for
 // calls of that size is held fixed by the library's tests.
-inline bool rounds_on_128_tiles(bool mx, bool fp4, long long m, long long n, long long k_steps, long long batch, bool fp32_c, long long cus)
+// Against the eight-wave kernel, 128-tiles / 256-tiles, block scales bf16 C, fp32, row-major MXFP8 bf16, fp32:
+//   6144 x 3072  8 steps 29.5 / 33.7, 32.3 / 41.6, 31.2 / 34.6, 34.0 / 41.9   16: 47.0 / 54.8, 50.0 / 62.3, 50.9 / 55.2, 54.0 / 62.9   32: 84.8 / 98.0, 90.7 / 105, 99.8 / 95.6, 106 / 106
+//   5376 x 4096  8: 33.6 / 36.0, 37.9 / 43.6, 35.7 / 36.9, 39.6 / 42.8   12: 44.6 / 48.3, 48.8 / 56.0, 46.9 / 48.1, 50.7 / 53.1   24: 75.9 / 80.6, 81.4 / 87.7, 89.1 / 80.5, 94.2 / 85.6
+//   2304 x 4096  8: 19.5 / 19.1, 21.9 / 23.1, 20.1 / 19.5, 22.7 / 23.4   16: 30.4 / 29.5, 31.9 / 33.7, 32.0 / 31.3, 33.8 / 34.6
+enum RoundsKind { ROUNDS_PLAIN, ROUNDS_MXFP8_TILED, ROUNDS_MXFP4_TILED, ROUNDS_BLOCK, ROUNDS_MXFP8_ROWS };      // (plain: per-tensor and row/col scales, bf16)
+inline bool rounds_on_128_tiles(RoundsKind kind, long long m, long long n, long long k_steps, long long batch, bool fp32_c, long long cus)
 {
     const Rounds rounds = tile_rounds(m, n, batch, cus);
     if (k_steps < 5 || rounds.of256 > 2 || rounds.of128 > 3 * rounds.of256) return false;
-    if (rounds.of128 < 3 * rounds.of256) return k_steps <= (mx && !fp4 ? 20 : 32);
-    return k_steps <= (!mx ? 16 : fp4 ? (fp32_c ? 16 : 8) : fp32_c ? 8 : 0);
+    const bool finer = rounds.of128 < 3 * rounds.of256, two = rounds.of256 == 2;
+    switch (kind) {
+        case ROUNDS_MXFP8_TILED: return k_steps <= (finer ? 20 : fp32_c ? 8 : 0);
+        case ROUNDS_MXFP4_TILED: return k_steps <= (finer ? 32 : fp32_c ? 16 : 8);
+        case ROUNDS_BLOCK: return k_steps <= (finer ? 32 : two ? 24 : fp32_c ? 16 : 0);
+        case ROUNDS_MXFP8_ROWS: return k_steps <= (finer ? 16 : fp32_c ? 12 : two ? 8 : 0);
+        default: return k_steps <= (finer ? 32 : 16);
+    }
 }
 
 // MXFP4 on row-major scales, more than two 128-tiles per compute unit: the four-wave kernel (256-tiles, one workgroup per compute

@@ -31,9 +31,9 @@ int route_flat_is_faster(long long m, long long n, long long row_bytes, long lon
 {
     return a8w8::flat_is_faster(m, n, row_bytes, batch, layout_factor, cus);
 }
-int route_rounds_on_128_tiles(int mx, int fp4, long long m, long long n, long long k_steps, long long batch, int fp32_c, long long cus)
+int route_rounds_on_128_tiles(int kind, long long m, long long n, long long k_steps, long long batch, int fp32_c, long long cus)
 {
-    return a8w8::rounds_on_128_tiles(mx != 0, fp4 != 0, m, n, k_steps, batch, fp32_c != 0, cus);
+    return a8w8::rounds_on_128_tiles((a8w8::RoundsKind)kind, m, n, k_steps, batch, fp32_c != 0, cus);
 }
 int route_fits_128_tiles(long long m, long long n, long long batch, long long cus) { return a8w8::fits_128_tiles(m, n, batch, cus); }
 int route_tile128_variant(long long m, long long n, long long k_bytes, long long batch, int has_tall, int cheap_steps, long long cus, int block)

@@ -82,8 +82,8 @@ def flat_is_faster(kind, row_major, m, n, k, batch=1, cus=256):
 
 
 def rounds_on_128_tiles(m, n, steps, kind="fp8", batch=1, fp32=False, cus=256):
-    """kind: "fp8" (per-tensor and row/col scales), "bf16", "mxfp8", "mxfp4" (tiled scales)."""
-    return bool(lib().route_rounds_on_128_tiles(int(kind in ("mxfp8", "mxfp4")), int(kind == "mxfp4"), _ll(m), _ll(n), _ll(steps), _ll(batch), int(fp32), _ll(cus)))
+    """kind: "fp8" (per-tensor and row/col scales), "bf16", "mxfp8", "mxfp4" (tiled scales), "block", "mx" (row-major scales)."""
+    return bool(lib().route_rounds_on_128_tiles({"fp8": 0, "bf16": 0, "mxfp8": 1, "mxfp4": 2, "block": 3, "mx": 4}[kind], _ll(m), _ll(n), _ll(steps), _ll(batch), int(fp32), _ll(cus)))
 
 
 TILE128 = ("128x64", "128, four stages", "256x128", "128, two stages", "64x64")     # enum Tile128

@@ -46,9 +46,10 @@ def test_partial_steps(m, n, k, variant, kind, mode):
 # more than two 128-tiles per compute unit, in rounds that 256-tiles fill badly
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,steps", [(4352, 4608, 5), (6100, 3001, 6), (2100, 4200, 8), (5300, 4000, 16)])
-@pytest.mark.parametrize("kind,mode,route", [k for k in KINDS if k[1] not in (g.BLOCK, g.MX)], ids=lambda v: str(v))
+@pytest.mark.parametrize("kind,mode,route", [k for k in KINDS if k != ("fp4", g.MX, "mxfp4")], ids=lambda v: str(v))
 def test_badly_filled_rounds(m, n, steps, kind, mode, route):
-    name = {"fp8": "mxfp8" if mode == g.MX_TILED else "fp8", "fp4": "mxfp4"}.get(kind, kind)
+    n = n // 128 * 128 if mode == g.BLOCK else n
+    name = {"fp8": {g.MX_TILED: "mxfp8", g.MX: "mx", g.BLOCK: "block"}.get(mode, "fp8"), "fp4": "mxfp4"}.get(kind, kind)
     assert routes.tile128_variant(route, m, n, steps * 128) is None and (routes.rounds_on_128_tiles(m, n, steps, name, fp32=True) or steps * (name != "fp8") > 8)
     check(kind, mode, m, n, steps * ELEMENTS[kind])
 
@@ -58,10 +59,13 @@ def test_rule_for_badly_filled_rounds():
                                            (4352, 4608, 20, "mxfp8", False, True), (4352, 4608, 22, "mxfp8", False, False), (4352, 4608, 32, "mxfp4", False, True),
                                            (2304, 4096, 16, "fp8", False, True), (2304, 4096, 18, "fp8", False, False), (2304, 4096, 6, "mxfp8", False, False), (2304, 4096, 8, "mxfp8", True, True),
                                            (2304, 4096, 10, "mxfp4", False, False), (2304, 4096, 16, "mxfp4", True, True), (4096, 4096, 8, "fp8", False, False),
-                                           (4096, 7168, 8, "fp8", False, False), (8192, 4608, 8, "fp8", False, False)):
+                                           (4096, 7168, 8, "fp8", False, False), (8192, 4608, 8, "fp8", False, False), (4352, 4608, 32, "block", False, True),
+                                           (5376, 4096, 24, "block", False, True), (5376, 4096, 26, "block", True, False), (2304, 4096, 8, "block", False, False),
+                                           (2304, 4096, 16, "block", True, True), (4352, 4608, 16, "mx", False, True), (4352, 4608, 18, "mx", True, False),
+                                           (5376, 4096, 8, "mx", False, True), (5376, 4096, 10, "mx", False, False), (2304, 4096, 12, "mx", True, True)):
         assert routes.rounds_on_128_tiles(m, n, steps, kind, fp32=fp32) is small, (m, n, steps, kind, fp32)
-        if kind in ("fp8", "mxfp8"):
-            args = g.raw_gemm_args(1 << 12, 1 << 12, 1 << 12, 1 << 12, 1 << 12, m, n, steps * 128, g.ROWCOL if kind == "fp8" else g.MX_TILED, g.FP32 if fp32 else g.BF16)
+        if kind in ("fp8", "mxfp8", "block", "mx"):
+            args = g.raw_gemm_args(1 << 12, 1 << 12, 1 << 12, 1 << 12, 1 << 12, m, n, steps * 128, {"fp8": g.ROWCOL, "mxfp8": g.MX_TILED, "block": g.BLOCK, "mx": g.MX}[kind], g.FP32 if fp32 else g.BF16)
             assert (g.kernel_name(args) == "gemm_a8w8_tile128") is small
             args.stride_c = 1 << 24          # past the 256-tile kernels' offsets: refused, as before
             if steps % 2 == 0:
