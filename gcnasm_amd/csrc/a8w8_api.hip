@@ -593,13 +593,23 @@ int fill_mx_tiled(int rows, int k, uint8_t* scale, hipStream_t s)
     return launch(mx_tiled_fill_kernel, dim3((unsigned)((dwords + 255) / 256)), dim3(256), 0, s, (uint32_t*)scale, dwords);
 }
 
-// The vectorised MX quantisers: by lines of the tiled scales or as many chunks per wave as the array fills the chip with (quant_mx_lines_kernel,
-// quant_mx_vec_kernel), over the padded array where mx_padding_in_launch says so.
+// The vectorised MX quantisers: row-major scales over the flattened array (quant_mx_flat_kernel); tiled ones by lines of the scales or as many chunks per
+// wave as the array fills the chip with (quant_mx_lines_kernel, quant_mx_vec_kernel), over the padded array where mx_padding_in_launch says so.
 template <bool FP4, bool TILED>
 int launch_quant_mx(const float* src, int rows, int k, int ld, uint8_t* q, uint8_t* scale, hipStream_t s)
 {
-    int rows_p = rows, k_p = k;
-    if constexpr (TILED) {
+    if constexpr (!TILED) {
+        const unsigned total = (unsigned)rows * (unsigned)k;
+        const auto flat = [&](auto kernel, unsigned chunks) {
+            return launch(kernel, dim3((total + 1024 * chunks - 1) / (1024 * chunks)), dim3(256), 0, s, src, total, (unsigned)k, (unsigned)ld, q, scale);
+        };
+        switch (quant_mx_chunks(FP4, total, ld != k)) {
+            case 1: return flat(quant_mx_flat_kernel<FP4, 1>, 1);
+            case 2: return flat(quant_mx_flat_kernel<FP4, 2>, 2);
+            default: return flat(quant_mx_flat_kernel<FP4, 4>, 4);
+        }
+    } else {
+        int rows_p = rows, k_p = k;
         if (mx_padding_in_launch(rows, k)) {
             rows_p = (rows + 63) / 64 * 64;
             k_p = (k + 511) / 512 * 512;
@@ -612,16 +622,15 @@ int launch_quant_mx(const float* src, int rows, int k, int ld, uint8_t* q, uint8
         } else if (const int st = fill_mx_tiled(rows, k, scale, s); st != A8W8_OK) {
             return st;
         }
-    }
-    const long long total = (long long)rows_p * k_p;
-    const auto grid = [&](int per_thread) { return dim3((unsigned)((total / per_thread + 255) / 256)); };
-    if (total >= QUANT_MX_FULL) return launch(quant_mx_vec_kernel<FP4, TILED, 4>, grid(16), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
-    if constexpr (FP4) {
-        return launch(quant_mxfp4_few_kernel<TILED>, grid(8), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
-    } else {
-        if (total > QUANT_MX_FEW)
-            return launch(quant_mx_vec_kernel<false, TILED, 2>, grid(8), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
-        return launch(quant_mx_vec_kernel<false, TILED, 1>, grid(4), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
+        const long long total = (long long)rows_p * k_p;
+        const auto grid = [&](int per_thread) { return dim3((unsigned)((total / per_thread + 255) / 256)); };
+        if (total >= QUANT_MX_FULL) return launch(quant_mx_vec_kernel<FP4, 4>, grid(16), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
+        if constexpr (FP4) {
+            return launch(quant_mxfp4_few_kernel, grid(8), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
+        } else {
+            if (total > QUANT_MX_FEW) return launch(quant_mx_vec_kernel<false, 2>, grid(8), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
+            return launch(quant_mx_vec_kernel<false, 1>, grid(4), dim3(256), 0, s, src, rows, k, rows_p, k_p, ld, q, scale);
+        }
     }
 }
 

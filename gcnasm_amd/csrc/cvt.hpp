@@ -372,25 +372,24 @@ A8W8_DEV float4 load_once4(const float* p)
     return make_float4(t.x, t.y, t.z, t.w);
 }
 
-// MX formats with one E8M0 exponent per 32 elements (bound: HBM).  A wave takes 256 CHUNKS consecutive elements of the
+// MX formats with one E8M0 exponent per 32 elements, tiled scales that do not leave by lines (bound: HBM).  A wave takes 256 CHUNKS consecutive elements of the
 // flattened [rows, k] array: lane l owns elements 4l..4l+3 of each chunk of 256, eight lanes share a block.  Every load and
 // store instruction of a wave covers one contiguous run of memory; all loads are issued before any chunk is processed.
 // Four chunks are what large arrays want (8192 x 8192 E4M3, tiled scales: 56.3 us, two 58.3, one 64.9), fewer where there are
 // not enough of them to fill the chip and a wave's own latency is the time (2560 x 2560: 8.2 / 7.4 / 8.5; 64 x 7168: 3.8 / 2.7 /
-// 2.7; 16 x 7168: 3.7 / 2.6 / 2.3).  Tiled scales of arrays past a million elements: quant_mx_lines_kernel below.
-// TILED: the grid covers the padded [rows_p, k_p] array of the tiled layout (rows_p % 64 == 0, k_p % 512 == 0), so that the
-// positions no (row, block) owns get their 127 here instead of from a launch of their own before this one (2.3 us).  Otherwise,
-// and where that launch precedes this one (much padding: mx_padding_in_launch of routes.hpp), rows_p = rows and k_p = k.
+// 2.7; 16 x 7168: 3.7 / 2.6 / 2.3).  Tiled scales of arrays past a million elements: quant_mx_lines_kernel below; row-major ones: quant_mx_flat_kernel.
+// The grid covers the padded [rows_p, k_p] array of the tiled layout (rows_p % 64 == 0, k_p % 512 == 0), so that the
+// positions no (row, block) owns get their 127 here instead of from a launch of their own before this one (2.3 us).  Where that
+// launch precedes this one (much padding: mx_padding_in_launch of routes.hpp), rows_p = rows and k_p = k.
 // FP4: packed E2M1, two bytes per lane and chunk; the hardware convert instead of seven comparisons per element (8192 x 8192
 // 62.6 -> 50.3 us, 4096 x 4096 16.8 -> 13.6).
-template <bool FP4, bool TILED, int CHUNKS>
+template <bool FP4, int CHUNKS>
 __global__ void __launch_bounds__(256) quant_mx_vec_kernel(const float* __restrict__ src, int rows, int k, int rows_p, int k_p, int ld,
                                                            uint8_t* __restrict__ q, uint8_t* __restrict__ scale)
 {
     const unsigned total = (unsigned)rows_p * (unsigned)k_p;        // < 2^31 (checked by the host)
     const unsigned wave = (blockIdx.x * 256u + threadIdx.x) >> 6;
     const unsigned lane = threadIdx.x & 63;
-    const int blocks = k >> 5;
     unsigned row[CHUNKS], col[CHUNKS];
     bool live[CHUNKS], owned[CHUNKS];
     float4 v[CHUNKS];
@@ -400,7 +399,7 @@ __global__ void __launch_bounds__(256) quant_mx_vec_kernel(const float* __restri
         live[c] = e0 < total;
         row[c] = live[c] ? e0 / (unsigned)k_p : 0u;
         col[c] = live[c] ? e0 % (unsigned)k_p : 0u;
-        owned[c] = live[c] && (!TILED || (row[c] < (unsigned)rows && col[c] < (unsigned)k));
+        owned[c] = live[c] && row[c] < (unsigned)rows && col[c] < (unsigned)k;
         v[c] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (owned[c]) v[c] = load_once4(src + (size_t)row[c] * ld + col[c]);
     }
@@ -411,10 +410,7 @@ __global__ void __launch_bounds__(256) quant_mx_vec_kernel(const float* __restri
         for (int off = 4; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
         const int e = FP4 ? mx_exponent_e2m1(amax) : mx_exponent_e4m3(amax);
         if (!live[c]) continue;
-        if ((lane & 7) == 0) {
-            const int g = (int)(col[c] >> 5);
-            scale[TILED ? mx_tiled_index(rows, (int)row[c], g) : (size_t)row[c] * blocks + g] = (uint8_t)((owned[c] ? e : 0) + 127);
-        }
+        if ((lane & 7) == 0) scale[mx_tiled_index(rows, (int)row[c], (int)(col[c] >> 5))] = (uint8_t)((owned[c] ? e : 0) + 127);
         if (!owned[c]) continue;
         if constexpr (FP4) {
             const float s = __uint_as_float((unsigned)(e + 127) << 23);      // (2^-127: the convert takes the exponent field)
@@ -426,10 +422,9 @@ __global__ void __launch_bounds__(256) quant_mx_vec_kernel(const float* __restri
     }
 }
 
-// MXFP4 below the size that fills the chip: lane l owns eight consecutive elements (two 16-byte loads, one 4-byte store), four
+// MXFP4 with tiled scales below the size that fills the chip: lane l owns eight consecutive elements (two 16-byte loads, one 4-byte store), four
 // lanes share a block, a wave takes 512 consecutive elements (256 x 8192: 2.7 us against 3.2-3.8 with chunks, 64 x 7168: 2.3
 // against 2.6; 4096 x 2048: 7.8 against 7.5).
-template <bool TILED>
 __global__ void __launch_bounds__(256) quant_mxfp4_few_kernel(const float* __restrict__ src, int rows, int k, int rows_p, int k_p, int ld,
                                                               uint8_t* __restrict__ q, uint8_t* __restrict__ scale)
 {
@@ -437,7 +432,7 @@ __global__ void __launch_bounds__(256) quant_mxfp4_few_kernel(const float* __res
     const unsigned e0 = (blockIdx.x * 256u + threadIdx.x) * 8u;
     const bool live = e0 < total;
     const unsigned row = live ? e0 / (unsigned)k_p : 0u, col = live ? e0 % (unsigned)k_p : 0u;
-    const bool owned = live && (!TILED || (row < (unsigned)rows && col < (unsigned)k));
+    const bool owned = live && row < (unsigned)rows && col < (unsigned)k;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
     if (owned) {
         const float* p = src + (size_t)row * ld + col;
@@ -450,14 +445,47 @@ __global__ void __launch_bounds__(256) quant_mxfp4_few_kernel(const float* __res
     for (int off = 2; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
     const int e = mx_exponent_e2m1(amax);
     if (!live) return;
-    if ((threadIdx.x & 3) == 0) {
-        const int g = (int)(col >> 5);
-        scale[TILED ? mx_tiled_index(rows, (int)row, g) : (size_t)row * (k >> 5) + g] = (uint8_t)((owned ? e : 0) + 127);
-    }
+    if ((threadIdx.x & 3) == 0) scale[mx_tiled_index(rows, (int)row, (int)(col >> 5))] = (uint8_t)((owned ? e : 0) + 127);
     if (!owned) return;
     const float s = __uint_as_float((unsigned)(e + 127) << 23);
     *(uint32_t*)(q + (((size_t)row * k + col) >> 1)) =
         e2m1_pair<3>(e2m1_pair<2>(e2m1_pair<1>(e2m1_pair<0>(0u, a.x, a.y, s), a.z, a.w, s), b.x, b.y, s), b.z, b.w, s);
+}
+
+// The same for row-major scales (bound: HBM).  Codes and scales then lie as the flattened array does, code and block numbers are the element's own, and
+// no row or column is computed unless the rows of the input are apart (ld != k): the divisions of quant_mx_vec_kernel stood before every load.  Two
+// chunks per wave for whole arrays, four for rows apart, one where there are too few to fill the chip (quant_mx_chunks of routes.hpp).  us, rows and
+// columns / flattened, E4M3, MXFP4: 8192 x 8192 54.5 -> 52.3, 50.8 -> 47.9 (6.0 TB/s), 4096 x 4096 16.5 -> 15.5, 14.6 -> 13.7, 2560 x 2560 7.6 -> 7.3,
+// 7.5 -> 6.9, 300 x 5632 3.9 -> 3.2, 3.6 -> 3.5.  Scale bytes gathered into lines in LDS first: 0.1 to 0.4 us longer.
+template <bool FP4, int CHUNKS>
+__global__ void __launch_bounds__(256) quant_mx_flat_kernel(const float* __restrict__ src, unsigned total, unsigned k, unsigned ld, uint8_t* __restrict__ q,
+                                                            uint8_t* __restrict__ scale)
+{
+    const unsigned lane = threadIdx.x & 63;
+    const unsigned first = ((blockIdx.x * 256u + threadIdx.x) >> 6) * (256u * CHUNKS) + lane * 4u;      // (total < 2^31, checked by the host)
+    float4 v[CHUNKS];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const unsigned e0 = first + c * 256u;
+        v[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (e0 < total) v[c] = load_once4(src + (ld == k ? (size_t)e0 : (size_t)(e0 / k) * ld + e0 % k));
+    }
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const unsigned e0 = first + c * 256u;
+        float amax = fmaxf(fmaxf(fabsf(v[c].x), fabsf(v[c].y)), fmaxf(fabsf(v[c].z), fabsf(v[c].w)));
+#pragma unroll
+        for (int off = 4; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+        const int e = FP4 ? mx_exponent_e2m1(amax) : mx_exponent_e4m3(amax);
+        if (e0 >= total) continue;
+        if ((lane & 7) == 0) scale[e0 >> 5] = (uint8_t)(e + 127);
+        if constexpr (FP4) {
+            const float s = __uint_as_float((unsigned)(e + 127) << 23);
+            *(uint16_t*)(q + (e0 >> 1)) = (uint16_t)e2m1_pair<1>(e2m1_pair<0>(0u, v[c].x, v[c].y, s), v[c].z, v[c].w, s);
+        } else {
+            *(uint32_t*)(q + e0) = pack4_e4m3(ldexpf(v[c].x, -e), ldexpf(v[c].y, -e), ldexpf(v[c].z, -e), ldexpf(v[c].w, -e));
+        }
+    }
 }
 
 // The same for tiled scales, by lines of the scale array (bound: HBM).  A workgroup takes the 16 rows and 256 columns whose scales are one
@@ -514,8 +542,7 @@ __global__ void __launch_bounds__(64 * WAVES) quant_mx_lines_kernel(const float*
     }
 }
 
-// elements from which the chip is full; elements up to which a chunk per wave is the fastest (64 x 7168 row-major 2.93 us with two, 2.68 with one, 128 x 8192
-// 3.05 / 2.97, 512 x 4096 3.87 / 3.97)
+// tiled scales: elements from which the chip is full; elements up to which a chunk per wave is the fastest (64 x 7168 3.3 us with two, 3.1 with one)
 constexpr long long QUANT_MX_FULL = 1ll << 23, QUANT_MX_FEW = 1ll << 20;
 
 // per-row scale, one workgroup per row.  HOLD: the row (at most 16 THREADS elements) stays in registers between the amax pass

@@ -30,6 +30,15 @@ inline MxLines quant_mx_by_lines(bool fp4, long long rows, long long k)
     return elements >= 5000000 && elements < 15000000 ? MX_LINES_FOUR_WAVES : MX_LINES_EIGHT_WAVES;
 }
 
+// Row-major MX scales: chunks of 256 elements per wave (quant_mx_flat_kernel).  us, one / two / four: E4M3 1024 x 2048 3.4 / 3.9 / 4.2, 2560 x 2560 8.0 / 7.3 / 7.7,
+// 8192 x 8192 59.0 / 52.3 / 53.6; MXFP4 128 x 8192 3.2 / 3.3 / 3.7, 1024 x 2048 3.5 / 3.2 / 4.2, 8192 x 8192 56.9 / 47.9 / 49.6.  Rows apart, from 8M elements:
+// 5831 x 2304 14.8 / 13.6 / 12.9, MXFP4 13.4 / 12.1 / 11.2 (below, 2560 x 2560 8.3 / 7.5 / 7.7).
+inline int quant_mx_chunks(bool fp4, long long elements, bool rows_apart)
+{
+    if (elements <= 1ll << (fp4 ? 20 : 21)) return 1;
+    return rows_apart && elements >= 1ll << 23 ? 4 : 2;
+}
+
 // The per-row quantiser: a wave per row for more than a thousand rows of at most 1024 elements, else a workgroup (quant_rowwise_wave_kernel).
 inline bool quant_rows_by_wave(long long rows, long long k)
 {

@@ -4,6 +4,7 @@
 extern "C" {
 int route_mx_padding_in_launch(long long rows, long long k) { return a8w8::mx_padding_in_launch(rows, k); }
 int route_quant_mx_by_lines(int fp4, long long rows, long long k) { return a8w8::quant_mx_by_lines(fp4 != 0, rows, k); }
+int route_quant_mx_chunks(int fp4, long long elements, int rows_apart) { return a8w8::quant_mx_chunks(fp4 != 0, elements, rows_apart != 0); }
 int route_quant_rows_by_wave(long long rows, long long k) { return a8w8::quant_rows_by_wave(rows, k); }
 int route_partial_steps_on_tiles(long long m, long long n, long long k_bytes, long long batch)
 {

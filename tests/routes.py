@@ -30,6 +30,10 @@ def quant_mx_by_lines(rows, k, fp4=False):
     return (None, 4, 8)[lib().route_quant_mx_by_lines(int(fp4), _ll(rows), _ll(k))]
 
 
+def quant_mx_chunks(elements, fp4=False, rows_apart=False):
+    return int(lib().route_quant_mx_chunks(int(fp4), _ll(elements), int(rows_apart)))
+
+
 def quant_rows_by_wave(rows, k):
     return bool(lib().route_quant_rows_by_wave(_ll(rows), _ll(k)))
 

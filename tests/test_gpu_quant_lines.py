@@ -1,4 +1,4 @@
-"""Tiled MX scales written by lines of the scale array, and per-row scales with a wave per row: the same bytes as the oracle's, at whole and
+"""Tiled MX scales written by lines of the scale array, row-major ones over the flattened array, and per-row scales with a wave per row: the same bytes as the oracle's, at whole and
 partial 64-row blocks and 256- and 512-column groups, with rows further apart than their elements."""
 import numpy as np
 import pytest
@@ -50,6 +50,18 @@ def test_tiled_scales_by_lines_of_infinities_and_nan(orc):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,k", [(1, 32), (3, 224), (33, 1056), (2049, 1024), (257, 4128), (1056, 8192)])
+@pytest.mark.parametrize("pad", [0, 4, 2048])
+def test_row_major_scales_of_the_flattened_array(orc, rows, k, pad):
+    """One, two and four chunks per wave, whole and partial last workgroups."""
+    x, view = _rows_apart(rows, k, pad, True)
+    # (finite values: blocks that hold an infinity, or zeros and NaN alone, keep exponent 0 on the device and not in the oracle; the test above compares
+    # those with the tiled quantiser's)
+    for (q, s), (q0, s0) in ((g.quantize(view, g.MX), orc.quantize(x, orc.MX)), (g.quantize_mxfp4(view), orc.quantize_mxfp4(x))):
+        assert (q.cpu().numpy() == q0).all() and (s.cpu().numpy().reshape(s0.shape) == s0).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,k", [(1025, 1024), (1027, 4), (1030, 256), (2306, 768), (1026, 1020), (5000, 260)])
 @pytest.mark.parametrize("pad", [0, 4])
 def test_a_wave_per_row(orc, rows, k, pad):
@@ -63,6 +75,8 @@ def test_a_wave_per_row(orc, rows, k, pad):
 
 
 def test_rules():
+    assert [routes.quant_mx_chunks(e, f, a) for f in (False, True) for a in (False, True) for e in (1 << 20, (1 << 20) + 32, 1 << 21, (1 << 21) + 32, 1 << 23)] == [
+        1, 1, 1, 2, 2, 1, 1, 1, 2, 4, 1, 2, 2, 2, 2, 1, 2, 2, 2, 4]
     for rows, k, fp8, fp4 in ((128, 8192, None, None), (129, 8192, 8, 8), (1, 65536, 8, None), (64, 7168, None, None), (256, 8192, 8, 8), (2560, 2560, 4, 4),
                               (4096, 4096, 8, 8), (8192, 8192, 8, 8)):
         assert routes.quant_mx_by_lines(rows, k) == fp8 and routes.quant_mx_by_lines(rows, k, fp4=True) == fp4
