@@ -235,17 +235,45 @@ def _out(c, shape, c_dtype, device):
         raise TypeError(f"output tensor must be bfloat16 or float32, got {c.dtype}")
     if tuple(c.shape) != tuple(shape):
         raise ValueError(f"output tensor has shape {tuple(c.shape)}, expected {tuple(shape)}")
+    if shape[-1] > 1 and c.stride(-1) != 1:
+        raise ValueError("c: the last dimension must be contiguous")
+    if not c.is_cuda:
+        raise ValueError("c must live on the GPU")
     return c, (BF16 if c.dtype == torch.bfloat16 else FP32)
 
 
-def _check_operand(t, name, dims, shape, strides):
-    """Operands are strided views of device memory whose rows are contiguous; anything else would be misread."""
+def _check_rows(t, name, element_bytes):
+    """What is read row by row: elements of the size that the kernel takes, side by side in GPU memory.  Anything else would be misread, and smaller
+    elements read past their end."""
+    if t.element_size() != element_bytes:
+        raise TypeError(f"{name} must have elements of {element_bytes} bytes, got {t.dtype}")
+    if t.shape[-1] > 1 and t.stride(-1) != 1:
+        raise ValueError(f"{name}: the last dimension must be contiguous (stride {t.stride(-1)})")
     if not t.is_cuda:
         raise ValueError(f"{name} must live on the GPU")
-    if len(shape) not in dims:
-        raise ValueError(f"{name} must have {' or '.join(str(d) for d in dims)} dimensions, got {len(shape)}")
-    if shape and shape[-1] > 1 and strides[-1] != 1:
-        raise ValueError(f"{name}: the last dimension must be contiguous (stride {strides[-1]})")
+
+
+def _check_fp32_rows(x, name="x"):
+    if x.dtype != torch.float32:
+        raise TypeError(f"{name} must be float32, got {x.dtype}")
+    _check_rows(x, name, 4)
+
+
+def _check_operands(a, b, element_bytes, dims, n=None):
+    """a [.., M, row], and b [.., N, row] or, with `n` given, the flat pre-shuffled weight of n rows (any element type)."""
+    for t, name, want in ((a, "a", dims), (b, "b", dims if n is None else (1, 2))):
+        if t.dim() not in want:
+            raise ValueError(f"{name} must have {' or '.join(str(d) for d in want)} dimensions, got {t.dim()}")
+    _check_rows(a, "a", element_bytes)
+    if n is None:
+        _check_rows(b, "b", element_bytes)
+        if b.shape[-1] < a.shape[-1]:
+            raise ValueError(f"rows of b hold {b.shape[-1]} elements, those of a {a.shape[-1]}")
+        return
+    if not b.is_contiguous() or not b.is_cuda:
+        raise ValueError("shuffled b must be a contiguous GPU tensor")
+    if b.numel() * b.element_size() < n * a.shape[-1] * element_bytes:
+        raise ValueError(f"shuffled b holds {b.numel() * b.element_size()} bytes, {n} rows are {n * a.shape[-1] * element_bytes}")
 
 
 def _check_scales(t, name, scale_mode):
@@ -287,11 +315,26 @@ def _check_scale_sizes(sfa, sfb, scale_mode, m, n, k, batch, b_shared):
         raise ValueError(f"b is shared by all {batch} batch entries but sfb holds a set of scales per entry; pass one set")
 
 
+def _check_fp4_scales(sfa, sfb, scale_mode, m, n, k):
+    """E8M0 bytes of any one-byte type, contiguous, on the GPU, as many as the kernels read (the library refuses other modes)."""
+    if scale_mode not in (MX, MX_TILED):
+        return
+    for t, name, rows in ((sfa, "sfa", m), (sfb, "sfb", n)):
+        if t.element_size() != 1:
+            raise TypeError(f"{name} must have elements of one byte, got {t.dtype}")
+        if not t.is_contiguous() or not t.is_cuda:
+            raise ValueError(f"{name} must be a contiguous GPU tensor")
+        need = scale_elements(scale_mode, rows, k, name == "sfb")
+        if t.numel() < need:
+            raise ValueError(f"{name} holds {t.numel()} elements, this problem reads {need}")
+
+
 def _args_from_tensors(a, b, sfa, sfb, scale_mode, c, c_dtype, b_preshuffled, n=None, scaled=True):
     _need_torch()
     a_shape, a_strides, b_shape, b_strides = a.shape, a.stride(), b.shape, b.stride()
-    _check_operand(a, "a", (2, 3), a_shape, a_strides)
-    _check_operand(b, "b", (1, 2) if b_preshuffled else (2, 3), b_shape, b_strides)
+    if b_preshuffled and n is None:
+        n = b_shape[-2]
+    _check_operands(a, b, 1 if scaled else 2, (2, 3), n=n if b_preshuffled else None)
     if scaled:
         _check_scales(sfa, "sfa", scale_mode)
         _check_scales(sfb, "sfb", scale_mode)
@@ -302,8 +345,6 @@ def _args_from_tensors(a, b, sfa, sfb, scale_mode, c, c_dtype, b_preshuffled, n=
         n = b_shape[-2]
     c, c_dtype = _out(c, (batch, m, n) if batched else (m, n), c_dtype, a.device)
     c_strides = c.stride()
-    if n > 1 and c_strides[-1] != 1:
-        raise ValueError("c: the last dimension must be contiguous")
     g = raw_gemm_args(a.data_ptr(), b.data_ptr(), c.data_ptr(), sfa.data_ptr(), sfb.data_ptr(), m, n, k, scale_mode,
                       c_dtype, batch, stride_a=a_strides[-2], stride_b=(k if b_preshuffled else b_strides[-2]),
                       stride_c=c_strides[-2], b_preshuffled=b_preshuffled)
@@ -378,6 +419,7 @@ def quantize_mxfp4(x, tiled=False):
         return _done(r, "a4w4_quantize_mx")
     _need_torch()
     rows, k = x.shape
+    _check_fp32_rows(x)
     q = torch.empty((rows, k // 2), dtype=torch.uint8, device=x.device)
     s = torch.empty(mx_tiled_bytes(rows, k) if tiled else (rows, k // 32), dtype=torch.uint8, device=x.device)
     _check(lib().a4w4_quantize_mx(x.data_ptr(), rows, k, x.stride(0), q.data_ptr(), s.data_ptr(), int(tiled), _stream()),
@@ -392,10 +434,12 @@ def gemm_a4w4(a, b, sfa, sfb, scale_mode=MX_TILED, c=None, c_dtype=BF16, n=None)
     if r is not None:
         return _done(r, "a4w4_gemm")
     _need_torch()
+    _check_operands(a, b, 1, (2,), n=n)
     m, k = a.shape[-2], a.shape[-1] * 2
     shuffled = n is not None
     if not shuffled:
         n = b.shape[-2]
+    _check_fp4_scales(sfa, sfb, scale_mode, m, n, k)
     c, c_dtype = _out(c, (m, n), c_dtype, a.device)
     g = raw_gemm_args(a.data_ptr(), b.data_ptr(), c.data_ptr(), sfa.data_ptr(), sfb.data_ptr(), m, n, k, scale_mode, c_dtype,
                       stride_a=a.stride(-2) * 2, stride_b=(k if shuffled else b.stride(-2) * 2), stride_c=c.stride(-2),
@@ -411,7 +455,10 @@ def flatmm_a4w4(a, b_shuffled, sfa_tiled, sfb_tiled, n, c=None, c_dtype=BF16):
     if r is not None:
         return _done(r, "a4w4_flatmm")
     _need_torch()
+    _check_operands(a, b_shuffled, 1, (2,), n=n)
     m, k = a.shape[-2], a.shape[-1] * 2
+    if m <= 128:      # (more rows are the library's to refuse)
+        _check_fp4_scales(sfa_tiled, sfb_tiled, MX_TILED, m, n, k)
     c, c_dtype = _out(c, (m, n), c_dtype, a.device)
     g = raw_gemm_args(a.data_ptr(), b_shuffled.data_ptr(), c.data_ptr(), sfa_tiled.data_ptr(), sfb_tiled.data_ptr(), m, n, k,
                       MX_TILED, c_dtype, stride_a=a.stride(-2) * 2, stride_b=k, stride_c=c.stride(-2), b_preshuffled=1)
@@ -461,6 +508,9 @@ def unshuffle_b(bs_np, n, k):
 def preshuffle_b_device(b):
     _need_torch()
     n, k = b.shape
+    _check_rows(b, "b", 1)
+    if not b.is_contiguous():
+        raise ValueError("b must be contiguous")
     out = torch.empty(n * k, dtype=torch.uint8, device=b.device)
     _check(lib().a8w8_preshuffle_b_device(b.data_ptr(), out.data_ptr(), n, k, _stream()), "a8w8_preshuffle_b_device")
     return out
@@ -472,6 +522,10 @@ def cvt_f32_to_e4m3(x, dialect=OCP, clamp240=False):
         return _done(r, "a8w8_cvt_f32_to_e4m3")
     _need_torch()
     x = x.contiguous()
+    if x.dtype != torch.float32:
+        raise TypeError(f"x must be float32, got {x.dtype}")
+    if not x.is_cuda:
+        raise ValueError("x must live on the GPU")
     out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
     _check(lib().a8w8_cvt_f32_to_e4m3(x.data_ptr(), out.data_ptr(), x.numel(), dialect, int(clamp240), _stream()),
            "a8w8_cvt_f32_to_e4m3")
@@ -484,6 +538,10 @@ def cvt_e4m3_to_f32(codes, dialect=OCP):
         return _done(r, "a8w8_cvt_e4m3_to_f32")
     _need_torch()
     codes = codes.contiguous()
+    if codes.element_size() != 1:
+        raise TypeError(f"codes must have elements of one byte, got {codes.dtype}")
+    if not codes.is_cuda:
+        raise ValueError("codes must live on the GPU")
     out = torch.empty(codes.shape, dtype=torch.float32, device=codes.device)
     _check(lib().a8w8_cvt_e4m3_to_f32(codes.data_ptr(), out.data_ptr(), codes.numel(), dialect, _stream()),
            "a8w8_cvt_e4m3_to_f32")
@@ -497,6 +555,7 @@ def quantize(x, scale_mode, group_rows=1):
         return _done(r, "a8w8_quantize")
     _need_torch()
     rows, k = x.shape
+    _check_fp32_rows(x)
     q = torch.empty((rows, k), dtype=torch.uint8, device=x.device)
     if scale_mode == TENSOR:
         s = torch.empty(1, dtype=torch.float32, device=x.device)
@@ -521,6 +580,9 @@ def mx_tile_scales(sf, out=None):
     """Row-major E8M0 scales [rows, K/32] (u8, on the GPU) -> the MX_TILED layout (flat u8 tensor)."""
     _need_torch()
     rows, kb = sf.shape
+    _check_rows(sf, "sf", 1)
+    if out is not None and (not out.is_contiguous() or not out.is_cuda or out.numel() * out.element_size() < mx_tiled_bytes(rows, kb * 32)):
+        raise ValueError(f"out must be a contiguous GPU tensor of {mx_tiled_bytes(rows, kb * 32)} bytes")
     if out is None:
         out = torch.empty(mx_tiled_bytes(rows, kb * 32), dtype=torch.uint8, device=sf.device)
     _check(lib().a8w8_mx_tile_scales(sf.data_ptr(), rows, kb * 32, sf.stride(0), out.data_ptr(), _stream()),
@@ -533,6 +595,10 @@ def mx_tile_scales_ab(sfa, sfb):
     _need_torch()
     m, kb = sfa.shape
     n = sfb.shape[0]
+    _check_rows(sfa, "sfa", 1)
+    _check_rows(sfb, "sfb", 1)
+    if sfb.dim() != 2 or sfb.shape[1] < kb:
+        raise ValueError(f"sfb must have rows of {kb} scales, got {tuple(sfb.shape)}")
     ta = torch.empty(mx_tiled_bytes(m, kb * 32), dtype=torch.uint8, device=sfa.device)
     tb = torch.empty(mx_tiled_bytes(n, kb * 32), dtype=torch.uint8, device=sfb.device)
     _check(lib().a8w8_mx_tile_scales_ab(sfa.data_ptr(), m, sfa.stride(0), ta.data_ptr(), sfb.data_ptr(), n,

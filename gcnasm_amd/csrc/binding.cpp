@@ -49,6 +49,16 @@ const at::Tensor* plain(PyObject* o)
     return &t;
 }
 
+// elements side by side along the last dimension
+bool rows_contiguous(const at::Tensor& t) { return t.size(-1) <= 1 || t.stride(-1) == 1; }
+
+// fp32 [rows, k] that a quantiser reads row by row (narrower elements would be read past their end)
+const at::Tensor* fp32_rows(PyObject* o)
+{
+    const at::Tensor* x = plain(o);
+    return x && x->scalar_type() == at::kFloat && x->dim() == 2 && x->size(0) > 0 && x->size(1) > 0 && rows_contiguous(*x) ? x : nullptr;
+}
+
 bool as_int(PyObject* o, long& v)
 {
     if (!PyLong_Check(o)) return false;      // (bools are ints)
@@ -81,8 +91,8 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
     HANDLE_TH_ERRORS
     long mode, group;
-    const at::Tensor* x = count == 3 && !modes_active() ? plain(args[0]) : nullptr;
-    if (!x || x->dim() != 2 || !as_int(args[1], mode) || !as_int(args[2], group) || x->size(0) <= 0 || x->size(1) <= 0) Py_RETURN_NONE;
+    const at::Tensor* x = count == 3 && !modes_active() ? fp32_rows(args[0]) : nullptr;
+    if (!x || !as_int(args[1], mode) || !as_int(args[2], group)) Py_RETURN_NONE;
     const int64_t rows = x->size(0), k = x->size(1);
     if (mode < A8W8_SCALE_TENSOR || mode > A8W8_SCALE_MX_E8M0_TILED) Py_RETURN_NONE;
     const at::Tensor q = allocate({rows, k}, at::kByte, *x);
@@ -112,8 +122,8 @@ PyObject* quantize_mxfp4(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
     HANDLE_TH_ERRORS
     long tiled;
-    const at::Tensor* x = count == 2 && !modes_active() ? plain(args[0]) : nullptr;
-    if (!x || x->dim() != 2 || !as_int(args[1], tiled) || x->size(0) <= 0 || x->size(1) <= 0) Py_RETURN_NONE;
+    const at::Tensor* x = count == 2 && !modes_active() ? fp32_rows(args[0]) : nullptr;
+    if (!x || !as_int(args[1], tiled)) Py_RETURN_NONE;
     const int64_t rows = x->size(0), k = x->size(1), ld = x->stride(0);
     const at::Tensor q = allocate({rows, k / 2}, at::kByte, *x);
     const at::Tensor s = tiled ? allocate({mx_tiled(rows, k)}, at::kByte, *x) : allocate({rows, k / 32}, at::kByte, *x);
@@ -133,7 +143,7 @@ PyObject* encode(PyObject*, PyObject* const* args, Py_ssize_t count)
     HANDLE_TH_ERRORS
     long dialect, clamp;
     const at::Tensor* x = count == 3 && !modes_active() ? plain(args[0]) : nullptr;
-    if (!x || !x->is_contiguous() || !as_int(args[1], dialect) || !as_int(args[2], clamp)) Py_RETURN_NONE;
+    if (!x || x->scalar_type() != at::kFloat || !x->is_contiguous() || !as_int(args[1], dialect) || !as_int(args[2], clamp)) Py_RETURN_NONE;
     const at::Tensor out = allocate(x->sizes(), at::kByte, *x);
     const void* src = x->data_ptr();
     void *dst = out.data_ptr(), *st = stream();
@@ -151,7 +161,7 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t count)
     HANDLE_TH_ERRORS
     long dialect;
     const at::Tensor* x = count == 2 && !modes_active() ? plain(args[0]) : nullptr;
-    if (!x || !x->is_contiguous() || !as_int(args[1], dialect)) Py_RETURN_NONE;
+    if (!x || x->element_size() != 1 || !x->is_contiguous() || !as_int(args[1], dialect)) Py_RETURN_NONE;
     const at::Tensor out = allocate(x->sizes(), at::kFloat, *x);
     const void* src = x->data_ptr();
     void *dst = out.data_ptr(), *st = stream();
@@ -178,7 +188,8 @@ int64_t scale_elements(long mode, int64_t rows, int64_t k, bool weight_side)
     }
 }
 
-bool rows_contiguous(const at::Tensor& t) { return t.size(-1) <= 1 || t.stride(-1) == 1; }
+// a one-byte array of a contiguous tensor, as many elements as the kernels read
+bool fp4_scales_ok(const at::Tensor& t, int64_t need) { return t.is_contiguous() && t.element_size() == 1 && t.numel() >= need; }
 
 PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
@@ -193,7 +204,10 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t count)
     const bool batched = a->dim() == 3;
     if ((a->dim() != 2 && !batched) || (fp4 && batched) || !(shuffled ? b->dim() == 1 || b->dim() == 2 : b->dim() == 2 || (b->dim() == 3 && batched)))
         Py_RETURN_NONE;
-    if (!rows_contiguous(*a) || !rows_contiguous(*b)) Py_RETURN_NONE;
+    const int64_t element_bytes = scaled ? 1 : 2;
+    if (!rows_contiguous(*a) || (int64_t)a->element_size() != element_bytes) Py_RETURN_NONE;
+    if (!shuffled && (!rows_contiguous(*b) || (int64_t)b->element_size() != element_bytes || b->size(-1) < a->size(-1))) Py_RETURN_NONE;
+    if (shuffled && (!b->is_contiguous() || (int64_t)b->nbytes() < n_given * a->size(-1) * element_bytes)) Py_RETURN_NONE;
     const int64_t per_byte = fp4 ? 2 : 1, batch = batched ? a->size(0) : 1, m = a->size(-2), k = a->size(-1) * per_byte, n = shuffled ? n_given : b->size(-2);
     if (batch <= 0 || m <= 0 || n <= 0 || k <= 0) Py_RETURN_NONE;
 
@@ -215,6 +229,7 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t count)
             b_batch = sfb_batch = 0;      // one weight matrix, and one set of weight scales, for every batch entry
         }
     }
+    if (fp4 && (mode < A8W8_SCALE_MX_E8M0_1x32 || !fp4_scales_ok(*sfa, sfa_batch) || !fp4_scales_ok(*sfb, sfb_batch))) Py_RETURN_NONE;
     if (scaled && !fp4) {
         const at::ScalarType want = mode >= A8W8_SCALE_MX_E8M0_1x32 ? at::kByte : at::kFloat;
         if (!sfa->is_contiguous() || !sfb->is_contiguous() || sfa->scalar_type() != want || sfb->scalar_type() != want) Py_RETURN_NONE;
