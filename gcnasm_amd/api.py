@@ -253,10 +253,17 @@ def _check_rows(t, name, element_bytes):
         raise ValueError(f"{name} must live on the GPU")
 
 
-def _check_fp32_rows(x, name="x"):
+def _check_ints(where, *values):
+    """The C ABI counts rows, columns and strides with an int; a larger one would be read modulo 2^32."""
+    if any(v > 0x7FFFFFFF for v in values):
+        raise A8W8Error(-7, where)
+
+
+def _check_fp32_rows(x, where):
     if x.dtype != torch.float32:
-        raise TypeError(f"{name} must be float32, got {x.dtype}")
-    _check_rows(x, name, 4)
+        raise TypeError(f"x must be float32, got {x.dtype}")
+    _check_rows(x, "x", 4)
+    _check_ints(where, x.shape[0], x.shape[1], x.stride(0))
 
 
 def _check_operands(a, b, element_bytes, dims, n=None):
@@ -345,6 +352,9 @@ def _args_from_tensors(a, b, sfa, sfb, scale_mode, c, c_dtype, b_preshuffled, n=
         n = b_shape[-2]
     c, c_dtype = _out(c, (batch, m, n) if batched else (m, n), c_dtype, a.device)
     c_strides = c.stride()
+    _check_ints("gemm", m, n, k, batch, a_strides[-2], k if b_preshuffled else b_strides[-2], c_strides[-2])
+    if batch > 1:
+        _check_ints("gemm", a_strides[0], b_strides[0] if len(b_shape) == 3 else n * k if b_preshuffled else 0, c_strides[0])
     g = raw_gemm_args(a.data_ptr(), b.data_ptr(), c.data_ptr(), sfa.data_ptr(), sfb.data_ptr(), m, n, k, scale_mode,
                       c_dtype, batch, stride_a=a_strides[-2], stride_b=(k if b_preshuffled else b_strides[-2]),
                       stride_c=c_strides[-2], b_preshuffled=b_preshuffled)
@@ -419,7 +429,7 @@ def quantize_mxfp4(x, tiled=False):
         return _done(r, "a4w4_quantize_mx")
     _need_torch()
     rows, k = x.shape
-    _check_fp32_rows(x)
+    _check_fp32_rows(x, "a4w4_quantize_mx")
     q = torch.empty((rows, k // 2), dtype=torch.uint8, device=x.device)
     s = torch.empty(mx_tiled_bytes(rows, k) if tiled else (rows, k // 32), dtype=torch.uint8, device=x.device)
     _check(lib().a4w4_quantize_mx(x.data_ptr(), rows, k, x.stride(0), q.data_ptr(), s.data_ptr(), int(tiled), _stream()),
@@ -441,6 +451,7 @@ def gemm_a4w4(a, b, sfa, sfb, scale_mode=MX_TILED, c=None, c_dtype=BF16, n=None)
         n = b.shape[-2]
     _check_fp4_scales(sfa, sfb, scale_mode, m, n, k)
     c, c_dtype = _out(c, (m, n), c_dtype, a.device)
+    _check_ints("a4w4_gemm", m, n, k, 2 * a.stride(-2), k if shuffled else 2 * b.stride(-2), c.stride(-2))
     g = raw_gemm_args(a.data_ptr(), b.data_ptr(), c.data_ptr(), sfa.data_ptr(), sfb.data_ptr(), m, n, k, scale_mode, c_dtype,
                       stride_a=a.stride(-2) * 2, stride_b=(k if shuffled else b.stride(-2) * 2), stride_c=c.stride(-2),
                       b_preshuffled=int(shuffled))
@@ -460,6 +471,7 @@ def flatmm_a4w4(a, b_shuffled, sfa_tiled, sfb_tiled, n, c=None, c_dtype=BF16):
     if m <= 128:      # (more rows are the library's to refuse)
         _check_fp4_scales(sfa_tiled, sfb_tiled, MX_TILED, m, n, k)
     c, c_dtype = _out(c, (m, n), c_dtype, a.device)
+    _check_ints("a4w4_flatmm", m, n, k, 2 * a.stride(-2), c.stride(-2))
     g = raw_gemm_args(a.data_ptr(), b_shuffled.data_ptr(), c.data_ptr(), sfa_tiled.data_ptr(), sfb_tiled.data_ptr(), m, n, k,
                       MX_TILED, c_dtype, stride_a=a.stride(-2) * 2, stride_b=k, stride_c=c.stride(-2), b_preshuffled=1)
     _check(lib().a4w4_flatmm(ctypes.byref(g), _stream()), "a4w4_flatmm")
@@ -555,7 +567,7 @@ def quantize(x, scale_mode, group_rows=1):
         return _done(r, "a8w8_quantize")
     _need_torch()
     rows, k = x.shape
-    _check_fp32_rows(x)
+    _check_fp32_rows(x, "a8w8_quantize")
     q = torch.empty((rows, k), dtype=torch.uint8, device=x.device)
     if scale_mode == TENSOR:
         s = torch.empty(1, dtype=torch.float32, device=x.device)

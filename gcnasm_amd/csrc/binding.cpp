@@ -17,6 +17,8 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 
+#include <climits>
+
 #include "../../include/mi355_a8w8.h"
 
 namespace {
@@ -52,11 +54,19 @@ const at::Tensor* plain(PyObject* o)
 // elements side by side along the last dimension
 bool rows_contiguous(const at::Tensor& t) { return t.size(-1) <= 1 || t.stride(-1) == 1; }
 
+// sizes and strides that the C ABI's ints hold
+template <class... I>
+bool ints(I... v)
+{
+    return ((v <= INT_MAX) && ...);
+}
+
 // fp32 [rows, k] that a quantiser reads row by row (narrower elements would be read past their end)
 const at::Tensor* fp32_rows(PyObject* o)
 {
     const at::Tensor* x = plain(o);
-    return x && x->scalar_type() == at::kFloat && x->dim() == 2 && x->size(0) > 0 && x->size(1) > 0 && rows_contiguous(*x) ? x : nullptr;
+    return x && x->scalar_type() == at::kFloat && x->dim() == 2 && x->size(0) > 0 && x->size(1) > 0 && rows_contiguous(*x) &&
+                   ints(x->size(0), x->size(1), x->stride(0)) ? x : nullptr;
 }
 
 bool as_int(PyObject* o, long& v)
@@ -252,6 +262,7 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t count)
             Py_RETURN_NONE;
         c_dtype = c->scalar_type() == at::kBFloat16 ? A8W8_C_BF16 : A8W8_C_FP32;
     }
+    if (!ints(m, n, k, batch, a->stride(-2) * per_byte, stride_b, c->stride(-2)) || (batch > 1 && !ints(a_batch, b_batch, c->stride(0), sfa_batch, sfb_batch))) Py_RETURN_NONE;
     a8w8_gemm_args g;
     g.a = a->data_ptr(); g.b = b->data_ptr(); g.c = c->data_ptr();
     g.m = (int)m; g.n = (int)n; g.k = (int)k; g.batch = (int)batch;

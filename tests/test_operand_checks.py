@@ -104,3 +104,28 @@ def test_still_taken():
     assert torch.equal(g.gemm_a4w4(a, b, bits(sa, torch.int8), bits(sb, torch.int8)), g.gemm_a4w4(a, b, sa, sb))
     one = torch.randn(40, 1, device="cuda").T      # a single row whose column stride is 1 and row stride is not its length
     assert torch.equal(g.cvt_f32_to_e4m3(one), g.cvt_f32_to_e4m3(one.clone()))
+
+
+@pytest.mark.gpu
+def test_strides_past_an_int():
+    """2^32 elements between rows or batch entries would arrive at the library as 0, i.e. as the first row or entry again."""
+    x = torch.empty((1 << 32) + 512, device="cuda").as_strided((2, 512), (1 << 32, 1))      # 16 GiB, of which nothing is read
+    for quantize in (lambda: g.quantize(x, g.ROWCOL), lambda: g.quantize_mxfp4(x)):
+        with pytest.raises(g.A8W8Error, match="-7"):
+            quantize()
+    del x
+    a = torch.empty((1 << 32) + 16 * 512, dtype=torch.uint8, device="cuda")
+    b, s = torch.zeros((256, 512), dtype=torch.uint8, device="cuda"), torch.ones(512, device="cuda")
+    for batched in (a.as_strided((2, 16, 512), (1 << 32, 512, 1)), a.as_strided((2, 512), (1 << 32, 1))):
+        with pytest.raises(g.A8W8Error, match="-7"):
+            g.gemm(batched, b, s, s, g.ROWCOL)
+    assert g.gemm(a.as_strided((1, 16, 512), (1 << 32, 512, 1)), b, s, s, g.ROWCOL).shape == (1, 16, 256)      # (no second entry)
+    e = torch.zeros(1 << 14, dtype=torch.uint8, device="cuda")
+    with pytest.raises(g.A8W8Error, match="-7"):
+        g.gemm_a4w4(a.as_strided((2, 512), (1 << 31, 1)), b, e, e)
+
+
+def test_ints():
+    api._check_ints("here", 0, (1 << 31) - 1)
+    with pytest.raises(g.A8W8Error, match="-7"):
+        api._check_ints("here", 5, 1 << 31)
