@@ -8,6 +8,7 @@ device-memory handles (data_ptr) plus the current HIP stream.
 import ctypes
 import os
 import subprocess
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # MI355_A8W8_LIBRARY: another build of the same sources (a measurement build made with `make EXTRA=-D... OUT=...`),
@@ -92,9 +93,10 @@ def lib():
         L.a8w8_cvt_e4m3_to_f32.argtypes = [vp, vp, ctypes.c_size_t, ctypes.c_int, vp]
         L.a8w8_quantize.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp, ctypes.c_int,
                                     ctypes.c_int, vp]
-        L.a8w8_quantize_ws.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp, ctypes.c_int, ctypes.c_int, vp, ctypes.c_size_t, vp]
-        L.a8w8_quantize_workspace_bytes.restype = ctypes.c_size_t
-        L.a8w8_quantize_workspace_bytes.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int]
+        if hasattr(L, "a8w8_quantize_ws"):      # (not in an older build named by MI355_A8W8_LIBRARY)
+            L.a8w8_quantize_ws.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp, ctypes.c_int, ctypes.c_int, vp, ctypes.c_size_t, vp]
+            L.a8w8_quantize_workspace_bytes.restype = ctypes.c_size_t
+            L.a8w8_quantize_workspace_bytes.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int]
         L.a8w8_mx_tile_scales.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp]
         L.a8w8_mx_tile_scales_ab.argtypes = [vp, ctypes.c_int, ctypes.c_int, vp, vp, ctypes.c_int, ctypes.c_int, vp,
                                              ctypes.c_int, vp]
@@ -128,16 +130,31 @@ _OPS = ("a8w8_gemm", "a8w8_gemm_blockscale", "a8w8_flatmm", "a16w16_gemm", "a16w
 _GEMM, _BLOCKSCALE, _FLATMM, _GEMM16, _FLATMM16, _GEMM4, _FLATMM4 = range(7)
 
 
+def _torch_build():
+    """What the Makefile compiles into the module as torch_build."""
+    return f"{torch.__version__} {torch.version.git_version}"
+
+
 def _connect():
-    """Load csrc/binding.cpp's module on the first call that takes tensors and hand it the library's entry points."""
+    """Load csrc/binding.cpp's module on the first call that takes tensors and hand it the library's entry points.  Without a module for this torch, or with
+    a library older than the module, the functions' own statements serve every call: the same kernels, 4 to 8 us of host time more per call."""
     global _fast_gemm, _fast_quantize, _fast_quantize_mxfp4, _fast_encode, _fast_decode
     _need_torch()
     L = lib()
+    why = None
     try:
         from . import _binding
+        if _binding.torch_build != _torch_build():
+            why = f"it was built for torch {_binding.torch_build}, this is {_torch_build()}"
+        elif not hasattr(L, "a8w8_quantize_ws"):
+            why = f"{_SO} has no a8w8_quantize_ws"
     except ImportError as e:
-        raise FileNotFoundError(f"{os.path.join(_HERE, '_binding.so')} is missing or was built for another torch: build it with "
-                                f"gcnasm_amd.build_library() or `make -C gcnasm_amd/csrc` ({e})") from e
+        why = str(e)
+    if why is not None:
+        warnings.warn(f"{os.path.join(_HERE, '_binding.so')} is not used: {why}.  Calls take longer on the host; build it with gcnasm_amd.build_library() or "
+                      "`make -C gcnasm_amd/csrc`.", RuntimeWarning, stacklevel=4)
+        _fast_gemm = _fast_quantize = _fast_quantize_mxfp4 = _fast_encode = _fast_decode = lambda *args: None
+        return
     _binding.connect(*(ctypes.cast(getattr(L, f), ctypes.c_void_p).value
                        for f in _OPS + ("a8w8_quantize_ws", "a4w4_quantize_mx", "a8w8_cvt_f32_to_e4m3", "a8w8_cvt_e4m3_to_f32",
                                         "a8w8_quantize_workspace_bytes")))

@@ -317,4 +317,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, methods, n
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__binding(void) { return PyModule_Create(&module); }
+// torch_build: the torch whose headers these are (api.py compares it with the torch that is loaded)
+PyMODINIT_FUNC PyInit__binding(void)
+{
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_build", A8W8_TORCH_BUILD) != 0) Py_CLEAR(m);
+    return m;
+}
