@@ -343,7 +343,7 @@ int launch_small(const GemmParams& p, int batch, hipStream_t stream)
 {
     // (256 x 128 tiles leave rows past the end to the buffer descriptors: the 32-bit offsets of a whole tile must not wrap)
     const bool tall = MODE != MODE_BLOCK && !RAGGED && (p.m + 256ll) * p.lda + p.k < (1ll << 32) && (p.n + 128ll) * p.ldb + p.k < (1ll << 32);
-    switch (tile128_variant(p.m, p.n, p.k, batch, tall, MODE == MODE_BF16 || MODE == MODE_F4T, num_cus(), MODE == MODE_BLOCK)) {
+    switch (tile128_variant(p.m, p.n, p.k, batch, tall, MODE == MODE_BF16 || MODE == MODE_F4T, num_cus(), MODE == MODE_BLOCK && CDT == C_FP32)) {
         case TILES_64x64: return launch_tiles<MODE, CDT, SHORT_STAGES, 64, RAGGED, 64>(p, batch, stream);
         case TILES_128x64:
             if constexpr (constexpr int deep = narrow_deep_stages(MODE, RAGGED); deep != 0)

@@ -218,14 +218,17 @@ constexpr int tall_min_ksteps(bool cheap_steps) { return cheap_steps ? 24 : 16; 
 //   12.5 / 10.3 / 7.9, 512 x 2048 x 8192 23.7 / 19.1 / 14.6, bf16 4 x 162 x 384 x 3840 23.9 / 19.4 / 15.1; block scales 1024 x 1024 x 4096 18.1 / 13.8 / 11.1;
 //   row-major MX 512 x 512 x 1024 7.4 / 6.3 / 5.0; K = 2000 (a partial step) 1000 x 1000 16.8 / 12.4 / 9.8.  Not for two workgroups per compute unit (700 x
 //   2048 x 2048, 352 tiles of 64 x 64 9.7 / 8.3 / 9.2).
-//  128 x 64: 1000 x 1536 x 1024 7.3 / 5.9, 1437 x 1280 x 1152 7.6 / 6.4, 1495 x 1344 x 7168 23.3 / 19.8, 512 x 4096 x 1024 on row-major MXFP4 8.9 / 7.5; with block
-//   scales also where 128 x 128 ones fill more than three quarters of the chip (two workgroups per compute unit hide each other's multiply-adds:
-//   2048 x 2048 x 1024 fp32 C 11.3 / 10.9; row/col 8.5 / 9.3).  Fewer than 16 steps: up to seven eighths of the compute units.
+//  128 x 64: 1000 x 1536 x 1024 7.3 / 5.9, 1437 x 1280 x 1152 7.6 / 6.4, 1495 x 1344 x 7168 23.3 / 19.8, 512 x 4096 x 1024 on row-major MXFP4 8.9 / 7.5.  Fewer than 16 steps: up
+//   to seven eighths of the compute units.  With block scales and fp32 C also where 128 x 128 ones fill more than three quarters of the chip, up to eight steps and from
+//   eight columns of them on (block_fp32: two workgroups per compute unit hide each other's multiply-adds and long stores).  128 x 64 / 128 x 128, operands in
+//   the caches, from HBM: 2048 x 2048 x 512 8.3 / 8.9, 9.7 / 10.0, x 1024 10.4 / 10.8, 12.4 / 12.2, 8 x 512 x 1024 x 1024 11.6 / 12.3, 3200 x 1024 x 1024 9.5 / 9.6, 11.1 / 11.1,
+//   7 x 512 x 1024 x 1024 10.9 / 11.5, 13.4 / 12.4.  Not with bf16 C (2048 x 2048 x 1024 9.0 / 8.6, 11.1 / 9.9), more steps (x 4096 fp32 22.6 / 22.2, 29.4 / 25.4, bf16 21.8 /
+//   19.8, 27.2 / 22.5) or fewer columns (16 x 512 x 512 x 4096 46.2 / 33.3, x 1024 15.2 / 13.6, 24640 x 128 x 1024 10.3 / 9.9, 13.5 / 12.2).
 // Then, up to one workgroup per compute unit: four LDS stages (deep prefetch).  More: 256 x 128 tiles
 // where they pay (has_tall: the variant exists for the operands), else two stages, so that two workgroups share a compute unit and
 // hide each other's waits.  cheap_steps: bf16, and MXFP4 on tiled scales.
 enum Tile128 { TILES_128x64, TILES_128_FOUR_STAGES, TILES_256x128, TILES_128_TWO_STAGES, TILES_64x64 };
-inline Tile128 tile128_variant(long long m, long long n, long long k_bytes, long long batch, bool has_tall, bool cheap_steps, long long cus, bool block = false)
+inline Tile128 tile128_variant(long long m, long long n, long long k_bytes, long long batch, bool has_tall, bool cheap_steps, long long cus, bool block_fp32 = false)
 {
     const long long tiles_n = (n + 127) / 128, items = batch * ((m + 127) / 128) * tiles_n;
     if (m <= 128) {
@@ -234,7 +237,7 @@ inline Tile128 tile128_variant(long long m, long long n, long long k_bytes, long
         const long long columns64 = (n + 63) / 64, items64 = batch * ((m + 127) / 128) * columns64;
         if (batch * ((m + 63) / 64) * columns64 <= cus) return TILES_64x64;
         if (8 * items64 <= (k_bytes / 128 >= A8W8_NARROW_MIN_KSTEPS ? 8 : 7) * cus) return TILES_128x64;
-        if (block && 4 * items > 3 * cus && items <= cus) return TILES_128x64;
+        if (block_fp32 && 4 * items > 3 * cus && items <= cus && tiles_n >= 8 && k_bytes <= 8 * 128) return TILES_128x64;
     }
     if (items <= A8W8_SMALL_DEEP_UP_TO * cus) return TILES_128_FOUR_STAGES;
     if (has_tall && batch * ((m + 255) / 256) * tiles_n <= cus && k_bytes / 128 >= tall_min_ksteps(cheap_steps)) return TILES_256x128;

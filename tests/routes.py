@@ -93,9 +93,9 @@ def rounds_on_128_tiles(m, n, steps, kind="fp8", batch=1, fp32=False, cus=256):
 TILE128 = ("128x64", "128, four stages", "256x128", "128, two stages", "64x64")     # enum Tile128
 
 
-def tile128_variant(kind, m, n, k_bytes, batch=1, cus=256):
+def tile128_variant(kind, m, n, k_bytes, batch=1, cus=256, fp32=True):
     """The variant of the 128-tile kernel, or None for a problem of more than two 128-tiles per compute unit.  kind: "fp8", "mx", "block",
-    "bf16", "mxfp4" (row-major scales), "mxfp4_tiled"; whole K steps."""
+    "bf16", "mxfp4" (row-major scales), "mxfp4_tiled"; whole K steps.  fp32: the type of C (block scales)."""
     if not lib().route_fits_128_tiles(_ll(m), _ll(n), _ll(batch), _ll(cus)):
         return None
-    return TILE128[lib().route_tile128_variant(_ll(m), _ll(n), _ll(k_bytes), _ll(batch), int(kind != "block"), int(kind in ("bf16", "mxfp4_tiled")), _ll(cus), int(kind == "block"))]
+    return TILE128[lib().route_tile128_variant(_ll(m), _ll(n), _ll(k_bytes), _ll(batch), int(kind != "block"), int(kind in ("bf16", "mxfp4_tiled")), _ll(cus), int(kind == "block" and fp32))]

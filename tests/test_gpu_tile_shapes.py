@@ -78,3 +78,12 @@ def test_rule():
                                        (2048, 2048, 8, "block", "128x64"), (1536, 1920, 8, "block", "128, four stages"), (128, 2048, 64, "fp8", "128x64"),
                                        (128, 2048, 8, "fp8", "128, four stages")):
         assert routes.tile128_variant(kind, m, n, steps * 128) == variant, (m, n, steps, kind)
+
+
+@pytest.mark.parametrize("m,n,batch", [(24640, 128, 1), (3200, 1024, 1), (1600, 2048, 1), (2300, 1536, 1), (4500, 896, 1), (2048, 2048, 1), (512, 512, 16), (976, 512, 8), (512, 1024, 7)])
+@pytest.mark.parametrize("steps", [3, 8, 9, 32])
+def test_block_scales_up_to_one_tile_per_compute_unit(m, n, batch, steps):
+    """193 to 256 tiles of 128 x 128 are halved for fp32 C, few steps and eight columns of them only: elsewhere two halves on a compute unit take up to 1.5 times as long."""
+    assert 192 < batch * -(-m // 128) * (n // 128) <= 256
+    assert routes.tile128_variant("block", m, n, steps * 128, batch, fp32=False) == "128, four stages"
+    assert routes.tile128_variant("block", m, n, steps * 128, batch, fp32=True) == ("128x64" if steps <= 8 and n >= 1024 else "128, four stages")
