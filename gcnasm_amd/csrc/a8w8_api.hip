@@ -46,12 +46,9 @@ constexpr int persist_lds_bytes(int mode)
     return mode == MODE_MX ? PERSIST_LDS_BYTES_MX : mode == MODE_ROWCOL ? PERSIST_LDS_BYTES_ROWCOL : PERSIST_LDS_BYTES;
 }
 
-// LDS stages of the 128 x 64 variant of the 128-tile kernel: three, and as many as fit 160 KiB for the modes that narrow_tiles_deep is for
+// LDS stages of the 128 x 64 variant of the 128-tile kernel: three, and as many as fit 160 KiB (narrow_tiles_deep)
 constexpr int NARROW_STAGES = 3, SHORT_STAGES = 4;      // (64 x 64 tiles: four; six and eight are 2 to 10% slower)
-constexpr int narrow_deep_stages(int mode, bool ragged)
-{
-    return ragged ? 0 : mode == MODE_MXT ? 5 : mode == MODE_TENSOR || mode == MODE_ROWCOL || mode == MODE_BF16 ? 6 : 0;
-}
+constexpr int narrow_deep_stages(int mode) { return mode == MODE_MXT || mode == MODE_F4T ? 5 : 6; }
 
 template <int MODE>
 bool raise_lds_limits_of_mode()
@@ -73,9 +70,9 @@ bool raise_lds_limits_of_mode()
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, SHORT_STAGES, 64, false, 64>, small_lds_bytes(MODE, SHORT_STAGES, 64, 64)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, SHORT_STAGES, 64, false, 64>, small_lds_bytes(MODE, SHORT_STAGES, 64, 64));
     }
-    if constexpr (constexpr int deep = narrow_deep_stages(MODE, false); deep != 0)
-        ok = ok && raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, deep, 64>, small_lds_bytes(MODE, deep, 64)) &&
-             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, deep, 64>, small_lds_bytes(MODE, deep, 64));
+    constexpr int deep = narrow_deep_stages(MODE);
+    ok = ok && raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, deep, 64>, small_lds_bytes(MODE, deep, 64)) &&
+         raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, deep, 64>, small_lds_bytes(MODE, deep, 64));
     if constexpr (MODE != MODE_BLOCK)
         ok = ok && raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, 3, SM_BN, false, 256>, small_lds_bytes(MODE, 3, SM_BN, 256)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 3, SM_BN, false, 256>, small_lds_bytes(MODE, 3, SM_BN, 256));
@@ -86,6 +83,8 @@ bool raise_lds_limits_of_mode()
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, 4, SM_BN, true>, small_lds_bytes(MODE, 4)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, NARROW_STAGES, 64, true>, small_lds_bytes(MODE, NARROW_STAGES, 64)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, NARROW_STAGES, 64, true>, small_lds_bytes(MODE, NARROW_STAGES, 64)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, deep, 64, true>, small_lds_bytes(MODE, deep, 64)) &&
+             raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, deep, 64, true>, small_lds_bytes(MODE, deep, 64)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_BF16, SHORT_STAGES, 64, true, 64>, small_lds_bytes(MODE, SHORT_STAGES, 64, 64)) &&
              raise_lds_limit(gemm_a8w8_tile128<MODE, C_FP32, SHORT_STAGES, 64, true, 64>, small_lds_bytes(MODE, SHORT_STAGES, 64, 64));
     return ok;
@@ -346,8 +345,8 @@ int launch_small(const GemmParams& p, int batch, hipStream_t stream)
     switch (tile128_variant(p.m, p.n, p.k, batch, tall, MODE == MODE_BF16 || MODE == MODE_F4T, num_cus(), MODE == MODE_BLOCK && CDT == C_FP32)) {
         case TILES_64x64: return launch_tiles<MODE, CDT, SHORT_STAGES, 64, RAGGED, 64>(p, batch, stream);
         case TILES_128x64:
-            if constexpr (constexpr int deep = narrow_deep_stages(MODE, RAGGED); deep != 0)
-                if (narrow_tiles_deep(p.k)) return launch_tiles<MODE, CDT, deep, 64, false, 128>(p, batch, stream);
+            if (narrow_tiles_deep(p.m, p.k, !RAGGED && (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16)))
+                return launch_tiles<MODE, CDT, narrow_deep_stages(MODE), 64, RAGGED, 128>(p, batch, stream);
             return launch_tiles<MODE, CDT, NARROW_STAGES, 64, RAGGED, 128>(p, batch, stream);
         case TILES_128_FOUR_STAGES: return launch_tiles<MODE, CDT, 4, 128, RAGGED, 128>(p, batch, stream);
         case TILES_256x128:

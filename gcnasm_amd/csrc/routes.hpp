@@ -203,13 +203,15 @@ inline bool narrow_tiles_pay(long long items128, long long n, long long k_bytes,
 //   2048x4096x2048    18.0 -> 18.1, 21.3 -> 20.2, 19.4 -> 18.6, 15.2 / 12.7 -> 15.8 / 13.5, 31.1 -> 30.1
 //   1000x8192x1024    14.2 -> 14.7, 14.9 -> 15.2, 14.3 -> 14.4, 11.8 / 10.7 -> 13.3 / 12.1, 19.1 -> 20.1
 // i.e. the line lies at 16 steps of 128 bytes, and where a step's scales cost next to nothing beside its short MFMAs at 24.
-// LDS stages of 128 x 64 tiles: three, or as many as fit 160 KiB from 28 steps on where a step is little more than its operands (per-tensor, row/col and
-// tiled MXFP8 scales, bf16).  us, three / six: 1000 x 1536 x 1024 5.9 / 6.3, 402 x 1920 x 3072 10.3 / 10.5, 1024 x 2048 x 4096 13.7 / 13.0, 1495 x 1344 x 7168
+constexpr int tall_min_ksteps(bool cheap_steps) { return cheap_steps ? 24 : 16; }
+
+// LDS stages of 128 x 64 tiles: three, or as many as fit 160 KiB (five or six).  Up to 128 rows always those: the workgroup's share of the weights comes from HBM, and a
+// deep queue hides its latency (us, three / six, weights from HBM: row-major MX 5 x 3328 x 2688 11.5 / 10.2, 1 x 8064 x 3584 15.4 / 13.8, 13 x 9344 x 2688 12.4 / 11.8,
+// MXFP4 2 x 768 x 13312 28.7 / 26.7, 3 x 4736 x 13312 30.0 / 28.7).  Beyond, from 28 steps on where a step is little more than its operands (light_steps: per-tensor,
+// row/col and tiled MXFP8 scales, bf16; whole steps): 1000 x 1536 x 1024 5.9 / 6.3, 402 x 1920 x 3072 10.3 / 10.5, 1024 x 2048 x 4096 13.7 / 13.0, 1495 x 1344 x 7168
 // 20.6 / 19.8; tiled MXFP8 11.0 / 11.4 at 24 steps, 14.5 / 14.2 at 32.  Others: block scales 1024 x 2048 x 4096 14.9 / 15.4, row-major MX 20.8 / 22.2, MXFP4 23.5 /
 // 24.9, tiled 14.7 / 14.9; partial steps 800 x 2000 x 2000 12.8 / 14.2.
-inline bool narrow_tiles_deep(long long k_bytes) { return k_bytes / 128 >= 28; }
-
-constexpr int tall_min_ksteps(bool cheap_steps) { return cheap_steps ? 24 : 16; }
+inline bool narrow_tiles_deep(long long m, long long k_bytes, bool light_steps) { return m <= 128 || (light_steps && k_bytes / 128 >= 28); }
 
 // The variant of the 128-tile kernel: the smallest tile whose workgroups do not outnumber the compute units, since a workgroup alone on its
 // compute unit takes as long as its own K loop, and that as long as its tile's rows take from L2 (16, 24, 32 KiB a step: 0.18, 0.27, 0.36 us).

@@ -87,3 +87,28 @@ def test_block_scales_up_to_one_tile_per_compute_unit(m, n, batch, steps):
     assert 192 < batch * -(-m // 128) * (n // 128) <= 256
     assert routes.tile128_variant("block", m, n, steps * 128, batch, fp32=False) == "128, four stages"
     assert routes.tile128_variant("block", m, n, steps * 128, batch, fp32=True) == ("128x64" if steps <= 8 and n >= 1024 else "128, four stages")
+
+
+def test_stages_of_128x64_tiles():
+    """Up to 128 rows the weights come from HBM: deep staging for every kind of step."""
+    for kind in ("fp8", "bf16", "mxfp8", "block", "mx", "mxfp4", "mxfp4_tiled", "ragged"):
+        light = kind in ("fp8", "bf16", "mxfp8")
+        assert [routes.narrow_tiles_deep(kind, m, s * 128) for m, s in ((1, 16), (128, 16), (128, 64), (129, 27), (129, 28))] == [True, True, True, False, light]
+
+
+# deep staging up to 128 rows: fewer, as many and more K steps than twice the stages; the last one a partial step
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,steps", [(1, 200, 16), (100, 1000, 17), (128, 1990, 30)])
+@pytest.mark.parametrize("kind,mode", [("fp8", g.MX), ("fp4", g.MX), ("fp8", g.BLOCK)], ids=lambda v: str(v))
+def test_up_to_128_rows(m, n, steps, kind, mode):
+    n = (n + 127) // 128 * 128 if mode == g.BLOCK else n
+    assert routes.tile128_variant("block", m, n, steps * 128) == "128x64"
+    check(kind, mode, m, n, steps * ELEMENTS[kind])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1, 200, 2064), (100, 1000, 2032), (128, 1990, 4016)])
+@pytest.mark.parametrize("kind,mode", [("fp8", g.ROWCOL), ("fp8", g.TENSOR), ("bf16", g.TENSOR)], ids=lambda v: str(v))
+def test_up_to_128_rows_partial_steps(m, n, k, kind, mode):
+    assert routes.tile128_variant("block", m, n, k) == "128x64" or k < 2048
+    check(kind, mode, m, n, k // 2 if kind == "bf16" else k)
