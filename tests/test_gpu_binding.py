@@ -108,6 +108,25 @@ def _other_forms():
             yield g.cvt_e4m3_to_f32, ((t * 50).to(torch.int32).to(torch.uint8), dialect), {}
 
 
+def _ordinary(f, args, kw):
+    """What csrc/binding.cpp is for: torch's own tensors in GPU memory, contiguous ones for the conversions, and no batch of b alone."""
+    tensors = [t for t in (*args, kw.get("c")) if isinstance(t, torch.Tensor)]
+    if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda for t in tensors):
+        return False
+    return args[0].is_contiguous() if f in (g.cvt_f32_to_e4m3, g.cvt_e4m3_to_f32) else f is not g.gemm or args[1].dim() <= args[0].dim()
+
+
+def _recorded(patch):
+    """Answers of the compiled path from here on, None where it declines."""
+    answers = []
+    for name in FAST:
+        def call(*args, fast=getattr(api, name)):
+            answers.append(fast(*args))
+            return answers[-1]
+        patch.setattr(api, name, call)
+    return answers
+
+
 def _outcome(f, args, kw):
     kw = dict(kw)
     given = kw.get("c")
@@ -127,9 +146,12 @@ def _outcome(f, args, kw):
 @pytest.mark.parametrize("forms", [_gemm_forms, _other_forms], ids=lambda f: f.__name__)
 def test_same_as_the_statements_of_the_functions(forms, monkeypatch):
     g.quantize(_rand(4, 128), g.ROWCOL)      # connects
-    served = 0
+    served, declined = set(), 0
     for i, (f, args, kw) in enumerate(forms()):
-        fast = _outcome(f, args, kw)
+        with monkeypatch.context() as patch:
+            answers = _recorded(patch)
+            fast = _outcome(f, args, kw)
+        assert len(answers) == 1, (i, f.__name__)
         with monkeypatch.context() as patch:
             for name in FAST:
                 patch.setattr(api, name, lambda *a: None)
@@ -137,16 +159,21 @@ def test_same_as_the_statements_of_the_functions(forms, monkeypatch):
         if isinstance(slow, tuple):
             assert fast == slow, (i, f.__name__, kw, fast, slow)
         else:
-            served += 1
+            assert (answers[0] is not None) == _ordinary(f, args, kw), (i, f.__name__, kw)
+            if answers[0] is None:
+                declined += 1
+            else:
+                served.add(i)
             for u, v in zip(fast, slow):
                 assert type(u) is type(v) and u.dtype == v.dtype and u.shape == v.shape and u.stride() == v.stride() and torch.equal(u.view(torch.uint8) if u.dim() else u, v.view(torch.uint8) if v.dim() else v), (i, f.__name__, kw)
-    assert served >= 40
+    assert len(served) >= 40 and declined > 0
 
 
 @pytest.mark.gpu
-def test_on_the_current_stream_and_under_modes():
+def test_on_the_current_stream_and_under_modes(monkeypatch):
     x = _rand(64, 1024)
     want = g.quantize(x, g.ROWCOL)
+    answers = _recorded(monkeypatch)
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
         y = x * 1.0
@@ -156,6 +183,7 @@ def test_on_the_current_stream_and_under_modes():
     with torch.inference_mode():
         q, _ = g.quantize(x, g.ROWCOL)
         assert q.is_inference()
+    assert len(answers) == 2 and all(r is not None for r in answers)
     with torch.device("cpu"):                # a function mode: the functions' own statements
         assert torch.equal(g.quantize(x, g.ROWCOL)[0], want[0])
     seen = []
@@ -168,6 +196,7 @@ def test_on_the_current_stream_and_under_modes():
     with Log():
         assert torch.equal(g.quantize(x, g.ROWCOL)[0], want[0])
     assert torch.ops.aten.empty.memory_format in seen      # allocations go through the mode
+    assert len(answers) == 4 and answers[2] is None and answers[3] is None
     with pytest.raises(Exception):           # no address behind a batched tensor
         torch.vmap(lambda t: g.quantize(t, g.ROWCOL)[0])(torch.stack([x, x]))
 
