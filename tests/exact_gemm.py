@@ -43,7 +43,8 @@ def _mx_scales(rows, k, tiled, pad):
 
 
 def check(kind, mode, m, n, k, batch=1, pad=0, shuffled=False, c_pad=0, c_shift=0):
-    """c_pad: elements between C's rows, c_shift: in front of its first one; neither may be written."""
+    """c_pad: elements between C's rows, c_shift: in front of its first one; neither may be written, nor may the 256 rows behind C, which is as far as a tile on its
+    edge reaches."""
     rng = np.random.Generator(np.random.Philox(m + n + k))
     per_byte = {"fp4": 2, "bf16": 0.5}.get(kind, 1)
     a, b = [[_operand(rng, rows, k, kind) for _ in range(batch)] for rows in (m, n)]
@@ -66,7 +67,7 @@ def check(kind, mode, m, n, k, batch=1, pad=0, shuffled=False, c_pad=0, c_shift=
         b_all = torch.stack([g.preshuffle_b_device(o[0][:, :row_bytes].contiguous()) for o in b])
         b_batch = n * k
     for c_dtype, dtype in ((g.FP32, torch.float32), (g.BF16, torch.bfloat16)):
-        store = torch.full((c_shift + batch * m * (n + c_pad) + 64,), -7.0, dtype=dtype, device="cuda")
+        store = torch.full((c_shift + (batch * m + 256) * (n + c_pad),), -7.0, dtype=dtype, device="cuda")
         c = store[c_shift:c_shift + batch * m * (n + c_pad)].view(batch, m, n + c_pad)
         args = g.raw_gemm_args(a_all.data_ptr(), b_all.data_ptr(), c.data_ptr(), s_all[0].data_ptr(), s_all[1].data_ptr(), m, n, k, mode, c_dtype, batch,
                                stride_a=stride, stride_b=stride, stride_c=n + c_pad, stride_sfa=sa[1], stride_sfb=sb[1],
