@@ -42,9 +42,9 @@ def _mx_scales(rows, k, tiled, pad):
     return g.mx_tile_scales(whole), 0, value
 
 
-def check(kind, mode, m, n, k, batch=1, pad=0, shuffled=False, c_pad=0, c_shift=0):
+def check(kind, mode, m, n, k, batch=1, pad=0, shuffled=False, c_pad=0, c_shift=0, kernel=None):
     """c_pad: elements between C's rows, c_shift: in front of its first one; neither may be written, nor may the 256 rows behind C, which is as far as a tile on its
-    edge reaches."""
+    edge reaches.  kernel: what serves FP8 operands, by type of C."""
     rng = np.random.Generator(np.random.Philox(m + n + k))
     per_byte = {"fp4": 2, "bf16": 0.5}.get(kind, 1)
     a, b = [[_operand(rng, rows, k, kind) for _ in range(batch)] for rows in (m, n)]
@@ -72,6 +72,7 @@ def check(kind, mode, m, n, k, batch=1, pad=0, shuffled=False, c_pad=0, c_shift=
         args = g.raw_gemm_args(a_all.data_ptr(), b_all.data_ptr(), c.data_ptr(), s_all[0].data_ptr(), s_all[1].data_ptr(), m, n, k, mode, c_dtype, batch,
                                stride_a=stride, stride_b=stride, stride_c=n + c_pad, stride_sfa=sa[1], stride_sfb=sb[1],
                                b_preshuffled=int(shuffled), batch_strides=(m * stride, b_batch, m * (n + c_pad), s_all[0].shape[1], s_all[1].shape[1]))
+        assert kernel is None or g.kernel_name(args) == kernel[c_dtype], (m, n, k, c_dtype, g.kernel_name(args))
         entry = {"fp4": g.lib().a4w4_gemm, "bf16": g.lib().a16w16_gemm}.get(kind, g.lib().a8w8_gemm)
         assert entry(ctypes.byref(args), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
         for e in range(batch):

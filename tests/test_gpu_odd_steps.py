@@ -11,7 +11,9 @@ from exact_gemm import check
 @pytest.mark.parametrize("m,n,steps", [(2790, 5111, 5), (2816, 5120, 7), (4090, 7100, 11), (2790, 5111, 13), (4350, 4200, 33)])
 @pytest.mark.parametrize("kind", ["fp8", "fp4"])
 def test_tiled_scales(m, n, steps, kind):
-    assert routes.odd_tiled_mx_on_four_waves(m, n, steps, fp4=kind == "fp4") or (kind, steps) == ("fp4", 33)
+    # (bf16 C, fp32 C); the others run on the 128-tile kernel
+    wide = {5: (True, False), 7: (True, False), 11: (True, kind == "fp8"), 13: (True, True), 33: (kind == "fp8", kind == "fp8")}[steps]
+    assert tuple(routes.odd_tiled_mx_on_four_waves(m, n, steps, fp4=kind == "fp4", fp32=fp32) for fp32 in (False, True)) == wide
     check(kind, g.MX_TILED, m, n, steps * (256 if kind == "fp4" else 128))
 
 

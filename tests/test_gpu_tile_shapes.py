@@ -22,8 +22,10 @@ ELEMENTS = {"fp4": 256, "bf16": 64, "fp8": 128}               # of a K step
 def test_shapes(m, n, steps, batch, variant, kind, mode, route):
     if mode == g.BLOCK:
         n = (n + 127) // 128 * 128
-    got = routes.tile128_variant(route, m, n, steps * 128, batch)
-    assert got == variant or mode == g.BLOCK      # (whole blocks of columns are other sizes)
+    want = {g.BF16: variant, g.FP32: variant}
+    if mode == g.BLOCK:      # whole blocks of columns are other sizes, and fp32 C has a line of its own
+        want.update({(1500, 1408): {g.BF16: "128, four stages", g.FP32: "128, four stages"}, (2000, 2048): {g.FP32: "128x64"}, (1600, 2176): {g.FP32: "128x64"}}.get((m, n), {}))
+    assert {c: routes.tile128_variant(route, m, n, steps * 128, batch, fp32=c == g.FP32) for c in want} == want
     check(kind, mode, m, n, steps * ELEMENTS[kind], batch=batch)
 
 
@@ -39,7 +41,7 @@ def test_shuffled_weights(m, n, steps, batch, kind, mode):
                                            (1990, 2010, 336, "128, four stages")])
 @pytest.mark.parametrize("kind,mode", [("fp8", g.ROWCOL), ("fp8", g.TENSOR), ("bf16", g.TENSOR)], ids=lambda v: str(v))
 def test_partial_steps(m, n, k, variant, kind, mode):
-    assert routes.tile128_variant("block", m, n, k, 1) == variant or variant == "128, four stages"      # (no 256 x 128 tiles here either)
+    assert routes.tile128_variant("fp8", m, n, k, 1) == variant
     check(kind, mode, m, n, k // 2 if kind == "bf16" else k)
 
 
@@ -50,7 +52,10 @@ def test_partial_steps(m, n, k, variant, kind, mode):
 def test_badly_filled_rounds(m, n, steps, kind, mode, route):
     n = n // 128 * 128 if mode == g.BLOCK else n
     name = {"fp8": {g.MX_TILED: "mxfp8", g.MX: "mx", g.BLOCK: "block"}.get(mode, "fp8"), "fp4": "mxfp4"}.get(kind, kind)
-    assert routes.tile128_variant(route, m, n, steps * 128) is None and (routes.rounds_on_128_tiles(m, n, steps, name, fp32=True) or steps * (name != "fp8") > 8)
+    # (bf16 C, fp32 C); the others run on 256-tiles
+    small = {8: {"mxfp8": (False, True), "mx": (False, True), "block": (False, True)}, 16: {"mxfp8": (False, False), "mx": (False, False), "mxfp4": (False, True)}}.get(steps, {})
+    assert routes.tile128_variant(route, m, n, steps * 128) is None
+    assert tuple(routes.rounds_on_128_tiles(m, n, steps, name, fp32=fp32) for fp32 in (False, True)) == small.get(name, (True, True))
     check(kind, mode, m, n, steps * ELEMENTS[kind])
 
 
@@ -110,5 +115,5 @@ def test_up_to_128_rows(m, n, steps, kind, mode):
 @pytest.mark.parametrize("m,n,k", [(1, 200, 2064), (100, 1000, 2032), (128, 1990, 4016)])
 @pytest.mark.parametrize("kind,mode", [("fp8", g.ROWCOL), ("fp8", g.TENSOR), ("bf16", g.TENSOR)], ids=lambda v: str(v))
 def test_up_to_128_rows_partial_steps(m, n, k, kind, mode):
-    assert routes.tile128_variant("block", m, n, k) == "128x64" or k < 2048
+    assert routes.tile128_variant("fp8", m, n, k) == ("128, four stages" if k == 2032 else "128x64")      # (2032: a step short of narrow tiles)
     check(kind, mode, m, n, k // 2 if kind == "bf16" else k)
