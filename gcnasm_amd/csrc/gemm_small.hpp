@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(SM_THREADS, BM_ == 256 ? 1 : 2) __attribute__(
     static_assert(BM_ == 128 || (SHORT && BN_ == 64 && SM_STAGES > 2) || (TALL && SM_STAGES == 3 && BN_ == 128 && !RAGGED && MODE != MODE_BLOCK), "tile height");
     static_assert(!RAGGED || MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_BF16, "partial K steps: no scales that change with K");
     constexpr bool BY_BF16 = RAGGED && MODE != MODE_BF16;      // FP8 operands converted to bf16
-    static_assert(SM_STAGES == 2 || SM_STAGES == 3 || SM_STAGES == 4 || SM_STAGES == 5 || SM_STAGES == 6 || SM_STAGES == 8, "LDS stages");
+    static_assert(SM_STAGES == 2 || SM_STAGES == 3 || SM_STAGES == 4 || SM_STAGES == 5 || SM_STAGES == 6, "LDS stages");
     static_assert(BN_ == 128 || BN_ == 64, "tile width");
     constexpr int SM_BN = BN_;
     constexpr int SM_BM = BM_;

@@ -55,8 +55,8 @@ def test_tiled_scales_by_lines_of_infinities_and_nan(orc):
 def test_row_major_scales_of_the_flattened_array(orc, rows, k, pad):
     """One, two and four chunks per wave, whole and partial last workgroups."""
     x, view = _rows_apart(rows, k, pad, True)
-    # (finite values: blocks that hold an infinity, or zeros and NaN alone, keep exponent 0 on the device and not in the oracle; the test above compares
-    # those with the tiled quantiser's)
+    # (finite values: a block that holds an infinity gets scale 1 on the device and 2^127 in the oracle, and NaN codes differ in their sign bit; the test
+    # above compares such blocks with the tiled quantiser's)
     for (q, s), (q0, s0) in ((g.quantize(view, g.MX), orc.quantize(x, orc.MX)), (g.quantize_mxfp4(view), orc.quantize_mxfp4(x))):
         assert (q.cpu().numpy() == q0).all() and (s.cpu().numpy().reshape(s0.shape) == s0).all()
 
