@@ -200,6 +200,7 @@ GemmParams make_params(const a8w8_gemm_args* g)
     p.tiles_m = (g->m + BM - 1) / BM;
     p.tiles_n = (g->n + BN - 1) / BN;
     p.inv_per_group = p.inv_rem = 0;
+    p.runs = 0;
     return p;
 }
 
@@ -332,6 +333,7 @@ int launch_tiles(const GemmParams& p, int batch, hipStream_t stream)
     q.tiles_n = (p.n + BN_ - 1) / BN_;
     q.inv_per_group = tile_map_inverse(8 * q.tiles_n);
     q.inv_rem = tile_map_inverse(q.tiles_m % 8);
+    q.runs = tiles_in_runs(q.tiles_m, q.tiles_n, p.k / BK, batch, BM_ > BN_, num_cus());
     const dim3 grid((unsigned)(q.tiles_m * q.tiles_n), 1, (unsigned)batch);
     return launch(gemm_a8w8_tile128<MODE, CDT, STAGES, BN_, RAGGED, BM_>, grid, dim3(SM_THREADS), small_lds_bytes(MODE, STAGES, BN_, BM_), stream, q);
 }
@@ -371,7 +373,7 @@ int launch_persist(const GemmParams& p, int batch, hipStream_t stream)
     pp.g = p;
     pp.batch = batch;
     pp.items = batch * p.tiles_m * p.tiles_n;
-    pp.map = make_tile_map(p.tiles_m, p.tiles_n);
+    pp.map = make_tile_map(p.tiles_m, p.tiles_n, items_in_runs(p.tiles_m, p.tiles_n, p.k / BK, batch, num_cus()));
     const int cus = num_cus();
     dim3 grid((unsigned)(pp.items < cus ? pp.items : cus), 1, 1);
     return launch(gemm_a8w8_persist<MODE, CDT>, grid, dim3(GEMM_THREADS), persist_lds_bytes(MODE), stream, pp);
@@ -388,7 +390,7 @@ int launch_wide(const GemmParams& p, int batch, hipStream_t stream)
         pp.g = p;
         pp.batch = batch;
         pp.items = batch * p.tiles_m * p.tiles_n;
-        pp.map = make_tile_map(p.tiles_m, p.tiles_n);
+        pp.map = make_tile_map(p.tiles_m, p.tiles_n, items_in_runs(p.tiles_m, p.tiles_n, p.k / BK, batch, num_cus()));
         const int cus = num_cus();
         dim3 grid((unsigned)(pp.items < cus ? pp.items : cus), 1, 1);
         return launch(gemm_a8w8_wide<MODE, CDT>, grid, dim3(WIDE_THREADS), wide_lds_bytes(MODE), stream, pp);

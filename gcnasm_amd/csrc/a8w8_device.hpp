@@ -57,6 +57,7 @@ struct GemmParams {
     // the a8w8_preshuffle_b layout (two 1 KiB blocks per step; ldb = k there, so that 16 r rows are 16 r * ldb bytes)
     int b_kshift;
     uint32_t inv_per_group, inv_rem;      // 128-tile kernel: tile_map_inverse of 8 tiles_n and of tiles_m % 8 (tile_of_block)
+    int runs;                             // 128-tile kernel: tiles_in_runs (routes.hpp)
 };
 
 // Raw buffer descriptor over [base, base + bytes): dword 3 = 0x00020000 selects the raw

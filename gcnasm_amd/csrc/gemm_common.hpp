@@ -32,8 +32,8 @@ constexpr int TM = WAVE_M / 16, TN = WAVE_N / 16;    // 4 x 8 MFMA tiles per wav
 
 // Workgroup id -> tile (tile_of_block).  Consecutive workgroup ids land on different XCDs (round-robin over
 // 8), each with its own L2, so ids are first regrouped so that one XCD works on a
-// contiguous run of tiles (without it, on tile counts that 8 does not divide, 210 tiles of 64 x 64 with K = 3072 took 10.8 us instead of 7.8); inside the run, tiles are walked down 8 tile-rows before moving
-// to the next tile-column so that concurrently resident tiles share A rows and B rows.
+// contiguous run of tiles, except on some tile counts that 8 does not divide (`runs`: tiles_in_runs and items_in_runs of routes.hpp); inside the run, tiles are
+// walked down 8 tile-rows before moving to the next tile-column so that concurrently resident tiles share A rows and B rows.
 // Nothing hides the lookup (the persistent kernels look tiles up at every tile change, the 128-tile kernel in front of its first load): every division is by a value the host knows, so the host passes floor(2^32 / d) for each of them and the
 // kernel divides with one multiply and one correction (exact for 0 <= n < 2^31 and any d >= 1: the estimate
 // mulhi(n, floor(2^32 / d)) is the quotient or one less).  Measured against run-time divisors: 0.25% of the MXFP8 8192^3
@@ -44,12 +44,13 @@ struct TileMap {
     int per_group;             // 8 * tiles_n: the tiles of eight tile rows
     int rem;                   // tiles_m % 8: tile rows of the last group when it is not a full one (0: none)
     uint32_t inv_tiles, inv_per_group, inv_rem;      // floor(2^32 / d) of the three divisors (d = 1: 2^32 - 1)
+    int runs;                  // a run of tiles per XCD
 };
 __host__ __device__ inline uint32_t tile_map_inverse(int d)
 {
     return d <= 1 ? 0xFFFFFFFFu : (uint32_t)((1ull << 32) / (uint32_t)d);
 }
-__host__ inline TileMap make_tile_map(int tiles_m, int tiles_n)
+__host__ inline TileMap make_tile_map(int tiles_m, int tiles_n, bool runs)
 {
     TileMap t;
     t.tiles_m = tiles_m; t.tiles_n = tiles_n;
@@ -59,6 +60,7 @@ __host__ inline TileMap make_tile_map(int tiles_m, int tiles_n)
     t.inv_tiles = tile_map_inverse(t.tiles);
     t.inv_per_group = tile_map_inverse(t.per_group);
     t.inv_rem = tile_map_inverse(t.rem);
+    t.runs = runs;
     return t;
 }
 A8W8_DEV int div_by_known(int n, int d, uint32_t inv)
@@ -71,7 +73,7 @@ A8W8_DEV void tile_of_block(const GemmParams& p, int bid, int& tm, int& tn)
 {
     const int nt = p.tiles_m * p.tiles_n;
     // (runs of nt / 8 tiles, the first nt % 8 of them one longer)
-    const int id = (bid & 7) * (nt >> 3) + min(bid & 7, nt & 7) + (bid >> 3);
+    const int id = p.runs ? (bid & 7) * (nt >> 3) + min(bid & 7, nt & 7) + (bid >> 3) : bid;
     const int per_group = 8 * p.tiles_n, group = div_by_known(id, per_group, p.inv_per_group), first_m = group * 8, in_group = id - group * per_group;
     if (p.tiles_m - first_m >= 8) {
         tn = in_group >> 3;
@@ -87,8 +89,7 @@ A8W8_DEV void tile_of_item(const TileMap& t, int item, int& batch, int& tm, int&
 {
     batch = div_by_known(item, t.tiles, t.inv_tiles);
     const int bid = item - batch * t.tiles;
-    // (220 tiles, 2816 x 5120 x 5120: 59.0 -> 58.0 us; 209, 2700 x 4736 x 5120: 63.5 -> 61.3)
-    const int id = (bid & 7) * (t.tiles >> 3) + min(bid & 7, t.tiles & 7) + (bid >> 3);
+    const int id = t.runs ? (bid & 7) * (t.tiles >> 3) + min(bid & 7, t.tiles & 7) + (bid >> 3) : bid;
     const int group = div_by_known(id, t.per_group, t.inv_per_group);
     const int first_m = group * 8;
     const int in_group = id - group * t.per_group;

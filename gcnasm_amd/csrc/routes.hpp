@@ -246,6 +246,31 @@ inline Tile128 tile128_variant(long long m, long long n, long long k_bytes, long
     return TILES_128_TWO_STAGES;
 }
 
+// ---------------------------------------------------------------- tiles and XCDs
+// Whether an XCD (workgroup ids modulo 8) takes a run of consecutive tiles, which are numbered down eight tile rows and then along the columns, or every eighth
+// tile.  The former where 8 divides the tiles.  Elsewhere too up to seven tile rows: a run holds all rows of a few columns, every eighth tile nearly all columns.
+// With more rows every eighth tile is one row of the eight, with all columns, and a run of the last, lower group of rows has many more of its columns than the
+// other runs have; runs pay where a launch has several tiles per compute unit, so that an XCD's are not all read at once, or many columns and a long K loop.
+// us, every eighth tile / runs, tile rows x columns: 128-tile kernel 3 x 52 12.2 / 11.3, 5 x 23 10.6 / 10.0, batch of 8 of 7 x 3 18.0 / 14.9; 17 x 12 12.9 / 13.9,
+// 28 x 9 25.2 / 26.3, 42 x 6 29.5 / 31.7, 52 x 7 17.4 / 18.8, 41 x 5 19.0 / 20.8; 25 x 57 63.7 / 55.2, 59 x 13 23.3 / 24.6; 9 x 28 of 55 steps 52.0 / 47.7.  By groups of shapes,
+// runs against every eighth tile: fewer than 8 rows 2.5% faster, 9 to 15 rows 2%, 17 and more 4% slower; more than one tile per compute unit and 9 to 15
+// rows 1.5% faster, more than two and 21 columns 6%; 40 steps and 13 columns 2% faster.  A batch of two rows of tall tiles (128 x 64) shares a tile row's A, the larger
+// operand, among every eighth tile: 16 of 2 x 6 12.0 / 12.9, 20.5 / 22.7.
+inline bool tiles_in_runs(long long tiles_m, long long tiles_n, long long k_steps, long long batch, bool tall, long long cus)
+{
+    const long long tiles = tiles_m * tiles_n;
+    if (tiles % 8 == 0) return true;
+    if (tiles_m < 8) return !(batch > 1 && tiles_m <= 2 && tall);
+    return (tiles > cus && tiles_m < 16) || (tiles > 2 * cus && tiles_n > 20) || (k_steps >= 40 && tiles_n > 12);
+}
+// The same for the 256-tile kernels, whose workgroups walk the tiles of all batch entries: up to two rounds of them and fewer than 16 steps runs are 2% slower (9 x 28 31.4 /
+// 33.4, 9 x 21 19.9 / 21.4), longer or more rounds 1 to 4% faster (220 tiles of 40 steps 59.0 / 58.0, 26 x 31 of 38 steps 300 / 281).
+inline bool items_in_runs(long long tiles_m, long long tiles_n, long long k_steps, long long batch, long long cus)
+{
+    const long long tiles = tiles_m * tiles_n;
+    return tiles % 8 == 0 || tiles_m < 8 || k_steps >= 16 || batch * tiles > 2 * cus;
+}
+
 // ---------------------------------------------------------------- flat GEMM (up to 128 activation rows)
 // Weight tiles (nt) and groups of 16 activation rows (mt) per workgroup of the flat GEMM.
 //

@@ -37,6 +37,14 @@ int route_rounds_on_128_tiles(int kind, long long m, long long n, long long k_st
     return a8w8::rounds_on_128_tiles((a8w8::RoundsKind)kind, m, n, k_steps, batch, fp32_c != 0, cus);
 }
 int route_narrow_tiles_deep(long long m, long long k_bytes, int light_steps) { return a8w8::narrow_tiles_deep(m, k_bytes, light_steps != 0); }
+int route_tiles_in_runs(long long tiles_m, long long tiles_n, long long k_steps, long long batch, int tall, long long cus)
+{
+    return a8w8::tiles_in_runs(tiles_m, tiles_n, k_steps, batch, tall != 0, cus);
+}
+int route_items_in_runs(long long tiles_m, long long tiles_n, long long k_steps, long long batch, long long cus)
+{
+    return a8w8::items_in_runs(tiles_m, tiles_n, k_steps, batch, cus);
+}
 int route_fits_128_tiles(long long m, long long n, long long batch, long long cus) { return a8w8::fits_128_tiles(m, n, batch, cus); }
 int route_tile128_variant(long long m, long long n, long long k_bytes, long long batch, int has_tall, int cheap_steps, long long cus, int block_fp32)
 {

@@ -95,6 +95,16 @@ def narrow_tiles_deep(kind, m, k_bytes):
     return bool(lib().route_narrow_tiles_deep(_ll(m), _ll(k_bytes), int(kind in ("fp8", "mxfp8", "bf16"))))
 
 
+def tiles_in_runs(tiles_m, tiles_n, steps, batch=1, tall=False, cus=256):
+    """128-tile kernel: a run of tiles per XCD, or every eighth; tall: tiles of more rows than columns."""
+    return bool(lib().route_tiles_in_runs(_ll(tiles_m), _ll(tiles_n), _ll(steps), _ll(batch), int(tall), _ll(cus)))
+
+
+def items_in_runs(tiles_m, tiles_n, steps, batch=1, cus=256):
+    """256-tile kernels."""
+    return bool(lib().route_items_in_runs(_ll(tiles_m), _ll(tiles_n), _ll(steps), _ll(batch), _ll(cus)))
+
+
 TILE128 = ("128x64", "128, four stages", "256x128", "128, two stages", "64x64")     # enum Tile128
 
 
