@@ -97,12 +97,18 @@ inline Rounds tile_rounds(long long m, long long n, long long batch, long long c
 //   6144 x 3072  8 steps 29.5 / 33.7, 32.3 / 41.6, 31.2 / 34.6, 34.0 / 41.9   16: 47.0 / 54.8, 50.0 / 62.3, 50.9 / 55.2, 54.0 / 62.9   32: 84.8 / 98.0, 90.7 / 105, 99.8 / 95.6, 106 / 106
 //   5376 x 4096  8: 33.6 / 36.0, 37.9 / 43.6, 35.7 / 36.9, 39.6 / 42.8   12: 44.6 / 48.3, 48.8 / 56.0, 46.9 / 48.1, 50.7 / 53.1   24: 75.9 / 80.6, 81.4 / 87.7, 89.1 / 80.5, 94.2 / 85.6
 //   2304 x 4096  8: 19.5 / 19.1, 21.9 / 23.1, 20.1 / 19.5, 22.7 / 23.4   16: 30.4 / 29.5, 31.9 / 33.7, 32.0 / 31.3, 33.8 / 34.6
+// A batch of small entries (up to 128 tiles of 128 x 128 each): every XCD's 128-tiles read nearly all of every entry, so that three rounds of them stand against one of 256-tiles
+// up to eight or ten steps only.  us, 128-tiles / 256-tiles: block fp32 16 x 953 x 640 8 steps 26.0 / 26.3, 10 30.3 / 29.2, 15 40.9 / 36.0; bf16 operands 16 x 953 x 640 bf16 C 8 22.1 / 25.9,
+// 15 35.0 / 28.7; 16 x 700 x 768 8 21.7 / 20.8, 10 25.6 / 23.1, 16 35.7 / 29.7; 8 x 1020 x 1280 8 20.5 / 20.5, 10 23.9 / 22.5, 16 32.9 / 28.8.  Larger entries as above:
+// 2 x 2600 x 2176 bf16 C 14 steps 28.2 / 31.5, block fp32 29.8 / 29.7 at 12.
 enum RoundsKind { ROUNDS_PLAIN, ROUNDS_MXFP8_TILED, ROUNDS_MXFP4_TILED, ROUNDS_BLOCK, ROUNDS_MXFP8_ROWS };      // (plain: per-tensor and row/col scales, bf16)
 inline bool rounds_on_128_tiles(RoundsKind kind, long long m, long long n, long long k_steps, long long batch, bool fp32_c, long long cus)
 {
     const Rounds rounds = tile_rounds(m, n, batch, cus);
     if (k_steps < 5 || rounds.of256 > 2 || rounds.of128 > 3 * rounds.of256) return false;
     const bool finer = rounds.of128 < 3 * rounds.of256, two = rounds.of256 == 2;
+    const long long entry_tiles = ((m + 127) / 128) * ((n + 127) / 128);
+    if (!finer && batch > 1 && entry_tiles <= 128 && k_steps > (entry_tiles <= 64 ? 8 : 10)) return false;
     switch (kind) {
         case ROUNDS_MXFP8_TILED: return k_steps <= (finer ? 20 : fp32_c ? 8 : 0);
         case ROUNDS_MXFP4_TILED: return k_steps <= (finer ? 32 : fp32_c ? 16 : 8);

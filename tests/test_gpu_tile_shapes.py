@@ -77,6 +77,13 @@ def test_rule_for_badly_filled_rounds():
                 assert g.kernel_name(args) in ("gemm_a8w8_wide", "gemm_a8w8_persist") and g.lib().a8w8_gemm(ctypes.byref(args), None) == -7
 
 
+@pytest.mark.parametrize("m,n,batch,most", [(953, 640, 16, 8), (700, 768, 16, 8), (1020, 1280, 8, 10), (2600, 2176, 2, 16), (2304, 4096, 1, 16)])
+def test_rounds_of_a_batch_of_small_entries(m, n, batch, most):
+    """Three rounds of 128-tiles against one of 256-tiles, up to `most` steps: beyond, small entries took up to 1.26 times as long."""
+    for kind, fp32 in (("bf16", False), ("bf16", True), ("fp8", False), ("block", True)):
+        assert [routes.rounds_on_128_tiles(m, n, s, kind, batch, fp32) for s in (5, most, most + 1)] == [True, True, False], (kind, fp32)
+
+
 def test_rule():
     for m, n, steps, kind, variant in ((129, 64, 1, "fp8", "64x64"), (1024, 1024, 64, "bf16", "64x64"), (1025, 1024, 64, "bf16", "128x64"), (1000, 1536, 8, "fp8", "128x64"),
                                        (256, 8192, 16, "mx", "128x64"), (256, 8192, 15, "mx", "128, four stages"), (2048, 2048, 8, "fp8", "128, four stages"),
