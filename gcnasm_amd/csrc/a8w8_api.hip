@@ -347,7 +347,8 @@ int launch_small(const GemmParams& p, int batch, hipStream_t stream)
     switch (tile128_variant(p.m, p.n, p.k, batch, tall, MODE == MODE_BF16 || MODE == MODE_F4T, num_cus(), MODE == MODE_BLOCK && CDT == C_FP32)) {
         case TILES_64x64: return launch_tiles<MODE, CDT, SHORT_STAGES, 64, RAGGED, 64>(p, batch, stream);
         case TILES_128x64:
-            if (narrow_tiles_deep(p.m, p.k, !RAGGED && (MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16)))
+            if (narrow_tiles_deep(p.m, p.n, p.k, RAGGED ? STEP_OTHER : MODE == MODE_BLOCK ? STEP_BLOCK
+                                                 : MODE == MODE_TENSOR || MODE == MODE_ROWCOL || MODE == MODE_MXT || MODE == MODE_BF16 ? STEP_LIGHT : STEP_OTHER))
                 return launch_tiles<MODE, CDT, narrow_deep_stages(MODE), 64, RAGGED, 128>(p, batch, stream);
             return launch_tiles<MODE, CDT, NARROW_STAGES, 64, RAGGED, 128>(p, batch, stream);
         case TILES_128_FOUR_STAGES: return launch_tiles<MODE, CDT, 4, 128, RAGGED, 128>(p, batch, stream);

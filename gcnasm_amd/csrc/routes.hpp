@@ -213,11 +213,19 @@ constexpr int tall_min_ksteps(bool cheap_steps) { return cheap_steps ? 24 : 16; 
 
 // LDS stages of 128 x 64 tiles: three, or as many as fit 160 KiB (five or six).  Up to 128 rows always those: the workgroup's share of the weights comes from HBM, and a
 // deep queue hides its latency (us, three / six, weights from HBM: row-major MX 5 x 3328 x 2688 11.5 / 10.2, 1 x 8064 x 3584 15.4 / 13.8, 13 x 9344 x 2688 12.4 / 11.8,
-// MXFP4 2 x 768 x 13312 28.7 / 26.7, 3 x 4736 x 13312 30.0 / 28.7).  Beyond, from 28 steps on where a step is little more than its operands (light_steps: per-tensor,
-// row/col and tiled MXFP8 scales, bf16; whole steps): 1000 x 1536 x 1024 5.9 / 6.3, 402 x 1920 x 3072 10.3 / 10.5, 1024 x 2048 x 4096 13.7 / 13.0, 1495 x 1344 x 7168
+// MXFP4 2 x 768 x 13312 28.7 / 26.7, 3 x 4736 x 13312 30.0 / 28.7).  The same up to 384 rows for weights that a cache does not keep from one layer's pass to the next, from 12 MiB where a
+// step is little more than its operands (STEP_LIGHT: per-tensor, row/col and tiled MXFP8 scales, bf16; whole steps) and from 20 MiB with block scales (from HBM, from the caches: row/col
+// 156 x 7936 x 2816 16.1 / 14.7, 13.9 / 13.9, tiled MXFP8 132 x 8064 x 2432 15.2 / 14.4, 13.4 / 13.8; block 186 x 6144 x 7936 34.4 / 30.5, 303 x 4736 x 7680 36.2 / 32.8,
+// 177 x 6144 x 5760 26.1 / 23.0, 21.6 / 22.1; not smaller ones, 6 to 12 MiB 1.05 times as long from either, nor other kinds of step: row-major MX 2 to 5% longer, MXFP4 2 to 6%,
+// partial steps 4%).  Otherwise beyond 128 rows from 28 light steps on: 1000 x 1536 x 1024 5.9 / 6.3, 402 x 1920 x 3072 10.3 / 10.5, 1024 x 2048 x 4096 13.7 / 13.0, 1495 x 1344 x 7168
 // 20.6 / 19.8; tiled MXFP8 11.0 / 11.4 at 24 steps, 14.5 / 14.2 at 32.  Others: block scales 1024 x 2048 x 4096 14.9 / 15.4, row-major MX 20.8 / 22.2, MXFP4 23.5 /
 // 24.9, tiled 14.7 / 14.9; partial steps 800 x 2000 x 2000 12.8 / 14.2.
-inline bool narrow_tiles_deep(long long m, long long k_bytes, bool light_steps) { return m <= 128 || (light_steps && k_bytes / 128 >= 28); }
+enum StepKind { STEP_LIGHT, STEP_BLOCK, STEP_OTHER };
+inline bool narrow_tiles_deep(long long m, long long n, long long k_bytes, StepKind kind)
+{
+    if (m <= 128 || (kind == STEP_LIGHT && k_bytes / 128 >= 28)) return true;
+    return m <= 384 && kind != STEP_OTHER && n * k_bytes >= (kind == STEP_LIGHT ? 12ll << 20 : 20ll << 20);
+}
 
 // The variant of the 128-tile kernel: the smallest tile whose workgroups do not outnumber the compute units, since a workgroup alone on its
 // compute unit takes as long as its own K loop, and that as long as its tile's rows take from L2 (16, 24, 32 KiB a step: 0.18, 0.27, 0.36 us).

@@ -36,7 +36,7 @@ int route_rounds_on_128_tiles(int kind, long long m, long long n, long long k_st
 {
     return a8w8::rounds_on_128_tiles((a8w8::RoundsKind)kind, m, n, k_steps, batch, fp32_c != 0, cus);
 }
-int route_narrow_tiles_deep(long long m, long long k_bytes, int light_steps) { return a8w8::narrow_tiles_deep(m, k_bytes, light_steps != 0); }
+int route_narrow_tiles_deep(long long m, long long n, long long k_bytes, int kind) { return a8w8::narrow_tiles_deep(m, n, k_bytes, (a8w8::StepKind)kind); }
 int route_tiles_in_runs(long long tiles_m, long long tiles_n, long long k_steps, long long batch, int tall, long long cus)
 {
     return a8w8::tiles_in_runs(tiles_m, tiles_n, k_steps, batch, tall != 0, cus);

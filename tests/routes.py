@@ -90,9 +90,9 @@ def rounds_on_128_tiles(m, n, steps, kind="fp8", batch=1, fp32=False, cus=256):
     return bool(lib().route_rounds_on_128_tiles({"fp8": 0, "bf16": 0, "mxfp8": 1, "mxfp4": 2, "block": 3, "mx": 4}[kind], _ll(m), _ll(n), _ll(steps), _ll(batch), int(fp32), _ll(cus)))
 
 
-def narrow_tiles_deep(kind, m, k_bytes):
+def narrow_tiles_deep(kind, m, k_bytes, n=1024):
     """More than three LDS stages for 128 x 64 tiles; kind as below, "mxfp8" (tiled scales), "ragged" (partial K steps)."""
-    return bool(lib().route_narrow_tiles_deep(_ll(m), _ll(k_bytes), int(kind in ("fp8", "mxfp8", "bf16"))))
+    return bool(lib().route_narrow_tiles_deep(_ll(m), _ll(n), _ll(k_bytes), 0 if kind in ("fp8", "mxfp8", "bf16") else 1 if kind == "block" else 2))
 
 
 def tiles_in_runs(tiles_m, tiles_n, steps, batch=1, tall=False, cus=256):

@@ -108,6 +108,13 @@ def test_stages_of_128x64_tiles():
         assert [routes.narrow_tiles_deep(kind, m, s * 128) for m, s in ((1, 16), (128, 16), (128, 64), (129, 27), (129, 28))] == [True, True, True, False, light]
 
 
+def test_stages_of_128x64_tiles_over_large_weights():
+    """Up to 384 rows too, light steps from 12 MiB of weights and block scales from 20: three stages took up to 13% longer from HBM."""
+    for kind, mib in (("fp8", 12), ("bf16", 12), ("mxfp8", 12), ("block", 20)):
+        assert [routes.narrow_tiles_deep(kind, m, 2048, n) for m, n in ((129, mib * 512), (384, mib * 512), (385, mib * 512), (384, mib * 512 - 1))] == [True, True, False, False]
+    assert not any(routes.narrow_tiles_deep(kind, 129, 8192, 8192) for kind in ("mx", "mxfp4", "mxfp4_tiled", "ragged"))
+
+
 # deep staging up to 128 rows: fewer, as many and more K steps than twice the stages; the last one a partial step
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,steps", [(1, 200, 16), (100, 1000, 17), (128, 1990, 30)])
@@ -116,6 +123,14 @@ def test_up_to_128_rows(m, n, steps, kind, mode):
     n = (n + 127) // 128 * 128 if mode == g.BLOCK else n
     assert routes.tile128_variant("block", m, n, steps * 128) == "128x64"
     check(kind, mode, m, n, steps * ELEMENTS[kind])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,steps,kind,mode", [(200, 6400, 26, "block", g.BLOCK), (300, 4992, 33, "block", g.BLOCK), (190, 6500, 16, "fp8", g.ROWCOL), (257, 5300, 19, "fp8", g.MX_TILED),
+                                                 (130, 7000, 27, "bf16", g.TENSOR)])
+def test_deep_staging_over_large_weights(m, n, steps, kind, mode):
+    assert routes.tile128_variant("fp8", m, n, steps * 128) == "128x64" and routes.narrow_tiles_deep({"fp8": "mxfp8"}.get(kind, kind), m, steps * 128, n)
+    check("fp8" if kind == "block" else kind, mode, m, n, steps * (64 if kind == "bf16" else 128))
 
 
 @pytest.mark.gpu
