@@ -268,13 +268,13 @@ inline Tile128 tile128_variant(long long m, long long n, long long k_bytes, long
 // us, every eighth tile / runs, tile rows x columns: 128-tile kernel 3 x 52 12.2 / 11.3, 5 x 23 10.6 / 10.0, batch of 8 of 7 x 3 18.0 / 14.9; 17 x 12 12.9 / 13.9,
 // 28 x 9 25.2 / 26.3, 42 x 6 29.5 / 31.7, 52 x 7 17.4 / 18.8, 41 x 5 19.0 / 20.8; 25 x 57 63.7 / 55.2, 59 x 13 23.3 / 24.6; 9 x 28 of 55 steps 52.0 / 47.7.  By groups of shapes,
 // runs against every eighth tile: fewer than 8 rows 2.5% faster, 9 to 15 rows 2%, 17 and more 4% slower; more than one tile per compute unit and 9 to 15
-// rows 1.5% faster, more than two and 21 columns 6%; 40 steps and 13 columns 2% faster.  A batch of two rows of tall tiles (128 x 64) shares a tile row's A, the larger
-// operand, among every eighth tile: 16 of 2 x 6 12.0 / 12.9, 20.5 / 22.7.
+// rows 1.5% faster, more than two and 21 columns 6%; 40 steps and 13 columns 2% faster.  A batch of two or four rows of tall tiles (128 x 64, 256 x 128) shares a tile row's
+// A, the larger operand, among every eighth tile: 16 of 2 x 6 12.0 / 12.9, 20.5 / 22.7, 16 of 4 x 3 42.1 / 46.6, 8 of 4 x 7 51.1 / 70.9.
 inline bool tiles_in_runs(long long tiles_m, long long tiles_n, long long k_steps, long long batch, bool tall, long long cus)
 {
     const long long tiles = tiles_m * tiles_n;
     if (tiles % 8 == 0) return true;
-    if (tiles_m < 8) return !(batch > 1 && tiles_m <= 2 && tall);
+    if (tiles_m < 8) return !(batch > 1 && 8 % tiles_m == 0 && tall);
     return (tiles > cus && tiles_m < 16) || (tiles > 2 * cus && tiles_n > 20) || (k_steps >= 40 && tiles_n > 12);
 }
 // The same for the 256-tile kernels, whose workgroups walk the tiles of all batch entries: up to two rounds of them and fewer than 16 steps runs are 2% slower (9 x 28 31.4 /

@@ -11,7 +11,7 @@ from exact_gemm import check
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,steps,batch,bm,bn,runs", [
     (200, 900, 3, 1, 64, 64, True), (440, 380, 3, 5, 64, 64, True), (580, 900, 3, 1, 64, 64, False), (1080, 700, 3, 1, 64, 64, False), (580, 400, 2, 3, 64, 64, False),
-    (600, 1088, 40, 1, 64, 64, True), (700, 1900, 3, 1, 128, 64, True), (200, 350, 17, 16, 128, 64, False), (2200, 700, 16, 1, 128, 64, False),
+    (600, 1088, 40, 1, 64, 64, True), (700, 1900, 3, 1, 128, 64, True), (200, 350, 17, 16, 128, 64, False), (900, 880, 30, 8, 256, 128, False), (2200, 700, 16, 1, 128, 64, False),
     (600, 4300, 3, 1, 128, 128, True), (2200, 1700, 3, 1, 128, 128, False), (1153, 3700, 3, 1, 128, 128, True), (2177, 2600, 3, 1, 128, 128, False),
     (700, 6700, 24, 1, 256, 128, True), (3300, 2300, 24, 1, 256, 128, False)])
 @pytest.mark.parametrize("kind,mode,route", [("fp8", g.ROWCOL, "fp8"), ("bf16", g.TENSOR, "bf16")], ids=lambda v: str(v))
@@ -45,7 +45,7 @@ def test_128_tiles_in_rounds(m, n, runs):
 
 def test_rules():
     assert all(routes.tiles_in_runs(a, b, 1) and routes.items_in_runs(a, b, 1) for a, b in ((8, 7), (16, 5), (100, 4), (9, 8)))
-    for tiles, steps, batch, tall, runs in (((7, 3), 9, 1, False, True), ((7, 3), 9, 8, False, True), ((2, 6), 9, 16, True, False), ((2, 6), 9, 16, False, True), ((2, 6), 9, 1, True, True),
+    for tiles, steps, batch, tall, runs in (((7, 3), 9, 1, False, True), ((7, 3), 9, 8, False, True), ((2, 6), 9, 16, True, False), ((2, 6), 9, 16, False, True), ((2, 6), 9, 1, True, True), ((4, 7), 50, 8, True, False), ((4, 7), 50, 8, False, True),
                                             ((3, 6), 9, 16, True, True), ((9, 9), 9, 1, False, False), ((9, 28), 39, 1, False, False), ((9, 28), 40, 1, False, True),
                                             ((17, 12), 50, 1, False, False), ((9, 29), 9, 1, False, True), ((17, 17), 9, 1, False, False), ((25, 21), 9, 1, False, True),
                                             ((59, 13), 9, 1, False, False)):
