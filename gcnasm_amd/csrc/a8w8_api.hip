@@ -320,7 +320,7 @@ bool small_ok(const a8w8_gemm_args* g, bool fp4)
     const bool fp32 = g->c_dtype == A8W8_C_FP32;
     const RoundsKind kind = mxt ? (fp4 ? ROUNDS_MXFP4_TILED : ROUNDS_MXFP8_TILED) : g->scale_mode == A8W8_SCALE_BLOCK_1x128_128x128 ? ROUNDS_BLOCK
                             : g->scale_mode == A8W8_SCALE_MX_E8M0_1x32 ? ROUNDS_MXFP8_ROWS : ROUNDS_PLAIN;
-    if (c_tile_fits(g->stride_c, fp32 ? 4 : 2) && rounds_on_128_tiles(kind, g->m, g->n, g->k / BK, g->batch, fp32, num_cus())) return true;
+    if (c_tile_fits(g->stride_c, fp32 ? 4 : 2) && rounds_on_128_tiles(kind, g->m, g->n, g->k / BK, g->batch, fp32, num_cus(), g->b_preshuffled != 0)) return true;
     return fits_128_tiles(g->m, g->n, g->batch, num_cus());
 }
 

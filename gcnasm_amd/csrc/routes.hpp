@@ -101,14 +101,23 @@ inline Rounds tile_rounds(long long m, long long n, long long batch, long long c
 // up to eight or ten steps only.  us, 128-tiles / 256-tiles: block fp32 16 x 953 x 640 8 steps 26.0 / 26.3, 10 30.3 / 29.2, 15 40.9 / 36.0; bf16 operands 16 x 953 x 640 bf16 C 8 22.1 / 25.9,
 // 15 35.0 / 28.7; 16 x 700 x 768 8 21.7 / 20.8, 10 25.6 / 23.1, 16 35.7 / 29.7; 8 x 1020 x 1280 8 20.5 / 20.5, 10 23.9 / 22.5, 16 32.9 / 28.8.  Larger entries as above:
 // 2 x 2600 x 2176 bf16 C 14 steps 28.2 / 31.5, block fp32 29.8 / 29.7 at 12.
+// Weights in the shuffled layout (b_shuffled): the 256-tiles gain by it what the 128-tiles do not, and only rounds of twice as many 128-tiles at most, 5 against 2 with tiled scales, and 5
+// against 2 with fp32 C over few steps go to 128-tiles.  128-tiles / 256-tiles, geometric means over 500 drawn shapes: 4 against 2 0.70 to 0.88 for every kind; 5 against 2 tiled MXFP4
+// 0.90 to 1.00, tiled MXFP8 0.86 to 0.98, fp32 C row/col 0.81 and 0.92 up to 8 and 12 steps, 1.01 to 1.06 beyond, block 0.91 to 0.96 up to 16, bf16 C 1.00 to 1.12; 6 against
+// 2 1.00 to 1.25; 3 against 1 row/col 1.13 to 1.24, block 1.08, row-major MX 1.10 to 1.17, tiled MXFP4 1.00 (2 x 3894 x 1280 x 1408 row/col 23.9 / 20.0 us).
 enum RoundsKind { ROUNDS_PLAIN, ROUNDS_MXFP8_TILED, ROUNDS_MXFP4_TILED, ROUNDS_BLOCK, ROUNDS_MXFP8_ROWS };      // (plain: per-tensor and row/col scales, bf16)
-inline bool rounds_on_128_tiles(RoundsKind kind, long long m, long long n, long long k_steps, long long batch, bool fp32_c, long long cus)
+inline bool rounds_on_128_tiles(RoundsKind kind, long long m, long long n, long long k_steps, long long batch, bool fp32_c, long long cus, bool b_shuffled = false)
 {
     const Rounds rounds = tile_rounds(m, n, batch, cus);
     if (k_steps < 5 || rounds.of256 > 2 || rounds.of128 > 3 * rounds.of256) return false;
     const bool finer = rounds.of128 < 3 * rounds.of256, two = rounds.of256 == 2;
     const long long entry_tiles = ((m + 127) / 128) * ((n + 127) / 128);
     if (!finer && batch > 1 && entry_tiles <= 128 && k_steps > (entry_tiles <= 64 ? 8 : 10)) return false;
+    if (b_shuffled && rounds.of128 > 2 * rounds.of256) {
+        if (!finer) return false;
+        if (kind != ROUNDS_MXFP8_TILED && kind != ROUNDS_MXFP4_TILED)
+            return fp32_c && k_steps <= (kind == ROUNDS_BLOCK ? 16 : kind == ROUNDS_MXFP8_ROWS ? 8 : 12);
+    }
     switch (kind) {
         case ROUNDS_MXFP8_TILED: return k_steps <= (finer ? 20 : fp32_c ? 8 : 0);
         case ROUNDS_MXFP4_TILED: return k_steps <= (finer ? 32 : fp32_c ? 16 : 8);

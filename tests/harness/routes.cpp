@@ -32,9 +32,9 @@ int route_flat_is_faster(long long m, long long n, long long row_bytes, long lon
 {
     return a8w8::flat_is_faster(m, n, row_bytes, batch, layout_factor, cus);
 }
-int route_rounds_on_128_tiles(int kind, long long m, long long n, long long k_steps, long long batch, int fp32_c, long long cus)
+int route_rounds_on_128_tiles(int kind, long long m, long long n, long long k_steps, long long batch, int fp32_c, long long cus, int b_shuffled)
 {
-    return a8w8::rounds_on_128_tiles((a8w8::RoundsKind)kind, m, n, k_steps, batch, fp32_c != 0, cus);
+    return a8w8::rounds_on_128_tiles((a8w8::RoundsKind)kind, m, n, k_steps, batch, fp32_c != 0, cus, b_shuffled != 0);
 }
 int route_narrow_tiles_deep(long long m, long long n, long long k_bytes, int kind) { return a8w8::narrow_tiles_deep(m, n, k_bytes, (a8w8::StepKind)kind); }
 int route_tiles_in_runs(long long tiles_m, long long tiles_n, long long k_steps, long long batch, int tall, long long cus)

@@ -85,9 +85,9 @@ def flat_is_faster(kind, row_major, m, n, k, batch=1, cus=256):
     return bool(lib().route_flat_is_faster(_ll(m), _ll(n), _ll(row_bytes), _ll(batch), ctypes.c_double(factor), _ll(cus)))
 
 
-def rounds_on_128_tiles(m, n, steps, kind="fp8", batch=1, fp32=False, cus=256):
+def rounds_on_128_tiles(m, n, steps, kind="fp8", batch=1, fp32=False, cus=256, shuffled=False):
     """kind: "fp8" (per-tensor and row/col scales), "bf16", "mxfp8", "mxfp4" (tiled scales), "block", "mx" (row-major scales)."""
-    return bool(lib().route_rounds_on_128_tiles({"fp8": 0, "bf16": 0, "mxfp8": 1, "mxfp4": 2, "block": 3, "mx": 4}[kind], _ll(m), _ll(n), _ll(steps), _ll(batch), int(fp32), _ll(cus)))
+    return bool(lib().route_rounds_on_128_tiles({"fp8": 0, "bf16": 0, "mxfp8": 1, "mxfp4": 2, "block": 3, "mx": 4}[kind], _ll(m), _ll(n), _ll(steps), _ll(batch), int(fp32), _ll(cus), int(shuffled)))
 
 
 def narrow_tiles_deep(kind, m, k_bytes, n=1024):

@@ -45,6 +45,13 @@ def test_partial_steps(m, n, k, variant, kind, mode):
     check(kind, mode, m, n, k // 2 if kind == "bf16" else k)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,steps", [(3080, 5120, 5), (4352, 4608, 6), (5300, 4096, 8)])
+@pytest.mark.parametrize("kind,mode", [("fp8", g.ROWCOL), ("fp8", g.BLOCK), ("fp8", g.MX), ("fp8", g.MX_TILED), ("bf16", g.TENSOR), ("fp4", g.MX_TILED)], ids=lambda v: str(v))
+def test_shuffled_weights_in_badly_filled_rounds(m, n, steps, kind, mode):
+    check(kind, mode, m, n, steps * ELEMENTS[kind], shuffled=True)
+
+
 # more than two 128-tiles per compute unit, in rounds that 256-tiles fill badly
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,steps", [(4352, 4608, 5), (6100, 3001, 6), (2100, 4200, 8), (5300, 4000, 16)])
@@ -82,6 +89,19 @@ def test_rounds_of_a_batch_of_small_entries(m, n, batch, most):
     """Three rounds of 128-tiles against one of 256-tiles, up to `most` steps: beyond, small entries took up to 1.26 times as long."""
     for kind, fp32 in (("bf16", False), ("bf16", True), ("fp8", False), ("block", True)):
         assert [routes.rounds_on_128_tiles(m, n, s, kind, batch, fp32) for s in (5, most, most + 1)] == [True, True, False], (kind, fp32)
+
+
+def test_rounds_over_shuffled_weights():
+    """Measured on row-major weights, the rounds made shuffled ones up to 1.25 times as slow."""
+    four, five, six, three = (3080, 5120), (4352, 4608), (5376, 4096), (2304, 4096)      # rounds of 128-tiles, against 2, 2, 2 and 1 of 256-tiles
+    for kind, bf16_most, fp32_most in (("fp8", 0, 12), ("bf16", 0, 12), ("block", 0, 16), ("mx", 0, 8), ("mxfp8", 20, 20), ("mxfp4", 32, 32)):
+        for fp32, most in ((False, bf16_most), (True, fp32_most)):
+            assert [routes.rounds_on_128_tiles(*five, s, kind, fp32=fp32, shuffled=True) for s in (5, most, most + 1)] == [most > 0, most > 0, False], (kind, fp32)
+            assert not routes.rounds_on_128_tiles(*six, 5, kind, fp32=fp32, shuffled=True) and not routes.rounds_on_128_tiles(*three, 5, kind, fp32=fp32, shuffled=True)
+            assert routes.rounds_on_128_tiles(*four, 8, kind, fp32=fp32, shuffled=True) and routes.rounds_on_128_tiles(*four, 8, kind, fp32=fp32)
+    for mode, shuffled, name in ((g.ROWCOL, 0, "gemm_a8w8_tile128"), (g.ROWCOL, 1, "gemm_a8w8_wide"), (g.BLOCK, 0, "gemm_a8w8_tile128"), (g.BLOCK, 1, "gemm_a8w8_persist")):
+        args = g.raw_gemm_args(1 << 12, 1 << 12, 1 << 12, 1 << 12, 1 << 12, *six, 1024, mode, b_preshuffled=shuffled)
+        assert g.kernel_name(args) == name
 
 
 def test_rule():
